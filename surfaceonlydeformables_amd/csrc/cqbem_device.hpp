@@ -145,6 +145,14 @@ __device__ inline double rsqrt_nr(double d) {
     return fma(0.5 * y, e, y);
 }
 
+// 1/sqrt(d), d > 0, in one third-order step y += y e (1/2 + 3 e/8), e = 1 - d y^2, from the hardware estimate
+// (relative error below 2^-22, so the step's own error is below 2^-64).
+__device__ inline double rsqrt_h3(double d) {
+    const double y = __builtin_amdgcn_rsq(d);
+    const double e = fma(-d * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
 // ---------------------------------------------------------------------------
 // Table-driven variants (P. T. P. Tang, "Table-driven implementation of the
 // exponential function in IEEE floating-point arithmetic", ACM TOMS 15, 1989;
@@ -172,60 +180,63 @@ __device__ inline void load_math_tables(MathTables *s) {
     }
 }
 
-// e^{-a}, a >= -700, as exp_neg.  k = rint(t 64/ln2), t = -a clamped to [-740, 700];
-// r = t - k ln2/64 (the k hi product and the first subtraction exact); e^r - 1 through r^6
-// (next term < 3e-20); 2^(k/64) = 2^(k >> 6) T[k & 63], and T_hi + (T_hi p + T_lo) last.
-__host__ __device__ inline double exp_neg_tab(double a, const double2 *T) {
+// Both find k by adding 1.5 2^52, which leaves rint in the low bits of the sum's significand: the integer is read
+// from there (no conversion) and the subtraction gives it back as a double.
+constexpr double kRoundMagic = 6755399441055744.0;  // 1.5 2^52
+__host__ __device__ inline int magic_int(double t) { return (int)(unsigned)__builtin_bit_cast(unsigned long long, t); }
+
+// e^t, -740 <= t <= 700.  k = rint(t 64/ln2); r = t - k ln2/64 (the k hi product and the first subtraction exact);
+// e^r - 1 = r + r^2 q(r), q the degree-4 Taylor polynomial with its last term replaced by its Chebyshev economization
+// on |r| <= ln2/128 (error 5e-18 of the result); 2^(k/64) = 2^(k >> 6) T[k & 63], and T_hi + (T_hi p + T_lo) last.
+__host__ __device__ inline double exp_tab_core(double t, const double2 *T) {
 #pragma clang fp contract(off)
-    const double t = fmin(fmax(-a, -740.0), 700.0);
-    const double k = rint(t * CQBEM_64_OVER_LN2);
+    constexpr double kR = 0.005415212348514945;  // ln2/128
+    const double km = fma(t, CQBEM_64_OVER_LN2, kRoundMagic);
+    const double k = km - kRoundMagic;
     const double r1 = fma(-k, CQBEM_LN2_OVER_64_HI, t);
     const double r = fma(-k, CQBEM_LN2_OVER_64_LO, r1);
-    double q = fma(r, 1.0 / 720.0, 1.0 / 120.0);
-    q = fma(q, r, 1.0 / 24.0);
+    double q = fma(r, 1.0 / 120.0, 1.0 / 24.0 + kR * kR / 720.0);
     q = fma(q, r, 1.0 / 6.0);
-    q = fma(q, r, 0.5);
+    q = fma(q, r, 0.5 - kR * kR * kR * kR / 5760.0);
     const double p = fma(r * r, q, r);
-    const int ki = (int)k;
+    const int ki = magic_int(km);
     const double2 e = T[ki & 63];
     return ldexp(e.x + fma(e.x, p, e.y), ki >> 6);
 }
+// e^{-a}, clamped at a = 740 (underflowed to 0) and a = -700.
+__host__ __device__ inline double exp_neg_tab(double a, const double2 *T) {
+    return exp_tab_core(fmin(fmax(-a, -740.0), 700.0), T);
+}
 
-// sin y, cos y for |y| < kTrigArgMax, as cq_sincos.  k = rint(32 y/pi); r + rr = y - k pi/32 to
-// ~1e-28 (three-part pi/32, the first two products exact, TwoSum on the subtraction; |rr| reaches
-// 1e-12 at |k| ~ 1e7, so rr enters to first order, sin(r + rr) = sin r + rr cos r and
-// cos(r + rr) - 1 = cos r - 1 - rr sin r, the rr^2 terms below 1e-24); sin r through r^9 and
-// cos r - 1 through r^8 (next terms < 1e-19); then sin(a + r) = S + (S (cos r - 1) + C sin r) and
-// cos(a + r) = C + (C (cos r - 1) - S sin r) with a = (k mod 64) pi/32 and the table's lo parts
-// added inside the brackets.
+// sin y, cos y for |y| < kTrigArgMax, as cq_sincos.  k = rint(32 y/pi); r = y - k pi/32 in two FMAs (k A exact, so the
+// first has no rounding error; the second part holds the next 53 bits of pi/32: r is off by 2^-58 at most, 0.02 ulp
+// of 1); sin r - r = r^3 times the degree-3 Taylor polynomial in r^2 with its last term economized on |r| <= pi/64
+// (error 2e-19), cos r - 1 through r^8 (next term < 1e-19); then sin(a + r) = S + (S (cos r - 1) + C sin r) and
+// cos(a + r) = C + (C (cos r - 1) - S sin r) with a = (k mod 64) pi/32 and the table's lo parts added inside the
+// brackets.
 __host__ __device__ inline void sincos_tab(double y, const double4 *T, double *s, double *c) {
 #pragma clang fp contract(off)
-    const double k = rint(y * CQBEM_32_OVER_PI);
+    constexpr double kX = 0.0024094971401247595;  // (pi/64)^2
+    const double km = fma(y, CQBEM_32_OVER_PI, kRoundMagic);
+    const double k = km - kRoundMagic;
     const double r1 = fma(-k, CQBEM_PI_OVER_32_A, y);
-    const double tb = k * CQBEM_PI_OVER_32_B;
-    const double r = r1 - tb;
-    const double bb = r - r1;
-    double rr = (r1 - (r - bb)) - (tb + bb);
-    rr = fma(-k, CQBEM_PI_OVER_32_C, rr);
+    const double r = fma(-k, CQBEM_PI_OVER_32_B + CQBEM_PI_OVER_32_C, r1);
     const double x = r * r;
-    double ps = fma(x, 1.0 / 362880.0, -1.0 / 5040.0);
-    ps = fma(ps, x, 1.0 / 120.0);
-    ps = fma(ps, x, -1.0 / 6.0);
-    const double s0 = (r * x) * ps;  // sin r - r
+    double ps = fma(x, -1.0 / 5040.0 + 1.5 * kX / 362880.0, 1.0 / 120.0 - 0.5625 * kX * kX / 362880.0);
+    ps = fma(ps, x, -1.0 / 6.0 + kX * kX * kX / 32.0 / 362880.0);
+    const double sr = fma(r * x, ps, r);  // sin r
     double pc = fma(x, 1.0 / 40320.0, -1.0 / 720.0);
     pc = fma(pc, x, 1.0 / 24.0);
     pc = fma(pc, x, -0.5);
-    const double c0 = x * pc;                        // cos r - 1
-    const double sr = r + fma(rr, 1.0 + c0, s0);     // sin(r + rr)
-    const double cm1 = fma(-rr, r + s0, c0);         // cos(r + rr) - 1
-    const double4 e = T[(int)k & 63];
+    const double cm1 = x * pc;  // cos r - 1
+    const double4 e = T[magic_int(km) & 63];
     *s = e.x + fma(e.z, sr, fma(e.x, cm1, e.y));
     *c = e.z + fma(-e.x, sr, fma(e.z, cm1, e.w));
 }
 
 // exp(-z), Re z >= 0, through the tables
 __host__ __device__ inline cd cexp_neg_tab(cd z, const MathTables *M) {
-    const double m = exp_neg_tab(z.x, M->e);
+    const double m = exp_tab_core(fmax(-z.x, -740.0), M->e);
     double sn, cs;
     sincos_tab(z.y, M->t, &sn, &cs);
     return cd{m * cs, -m * sn};
@@ -289,26 +300,12 @@ __device__ inline Expo expo(double r, const Freq &f, const MathTables *M) {
     return E;
 }
 
-// The exponentials G and H need: e1, e2 and dA, the last formed as ((z1 + 1) e1 - (z2 + 1) e2) / s^2 with one product
-// by 1/s^2 (A2 is not formed: it is left zero).
-__device__ inline Expo expo_gh(double r, const Freq &f, const MathTables *M) {
-    Expo E;
-    const cd z1 = f.sc1 * r, z2 = f.sc2 * r;
-    E.e1 = cexp_neg_tab(z1, M);
-    E.e2 = cexp_neg_tab(z2, M);
-    E.dA = ((z1 + cd{1.0, 0.0}) * E.e1 - (z2 + cd{1.0, 0.0}) * E.e2) * f.is2;
-    E.A2 = cd{0.0, 0.0};
-    return E;
-}
-
-// u_hat = alpha rh rh^T + beta I  (times r if `times_r`: r*u_hat for polar rules).  SCALED = false leaves out the
-// factor g_scale = 1/(4 pi rho), for callers that apply it to their sums.
-template <bool SCALED = true>
+// u_hat = alpha rh rh^T + beta I  (times r if `times_r`: r*u_hat for polar rules).
 __device__ inline void g_coef(const Expo &E, double ir, double ir2, const Mat &m, cd &alpha, cd &beta) {
     const cd t = E.dA * ir2;
     alpha = 3.0 * t + E.e1 * m.ic1s - E.e2 * m.ic2s;
     beta = E.e2 * m.ic2s - t;
-    if (SCALED) alpha = alpha * m.g_scale, beta = beta * m.g_scale;
+    alpha = alpha * m.g_scale, beta = beta * m.g_scale;
 }
 
 // p_hat coefficients without the 1/(4 pi) factor.
@@ -325,6 +322,122 @@ __device__ inline void h_coef(const Expo &E, double ir, double ir2, const Freq &
 
 constexpr double kInv4Pi = 0.079577471545947667884;  // 1/(4 pi)
 constexpr double kInv8Pi = 0.039788735772973833942;  // 1/(8 pi)
+
+// symmetric 3x3 packed index: 00 11 22 01 02 12
+__host__ __device__ inline int sidx(int a, int b) {
+    if (a == b) return a;
+    const int lo = a < b ? a : b, hi = a < b ? b : a;
+    return lo == 0 ? (hi == 1 ? 3 : 4) : 5;
+}
+
+// ---------------------------------------------------------------------------
+// Regular faces in the face's own frame.  With the axes t1, t2 in the face's plane and n its normal, a source point
+// y of the face seen from x is y - x = (ar, br, cr) with cr the same at every point of the face, and the direction is
+// h = (a, b, c).  The traction kernel then has 8 different entries (xy = yx) and no separate normal:
+//   p_xx = h2 c + h4 c a^2, p_yy = h2 c + h4 c b^2, p_xy = h4 c a b, p_xz = a (h1 + h4 c^2), p_zx = a (h2 + h4 c^2),
+//   p_yz, p_zy alike with b, p_zz = c (h1 + 2 h2 + h4 c^2)
+// and one rotation per face and corner, after the quadrature, brings the sums to the global axes.
+// ---------------------------------------------------------------------------
+struct FaceFrame {
+    double L1, u, v;       // corners in the plane: (0, 0), (L1, 0), (u, v)
+    double xa, xb, cr;     // -x in the plane, and the constant third coordinate of y - x
+};
+// Columns t1, t2, n of the axes of the face with edges e1 = y1 - y0 and e2 = y2 - y0, and twice its area.
+__device__ inline void face_axes(const double *e1, const double *e2, double Q[3][3], double *L1, double *area2) {
+    const double l2 = e1[0] * e1[0] + e1[1] * e1[1] + e1[2] * e1[2], il = rsqrt_h3(l2);
+    double c[3], c2 = 0;
+    for (int k = 0; k < 3; k++) c[k] = e1[(k + 1) % 3] * e2[(k + 2) % 3] - e1[(k + 2) % 3] * e2[(k + 1) % 3], c2 = fma(c[k], c[k], c2);
+    const double ic = rsqrt_h3(c2);
+    for (int k = 0; k < 3; k++) Q[0][k] = e1[k] * il, Q[2][k] = c[k] * ic;
+    for (int k = 0; k < 3; k++) Q[1][k] = Q[2][(k + 1) % 3] * Q[0][(k + 2) % 3] - Q[2][(k + 2) % 3] * Q[0][(k + 1) % 3];
+    *L1 = l2 * il, *area2 = c2 * ic;
+}
+// Frame of the face (y0, y1, y2) seen from x.
+__device__ inline FaceFrame face_frame(const double y[3][3], double x0, double x1, double x2) {
+    FaceFrame F;
+    double e1[3], e2[3], Q[3][3], area2;
+    for (int k = 0; k < 3; k++) e1[k] = y[1][k] - y[0][k], e2[k] = y[2][k] - y[0][k];
+    const double xr[3] = {y[0][0] - x0, y[0][1] - x1, y[0][2] - x2};
+    face_axes(e1, e2, Q, &F.L1, &area2);
+    auto dot = [](const double *a, const double *b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; };
+    F.u = dot(e2, Q[0]), F.v = dot(e2, Q[1]);
+    F.xa = dot(xr, Q[0]), F.xb = dot(xr, Q[1]), F.cr = dot(xr, Q[2]);
+    return F;
+}
+
+// Frequency- and material-dependent factors of one point: with w_k = z_k e_k and dd = (A1 - A2) / r^2 every
+// coefficient is a short sum, the traction's in units of 1/r^2 (their static part 6 c2^2 dd is the first bracket of
+// H_collocation.cu:45-76, which the displacement kernel shares).
+struct PointExpo {
+    double ir, ir2, r;
+    cd e1, e2, w1, w2, s2, q2;  // s2 = (z2 + 1) e2, q2 = 1 / (s r)^2
+    cd dd;
+};
+__device__ inline PointExpo point_expo(double d2, const Freq &f, const MathTables *M) {
+    PointExpo E;
+    E.ir = rsqrt_h3(d2), E.r = d2 * E.ir, E.ir2 = E.ir * E.ir;
+    const cd z1 = f.sc1 * E.r, z2 = f.sc2 * E.r;
+    E.e1 = cexp_neg_tab(z1, M), E.e2 = cexp_neg_tab(z2, M);
+    E.w1 = z1 * E.e1, E.w2 = z2 * E.e2;
+    E.s2 = E.w2 + E.e2, E.q2 = f.is2 * E.ir2;
+    E.dd = ((E.w1 + E.e1) - E.s2) * E.q2;
+    return E;
+}
+
+// Local entries of one point in direction (a, b, c), not weighted: G (xx yy zz xy xz yz) = (alpha h h^T + beta I) / r
+// without 1/(4 pi rho), and H (xx yy zz xy xz yz zx zy) without 1/(4 pi).
+__device__ inline void point_g(const PointExpo &E, double a, double b, double c, const Mat &m, cd *G) {
+    const cd t = E.e2 * m.ic2s;
+    const cd al = (3.0 * E.dd + (E.e1 * m.ic1s - t)) * E.ir, be = (t - E.dd) * E.ir;
+    G[0] = G[1] = G[2] = be;
+    fma_cr(G[0], al, a * a), fma_cr(G[1], al, b * b), fma_cr(G[2], al, c * c);
+    G[3] = al * (a * b), G[4] = al * (a * c), G[5] = al * (b * c);
+}
+__device__ inline void point_h(const PointExpo &E, double a, double b, double c, const Mat &m, cd *H) {
+    const double k = m.kap, a2 = a * E.ir2, b2 = b * E.ir2, c2 = c * E.ir2, cc = c * c;
+    const cd d6 = E.dd * m.six_c2s;
+    cd h1 = d6, h2 = d6, h4 = d6 * (-5.0);
+    fma_cr(h1, E.e1, 4.0 * k - 1.0), fma_cr(h1, E.e2, -2.0), fma_cr(h1, E.w1, 2.0 * k - 1.0);
+    fma_cr(h2, E.e1, 2.0 * k), fma_cr(h2, E.e2, -3.0), h2 -= E.w2;
+    fma_cr(h4, E.e1, -12.0 * k), fma_cr(h4, E.e2, 12.0), fma_cr(h4, E.w1, -2.0 * k), fma_cr(h4, E.w2, 2.0);
+    const cd hc = h4 * c2;
+    H[0] = H[1] = h2 * c2;
+    fma_cr(H[0], hc, a * a), fma_cr(H[1], hc, b * b);
+    H[3] = hc * (a * b);
+    cd p1 = h1, p2 = h2;
+    fma_cr(p1, h4, cc), fma_cr(p2, h4, cc);
+    H[4] = p1 * a2, H[5] = p1 * b2, H[6] = p2 * a2, H[7] = p2 * b2;
+    fma_cr(p1, h2, 2.0);
+    H[2] = p1 * c2;
+}
+
+// out (xx yy zz xy xz yz) = Q S Q^T for one real part of a symmetric local block S, columns t1, t2, n of Q; `A` holds
+// Q times a factor (the face's area).
+__device__ inline void rotate_sym(const double S[6], const double Q[3][3], const double A[3][3], double *out) {
+    const int ix[3][3] = {{0, 3, 4}, {3, 1, 5}, {4, 5, 2}};
+    double P[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) P[i][b] = fma(S[ix[i][0]], Q[0][b], fma(S[ix[i][1]], Q[1][b], S[ix[i][2]] * Q[2][b]));
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int b = a; b < 3; b++) out[sidx(a, b)] = fma(A[0][a], P[0][b], fma(A[1][a], P[1][b], A[2][a] * P[2][b]));
+}
+// The same for a general block given as xx yy zz xy(= yx) xz yz zx zy; out is row-major.
+__device__ inline void rotate_gen(const double S[8], const double Q[3][3], const double A[3][3], double *out) {
+    const int ix[3][3] = {{0, 3, 4}, {3, 1, 5}, {6, 7, 2}};
+    double P[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) P[i][b] = fma(S[ix[i][0]], Q[0][b], fma(S[ix[i][1]], Q[1][b], S[ix[i][2]] * Q[2][b]));
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) out[a * 3 + b] = fma(A[0][a], P[0][b], fma(A[1][a], P[1][b], A[2][a] * P[2][b]));
+}
 
 // b_hat (translational) and b_hat_ijk (angular) coefficients.
 __device__ inline void b_coef(const Expo &E, double ir, double ir2, const Freq &f, const Mat &m, cd &t1, cd &t2, cd &u1,
@@ -347,13 +460,6 @@ __device__ inline void b_coef_8pi(const Expo &E, double ir, double ir2, const Fr
     const cd u2 = ((E.e2 * m.ic2) - (E.e1 * m.ic1)) * f.is;
     u12 = u1 + u2;
     u3 = E.e2 * f.is * (2.0 * m.ic2);
-}
-
-// symmetric 3x3 packed index: 00 11 22 01 02 12
-__host__ __device__ inline int sidx(int a, int b) {
-    if (a == b) return a;
-    const int lo = a < b ? a : b, hi = a < b ? b : a;
-    return lo == 0 ? (hi == 1 ? 3 : 4) : 5;
 }
 
 }  // namespace cqbem

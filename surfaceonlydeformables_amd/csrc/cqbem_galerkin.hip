@@ -986,13 +986,13 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
                 const int row0 = fi0 * npts, nrows = nfc * npts;
                 if (U || P) {
                     {
-                        // the pair kernel at the test points: timed on its own, with its launches and its unique
+                        // the patch kernel at the test points: timed on its own, with its launches and its unique
                         // evaluations (test point, regular source face, source point, frequency)
                         EvTimer tp(st, &tm[2]);
-                        check(launch_colloc_gh_pair(g, job.pair_pts, job.npts_even, job.freqs, 0, nl, job.mat, row0, nrows,
-                                                    tpts, job.patch_pass, job.pass_info, job.pass_faces, job.patch_verts,
+                        check(launch_colloc_gh_patch(g, job.patch_pts, npts, job.freqs, 0, nl, job.mat, row0, nrows,
+                                                    tpts, job.patch_chunk, job.chunk_info, job.chunk_faces, job.patch_verts,
                                                     job.npatches, sG, sH, n3, ls, st),
-                              "k_colloc_gh_pair (test points)");
+                              "k_colloc_gh_patch (test points)");
                     }
                     tm[6] += 1;
                     for (int fi = fi0; fi < fi0 + nfc; fi++)

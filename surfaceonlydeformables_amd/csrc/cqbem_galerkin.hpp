@@ -19,12 +19,11 @@ struct GalerkinJob {
     int nl;               // number of frequencies
     Mat mat;
     int num_cus;
-    // pair-form tables of the collocation G/H kernel (column patches; see launch_colloc_gh_pair)
-    const double4 *pair_pts;
-    int npts_even;
-    const int *patch_pass;
-    const int2 *pass_info;
-    const int4 *pass_faces;
+    // patch-form tables of the collocation G/H kernel (column patches; see launch_colloc_gh_patch)
+    const double4 *patch_pts;
+    const int *patch_chunk;
+    const int4 *chunk_info;
+    const int4 *chunk_faces;
     const int *patch_verts;
     int npatches;
     size_t scratch_bytes;  // bound of the per-test-point row scratch (at least one face is always processed)

@@ -115,9 +115,9 @@ void check_inputs(const cqbem_mesh *mesh, const cqbem_params *p) {
     if (p->quad_policy != CQBEM_QUAD_REFERENCE && p->quad_policy != CQBEM_QUAD_BANDED)
         throw Err{CQBEM_ERR_ARG, "unknown quad_policy"};
     if (p->quad_policy == CQBEM_QUAD_BANDED) {
-        // the bands apply to the pair kernel: collocation G/H, in FP64 or CQBEM_MIXED with G in that kernel
+        // the bands apply to the patch kernel: collocation G/H, in FP64 or CQBEM_MIXED with G in that kernel
         if (p->galerkin || (p->precision == CQBEM_MIXED && mixed_float_g()))
-            throw Err{CQBEM_ERR_UNSUPPORTED, "CQBEM_QUAD_BANDED is implemented for collocation G/H in the pair kernel"};
+            throw Err{CQBEM_ERR_UNSUPPORTED, "CQBEM_QUAD_BANDED is implemented for collocation G/H in the patch kernel"};
         if (p->far_order < 0 || p->far_order > 5 || p->far_subdivision < 0 || p->far_subdivision > 16 ||
             !(p->band_kappa >= 0) || !(p->band_kappa_b >= 0))
             throw Err{CQBEM_ERR_ARG, "far rule or band threshold out of range"};
@@ -186,17 +186,17 @@ struct Prepared {
     int nv, nf, L, Lf;
     std::vector<double> N, area;
     std::vector<int> vs_ptr, vs_face, sg_ptr, sg_face;
-    // pair form: patches of pair_patch_size() vertices, passes of pair_pass_faces() faces
-    std::vector<int> pair_patch_pass, pair_patch_verts;
-    std::vector<int2> pair_pass_info;   // (first face entry, nfaces | nsub << 16)
-    std::vector<int4> pair_pass_faces;  // (face, corner codes), code = slot | sub-step << 10, -1 outside
-    int pair_npatches = 0;
+    // patch form: patches of patch_size() vertices, chunks of chunk_face_count() faces
+    std::vector<int> patch_chunk, patch_verts;
+    std::vector<int4> chunk_info;   // (first face entry, nfaces, sub-steps of corner 0 | 1 << 8 | 2 << 16, 0)
+    std::vector<int4> chunk_faces;  // vertex | slot << 24 of the corners, sub-steps (8 bits each, 255 outside)
+    int npatches = 0;
     int npts = 0;               // points of the composite triangle rule
-    std::vector<double4> quad;  // the rule, padded to an even count with a zero-weight point
-    std::vector<double4> pair_pts;  // per padded point: (b0, b1, b2, w), (phi_F own, phi_F partner, 0, 0)
-    // CQBEM_QUAD_BANDED: the far rule's pair point table and, per patch, its bounding sphere's centre and the far
+    std::vector<double4> quad;  // the rule: (b0, b1, b2, w) per point
+    std::vector<double4> patch_pts;  // the rule as the patch kernel reads it: (b1, b2, 0, 0), w (b0, b1, b2, 1)
+    // CQBEM_QUAD_BANDED: the far rule's patch point table and, per patch, its bounding sphere's centre and the far
     // distance (radius + kappa h)
-    std::vector<double4> far_pair_pts;
+    std::vector<double4> far_patch_pts;
     int far_npts = 0;  // points of the far rule (unpadded)
     std::vector<double4> patch_sphere;
     std::vector<double> patch_weight;  // per patch: sum over its faces of 1 / (patches listing the face)
@@ -292,19 +292,18 @@ Prepared prepare(const cqbem_mesh *mesh, const cqbem_params *p) {
         std::sort(key.begin(), key.end());
         for (int r = 0; r < P.nv; r++) order[r] = key[r].second;
     }
-    // Pair-form patches, grown one at a time.  A patch lists every face with a corner in it; the list is ordered by
-    // a vertex-disjoint colouring and cut into passes of pair_pass_faces() faces.  A patch starts from the first
+    // Patches, grown one at a time.  A patch lists every face with a corner in it; the list is ordered by
+    // a vertex-disjoint colouring and cut into chunks of chunk_face_count() faces.  A patch starts from the first
     // unassigned vertex in Morton order and takes, among the unassigned vertices that share a face with it, the
     // one adding the fewest faces to its list, then the one with the most assigned neighbours, then the first in
-    // Morton order.  It closes at pair_patch_size() vertices, or when the next vertex would take its face list
-    // beyond kPairTargetPasses full passes; a patch whose neighbours run out (a mesh in several pieces) goes on
+    // Morton order.  It closes at patch_size() vertices, or when the next vertex would take its face list
+    // beyond kTargetChunks full chunks; a patch whose neighbours run out (a mesh in several pieces) goes on
     // from the next unassigned vertex in Morton order.  Compact patches list fewer faces twice than runs of the
     // Morton order (icosphere level 4: 1.14 face listings per face instead of 1.22).  A patch's slots are its
-    // vertices in ascending order.  Within a pass every in-patch corner gets a sub-step: its rank among the pass's
-    // updates of that vertex, in face order.
+    // vertices in ascending order.
     {
-        constexpr int kPairTargetPasses = 4;
-        const int C = pair_patch_size(), PF = pair_pass_faces(), cap = kPairTargetPasses * PF;
+        constexpr int kTargetChunks = 8;
+        const int C = patch_size(), PF = chunk_face_count(), cap = kTargetChunks * PF;
         std::vector<int> nb_ptr(P.nv + 1, 0), nb;  // distinct neighbours: the other corners of the vertex's faces
         {
             std::vector<int> tmp;
@@ -374,17 +373,17 @@ Prepared prepare(const cqbem_mesh *mesh, const cqbem_params *p) {
             std::sort(members.begin(), members.end());
             for (size_t k = 0; k < members.size(); k++) slot[members[k]] = (int)k;
         }
-        P.pair_npatches = (int)lists.size();
-        P.pair_patch_verts.assign((size_t)P.pair_npatches * C, -1);
-        for (int v = 0; v < P.nv; v++) P.pair_patch_verts[(size_t)patch[v] * C + slot[v]] = v;
-        P.pair_patch_pass.assign(1, 0);
-        std::vector<int> cnt(C);
+        P.npatches = (int)lists.size();
+        P.patch_verts.assign((size_t)P.npatches * C, -1);
+        for (int v = 0; v < P.nv; v++) P.patch_verts[(size_t)patch[v] * C + slot[v]] = v;
+        P.patch_chunk.assign(1, 0);
+        std::vector<int> cnt[3] = {std::vector<int>(C), std::vector<int>(C), std::vector<int>(C)};
         std::vector<std::vector<int>> used;  // per colour, per slot: taken
-        for (int pc = 0; pc < P.pair_npatches; pc++) {
+        for (int pc = 0; pc < P.npatches; pc++) {
             auto &l = lists[pc];
             std::sort(l.begin(), l.end());
-            // greedy colouring: faces of one colour share no in-patch vertex; ordering the passes by colour keeps
-            // the updates per vertex and pass (the sub-steps) near 2-3 instead of the full valence
+            // greedy colouring: faces of one colour share no in-patch vertex; ordering the chunks by colour keeps
+            // the updates per vertex and chunk (the sub-steps) near one per corner
             used.clear();
             std::vector<std::pair<int, int>> keyed;
             keyed.reserve(l.size());
@@ -403,35 +402,44 @@ Prepared prepare(const cqbem_mesh *mesh, const cqbem_params *p) {
             }
             std::sort(keyed.begin(), keyed.end());
             for (size_t k = 0; k < l.size(); k++) l[k] = keyed[k].second;
+            // each chunk's corner updates in sub-steps, corner 0 first: the sub-step of a corner is its rank among the
+            // chunk's updates of that vertex from the same corner position.  A face's corners may be taken from any of
+            // the three (in order): the one that adds the fewest sub-steps, then the one with the lowest ranks.
             for (size_t b = 0; b < l.size(); b += PF) {
                 const int nf = (int)std::min<size_t>(PF, l.size() - b);
-                std::fill(cnt.begin(), cnt.end(), 0);
-                int nsub = 0;
-                const int first = (int)P.pair_pass_faces.size();
+                int nsub[3] = {0, 0, 0};
+                for (auto &c : cnt) std::fill(c.begin(), c.end(), 0);
+                const int first = (int)P.chunk_faces.size();
                 for (int k = 0; k < nf; k++) {
                     const int f = l[b + k];
-                    int code[3];
-                    for (int c = 0; c < 3; c++) {
-                        const int v = F[3 * f + c];
-                        if (patch[v] != pc) {
-                            code[c] = -1;
-                            continue;
+                    int best = 0, best_steps = 0, best_ranks = 0;
+                    for (int rot = 0; rot < 3; rot++) {
+                        int steps = 0, ranks = 0;
+                        for (int c = 0; c < 3; c++) {
+                            const int v = F[3 * f + (c + rot) % 3];
+                            const int r = patch[v] == pc ? cnt[c][slot[v]] + 1 : 0;
+                            steps += std::max(nsub[c], r), ranks += r * r;
                         }
-                        const int sub = cnt[slot[v]]++;
-                        nsub = std::max(nsub, sub + 1);
-                        code[c] = slot[v] | sub << 10;
+                        if (rot == 0 || steps < best_steps || (steps == best_steps && ranks < best_ranks))
+                            best = rot, best_steps = steps, best_ranks = ranks;
                     }
-                    P.pair_pass_faces.push_back(make_int4(f, code[0], code[1], code[2]));
+                    unsigned corner[3], steps = 0;
+                    for (int c = 0; c < 3; c++) {
+                        const int v = F[3 * f + (c + best) % 3];
+                        unsigned step = 0xff, sl = 0;
+                        if (patch[v] == pc) sl = slot[v], step = cnt[c][slot[v]]++, nsub[c] = std::max<int>(nsub[c], step + 1);
+                        corner[c] = (unsigned)v | sl << 24, steps |= step << (8 * c);
+                    }
+                    P.chunk_faces.push_back(make_int4((int)corner[0], (int)corner[1], (int)corner[2], (int)steps));
                 }
-                if (nsub > 0x7fff) throw Err{CQBEM_ERR_UNSUPPORTED, "vertex valence too large for the pair schedule"};
-                P.pair_pass_info.push_back(make_int2(first, nf | nsub << 16));
+                P.chunk_info.push_back(make_int4(first, nf, nsub[0] | nsub[1] << 8 | nsub[2] << 16, 0));
             }
-            P.pair_patch_pass.push_back((int)P.pair_pass_info.size());
+            P.patch_chunk.push_back((int)P.chunk_info.size());
         }
         if (p->quad_policy == CQBEM_QUAD_BANDED) {
             // per patch: bounding sphere of its faces (centre: mean of their corners) and largest face diameter
             const double kappa = p->band_kappa > 0 ? p->band_kappa : kBandKappa;
-            for (int pc = 0; pc < P.pair_npatches; pc++) {
+            for (int pc = 0; pc < P.npatches; pc++) {
                 double c[3] = {0, 0, 0};
                 for (int f : lists[pc])
                     for (int k = 0; k < 3; k++)
@@ -475,28 +483,25 @@ Prepared prepare(const cqbem_mesh *mesh, const cqbem_params *p) {
             }
         }
     }
-    for (const TriPoint &t : composite_tri_rule(p->order, p->subdivision)) P.quad.push_back(make_double4(t.b[0], t.b[1], t.b[2], t.w));
-    P.npts = (int)P.quad.size();
-    if (P.quad.size() & 1) P.quad.push_back(make_double4(1.0 / 3.0, 1.0 / 3.0, 1.0 / 3.0, 0.0));
-    // pair-kernel point table: even points go to lane A (corner 0), odd points to lane B (corner 2)
-    for (size_t q = 0; q < P.quad.size(); q++) {
-        const double4 &Q = P.quad[q], &Qp = P.quad[q ^ 1];
-        P.pair_pts.push_back(Q);
-        P.pair_pts.push_back((q & 1) ? make_double4(Q.z, Qp.z, 0.0, 0.0) : make_double4(Q.x, Qp.x, 0.0, 0.0));
-    }
-    if (p->quad_policy == CQBEM_QUAD_BANDED) {
-        std::vector<double4> fq;
-        for (const TriPoint &t : composite_tri_rule(p->far_order > 0 ? p->far_order : p->order,
-                                                    p->far_subdivision > 0 ? p->far_subdivision : 1))
-            fq.push_back(make_double4(t.b[0], t.b[1], t.b[2], t.w));
-        P.far_npts = (int)fq.size();
-        P.far_quad = fq;
-        if (fq.size() & 1) fq.push_back(make_double4(1.0 / 3.0, 1.0 / 3.0, 1.0 / 3.0, 0.0));
-        for (size_t q = 0; q < fq.size(); q++) {
-            const double4 &Q = fq[q], &Qp = fq[q ^ 1];
-            P.far_pair_pts.push_back(Q);
-            P.far_pair_pts.push_back((q & 1) ? make_double4(Q.z, Qp.z, 0.0, 0.0) : make_double4(Q.x, Qp.x, 0.0, 0.0));
+    // the patch kernel's point table of a rule: (b1, b2, 0, 0) and w (b0, b1, b2, 1) per point
+    auto patch_points = [](const std::vector<double4> &rule, std::vector<double4> &pts) {
+        for (const double4 &Q : rule) {
+            pts.push_back(make_double4(Q.y, Q.z, 0.0, 0.0));
+            pts.push_back(make_double4(Q.w * Q.x, Q.w * Q.y, Q.w * Q.z, Q.w));
         }
+    };
+    auto rule_points = [](int order, int subdivision) {
+        std::vector<double4> rule;
+        for (const TriPoint &t : composite_tri_rule(order, subdivision)) rule.push_back(make_double4(t.b[0], t.b[1], t.b[2], t.w));
+        return rule;
+    };
+    P.quad = rule_points(p->order, p->subdivision);
+    P.npts = (int)P.quad.size();
+    patch_points(P.quad, P.patch_pts);
+    if (p->quad_policy == CQBEM_QUAD_BANDED) {
+        P.far_quad = rule_points(p->far_order > 0 ? p->far_order : p->order, p->far_subdivision > 0 ? p->far_subdivision : 1);
+        P.far_npts = (int)P.far_quad.size();
+        patch_points(P.far_quad, P.far_patch_pts);
     }
     for (auto &xw : composite_line01(p->order, p->subdivision)) P.line.push_back(make_double2(xw.first, xw.second));
     const auto s = cq_frequencies(p->L, p->R, p->dt, p->bdf);
@@ -519,20 +524,20 @@ Prepared prepare(const cqbem_mesh *mesh, const cqbem_params *p) {
 
 struct DevMesh {
     DBuf V, F, N, area, vs_ptr, vs_face, sg_ptr, sg_face, vmap, quad, line, freqs, tab;
-    DBuf pair_patch_pass, pair_pass_info, pair_pass_faces, pair_patch_verts, pair_pts;
+    DBuf patch_chunk, chunk_info, chunk_faces, patch_verts, patch_pts;
     DBuf far_pts, patch_sphere, far_quad, face_sphere;  // CQBEM_QUAD_BANDED
     Geom g;
 };
 
-// Collocation G/H regular-face kernel variant: "pair" (default: compact vertex patches, each face evaluated once
-// per patch by a lane pair) or "star" (one lane per column vertex over its vertex star, each face
+// Collocation G/H regular-face kernel variant: "patch" (default: compact vertex patches, each face evaluated once
+// per patch by one lane) or "star" (one lane per column vertex over its vertex star, each face
 // evaluated once per corner); CQBEM_COLLOC_KERNEL=star selects the latter.
 bool colloc_star() {
     const char *e = std::getenv("CQBEM_COLLOC_KERNEL");
     return e && !std::strcmp(e, "star");
 }
 
-// CQBEM_MIXED's far-field G: by default in the FP64 pair kernel together with H (G shares H's exponentials there,
+// CQBEM_MIXED's far-field G: by default in the FP64 patch kernel together with H (G shares H's exponentials there,
 // which costs less than a float kernel of its own on MI355X); CQBEM_MIXED_G=float selects the float star kernel
 // (the reference's own typedef for G).
 bool mixed_float_g() {
@@ -543,8 +548,8 @@ bool mixed_float_g() {
 // The band descriptor of a prepared job (empty unless CQBEM_QUAD_BANDED).
 Bands bands_of(const DevMesh &d, const Prepared &P) {
     Bands b;
-    if (P.far_pair_pts.empty()) return b;
-    b.far_pts = d.far_pts.as<double4>(), b.far_rounds = (int)P.far_pair_pts.size() / 4;
+    if (P.far_patch_pts.empty()) return b;
+    b.far_pts = d.far_pts.as<double4>(), b.far_npts = P.far_npts;
     b.sphere = d.patch_sphere.as<double4>();
     return b;
 }
@@ -557,10 +562,10 @@ FaceBands fbands_of(const DevMesh &d, const Prepared &P) {
     return b;
 }
 
-// Host replica of the pair kernel's per-tile rule choice (CQBEM_QUAD_BANDED): whether tile (patch pc, row point x)
+// Host replica of the patch kernel's per-tile rule choice (CQBEM_QUAD_BANDED): whether tile (patch pc, row point x)
 // takes the far rule.
 bool tile_is_far(const Prepared &P, int pc, const double *x) {
-    if (P.far_pair_pts.empty()) return false;
+    if (P.far_patch_pts.empty()) return false;
     return beyond_sphere(x[0], x[1], x[2], P.patch_sphere[pc]);
 }
 
@@ -575,19 +580,19 @@ bool face_is_far(const Prepared &P, int f, const double *x) {
 // faces of a row lie in near tiles: the patch listing them contains the row vertex).
 double regular_evals(const Prepared &P, const double *V, int i) {
     const int nsing = P.sg_ptr[i + 1] - P.sg_ptr[i];
-    if (P.far_pair_pts.empty()) return (double)(P.nf - nsing) * P.npts * P.Lf;
+    if (P.far_patch_pts.empty()) return (double)(P.nf - nsing) * P.npts * P.Lf;
     double e = -(double)nsing * P.npts;
-    for (int pc = 0; pc < P.pair_npatches; pc++) e += P.patch_weight[pc] * (tile_is_far(P, pc, V + 3 * i) ? P.far_npts : P.npts);
+    for (int pc = 0; pc < P.npatches; pc++) e += P.patch_weight[pc] * (tile_is_far(P, pc, V + 3 * i) ? P.far_npts : P.npts);
     return e * P.Lf;
 }
 
 hipError_t launch_gh(const DevMesh &d, const Prepared &P, const Freq *freqs, int l0, int nl, int row0, int nrows, cd *UG,
                      cd *UH, long long ld, long long lstride, hipStream_t st) {
-    if (colloc_star() && P.far_pair_pts.empty())
+    if (colloc_star() && P.far_patch_pts.empty())
         return launch_colloc_gh(d.g, d.quad.as<double4>(), P.npts, freqs, l0, nl, P.mat, row0, nrows, UG, UH, ld, lstride, st);
-    return launch_colloc_gh_pair(d.g, d.pair_pts.as<double4>(), (int)P.quad.size(), freqs, l0, nl, P.mat, row0, nrows,
-                                 nullptr, d.pair_patch_pass.as<int>(), d.pair_pass_info.as<int2>(), d.pair_pass_faces.as<int4>(),
-                                 d.pair_patch_verts.as<int>(), P.pair_npatches, UG, UH, ld, lstride, st, bands_of(d, P));
+    return launch_colloc_gh_patch(d.g, d.patch_pts.as<double4>(), P.npts, freqs, l0, nl, P.mat, row0, nrows,
+                                 nullptr, d.patch_chunk.as<int>(), d.chunk_info.as<int4>(), d.chunk_faces.as<int4>(),
+                                 d.patch_verts.as<int>(), P.npatches, UG, UH, ld, lstride, st, bands_of(d, P));
 }
 
 void upload_mesh(DevMesh &d, const cqbem_mesh *mesh, const Prepared &P, hipStream_t st) {
@@ -602,11 +607,11 @@ void upload_mesh(DevMesh &d, const cqbem_mesh *mesh, const Prepared &P, hipStrea
     upload(d.N, P.N, st), upload(d.area, P.area, st), upload(d.vs_ptr, P.vs_ptr, st), upload(d.vs_face, P.vs_face, st);
     upload(d.sg_ptr, P.sg_ptr, st), upload(d.sg_face, P.sg_face, st), upload(d.quad, P.quad, st), upload(d.line, P.line, st);
     upload(d.freqs, P.freqs, st), upload(d.tab, P.tab, st);
-    upload(d.pair_patch_pass, P.pair_patch_pass, st), upload(d.pair_pass_info, P.pair_pass_info, st);
-    upload(d.pair_pass_faces, P.pair_pass_faces, st), upload(d.pair_patch_verts, P.pair_patch_verts, st);
-    upload(d.pair_pts, P.pair_pts, st);
-    if (!P.far_pair_pts.empty()) {
-        upload(d.far_pts, P.far_pair_pts, st), upload(d.patch_sphere, P.patch_sphere, st);
+    upload(d.patch_chunk, P.patch_chunk, st), upload(d.chunk_info, P.chunk_info, st);
+    upload(d.chunk_faces, P.chunk_faces, st), upload(d.patch_verts, P.patch_verts, st);
+    upload(d.patch_pts, P.patch_pts, st);
+    if (!P.far_patch_pts.empty()) {
+        upload(d.far_pts, P.far_patch_pts, st), upload(d.patch_sphere, P.patch_sphere, st);
         if (!P.face_sphere.empty()) upload(d.far_quad, P.far_quad, st), upload(d.face_sphere, P.face_sphere, st);
     }
     Geom &g = d.g;
@@ -829,9 +834,9 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
                 HIPCHK(launch_add_c_colloc(H, dC.as<double>(), nv, st));
         }
     } else {
-        GalerkinJob gj{g, quad, npts, line, nline, freqs, Lf, P.mat, ctx->num_cus, d.pair_pts.as<double4>(), (int)P.quad.size(),
-                       d.pair_patch_pass.as<int>(), d.pair_pass_info.as<int2>(), d.pair_pass_faces.as<int4>(),
-                       d.pair_patch_verts.as<int>(), P.pair_npatches, galerkin_budget(slab_budget)};
+        GalerkinJob gj{g, quad, npts, line, nline, freqs, Lf, P.mat, ctx->num_cus, d.patch_pts.as<double4>(),
+                       d.patch_chunk.as<int>(), d.chunk_info.as<int4>(), d.chunk_faces.as<int4>(),
+                       d.patch_verts.as<int>(), P.npatches, galerkin_budget(slab_budget)};
         if (mixed) gj.freqs32 = freqs32, gj.mat32 = mat32;  // far-field B at the test points in float
         check_cancel();
         const int nmat = (wantG ? 1 : 0) + (wantH ? 1 : 0);
@@ -968,9 +973,9 @@ template <class Fn> void parallel_for(size_t n, Fn fn) {
     if (err) std::rethrow_exception(err);
 }
 
-// A scene: every object's G/H regular-face tiles go through shared launches of the pair kernel (k_scene_gh_tiles:
+// A scene: every object's G/H regular-face tiles go through shared launches of the patch kernel (k_scene_gh_tiles:
 // all objects' tiles in one grid, largest pieces first), in waves whose spectra fit the scratch budget; each wave's
-// launches -- the shared pair kernel, the float G kernel of objects that use it (CQBEM_MIXED_G=float), the singular
+// launches -- the shared patch kernel, the float G kernel of objects that use it (CQBEM_MIXED_G=float), the singular
 // faces and the transforms of
 // every piece -- are captured in one HIP graph and launched once.  B, C and the B post-processing of all objects
 // follow in a last graph.  Galerkin objects run one after another through run_job.
@@ -1069,7 +1074,7 @@ void run_scene(cqbem_context *ctx, hipStream_t st, int n, const cqbem_mesh *mesh
         const int rows = (int)std::min<uint64_t>(std::min<uint64_t>(std::max<uint64_t>(W / per_row, 1), o->P.nv), 65535);
         for (int r0 = 0; r0 < o->P.nv; r0 += rows) {
             const int nr = std::min(rows, o->P.nv - r0);
-            pieces.push_back(Piece{o, r0, nr, per_row * nr, (long long)o->P.pair_npatches * o->P.Lf * nr});
+            pieces.push_back(Piece{o, r0, nr, per_row * nr, (long long)o->P.npatches * o->P.Lf * nr});
         }
     }
     // waves: first fit of the pieces, largest first, into the budget
@@ -1105,19 +1110,21 @@ void run_scene(cqbem_context *ctx, hipStream_t st, int n, const cqbem_mesh *mesh
             if (o->wantH) sH = reinterpret_cast<cd *>(spec.as<char>() + off), off += (size_t)o->P.Lf * lstride * sizeof(cd);
             slabs.push_back(Slab{pc, sG, sH, lstride});
             // objects with the float G kernel: H through the shared launch, G through the float kernel
-            const bool g_in_pair = o->wantG && !o->g32;
-            if (!g_in_pair && !o->wantH) continue;
-            ScenePiece sp{o->d.g, o->d.pair_pts.as<double4>(), (int)o->P.quad.size() / 2, o->d.freqs.as<Freq>(), o->P.mat,
-                          pc.row0, pc.nrows, o->P.Lf, o->P.pair_npatches, o->d.pair_patch_pass.as<int>(),
-                          o->d.pair_pass_info.as<int2>(), o->d.pair_pass_faces.as<int4>(), o->d.pair_patch_verts.as<int>(),
-                          g_in_pair ? sG : nullptr, o->wantH ? sH : nullptr, n3, lstride, 0u, bands_of(o->d, o->P)};
-            (g_in_pair ? (o->wantH ? gh : gonly) : honly).push_back(sp);
+            const bool g_in_patch = o->wantG && !o->g32;
+            if (!g_in_patch && !o->wantH) continue;
+            ScenePiece sp{o->d.g, o->d.patch_pts.as<double4>(), o->P.npts, o->d.freqs.as<Freq>(), o->P.mat,
+                          pc.row0, pc.nrows, 1, o->P.Lf, o->P.npatches, o->d.patch_chunk.as<int>(),
+                          o->d.chunk_info.as<int4>(), o->d.chunk_faces.as<int4>(), o->d.patch_verts.as<int>(),
+                          g_in_patch ? sG : nullptr, o->wantH ? sH : nullptr, n3, lstride, 0u, bands_of(o->d, o->P)};
+            (g_in_patch ? (o->wantH ? gh : gonly) : honly).push_back(sp);
         }
         auto number = [](std::vector<ScenePiece> &v) {
-            long long base = 0;
+            long long base = 0, tiles = 0;
+            for (auto &sp : v) tiles += (long long)sp.npatches * sp.nl * sp.nrows;
             for (auto &sp : v) {
+                sp.rpt = patch_rows_per_tile(tiles);
                 sp.base = (unsigned)base;
-                base += (long long)sp.npatches * sp.nl * sp.nrows;
+                base += (long long)sp.npatches * sp.nl * ((sp.nrows + sp.rpt - 1) / sp.rpt);
             }
             if (base >= (1LL << 31)) throw Err{CQBEM_ERR_UNSUPPORTED, "assemble_scene: too many tiles in one wave"};
             return base;
@@ -1133,9 +1140,9 @@ void run_scene(cqbem_context *ctx, hipStream_t st, int n, const cqbem_mesh *mesh
         {
             // the shared launches run one after another on the stream (they share the tile counter)
             GraphRun gr(st);
-            if (ngh) HIPCHK(launch_scene_gh_pair(dgh, (int)gh.size(), ngh, counter.as<unsigned>(), true, true, ctx->num_cus, st));
-            if (nho) HIPCHK(launch_scene_gh_pair(dho, (int)honly.size(), nho, counter.as<unsigned>(), false, true, ctx->num_cus, st));
-            if (ngo) HIPCHK(launch_scene_gh_pair(dgo, (int)gonly.size(), ngo, counter.as<unsigned>(), true, false, ctx->num_cus, st));
+            if (ngh) HIPCHK(launch_scene_gh(dgh, (int)gh.size(), ngh, counter.as<unsigned>(), true, true, ctx->num_cus, st));
+            if (nho) HIPCHK(launch_scene_gh(dho, (int)honly.size(), nho, counter.as<unsigned>(), false, true, ctx->num_cus, st));
+            if (ngo) HIPCHK(launch_scene_gh(dgo, (int)gonly.size(), ngo, counter.as<unsigned>(), true, false, ctx->num_cus, st));
             // each slab's float G, singular faces and transforms: one branch per slab (uncaptured), after the shared
             // launches
             Branches br(ctx, st, gr.capture);
@@ -1398,18 +1405,18 @@ int cqbem_band_plan(const cqbem_mesh *mesh, const cqbem_params *params, int32_t 
         check_inputs(mesh, params);
         if (params->quad_policy != CQBEM_QUAD_BANDED) throw Err{CQBEM_ERR_ARG, "quad_policy is not CQBEM_QUAD_BANDED"};
         const Prepared P = prepare(mesh, params);
-        *npatches = P.pair_npatches;
-        const int PV = pair_patch_size();
+        *npatches = P.npatches;
+        const int PV = patch_size();
         if (patch_of_vertex)
-            for (int pc = 0; pc < P.pair_npatches; pc++)
+            for (int pc = 0; pc < P.npatches; pc++)
                 for (int sl = 0; sl < PV; sl++) {
-                    const int v = P.pair_patch_verts[(size_t)pc * PV + sl];
+                    const int v = P.patch_verts[(size_t)pc * PV + sl];
                     if (v >= 0) patch_of_vertex[v] = pc;
                 }
         if (far)
             for (int i = 0; i < P.nv; i++)
-                for (int pc = 0; pc < P.pair_npatches; pc++)
-                    far[(size_t)i * P.pair_npatches + pc] = tile_is_far(P, pc, mesh->V + 3 * i) ? 1 : 0;
+                for (int pc = 0; pc < P.npatches; pc++)
+                    far[(size_t)i * P.npatches + pc] = tile_is_far(P, pc, mesh->V + 3 * i) ? 1 : 0;
     } catch (const Err &e) {
         return e.code;
     } catch (const std::exception &) {
@@ -1595,9 +1602,9 @@ int cqbem_laplace(cqbem_context *ctx, const cqbem_mesh *mesh, const cqbem_params
                                               dBa.as<cd>(), st));
             }
         } else {
-            GalerkinJob gj{d.g, quad, npts, line, nline, freqs + l, 1, P.mat, ctx->num_cus, d.pair_pts.as<double4>(),
-                           (int)P.quad.size(), d.pair_patch_pass.as<int>(), d.pair_pass_info.as<int2>(),
-                           d.pair_pass_faces.as<int4>(), d.pair_patch_verts.as<int>(), P.pair_npatches, (size_t)1 << 30};
+            GalerkinJob gj{d.g, quad, npts, line, nline, freqs + l, 1, P.mat, ctx->num_cus, d.patch_pts.as<double4>(),
+                           d.patch_chunk.as<int>(), d.chunk_info.as<int4>(),
+                           d.chunk_faces.as<int4>(), d.patch_verts.as<int>(), P.npatches, (size_t)1 << 30};
             if (mixed) gj.freqs32 = dfreq32.as<FreqF>() + l, gj.mat32 = mat32;
             double tm[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             run_galerkin(gj, mesh->F, mesh->vertex_map_inverse, wG ? dU.as<cd>() : nullptr, wH ? dP.as<cd>() : nullptr,
@@ -1670,7 +1677,7 @@ static int submit_impl(cqbem_context *ctx, const cqbem_mesh *mesh, const cqbem_p
             throw Err{CQBEM_ERR_NOMEM, "job footprint (" + std::to_string((fixed + res) >> 20) +
                                            " MiB) exceeds the HBM budget"};
         // the spectra slab: half of what the budget leaves (all of it up to 256 MiB), at most 2 GiB (a slab of that
-        // size already holds ~30k tiles of the pair kernel, and smaller slabs leave room for the other slots' jobs);
+        // size already holds ~30k tiles of the patch kernel, and smaller slabs leave room for the other slots' jobs);
         // one-row slabs when even that does not fit
         const uint64_t used = ctx->reserved + fixed + res;
         const uint64_t left = ctx->budget > used ? ctx->budget - used : 0;

@@ -18,6 +18,7 @@
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include "cqbem_device.hpp"
 #include "cqbem_kernels.hpp"
@@ -132,276 +133,348 @@ __global__ void __launch_bounds__(64) k_colloc_gh(Geom g, const double4 *__restr
 
 
 // ------------------------------------------------------------------------
-// G and H, regular faces, pair form.  Column vertices are grouped into
-// compact patches of at most kPairPV vertices; a block owns one (patch,
-// frequency, row vertex) and evaluates every face touching the patch once.
-// Two adjacent lanes share a face: per round each evaluates one quadrature
-// point, forms its 3x3 G and H blocks K (7 + 9 complex), and the two swap K
-// with a DPP quad permutation, so both see both points.  Lane A (even)
-// accumulates corner 0 and lane B (odd) corner 2 over both points; corner 1
-// is summed over each lane's own points and the two halves are added after
-// the face (lane A keeps its G part, lane B its H part) -- each point is
-// evaluated once for all three corner basis functions.  The face sums are added into
-// per-vertex LDS accumulators in sub-steps that the host schedules so that
-// no vertex is updated twice in one sub-step, in face order: deterministic,
-// no atomics.  The block then writes each (row, column) block once.
+// G and H, regular faces, patch form.  Column vertices are grouped into
+// compact patches of at most kPatchVerts vertices; a block owns one (patch,
+// frequency, row vertex) and evaluates every face touching the patch once, one
+// lane per face, 64 faces (a chunk) per wave.  The lane runs the rule in the
+// face's own frame (FaceFrame, point_g, point_h), where G has 6 and H 8
+// different entries, and keeps the sums of all three corner basis functions in
+// registers (84 doubles with G and H); the rule's points and weights are
+// wave-uniform (scalar loads).  After the rule it rotates each corner's sums to
+// the global axes and adds them to per-vertex LDS accumulators.  The waves add in chunk order (an LDS turn counter) and, within a chunk, in
+// sub-steps that the host schedules so that no vertex is updated twice in one
+// sub-step: every sum has one order, whatever the hardware's.  The block then
+// writes each (row, column) block once.
+//
+// Bound by FP64 VALU issue (and, near full issue, by the clock that the power
+// limit leaves): 292 VALU instructions per point, of which 84 are the corner
+// sums and 78 the two complex exponentials, and 1100 per face and row outside
+// the rule.  Icosphere level 4, L = 32, 28 points (6.2e9 unique evaluations):
+// 80.9 ms, 2.25 ms per point of the rule plus 18 ms.  The form it replaces, two
+// lanes per face that swapped every point's 16 global entries through DPP, took
+// 128 ms at 516 instructions per point.  Tried and slower: the same with a
+// block barrier per sub-step (86.5 ms), the rotation inside the wave's turn
+// (84 ms: it serializes the block), LDS atomic adds instead of the turn's
+// 16-byte read-modify-writes (84 ms).  FP64 matrix instructions share the
+// vector FP64 unit here (a 4x4x4 one takes 16 cycles and does not overlap with
+// vector FMAs), so corner sums on them would cost 4 slots where 3 FMAs do.
 // ------------------------------------------------------------------------
-constexpr int kPairPV = 256;                   // vertex slots per patch (64 KB of LDS accumulators)
-constexpr int kPairThreads = 256;
-constexpr int kPairFaces = kPairThreads / 2;  // faces per pass
-constexpr int kPairWords = 32;                // doubles per slot: G (6 sym + beta) then H (9), complex
-constexpr int kFaceWords = 13;                // per face of a pass: 3 corners, normal, area (16 KB per block)
+constexpr int kPatchVerts = 256;    // vertex slots per patch (60 KB of LDS accumulators)
+constexpr int kPatchThreads = 256;
+constexpr int kPatchPairs = 15;     // complex words per slot: G (6, packed symmetric) then H (9)
+constexpr int kRmw = 8;             // slot words read at a time when a corner is added
+constexpr int kNoStep = 0xff;       // sub-step code of a corner outside the patch
+constexpr int kFramePairs = 3;      // per lane, read at every point: the FaceFrame
 
-// Swap a double with the neighbouring lane of the pair (DPP quad_perm [1,0,3,2]).
-__device__ inline double pair_swap(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)b, 0xB1, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0xB1, 0xF, 0xF, false);
-    return __longlong_as_double(((long long)(unsigned)hi << 32) | (unsigned)lo);
+// Tables that no kernel writes, read through the constant address space: uniform indices become scalar loads also where
+// the pointer itself came from memory (scenes).
+typedef const __attribute__((address_space(4))) double const_double;
+typedef const __attribute__((address_space(4))) int const_int;
+__device__ inline const_double *as_const(const double4 *p) { return (const_double *)p; }
+__device__ inline const_int *as_const(const int4 *p) { return (const_int *)p; }
+// A pointer read from memory, known to be to global memory.
+template <class T> __device__ inline T *as_global(T *p) { return (T *)(__attribute__((address_space(1))) T *)p; }
+
+// Waits until the LDS counter holds `v`.  Every wave of the block is resident and every wave's waits are for events that
+// earlier program points of the others raise, so each wait ends.
+__device__ inline void wait_for(int *counter, int v) {
+    while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(counter, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)) != v)
+        __builtin_amdgcn_s_sleep(1);
 }
 
-// One (patch pc, frequency l, row il) tile of the pair form, for a block of kPairThreads threads.  acc, fgeo and
-// mtab are the block's LDS (mtab loaded and visible); the tile zeroes acc itself and ends with its write-out
-// (callers that run another tile on the same LDS synchronise first).
+// The rows il0 .. il0 + nr - 1 of one (patch pc, frequency l) for a block of kPatchThreads threads.  acc, frame,
+// counters (2) and mtab are the block's LDS (mtab loaded); callers that run another tile on the same LDS synchronise
+// first.  The block has no barrier between its rows: a wave evaluates its first chunk of the next row before it writes
+// out (and clears) its 64 vertex slots of the last one, so neither the other waves' adds nor the stores are waited for.
 template <bool DG, bool DH, bool GAL>
-__device__ __attribute__((always_inline)) inline void pair_tile(const Geom &g, const double4 *__restrict__ pts, int nrounds,
+__device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, const double4 *__restrict__ ref_pts, int ref_npts,
                                  const Bands &bands, const Freq *__restrict__ freqs,
                                  int l0, const Mat &m, int row0, const double4 *__restrict__ tpts,
-                                 const int *__restrict__ patch_pass, const int2 *__restrict__ pass_info,
-                                 const int4 *__restrict__ pass_faces, const int *__restrict__ patch_verts,
+                                 const int *__restrict__ patch_chunk, const int4 *__restrict__ chunk_info,
+                                 const int4 *__restrict__ chunk_faces, const int *__restrict__ patch_verts,
                                  cd *__restrict__ UG, cd *__restrict__ UH, long long ld, long long lstride, int pc, int l,
-                                 int il, double *acc, double *fgeo, const MathTables &mtab) {
-    const int i = row0 + il;
-    const int tid = threadIdx.x, pr = tid >> 1, side = tid & 1;
-    const Freq f = freqs[l0 + l];
-    // the row point: vertex i (collocation), or test point i with its face's corners t[] excluded (Galerkin)
-    double x0, x1, x2;
-    int t[3] = {i, i, i};
-    if (GAL) {
-        const double4 T = tpts[i];
-        x0 = T.x, x1 = T.y, x2 = T.z;
-        const int f1 = (int)T.w;
-        t[0] = g.F[3 * f1], t[1] = g.F[3 * f1 + 1], t[2] = g.F[3 * f1 + 2];
-    } else {
-        x0 = g.V[3 * i], x1 = g.V[3 * i + 1], x2 = g.V[3 * i + 2];
+                                 int il0, int nr, double2 *acc, double2 *frame, int *counters, const MathTables &mtab) {
+    constexpr int kWaves = kPatchThreads / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    Freq f;  // one frequency's constants, in scalar registers
+    {
+        const_double *src = (const_double *)(freqs + (l0 + l));
+        f.s = cd{src[0], src[1]}, f.sc1 = cd{src[2], src[3]}, f.sc2 = cd{src[4], src[5]}, f.is = cd{src[6], src[7]},
+        f.is2 = cd{src[8], src[9]};
     }
-    if (bands.far_pts) {  // the tile's rule: block-uniform (patch and row are)
-        if (__builtin_amdgcn_readfirstlane((int)beyond_sphere(x0, x1, x2, bands.sphere[pc])))
-            pts = bands.far_pts, nrounds = bands.far_rounds;
-    }
-    for (int k = tid; k < kPairWords * kPairPV; k += kPairThreads) acc[k] = 0.0;
+    for (int k = tid; k < kPatchPairs * kPatchVerts; k += kPatchThreads) acc[k] = make_double2(0.0, 0.0);
+    int *turns = counters, *cleared = counters + 1;  // chunks added so far; waves that cleared their slots, over all rows
+    if (tid < 2) counters[tid] = 0;
     __syncthreads();
+    // Waves take the patch's chunks in turn.  With one or two chunks, 4 or 2 waves share a chunk, each taking every 4th
+    // or 2nd point of the rule, as long as 7 points are left to each.
+    const int c0 = patch_chunk[pc], nchunk = patch_chunk[pc + 1] - c0;
+    const int split = nchunk == 1 && ref_npts >= 28 ? 4 : nchunk <= 2 && ref_npts >= 14 ? 2 : 1;
+    const int nturn = nchunk * split;
 
-    for (int pass = patch_pass[pc]; pass < patch_pass[pc + 1]; ++pass) {
-        const int2 info = pass_info[pass];
-        const int nfaces = info.y & 0xffff, nsub = info.y >> 16;
-        // pair-uniform: both lanes of a pair take the same branches around the swaps
-        int4 fe = make_int4(-1, -1, -1, -1);
-        bool active = pr < nfaces;
-        if (active) {
-            fe = pass_faces[info.x + pr];
-            const int a0 = g.F[3 * fe.x], a1 = g.F[3 * fe.x + 1], a2 = g.F[3 * fe.x + 2];
-            for (int k = 0; k < (GAL ? 3 : 1); k++)
-                active = active && !(same_vertex(g, t[k], a0) || same_vertex(g, t[k], a1) || same_vertex(g, t[k], a2));
-        }
-        cd accF[16], accX[16];
+    // writes the G and H blocks of (row r of the tile, the wave's vertex slots) and clears the slots
+    auto write_row = [&](int r) {
+        wait_for(turns, (r + 1) * nturn);
+        const int j = patch_verts[pc * kPatchVerts + tid];
+        if (j >= 0) {
+            const long long obase = (long long)l * lstride + (long long)(3 * (il0 + r)) * ld + 3 * (long long)j;
 #pragma unroll
-        for (int k = 0; k < 16; k++) accF[k] = cd{0, 0}, accX[k] = cd{0, 0};
-        if (active) {
-            const int fc = fe.x;
-            if (side == 0) {
-                const int a0 = g.F[3 * fc], a1 = g.F[3 * fc + 1], a2 = g.F[3 * fc + 2];
-                double *dst = fgeo + pr;
-                for (int k = 0; k < 3; k++) {
-                    dst[k * kPairFaces] = g.V[3 * a0 + k];
-                    dst[(3 + k) * kPairFaces] = g.V[3 * a1 + k];
-                    dst[(6 + k) * kPairFaces] = g.V[3 * a2 + k];
-                    dst[(9 + k) * kPairFaces] = g.N[3 * fc + k];
-                }
-                dst[12 * kPairFaces] = g.area[fc];
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            double4 qcur = pts[2 * side], wcur = pts[2 * side + 1];  // next round's point, prefetched
-            for (int rd = 0; rd < nrounds; ++rd) {
-                // the face slot is made opaque per round so that the loads below stay in the loop (LDS reads
-                // instead of 13 loop-invariant values held in VGPRs)
-                int slot = pr;
-                asm volatile("" : "+v"(slot));
-                const double *fg = fgeo + slot;
-                const double y00 = fg[0], y01 = fg[kPairFaces], y02 = fg[2 * kPairFaces];
-                const double y10 = fg[3 * kPairFaces], y11 = fg[4 * kPairFaces], y12 = fg[5 * kPairFaces];
-                const double y20 = fg[6 * kPairFaces], y21 = fg[7 * kPairFaces], y22 = fg[8 * kPairFaces];
-                const double ar = fg[12 * kPairFaces];
-                const double4 Qo = qcur, Wt = wcur;  // this lane's point and its corner weights
-                if (rd + 1 < nrounds) qcur = pts[4 * (rd + 1) + 2 * side], wcur = pts[4 * (rd + 1) + 2 * side + 1];
-                const double r0 = Qo.x * y00 + Qo.y * y10 + Qo.z * y20 - x0;
-                const double r1 = Qo.x * y01 + Qo.y * y11 + Qo.z * y21 - x1;
-                const double r2 = Qo.x * y02 + Qo.y * y12 + Qo.z * y22 - x2;
-                const double d2 = r0 * r0 + r1 * r1 + r2 * r2;
-                const double ir = rsqrt_nr(d2), r = d2 * ir, ir2 = ir * ir;
-                const double h[3] = {r0 * ir, r1 * ir, r2 * ir};
-                const double wL = Qo.w * ar;
-                const Expo E = expo_gh(r, f, &mtab);
-                cd al, be, c1, c2, c4;
-                if (DG) g_coef<false>(E, ir, ir2, m, al, be);  // 1/(4 pi rho) at the write-out
-                if (DH) h_coef(E, ir, ir2, f, m, c1, c2, c4);
-                // corner weights: the full corner (0 on lane A, 2 on lane B) takes the own and the partner point;
-                // corner 1 takes the own point only, and the pair adds its two halves after the face
-                const double fo = Wt.x, fp = Wt.y, xo = Qo.y;
-                auto consume = [&](const cd &Kk, cd &aF, cd &aX) {
-                    const cd Kq{pair_swap(Kk.x), pair_swap(Kk.y)};
-                    fma_cr(aF, Kk, fo);
-                    fma_cr(aF, Kq, fp);
-                    fma_cr(aX, Kk, xo);
-                };
-                if (DG) {  // G block: alpha rh rh^T + beta I, packed 00 11 22 01 02 12 then beta
-                    const double wr = wL * ir;
-                    al = al * wr;
+            for (int p = 0; p < 3; p++) {
 #pragma unroll
-                    for (int a = 0; a < 3; a++)
-#pragma unroll
-                        for (int b = a; b < 3; b++) consume(al * (h[a] * h[b]), accF[sidx(a, b)], accX[sidx(a, b)]);
-                    consume(be * wr, accF[6], accX[6]);
-                }
-                if (DH) {  // H block (without 1/4pi): rh_a u_b + n_a v_b + d I with u = c4 rn rh + c1 n, v = c2 rh, d = c2 rn
-                    const double n[3] = {fg[9 * kPairFaces], fg[10 * kPairFaces], fg[11 * kPairFaces]};
-                    const double rn = h[0] * n[0] + h[1] * n[1] + h[2] * n[2];
-                    c1 = c1 * wL;
-                    c2 = c2 * wL;
-                    c4 = c4 * (wL * rn);
-                    const cd d = c2 * rn;
-                    cd u[3], v[3];
-#pragma unroll
-                    for (int b = 0; b < 3; b++) {
-                        u[b] = c4 * h[b];
-                        fma_cr(u[b], c1, n[b]);
-                        v[b] = c2 * h[b];
+                for (int b = 0; b < 3; b++) {
+                    const int e = sidx(p, b);
+                    if (DG) {
+                        const double2 w = acc[e * kPatchVerts + tid];
+                        UG[obase + p * ld + b] = cd{w.x, w.y} * m.g_scale;
                     }
-#pragma unroll
-                    for (int a = 0; a < 3; a++)
-#pragma unroll
-                        for (int b = 0; b < 3; b++) {
-                            cd w = u[b] * h[a];
-                            fma_cr(w, v[b], n[a]);
-                            if (a == b) w += d;
-                            consume(w, accF[7 + a * 3 + b], accX[7 + a * 3 + b]);
-                        }
+                    if (DH) {
+                        const double2 w = acc[(6 + p * 3 + b) * kPatchVerts + tid];
+                        UH[obase + p * ld + b] = cd{w.x, w.y} * kInv4Pi;
+                    }
                 }
-            }
-#pragma unroll
-            for (int k = 0; k < 16; k++) accX[k] += cd{pair_swap(accX[k].x), pair_swap(accX[k].y)};
-        }
-        // scheduled updates of the vertex accumulators; corner code: slot | sub-step << 10, -1 = outside the patch
-        const int cF = side ? fe.w : fe.y, cX = fe.z;
-        // read-modify-write of n consecutive complex words of slot sl: all reads issued before the adds
-        auto rmw = [&](int sl, int w0, const cd *v, int n) {
-            double t[32];
-#pragma unroll
-            for (int k = 0; k < 16; k++)
-                if (k < n) t[2 * k] = acc[(w0 + 2 * k) * kPairPV + sl], t[2 * k + 1] = acc[(w0 + 2 * k + 1) * kPairPV + sl];
-#pragma unroll
-            for (int k = 0; k < 16; k++)
-                if (k < n) acc[(w0 + 2 * k) * kPairPV + sl] = t[2 * k] + v[k].x, acc[(w0 + 2 * k + 1) * kPairPV + sl] = t[2 * k + 1] + v[k].y;
-        };
-        for (int sub = 0; sub < nsub; ++sub) {
-            __syncthreads();
-            if (!active) continue;
-            if (cF >= 0 && (cF >> 10) == sub) {
-                if (DG && DH) rmw(cF & 0x3ff, 0, accF, 16);
-                else if (DG) rmw(cF & 0x3ff, 0, accF, 7);
-                else rmw(cF & 0x3ff, 14, accF + 7, 9);
-            }
-            if (cX >= 0 && (cX >> 10) == sub) {
-                if (side == 0) {
-                    if (DG) rmw(cX & 0x3ff, 0, accX, 7);
-                } else if (DH) {
-                    rmw(cX & 0x3ff, 14, accX + 7, 9);
-                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-    }
-    __syncthreads();
-    // one thread per vertex slot writes its (row, column) G and H blocks
-    for (int sl = tid; sl < kPairPV; sl += kPairThreads) {
-        const int j = patch_verts[pc * kPairPV + sl];
-        if (j < 0) continue;
-        auto a = [&](int e) { return acc[e * kPairPV + sl]; };
-        const long long obase = (long long)l * lstride + (long long)(3 * il) * ld + 3 * (long long)j;
 #pragma unroll
-        for (int p = 0; p < 3; p++)
+        for (int e = DG ? 0 : 6; e < (DH ? kPatchPairs : 6); e++) acc[e * kPatchVerts + tid] = make_double2(0.0, 0.0);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (lane == 0) __hip_atomic_fetch_add(cleared, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+
+#pragma unroll 1
+    for (int r = 0; r < nr; ++r) {
+        const int i = row0 + il0 + r;
+        // the row point: vertex i (collocation), or test point i with its face's corners t[] excluded (Galerkin)
+        double x0, x1, x2;
+        int t[3] = {i, i, i};
+        if (GAL) {
+            const double4 T = tpts[i];
+            x0 = T.x, x1 = T.y, x2 = T.z;
+            const int f1 = (int)T.w;
+            t[0] = g.F[3 * f1], t[1] = g.F[3 * f1 + 1], t[2] = g.F[3 * f1 + 2];
+        } else {
+            x0 = g.V[3 * i], x1 = g.V[3 * i + 1], x2 = g.V[3 * i + 2];
+        }
+        const double4 *pts = ref_pts;
+        int npts = ref_npts;
+        if (bands.far_pts) {  // the row's rule: block-uniform (patch and row are)
+            if (__builtin_amdgcn_readfirstlane((int)beyond_sphere(x0, x1, x2, bands.sphere[pc])))
+                pts = bands.far_pts, npts = bands.far_npts;
+        }
+        bool written = r == 0;  // whether the wave has written out the previous row
+#pragma unroll 1
+        for (int turn = wave; turn < nturn; turn += kWaves) {
+            const int part = turn % split;
+            const_int *ci = as_const(chunk_info + (c0 + turn / split));
+            const int4 info = make_int4(ci[0], ci[1], ci[2], 0);
+            // lanes past the chunk's faces repeat its last one; they and the faces touching the row point are not added
+            const int entry = info.x + min(lane, info.y - 1);
+            const int4 fe = chunk_faces[entry];
+            const int va[3] = {fe.x & 0xffffff, fe.y & 0xffffff, fe.z & 0xffffff};
+            bool active = lane < info.y;
+            for (int k = 0; k < (GAL ? 3 : 1); k++)
+                active = active && !(same_vertex(g, t[k], va[0]) || same_vertex(g, t[k], va[1]) || same_vertex(g, t[k], va[2]));
+            const unsigned long long act = __builtin_amdgcn_ballot_w64(active);
+            cd sg[3][6], sh[3][8];
+            if (act) {  // wave-uniform: no divergent merge of the sums
+                {
+                    double y[3][3];
 #pragma unroll
-            for (int b = 0; b < 3; b++) {
-                const int e = sidx(p, b);
-                if (DG) {
-                    cd v{a(2 * e), a(2 * e + 1)};
-                    if (p == b) v += cd{a(12), a(13)};
-                    UG[obase + p * ld + b] = v * m.g_scale;
+                    for (int k = 0; k < 3; k++)
+#pragma unroll
+                        for (int d = 0; d < 3; d++) y[k][d] = g.V[3 * va[k] + d];
+                    const FaceFrame F = face_frame(y, x0, x1, x2);
+                    frame[tid] = make_double2(F.L1, F.u), frame[kPatchThreads + tid] = make_double2(F.v, F.xa);
+                    frame[2 * kPatchThreads + tid] = make_double2(F.xb, F.cr);
                 }
-                if (DH) UH[obase + p * ld + b] = cd{a(14 + 2 * (p * 3 + b)), a(15 + 2 * (p * 3 + b))} * kInv4Pi;
+                // one point's entries into the sums; the first point starts them
+                auto point = [&](int q, auto first) __attribute__((always_inline)) {
+                    // the lane is made opaque per point so that the frame stays in LDS (14 VGPRs otherwise)
+                    int ln = tid;
+                    asm volatile("" : "+v"(ln));
+                    const double2 F0 = frame[ln], F1 = frame[kPatchThreads + ln], F2 = frame[2 * kPatchThreads + ln];
+                    const_double *B = as_const(pts + 2 * q);  // b1, b2, -, -, w (phi_0, phi_1, phi_2, 1)
+                    const double ar = fma(B[0], F0.x, fma(B[1], F0.y, F1.y)), br = fma(B[1], F1.x, F2.x), cr = F2.y;
+                    const PointExpo E = point_expo(fma(ar, ar, fma(br, br, cr * cr)), f, &mtab);
+                    const double w[3] = {B[4], B[5], B[6]};
+                    const double a = ar * E.ir, b = br * E.ir, c = cr * E.ir;
+                    auto add = [&](cd &s, const cd &v, double wk) {
+                        if (first()) s = v * wk;
+                        else fma_cr(s, v, wk);
+                    };
+                    // G and H one after the other, so that only one set of entries is live beside the sums
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (DG) {
+                        cd G[6];
+                        point_g(E, a, b, c, m, G);
+#pragma unroll
+                        for (int k = 0; k < 3; k++)
+#pragma unroll
+                            for (int e = 0; e < 6; e++) add(sg[k][e], G[e], w[k]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (DH) {
+                        cd H[8];
+                        point_h(E, a, b, c, m, H);
+#pragma unroll
+                        for (int k = 0; k < 3; k++)
+#pragma unroll
+                            for (int e = 0; e < 8; e++) add(sh[k][e], H[e], w[k]);
+                    }
+                };
+                point(part, std::true_type{});
+#pragma unroll 1
+                for (int q = part + split; q < npts; q += split) point(q, std::false_type{});
+            } else {
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+#pragma unroll
+                    for (int e = 0; e < 6; e++) sg[k][e] = cd{0, 0};
+#pragma unroll
+                    for (int e = 0; e < 8; e++) sh[k][e] = cd{0, 0};
+                }
             }
+            if (!written) write_row(r - 1), written = true;
+            // rotate each corner's sums and add them in the scheduled sub-steps, after every earlier chunk of the row and
+            // once all slots are cleared
+            const int4 ge = chunk_faces[info.x + min(lane, info.y - 1)];
+            double Q[3][3], A[3][3];
+            {
+                double e1[3], e2[3], L1, area2;
+                const int v0 = ge.x & 0xffffff, v1 = ge.y & 0xffffff, v2 = ge.z & 0xffffff;
+                for (int d = 0; d < 3; d++) e1[d] = g.V[3 * v1 + d] - g.V[3 * v0 + d], e2[d] = g.V[3 * v2 + d] - g.V[3 * v0 + d];
+                face_axes(e1, e2, Q, &L1, &area2);
+                for (int j = 0; j < 3; j++)
+                    for (int k = 0; k < 3; k++) A[j][k] = Q[j][k] * (0.5 * area2);
+            }
+            double v[3][2 * kPatchPairs];
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    if (DG) {
+                        double S[6], R[6];
+#pragma unroll
+                        for (int e = 0; e < 6; e++) S[e] = p ? sg[k][e].y : sg[k][e].x;
+                        rotate_sym(S, Q, A, R);
+#pragma unroll
+                        for (int e = 0; e < 6; e++) v[k][2 * e + p] = R[e];
+                    }
+                    if (DH) {
+                        double S[8], R[9];
+#pragma unroll
+                        for (int e = 0; e < 8; e++) S[e] = p ? sh[k][e].y : sh[k][e].x;
+                        rotate_gen(S, Q, A, R);
+#pragma unroll
+                        for (int e = 0; e < 9; e++) v[k][12 + 2 * e + p] = R[e];
+                    }
+                }
+                // formed here, not sunk behind the waits below
+#pragma unroll
+                for (int e = DG ? 0 : 12; e < (DH ? 2 * kPatchPairs : 12); e++) asm volatile("" : "+v"(v[k][e]));
+            }
+            wait_for(cleared, kWaves * r);
+            wait_for(turns, r * nturn + turn);
+            const int corner[3] = {ge.x, ge.y, ge.z};
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const int slot = (unsigned)corner[k] >> 24;
+                const int step = (act >> lane) & 1 ? (ge.w >> (8 * k)) & 0xff : kNoStep;
+                const int nsub = (info.z >> (8 * k)) & 0xff;
+                for (int s = 0; s < nsub; ++s) {
+                    if (step != s) continue;
+                    // read-modify-write of the slot's words, kRmw reads in flight
+#pragma unroll
+                    for (int e0 = DG ? 0 : 6; e0 < (DH ? kPatchPairs : 6); e0 += kRmw) {
+                        double2 u[kRmw];
+#pragma unroll
+                        for (int e = e0; e < e0 + kRmw && e < (DH ? kPatchPairs : 6); e++) u[e - e0] = acc[e * kPatchVerts + slot];
+#pragma unroll
+                        for (int e = e0; e < e0 + kRmw && e < (DH ? kPatchPairs : 6); e++)
+                            acc[e * kPatchVerts + slot] = make_double2(u[e - e0].x + v[k][2 * e], u[e - e0].y + v[k][2 * e + 1]);
+                    }
+                }
+            }
+            __hip_atomic_store(turns, r * nturn + turn + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        if (!written) write_row(r - 1);  // a wave without a chunk in this patch
     }
+    write_row(nr - 1);
 }
 
 // BANDED: the distance-banded rule (CQBEM_QUAD_BANDED) is compiled in; without it the tile rule check is not.
 template <bool DG, bool DH, bool GAL, bool BANDED>
-__global__ void __launch_bounds__(kPairThreads, 2) k_colloc_gh_pair(Geom g, const double4 *__restrict__ pts, int nrounds,
+__global__ void __launch_bounds__(kPatchThreads, 2) k_colloc_gh_patch(Geom g, const double4 *__restrict__ pts, int npts,
                                                                   const Freq *__restrict__ freqs, int l0, Mat m, int row0,
                                                                   const double4 *__restrict__ tpts,
-                                                                  const int *__restrict__ patch_pass,
-                                                                  const int2 *__restrict__ pass_info,
-                                                                  const int4 *__restrict__ pass_faces,
+                                                                  const int *__restrict__ patch_chunk,
+                                                                  const int4 *__restrict__ chunk_info,
+                                                                  const int4 *__restrict__ chunk_faces,
                                                                   const int *__restrict__ patch_verts, cd *__restrict__ UG,
                                                                   cd *__restrict__ UH, long long ld, long long lstride,
-                                                                  Bands bands) {
-    __shared__ double acc[kPairWords * kPairPV];      // [word][slot]
-    __shared__ double fgeo[kFaceWords * kPairFaces];  // [word][face of pass]: re-read every round, not held in VGPRs
+                                                                  int nrows, int rpt, Bands bands) {
+    __shared__ double2 acc[kPatchPairs * kPatchVerts];      // [word][slot]
+    __shared__ double2 frame[kFramePairs * kPatchThreads];
+    __shared__ int counters[2];  // [word pair][lane]
     __shared__ MathTables mtab;                       // tables of the exponentials
     load_math_tables(&mtab);
-    pair_tile<DG, DH, GAL>(g, pts, nrounds, BANDED ? bands : Bands{}, freqs, l0, m, row0, tpts, patch_pass, pass_info,
-                           pass_faces, patch_verts, UG, UH, ld, lstride, blockIdx.x, blockIdx.y, blockIdx.z, acc, fgeo, mtab);
+    patch_tile<DG, DH, GAL>(g, pts, npts, BANDED ? bands : Bands{}, freqs, l0, m, row0, tpts, patch_chunk, chunk_info,
+                           chunk_faces, patch_verts, UG, UH, ld, lstride, blockIdx.x, blockIdx.y, blockIdx.z * rpt,
+                           min(rpt, nrows - (int)blockIdx.z * rpt), acc, frame, counters, mtab);
 }
 
 // ------------------------------------------------------------------------
 // Several objects' G/H regular-face work in one launch: each piece (an object's row slab) contributes
 // npatches x nl x nrows tiles, numbered from its `base`, and each tile runs exactly the computation of
-// k_colloc_gh_pair's block for it, so every object's spectra are bit-identical to its own launch.  Two forms:
+// k_colloc_gh_patch's block for it, so every object's spectra are bit-identical to its own launch.  Two forms:
 //   k_scene_gh_tiles: one block per tile; the hardware's workgroup dispatcher hands tiles to CUs in tile order as
 //     they free up (pieces are ordered largest first by the host).  Same registers as the single-object kernel
 //     plus the piece lookup: 2 waves per SIMD.
-//   k_scene_gh_pair: persistent blocks (2 per CU) that take tile numbers from a device counter with one atomic add
+//   k_scene_gh_persistent: persistent blocks (2 per CU) that take tile numbers from a device counter with one atomic add
 //     per tile.  The loop-carried state costs 8 registers beyond 256, i.e. 1 wave per SIMD (CQBEM_SCENE_KERNEL=
 //     persistent selects it, for comparison).
 // ------------------------------------------------------------------------
 template <bool DG, bool DH>
-__device__ __attribute__((always_inline)) inline void scene_tile(const ScenePiece *__restrict__ pieces, int npieces, unsigned t, double *acc, double *fgeo,
+__device__ __attribute__((always_inline)) inline void scene_tile(const ScenePiece *__restrict__ pieces, int npieces, unsigned t, double2 *acc, double2 *frame, int *counters,
                                   const MathTables &mtab) {
     int pi = 0;
-    while (pi + 1 < npieces && pieces[pi + 1].base <= t) ++pi;
-    const ScenePiece *P = pieces + pi;
-    const unsigned local = t - P->base, np = (unsigned)P->npatches, nl = (unsigned)P->nl;
+    while (pi + 1 < npieces && (unsigned)*(const_int *)&pieces[pi + 1].base <= t) ++pi;
+    ScenePiece P;  // held in scalar registers
+    {
+        static_assert(sizeof(ScenePiece) % 4 == 0, "copied in words");
+        const_int *src = (const_int *)(pieces + pi);
+        int w[sizeof(ScenePiece) / 4];
+#pragma unroll
+        for (unsigned k = 0; k < sizeof(ScenePiece) / 4; k++) w[k] = src[k];
+        __builtin_memcpy(&P, w, sizeof(P));
+    }
+    P.g.V = as_global(P.g.V), P.g.vmap = as_global(P.g.vmap);
+    P.bands.sphere = as_global(P.bands.sphere);
+    const unsigned local = t - P.base, np = (unsigned)P.npatches, nl = (unsigned)P.nl;
     const unsigned rest = local / np;
-    pair_tile<DG, DH, false>(P->g, P->pts, P->nrounds, P->bands, P->freqs, 0, P->m, P->row0, nullptr, P->patch_pass, P->pass_info,
-                             P->pass_faces, P->patch_verts, P->UG, P->UH, P->ld, P->lstride, (int)(local - rest * np),
-                             (int)(rest % nl), (int)(rest / nl), acc, fgeo, mtab);
+    patch_tile<DG, DH, false>(P.g, P.pts, P.npts, P.bands, as_global(P.freqs), 0, P.m, P.row0, nullptr, as_global(P.patch_chunk),
+                              P.chunk_info, as_global(P.chunk_faces), as_global(P.patch_verts), as_global(P.UG), as_global(P.UH),
+                              P.ld, P.lstride, (int)(local - rest * np), (int)(rest % nl), (int)(rest / nl) * P.rpt,
+                              min(P.rpt, P.nrows - (int)(rest / nl) * P.rpt), acc, frame, counters, mtab);
 }
 
 template <bool DG, bool DH>
-__global__ void __launch_bounds__(kPairThreads, 2) k_scene_gh_tiles(const ScenePiece *__restrict__ pieces, int npieces,
+__global__ void __launch_bounds__(kPatchThreads, 2) k_scene_gh_tiles(const ScenePiece *__restrict__ pieces, int npieces,
                                                                   unsigned t0) {
-    __shared__ double acc[kPairWords * kPairPV];
-    __shared__ double fgeo[kFaceWords * kPairFaces];
+    __shared__ double2 acc[kPatchPairs * kPatchVerts];
+    __shared__ double2 frame[kFramePairs * kPatchThreads];
+    __shared__ int counters[2];
     __shared__ MathTables mtab;
     load_math_tables(&mtab);
-    scene_tile<DG, DH>(pieces, npieces, t0 + blockIdx.x, acc, fgeo, mtab);
+    scene_tile<DG, DH>(pieces, npieces, t0 + blockIdx.x, acc, frame, counters, mtab);
 }
 
 template <bool DG, bool DH>
-__global__ void __launch_bounds__(kPairThreads, 2) k_scene_gh_pair(const ScenePiece *__restrict__ pieces, int npieces,
+__global__ void __launch_bounds__(kPatchThreads, 2) k_scene_gh_persistent(const ScenePiece *__restrict__ pieces, int npieces,
                                                                  unsigned ntiles, unsigned *__restrict__ counter) {
-    __shared__ double acc[kPairWords * kPairPV];
-    __shared__ double fgeo[kFaceWords * kPairFaces];
+    __shared__ double2 acc[kPatchPairs * kPatchVerts];
+    __shared__ double2 frame[kFramePairs * kPatchThreads];
+    __shared__ int counters[2];
     __shared__ MathTables mtab;
     __shared__ unsigned next_tile;
     load_math_tables(&mtab);
@@ -411,7 +484,7 @@ __global__ void __launch_bounds__(kPairThreads, 2) k_scene_gh_pair(const ScenePi
         __syncthreads();
         const unsigned t = __builtin_amdgcn_readfirstlane(next_tile);
         if (t >= ntiles) break;  // uniform across the block: every wave leaves
-        scene_tile<DG, DH>(pieces, npieces, t, acc, fgeo, mtab);
+        scene_tile<DG, DH>(pieces, npieces, t, acc, frame, counters, mtab);
     }
 }
 
@@ -1182,33 +1255,38 @@ hipError_t launch_colloc_gh(const Geom &g, const double4 *quad, int npts, const 
 }
 
 
-hipError_t launch_colloc_gh_pair(const Geom &g, const double4 *pts, int npts_even, const Freq *freqs, int l0, int nl, const Mat &m,
-                                 int row0, int nrows, const double4 *tpts, const int *patch_pass, const int2 *pass_info,
-                                 const int4 *pass_faces, const int *patch_verts, int npatches, cd *UG, cd *UH, long long ld,
+// Rows per block of the patch kernel: enough to hide a row's start and write-out behind the next one's evaluation, and
+// still at least 8192 blocks (16 per resident block of 256 CUs) where there are as many tiles.
+int patch_rows_per_tile(long long tiles) { return (int)std::min<long long>(16, std::max<long long>(1, tiles / 8192)); }
+
+hipError_t launch_colloc_gh_patch(const Geom &g, const double4 *pts, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
+                                 int row0, int nrows, const double4 *tpts, const int *patch_chunk, const int4 *chunk_info,
+                                 const int4 *chunk_faces, const int *patch_verts, int npatches, cd *UG, cd *UH, long long ld,
                                  long long lstride, hipStream_t st, const Bands &bands) {
-    if ((!UG && !UH) || (npts_even & 1) || nrows <= 0 || nrows > 65535) return hipErrorInvalidValue;
-    if (bands.far_pts && (tpts || bands.far_rounds <= 0 || !bands.sphere)) return hipErrorInvalidValue;
-    dim3 grid(npatches, nl, nrows);
-#define CQBEM_PAIR(DG, DH, GAL, BANDED)                                                                                    \
-    hipLaunchKernelGGL((k_colloc_gh_pair<DG, DH, GAL, BANDED>), grid, dim3(kPairThreads), 0, st, g, pts, npts_even / 2, freqs, \
-                       l0, m, row0, tpts, patch_pass, pass_info, pass_faces, patch_verts, UG, UH, ld, lstride, bands)
+    if ((!UG && !UH) || npts <= 0 || nrows <= 0 || nrows > 65535) return hipErrorInvalidValue;
+    if (bands.far_pts && (tpts || bands.far_npts <= 0 || !bands.sphere)) return hipErrorInvalidValue;
+    const int rpt = patch_rows_per_tile((long long)npatches * nl * nrows);
+    dim3 grid(npatches, nl, (nrows + rpt - 1) / rpt);
+#define CQBEM_PATCH(DG, DH, GAL, BANDED)                                                                                    \
+    hipLaunchKernelGGL((k_colloc_gh_patch<DG, DH, GAL, BANDED>), grid, dim3(kPatchThreads), 0, st, g, pts, npts, freqs, \
+                       l0, m, row0, tpts, patch_chunk, chunk_info, chunk_faces, patch_verts, UG, UH, ld, lstride, nrows, rpt, bands)
     if (tpts) {  // test points: never banded (refused above)
-        if (UG && UH) CQBEM_PAIR(true, true, true, false);
-        else if (UG) CQBEM_PAIR(true, false, true, false);
-        else CQBEM_PAIR(false, true, true, false);
+        if (UG && UH) CQBEM_PATCH(true, true, true, false);
+        else if (UG) CQBEM_PATCH(true, false, true, false);
+        else CQBEM_PATCH(false, true, true, false);
     } else if (bands.far_pts) {
-        if (UG && UH) CQBEM_PAIR(true, true, false, true);
-        else if (UG) CQBEM_PAIR(true, false, false, true);
-        else CQBEM_PAIR(false, true, false, true);
+        if (UG && UH) CQBEM_PATCH(true, true, false, true);
+        else if (UG) CQBEM_PATCH(true, false, false, true);
+        else CQBEM_PATCH(false, true, false, true);
     } else {
-        if (UG && UH) CQBEM_PAIR(true, true, false, false);
-        else if (UG) CQBEM_PAIR(true, false, false, false);
-        else CQBEM_PAIR(false, true, false, false);
+        if (UG && UH) CQBEM_PATCH(true, true, false, false);
+        else if (UG) CQBEM_PATCH(true, false, false, false);
+        else CQBEM_PATCH(false, true, false, false);
     }
-#undef CQBEM_PAIR
+#undef CQBEM_PATCH
     return hipGetLastError();
 }
-hipError_t launch_scene_gh_pair(const ScenePiece *pieces, int npieces, long long ntiles, unsigned *counter, bool G, bool H,
+hipError_t launch_scene_gh(const ScenePiece *pieces, int npieces, long long ntiles, unsigned *counter, bool G, bool H,
                                 int num_cus, hipStream_t st) {
     if ((!G && !H) || npieces <= 0 || ntiles <= 0 || ntiles >= (1LL << 31)) return hipErrorInvalidValue;
     const char *env = std::getenv("CQBEM_SCENE_KERNEL");  // read per launch (tests switch it)
@@ -1219,30 +1297,30 @@ hipError_t launch_scene_gh_pair(const ScenePiece *pieces, int npieces, long long
         for (long long t0 = 0; t0 < ntiles; t0 += kChunk) {
             const dim3 grid((unsigned)std::min(kChunk, ntiles - t0));
             if (G && H)
-                hipLaunchKernelGGL((k_scene_gh_tiles<true, true>), grid, dim3(kPairThreads), 0, st, pieces, npieces, (unsigned)t0);
+                hipLaunchKernelGGL((k_scene_gh_tiles<true, true>), grid, dim3(kPatchThreads), 0, st, pieces, npieces, (unsigned)t0);
             else if (G)
-                hipLaunchKernelGGL((k_scene_gh_tiles<true, false>), grid, dim3(kPairThreads), 0, st, pieces, npieces, (unsigned)t0);
+                hipLaunchKernelGGL((k_scene_gh_tiles<true, false>), grid, dim3(kPatchThreads), 0, st, pieces, npieces, (unsigned)t0);
             else
-                hipLaunchKernelGGL((k_scene_gh_tiles<false, true>), grid, dim3(kPairThreads), 0, st, pieces, npieces, (unsigned)t0);
+                hipLaunchKernelGGL((k_scene_gh_tiles<false, true>), grid, dim3(kPatchThreads), 0, st, pieces, npieces, (unsigned)t0);
         }
         return hipGetLastError();
     }
     hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, st, counter);
     const unsigned blocks = (unsigned)std::min<long long>(ntiles, 2LL * num_cus);
     if (G && H)
-        hipLaunchKernelGGL((k_scene_gh_pair<true, true>), dim3(blocks), dim3(kPairThreads), 0, st, pieces, npieces,
+        hipLaunchKernelGGL((k_scene_gh_persistent<true, true>), dim3(blocks), dim3(kPatchThreads), 0, st, pieces, npieces,
                            (unsigned)ntiles, counter);
     else if (G)
-        hipLaunchKernelGGL((k_scene_gh_pair<true, false>), dim3(blocks), dim3(kPairThreads), 0, st, pieces, npieces,
+        hipLaunchKernelGGL((k_scene_gh_persistent<true, false>), dim3(blocks), dim3(kPatchThreads), 0, st, pieces, npieces,
                            (unsigned)ntiles, counter);
     else
-        hipLaunchKernelGGL((k_scene_gh_pair<false, true>), dim3(blocks), dim3(kPairThreads), 0, st, pieces, npieces,
+        hipLaunchKernelGGL((k_scene_gh_persistent<false, true>), dim3(blocks), dim3(kPatchThreads), 0, st, pieces, npieces,
                            (unsigned)ntiles, counter);
     return hipGetLastError();
 }
 
-int pair_patch_size() { return kPairPV; }
-int pair_pass_faces() { return kPairFaces; }
+int patch_size() { return kPatchVerts; }
+int chunk_face_count() { return 64; }
 
 hipError_t launch_colloc_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
                            int row0, int nrows, cd *Bt, cd *Ba, hipStream_t st, const FaceBands &fb) {

@@ -23,12 +23,12 @@ struct Geom {
 hipError_t launch_colloc_gh(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
                             int row0, int nrows, cd *UG, cd *UH, long long ld, long long lstride, hipStream_t st);
 
-// Distance bands of the pair kernel's regular-face rule (CQBEM_QUAD_BANDED).  A tile (patch, row point x) takes the
+// Distance bands of the patch kernel's regular-face rule (CQBEM_QUAD_BANDED).  A tile (patch, row point x) takes the
 // far rule at every frequency when |x - centre| >= radius + kappa h (h: the patch's largest face diameter);
 // otherwise the reference rule.  far_pts == nullptr: the reference rule for every tile.
 struct Bands {
-    const double4 *far_pts = nullptr;  // pair point table of the far rule (layout of the reference rule's)
-    int far_rounds = 0;                // its padded points / 2
+    const double4 *far_pts = nullptr;  // patch point table of the far rule (layout of the reference rule's)
+    int far_npts = 0;
     const double4 *sphere = nullptr;   // per patch: centre, radius + kappa h
 };
 // The bands' rule choice: whether row point x lies at or beyond distance S.w from (S.x, S.y, S.z).  Compiled without
@@ -46,33 +46,34 @@ struct FaceBands {
     int far_npts = 0;
     const double4 *sphere = nullptr;    // per face: centre, radius + kappa h
 };
-// Pair form of the G/H regular-face kernel (both matrices): per patch a range of passes
-// [patch_pass[p], patch_pass[p+1]); per pass (first face entry, nfaces | nsub << 16); per face entry
-// (face, corner 0, corner 1, corner 2) with corner = slot | sub-step << 10 or -1 outside the patch.
-// `pts` holds, for each point q of the (even-padded) rule, (b0, b1, b2, w) and (phi_F(q), phi_F(partner), 0, 0)
-// with phi_F the barycentric of corner 0 for even q (lane A) and of corner 2 for odd q (lane B), partner = q ^ 1.
+// Patch form of the G/H regular-face kernel (both matrices): per patch a range of chunks
+// [patch_chunk[p], patch_chunk[p+1]) of up to 64 faces; per chunk (first face entry, nfaces, sub-steps of corner 0 |
+// of corner 1 << 8 | of corner 2 << 16, 0); per face entry, for its corners k = 0..2 (the face's, from any of the
+// three), x, y, z = vertex | slot << 24 and w = the sub-steps, 8 bits each (255: outside the patch).
+// `pts` holds, for each point of the rule, (b1, b2, 0, 0) and w (b0, b1, b2, 1).
 // Rows are collocation vertices row0..row0+nrows-1 when tpts is null.  Otherwise they are the test points
 // tpts[row0..row0+nrows-1] = (x, y, z, test face), each excluding every face that shares a vertex with its
 // test face (the Galerkin non-singular set), and row r of the launch goes to rows 3r..3r+2 of UG/UH.
-hipError_t launch_colloc_gh_pair(const Geom &g, const double4 *pts, int npts_even, const Freq *freqs, int l0, int nl, const Mat &m,
-                                 int row0, int nrows, const double4 *tpts, const int *patch_pass, const int2 *pass_info,
-                                 const int4 *pass_faces, const int *patch_verts, int npatches, cd *UG, cd *UH, long long ld,
+hipError_t launch_colloc_gh_patch(const Geom &g, const double4 *pts, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
+                                 int row0, int nrows, const double4 *tpts, const int *patch_chunk, const int4 *chunk_info,
+                                 const int4 *chunk_faces, const int *patch_verts, int npatches, cd *UG, cd *UH, long long ld,
                                  long long lstride, hipStream_t st, const Bands &bands = Bands{});
-int pair_patch_size();
-int pair_pass_faces();
+int patch_size();       // vertex slots per patch
+int chunk_face_count();  // faces per chunk
+int patch_rows_per_tile(long long tiles);  // rows per block for a job of `tiles` (patch, frequency, row) tiles
 
-// One object's row slab in a multi-object launch of the pair kernel (collocation rows row0..row0+nrows-1 at all
-// nl frequencies of `freqs`): its npatches x nl x nrows tiles are numbered base .. base + npatches nl nrows - 1.
+// One object's row slab in a multi-object launch of the patch kernel (collocation rows row0..row0+nrows-1 at all
+// nl frequencies of `freqs`): its npatches x nl x ceil(nrows / rpt) tiles of rpt rows are numbered from base.
 struct ScenePiece {
     Geom g;
     const double4 *pts;
-    int nrounds;  // padded rule points / 2
+    int npts;
     const Freq *freqs;
     Mat m;
-    int row0, nrows, nl, npatches;
-    const int *patch_pass;
-    const int2 *pass_info;
-    const int4 *pass_faces;
+    int row0, nrows, rpt, nl, npatches;
+    const int *patch_chunk;
+    const int4 *chunk_info;
+    const int4 *chunk_faces;
     const int *patch_verts;
     cd *UG, *UH;
     long long ld, lstride;
@@ -81,7 +82,7 @@ struct ScenePiece {
 };
 // The pieces (device array, ascending base, all with the same G / H selection) in one persistent launch of
 // min(ntiles, 2 blocks per CU) blocks that take tiles from *counter (zeroed by the launcher with a kernel).
-hipError_t launch_scene_gh_pair(const ScenePiece *pieces, int npieces, long long ntiles, unsigned *counter, bool G, bool H,
+hipError_t launch_scene_gh(const ScenePiece *pieces, int npieces, long long ntiles, unsigned *counter, bool G, bool H,
                                 int num_cus, hipStream_t st);
 hipError_t launch_colloc_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
                            int row0, int nrows, cd *Bt, cd *Ba, hipStream_t st, const FaceBands &fb = FaceBands{});

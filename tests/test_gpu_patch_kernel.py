@@ -1,0 +1,83 @@
+"""The patch kernel of the regular-face G and H against the star kernel (CQBEM_COLLOC_KERNEL=star: one lane per column
+vertex, every face evaluated once per corner, another formulation of the same sums) where the patch kernel's work
+division changes: face counts at the edges of a 64-face chunk, of 1, 2 and several chunks per patch (a chunk shared by
+4, 2 or 1 waves), of several patches, and rules of 1 to 63 points; every face touching the row point; and several rows
+per block with a ragged last group.
+
+Tolerances.  One Laplace-domain matrix: each point's entries carry some 30 roundings of 1.1e-16 and a cancellation
+between the two waves' terms of at most 1/|z|^2 ~ 1e2, i.e. 4e-13 of the entry; 1e-12 of the matrix norm.  Weights:
+the inverse transform multiplies that by up to R^-(L-1) ~ 1e5 on weights that are small beside the first ones, over
+sums of Lf terms with independent errors; 1e-8 of the stack's norm."""
+import numpy as np
+import pytest
+
+from surfaceonlydeformables_amd import abi
+from surfaceonlydeformables_amd import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = abi.Context(0)
+    yield c
+    c.close()
+
+
+def sphere_with(nf):
+    """A closed mesh of nf faces (nf even), of about unit-ratio triangles."""
+    if nf == 4:
+        V = np.array([(1, 1, 1), (1, -1, -1), (-1, 1, -1), (-1, -1, 1)], float) * 0.1
+        return V, np.array([(0, 1, 2), (0, 3, 1), (0, 2, 3), (1, 3, 2)], np.int32)
+    level = 1
+    while 20 * 4 ** level < nf:
+        level += 1
+    V, F = M.icosphere(level, 0.2)
+    V = M.jitter(V, F, 0.01, nf)
+    return (V, F) if len(F) == nf else abi.decimate_mesh(V, F, nf)
+
+
+def params(L, order, sub, which=abi.G | abi.H, bdf=abi.BDF2):
+    _, c1, c2 = M.material_speeds(3e5, 0.33, 1000.0)
+    return abi.make_params(c1, c2, 1000.0, 0.33, 0.4 / (c2 * max(L - 2, 4)), 1e-10 ** (1 / (2 * L)), L, bdf=bdf, order=order,
+                           subdivision=sub, which=which)
+
+
+def off(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("nf,order,sub", [(4, 5, 2), (20, 5, 2), (62, 5, 1), (64, 5, 2), (66, 4, 2), (126, 1, 1), (128, 5, 2),
+                                          (130, 2, 1), (192, 3, 2), (258, 5, 2), (512, 5, 3), (520, 5, 2), (1100, 4, 1)])
+def test_one_frequency_against_the_star_kernel(ctx, monkeypatch, nf, order, sub):
+    V, F = sphere_with(nf)
+    assert len(F) == nf
+    V = M.center(V, F)
+    mesh, L = abi.make_mesh(V, F), 16
+    for which in (abi.G | abi.H, abi.G, abi.H):
+        p = params(L, order, sub, which)
+        for l in (0, 5):
+            print(f"patch kernel nf={nf} rule {order}x{sub} which={which} l={l}", flush=True)
+            monkeypatch.delenv("CQBEM_COLLOC_KERNEL", raising=False)
+            got = ctx.laplace(mesh, p, l)
+            monkeypatch.setenv("CQBEM_COLLOC_KERNEL", "star")
+            want = ctx.laplace(mesh, p, l)
+            for k in "UP":
+                assert (got[k] is None) == (want[k] is None)
+                if got[k] is not None:
+                    assert off(got[k], want[k]) <= 1e-12, k
+
+
+@pytest.mark.parametrize("nf,L", [(1280, 64), (1276, 61)])
+def test_rows_per_block_against_the_star_kernel(ctx, monkeypatch, nf, L):
+    """3 patches x 33 or 31 frequencies x 640-odd rows: 7 rows per block, the last group ragged."""
+    V, F = sphere_with(nf)
+    V = M.center(V, F)
+    mesh, p = abi.make_mesh(V, F), params(L, 2, 1)
+    print(f"patch kernel rows per block nf={nf} L={L}", flush=True)
+    monkeypatch.delenv("CQBEM_COLLOC_KERNEL", raising=False)
+    got = ctx.assemble(mesh, p, want=("G", "H"))
+    monkeypatch.setenv("CQBEM_COLLOC_KERNEL", "star")
+    want = ctx.assemble(mesh, p, want=("G", "H"))
+    for k in "GH":
+        assert off(got[k], want[k]) <= 1e-8, k
