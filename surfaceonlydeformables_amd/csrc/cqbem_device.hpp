@@ -450,16 +450,4 @@ __device__ inline void b_coef(const Expo &E, double ir, double ir2, const Freq &
     u3 = E.e2 * f.is * (m.ic2 * kInv4Pi);
 }
 
-// b_coef times 8 pi: t1, u1 and u12 without their factor 1/(8 pi), t2 and u3 without 1/(4 pi) but doubled (exact), so
-// that every sum of them takes the one factor 1/(8 pi) at its end.
-__device__ inline void b_coef_8pi(const Expo &E, double ir, double ir2, const Freq &f, const Mat &m, cd &t1, cd &t2,
-                                  cd &u1, cd &u12, cd &u3) {
-    t1 = E.dA * ir2;
-    t2 = (E.A2 - f.is2) * (2.0 * ir2);
-    u1 = E.dA * ir;
-    const cd u2 = ((E.e2 * m.ic2) - (E.e1 * m.ic1)) * f.is;
-    u12 = u1 + u2;
-    u3 = E.e2 * f.is * (2.0 * m.ic2);
-}
-
 }  // namespace cqbem

@@ -496,12 +496,21 @@ __global__ void k_zero_counter(unsigned *counter) {
 // ------------------------------------------------------------------------
 // B_trans and B_angular, regular faces.  Grid: (nl, rows), 256 threads; lanes
 // stride over the faces, then a wave shuffle reduction and one LDS pass.
+//
+// Bound by FP64 VALU issue.  A point adds to 12 complex moments of its face
+// (h, n.h, h h and two scalars, each times a function of r and s); every factor
+// that depends on the frequency alone (1/s^2, s, 1/s) waits until the face's
+// or the row's end, and the trace of the h h moment serves as the scalar moment
+// of the same function (|h| = 1).  156 instructions per point; with the factors
+// applied per point it was 203.  Icosphere level 4, L = 32: 34.0 ms (43.0).
 // ------------------------------------------------------------------------
 constexpr int kBWords = 48;  // B_trans (6 sym complex) + B_angular (18 complex), as doubles
 
 // GAL: the rows are test points tpts[row0 + y] (x, y, z, face) whose face's corners are excluded, written to
 // rows 3y..3y+2 of an nv3-row buffer; otherwise collocation vertex i = row0 + y, written to rows 3i..3i+2.
-template <bool GAL>
+// BANDED: each face takes the far rule or the reference rule (a lane then reads its own rule's points; without bands
+// they are wave-uniform).
+template <bool GAL, bool BANDED>
 __global__ void __launch_bounds__(256) k_colloc_b(Geom g, const double4 *__restrict__ quad, int npts,
                                                    const Freq *__restrict__ freqs, int l0, Mat m, int row0,
                                                    const double4 *__restrict__ tpts, cd *__restrict__ Bt,
@@ -513,18 +522,18 @@ __global__ void __launch_bounds__(256) k_colloc_b(Geom g, const double4 *__restr
     const int l = blockIdx.x;
     const int i = row0 + blockIdx.y;
     const Freq f = freqs[l0 + l];
-    double x0, x1, x2;
+    double x[3];
     int t[3] = {i, i, i};
     if (GAL) {
         const double4 T = tpts[i];
-        x0 = T.x, x1 = T.y, x2 = T.z;
+        x[0] = T.x, x[1] = T.y, x[2] = T.z;
         const int f1 = (int)T.w;
         t[0] = g.F[3 * f1], t[1] = g.F[3 * f1 + 1], t[2] = g.F[3 * f1 + 2];
     } else {
-        x0 = g.V[3 * i], x1 = g.V[3 * i + 1], x2 = g.V[3 * i + 2];
+        x[0] = g.V[3 * i], x[1] = g.V[3 * i + 1], x[2] = g.V[3 * i + 2];
     }
     const int io = GAL ? (int)blockIdx.y : i;
-    cd bt[6], ba[18];
+    cd bt[6], ba[18];  // the row's sums in units of 1/(8 pi s^2)
 #pragma unroll
     for (int k = 0; k < 6; k++) bt[k] = cd{0, 0};
 #pragma unroll
@@ -535,57 +544,75 @@ __global__ void __launch_bounds__(256) k_colloc_b(Geom g, const double4 *__restr
         for (int k = 0; k < (GAL ? 3 : 1); k++)
             touch = touch || same_vertex(g, t[k], a0) || same_vertex(g, t[k], a1) || same_vertex(g, t[k], a2);
         if (touch) continue;
-        const double *p0 = g.V + 3 * a0, *p1 = g.V + 3 * a1, *p2 = g.V + 3 * a2;
+        // y - x = o + b1 e1 + b2 e2, whose component along the normal is the same at every point
+        double o[3], e1[3], e2[3];
         const double n[3] = {g.N[3 * fc], g.N[3 * fc + 1], g.N[3 * fc + 2]};
-        const double ar = g.area[fc];
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            o[k] = g.V[3 * a0 + k] - x[k], e1[k] = g.V[3 * a1 + k] - g.V[3 * a0 + k], e2[k] = g.V[3 * a2 + k] - g.V[3 * a0 + k];
         const double4 *qf = quad;  // the face's rule
         int nq = npts;
-        if (fb.sphere && beyond_sphere(x0, x1, x2, fb.sphere[fc])) qf = fb.far_quad, nq = fb.far_npts;
+        if (BANDED && beyond_sphere(x[0], x[1], x[2], fb.sphere[fc])) qf = fb.far_quad, nq = fb.far_npts;
         cd mt[3] = {{0, 0}, {0, 0}, {0, 0}}, m2 = {0, 0}, M[6], S = {0, 0}, S3 = {0, 0};
 #pragma unroll
         for (int k = 0; k < 6; k++) M[k] = cd{0, 0};
+#pragma unroll 1
         for (int q = 0; q < nq; ++q) {
-            const double4 Q = qf[q];
-            const double r0 = Q.x * p0[0] + Q.y * p1[0] + Q.z * p2[0] - x0;
-            const double r1 = Q.x * p0[1] + Q.y * p1[1] + Q.z * p2[1] - x1;
-            const double r2 = Q.x * p0[2] + Q.y * p1[2] + Q.z * p2[2] - x2;
-            const double d2 = r0 * r0 + r1 * r1 + r2 * r2;
-            const double ir = rsqrt_nr(d2), r = d2 * ir, ir2 = ir * ir;
-            const double h[3] = {r0 * ir, r1 * ir, r2 * ir};
-            const double w = Q.w * ar;
-            const Expo E = expo(r, f, &mtab);
-            cd t1, t2, u1, u12, u3;
-            b_coef_8pi(E, ir, ir2, f, m, t1, t2, u1, u12, u3);  // 1/(8 pi) at the write-out
-            const double rn = h[0] * n[0] + h[1] * n[1] + h[2] * n[2];
-            t1 = t1 * w;
-            u1 = u1 * w;
+            double b1, b2, w;
+            if (BANDED) {
+                const double4 Q = qf[q];
+                b1 = Q.y, b2 = Q.z, w = Q.w;
+            } else {
+                const_double *Q = as_const(quad + q);
+                b1 = Q[1], b2 = Q[2], w = Q[3];
+            }
+            double d[3];
 #pragma unroll
-            for (int a = 0; a < 3; a++) fma_cr(mt[a], t1, h[a]);
-            fma_cr(m2, t2, w * rn);
+            for (int k = 0; k < 3; k++) d[k] = fma(b1, e1[k], fma(b2, e2[k], o[k]));
+            const double d2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+            const double ir = rsqrt_h3(d2), r = d2 * ir;
+            const cd z1 = f.sc1 * r, z2 = f.sc2 * r;
+            const cd E1 = cexp_neg_tab(z1, &mtab), E2 = cexp_neg_tab(z2, &mtab);
+            const cd s2 = z2 * E2 + E2, dS = (z1 * E1 + E1) - s2;  // s^2 A2, s^2 (A1 - A2)
+            const double w2 = (w * ir) * ir, w3 = w2 * ir;
+            const double h[3] = {w3 * d[0], w3 * d[1], w3 * d[2]};  // w h / r^2
 #pragma unroll
-            for (int a = 0; a < 3; a++)
+            for (int a = 0; a < 3; a++) {
+                fma_cr(mt[a], dS, h[a]);
 #pragma unroll
-                for (int b = a; b < 3; b++) fma_cr(M[sidx(a, b)], u1, h[a] * h[b]);
-            fma_cr(S, u12, w);
-            fma_cr(S3, u3, w);
+                for (int b = a; b < 3; b++) fma_cr(M[sidx(a, b)], dS, h[a] * d[b]);  // w h h / r
+            }
+            fma_cr(m2, cd{s2.x - 1.0, s2.y}, w3);
+            const cd v = E2 * m.ic2;
+            cd u = v;
+            fma_cr(u, E1, -m.ic1);
+            fma_cr(S, u, w);
+            fma_cr(S3, v, w);
         }
+        // the face's moments in units of area/s^2; m2 still lacks the normal component of y - x
+        const double ar = g.area[fc], rn = o[0] * n[0] + o[1] * n[1] + o[2] * n[2];
+        m2 = m2 * (2.0 * rn * ar);
+        S = (S * f.s + (M[0] + M[1] + M[2])) * ar, S3 = S3 * f.s * (2.0 * ar);
+#pragma unroll
+        for (int k = 0; k < 3; k++) mt[k] = mt[k] * ar;
+#pragma unroll
+        for (int k = 0; k < 6; k++) M[k] = M[k] * ar;
+#pragma unroll
+        for (int k = 0; k < 3; k++) M[k] += S;  // M_ak + S d_ak: both meet the same normal below
 #pragma unroll
         for (int a = 0; a < 3; a++)
 #pragma unroll
             for (int b = a; b < 3; b++) {
-                cd v = {0, 0};
+                cd &v = bt[sidx(a, b)];
                 fma_cr(v, mt[a], n[b]);
                 fma_cr(v, mt[b], n[a]);
                 if (a == b) v += m2;
-                bt[sidx(a, b)] += v;
 #pragma unroll
                 for (int k = 0; k < 3; k++) {
-                    cd u = {0, 0};
+                    cd &u = ba[sidx(a, b) * 3 + k];
                     fma_cr(u, M[sidx(a, k)], n[b]);
                     fma_cr(u, M[sidx(b, k)], n[a]);
-                    fma_cr(u, S, (b == k ? n[a] : 0.0) + (a == k ? n[b] : 0.0));
                     if (a == b) fma_cr(u, S3, n[k]);
-                    ba[sidx(a, b) * 3 + k] += u;
                 }
             }
     }
@@ -601,9 +628,11 @@ __global__ void __launch_bounds__(256) k_colloc_b(Geom g, const double4 *__restr
     __syncthreads();
     if (threadIdx.x < kBWords) {
         const int k = threadIdx.x;
-        const double v = ((red[0][k] + red[1][k]) + (red[2][k] + red[3][k])) * kInv8Pi;
+        const int c = k & 1, e0 = k & ~1;
+        auto total = [&](int j) { return (red[0][j] + red[1][j]) + (red[2][j] + red[3][j]); };
+        const cd sum = cd{total(e0), total(e0 + 1)} * f.is2;
+        const double v = (c ? sum.y : sum.x) * kInv8Pi;
         // scatter the packed symmetric entries to their full positions
-        const int c = k & 1;
         if (k < 12) {
             const int e = k >> 1;
             double *bt_out = reinterpret_cast<double *>(Bt + (long long)l * nv3 * 3 + (long long)(3 * io) * 3);
@@ -1325,15 +1354,19 @@ int chunk_face_count() { return 64; }
 hipError_t launch_colloc_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
                            int row0, int nrows, cd *Bt, cd *Ba, hipStream_t st, const FaceBands &fb) {
     if (nrows <= 0 || nrows > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_colloc_b<false>, dim3(nl, nrows), dim3(256), 0, st, g, quad, npts, freqs, l0, m, row0,
-                       (const double4 *)nullptr, Bt, Ba, 3LL * g.nv, fb);
+    if (fb.sphere)
+        hipLaunchKernelGGL((k_colloc_b<false, true>), dim3(nl, nrows), dim3(256), 0, st, g, quad, npts, freqs, l0, m, row0,
+                           (const double4 *)nullptr, Bt, Ba, 3LL * g.nv, fb);
+    else
+        hipLaunchKernelGGL((k_colloc_b<false, false>), dim3(nl, nrows), dim3(256), 0, st, g, quad, npts, freqs, l0, m, row0,
+                           (const double4 *)nullptr, Bt, Ba, 3LL * g.nv, fb);
     return hipGetLastError();
 }
 
 hipError_t launch_points_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
                            const double4 *tpts, int row0, int nrows, cd *Bt, cd *Ba, long long out_rows, hipStream_t st) {
     if (nrows <= 0 || nrows > 65535 || 3LL * nrows > out_rows) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_colloc_b<true>, dim3(nl, nrows), dim3(256), 0, st, g, quad, npts, freqs, l0, m, row0, tpts, Bt, Ba,
+    hipLaunchKernelGGL((k_colloc_b<true, false>), dim3(nl, nrows), dim3(256), 0, st, g, quad, npts, freqs, l0, m, row0, tpts, Bt, Ba,
                        out_rows, FaceBands{});
     return hipGetLastError();
 }
