@@ -250,6 +250,13 @@ __device__ inline cd cexp_neg(cd z) {
     return cd{m * cs, -m * sn};
 }
 
+// Tables that no kernel writes, read through the constant address space: uniform indices become scalar loads also where
+// the pointer itself came from memory (scenes).
+typedef const __attribute__((address_space(4))) double const_double;
+typedef const __attribute__((address_space(4))) int const_int;
+__device__ inline const_double *as_const(const double4 *p) { return (const_double *)p; }
+__device__ inline const_int *as_const(const int4 *p) { return (const_int *)p; }
+
 // Per-frequency constants, uniform across a wavefront (loaded with scalar loads).
 struct Freq {
     cd s;    // s_l

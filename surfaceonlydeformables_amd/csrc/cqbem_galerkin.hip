@@ -289,10 +289,7 @@ template <int MODE> struct SingAcc {
     cd v[MODE == 0 ? 63 : (MODE == 1 ? 81 : 36)];
 };
 
-// MIRROR (B of a coincident pair integrated over regions 1, 3, 5): the point also stands for its exchanged image,
-// whose test weight is Ly; the odd terms (t1 rh, t2 rh.n) change sign there and the even ones (u1 rh rh, u12, u3) do
-// not, so they take the weights wt (Lx - Ly) and wt (Lx + Ly).
-template <int MODE, bool MIRROR = false>
+template <int MODE>
 __device__ __forceinline__ void sing_eval(const double x[3], const double y[3], const double Lx[3], const double Ly[3], double wt,
                                  const double n[3], const Freq &f, const Mat &m, const MathTables *M, cd *acc) {
     const double r0 = y[0] - x[0], r1 = y[1] - x[1], r2 = y[2] - x[2];
@@ -346,19 +343,18 @@ __device__ __forceinline__ void sing_eval(const double x[3], const double y[3], 
         const double rn = h[0] * n[0] + h[1] * n[1] + h[2] * n[2];
         #pragma unroll
         for (int i = 0; i < 3; i++) {
-            const double wo = MIRROR ? wt * (Lx[i] - Ly[i]) : wt * Lx[i];  // odd terms
-            const double we = MIRROR ? wt * (Lx[i] + Ly[i]) : wt * Lx[i];  // even terms
+            const double wi = wt * Lx[i];
             cd *a = acc + i * 12;
-            const cd tw = t1 * wo, uw = u1 * we;
+            const cd tw = t1 * wi, uw = u1 * wi;
             #pragma unroll
             for (int p = 0; p < 3; p++) fma_cr(a[p], tw, h[p]);
-            fma_cr(a[3], t2, wo * rn);
+            fma_cr(a[3], t2, wi * rn);
             #pragma unroll
             for (int p = 0; p < 3; p++)
                 #pragma unroll
                 for (int b = p; b < 3; b++) fma_cr(a[4 + sidx(p, b)], uw, h[p] * h[b]);
-            fma_cr(a[10], u12, we);
-            fma_cr(a[11], u3, we);
+            fma_cr(a[10], u12, wi);
+            fma_cr(a[11], u3, wi);
         }
     }
 }
@@ -395,10 +391,10 @@ __device__ __forceinline__ void region_point(int r, double e1, double e2, double
     }
 }
 
-// HALF (B of coincident pairs): regions 1, 3, 5 only, each point standing for its exchanged image as well.
+// The lane variant (CQBEM_GALERKIN_SINGULAR=lane): every region of every ordered pair, one lane per 4D rule point.
 // B (MODE 2) is held to 2 waves per SIMD: its 36 accumulators and working set take 316 registers at 1 wave; at 2 it
 // spills 46-59 of them to scratch and still runs 15% faster.  G and H (the lane variant) keep 1 wave.
-template <int MODE, int KIND, bool HALF = false>
+template <int MODE, int KIND>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 2 : 1, 2))) k_gal_sing(Geom g, const Pair *__restrict__ pairs, int pair0,
                                                   const double2 *__restrict__ line, int nline,
                                                   const Freq *__restrict__ freqs, Mat m, cd *__restrict__ out) {
@@ -440,17 +436,16 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE ==
         const int ia = p / (nline * nline * nline), ib = (p / (nline * nline)) % nline, ic = (p / nline) % nline, id = p % nline;
         const double e1 = line[ia].x, e2 = line[ib].x, e3 = line[ic].x, xi = line[id].x;
         const double w = line[ia].y * line[ib].y * line[ic].y * line[id].y;
-        static_assert(!HALF || (MODE == 2 && KIND == 1), "the exchanged half is folded in for B of coincident pairs");
-        constexpr int NR = KIND == 1 ? (HALF ? 3 : 6) : (KIND == 2 ? 5 : 2);
+        constexpr int NR = KIND == 1 ? 6 : (KIND == 2 ? 5 : 2);
 #pragma unroll 1
         for (int r = 0; r < NR; r++) {
             double a0, a1, b0, b1, wt;
-            region_point<KIND>(HALF ? 2 * r : r, e1, e2, e3, xi, w, a0, a1, b0, b1, wt);
+            region_point<KIND>(r, e1, e2, e3, xi, w, a0, a1, b0, b1, wt);
             double x[3], y[3];
             #pragma unroll
             for (int k = 0; k < 3; k++) x[k] = px[k] + dx0[k] * a0 + dx1[k] * a1, y[k] = px[k] + dy0[k] * b0 + dy1[k] * b1;
             const double Lx[3] = {1.0 - a0, a0 - a1, a1}, Ly[3] = {1.0 - b0, b0 - b1, b1};
-            sing_eval<MODE, HALF>(x, y, Lx, Ly, wt, n, f, m, &mtab, acc);
+            sing_eval<MODE>(x, y, Lx, Ly, wt, n, f, m, &mtab, acc);
         }
     }
     // wave reduction; lane 0 expands and writes
@@ -513,196 +508,450 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE ==
 }
 
 // ---------------------------------------------------------------------------
-// Touching pairs, G and H, quad form.  The 9 (test corner i, source corner j) basis pairs of a point
-// pair need 63 (G) or 81 (H) complex accumulators when one lane takes all of them, which spills.  Here
-// the four lanes of a quad each evaluate their own point, pass the point's kernel data around the quad
-// (three DPP rotations), and each lane accumulates only its basis pairs c = q, q + 4, q + 8 over all four
-// points.  The quads' partial sums are added across the wavefront at the end.
+// Touching pairs, direction form.  Every Sauter-Schwab map scales with its last coordinate xi: both faces' points are
+// xi times a point that depends on the other three, so along xi the direction of y - x is constant, r = xi |d|, and
+// the basis products Lx_i Ly_j are polynomials of degree 2 in xi.  A lane takes one direction (e1, e2, e3, region),
+// sums the functions e^-z1, e^-z2 and s^2 (A1 - A2) times the needed powers of xi over the xi rule (24 or 18 FMAs per
+// point), and only then, once per direction, forms the kernel entries and multiplies them by the basis.  With the
+// reduced basis {1, Lx1, Lx2} x {1, Ly1, Ly2} (Lx0 = 1 - Lx1 - Lx2 is restored at the end) every product has a single
+// power of xi: T_0 for 1, T_1 for the four linear ones, T_2 for the four quadratic ones.  The two sets of four are the
+// rows of 4x4x4 FP64 matrix products: lane (j, b, k) = j + 4 b + 16 k holds item j's entry at direction (b, k) as the
+// B operand and row j's basis value at that direction as the A operand, which is the same for every item, since the
+// basis depends on the rule alone.  An item is a (pair, frequency); a wave works on four items and 16 directions.
+// The entries are those of the source face's frame (see FaceFrame).
+// Bound by FP64 VALU issue: 117 instructions per point for vertex-adjacent pairs and B, 190 where r is formed from
+// coordinates (touch_distance), and 450 to 700 per direction of n points; the per-point kernels took about 430 (G),
+// 520 (H) and 280 (B) per point and formed all 9 basis products at each.  Icosphere level 3, L = 32, rule 5 x 2 (n = 10):
+// all touching pairs 352 -> 101 ms.
 // ---------------------------------------------------------------------------
-template <int D> __device__ inline double quad_rot(double v) {  // lane q receives lane (q + D) mod 4's value
-    constexpr int sel = ((0 + D) & 3) | (((1 + D) & 3) << 2) | (((2 + D) & 3) << 4) | (((3 + D) & 3) << 6);
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)b, sel, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), sel, 0xF, 0xF, false);
-    return __longlong_as_double(((long long)(unsigned)hi << 32) | (unsigned)lo);
+constexpr int kTouchXi = 8;      // words of the xi table per point: xi, w / xi, w, w xi, .., w xi^4, -
+constexpr int kTouchMaxLine = 80;
+
+// The xi table of a composite rule of n points, and after it the sums of w xi and w xi^2.
+__global__ void k_gal_xi(const double2 *__restrict__ line, int n, double *__restrict__ tab) {
+    const int q = threadIdx.x;
+    if (q < n) {
+        const double xi = line[q].x, w = line[q].y;
+        double *t = tab + kTouchXi * q;
+        t[0] = xi, t[1] = w / xi, t[2] = w, t[3] = w * xi, t[4] = w * xi * xi, t[5] = w * xi * xi * xi, t[6] = w * xi * xi * xi * xi;
+        t[7] = 0.0;
+    }
+    if (q == 0) {
+        double k0 = 0, k1 = 0;
+        for (int k = 0; k < n; k++) k0 += line[k].y * line[k].x, k1 += line[k].y * line[k].x * line[k].x;
+        tab[kTouchXi * n] = k0, tab[kTouchXi * n + 1] = k1;
+    }
 }
 
-// Kernel data of one point pair.  G: alpha/r, beta/r, the 6 products rh_a rh_b; H: the 9 entries of p_hat.
-// Then Lx[3], Ly[3] and the weight.
-template <int MODE> struct QuadK {
-    static constexpr int NK = MODE == 0 ? 10 : 18;
-    double v[NK + 7];
+// One item's constants, in the LDS: the edges in the source face's frame (y's lie in its plane), the frequency and the
+// rotation back.
+struct TouchItem {
+    double dx0[3], dx1[3], dy0[2], dy1[2];
+    cd sc1, sc2, is2, is, s;
+    double Q[3][3], jac;
+    double px[3], gx0[3], gx1[3], gy0[3], gy1[3];  // the shared vertex and the edges in the global axes
 };
 
-template <int MODE>
-__device__ __forceinline__ void quad_point(const double x[3], const double y[3], const double Lx[3], const double Ly[3], double wt,
-                                           const double n[3], const Freq &f, const Mat &m, const MathTables *M,
-                                           QuadK<MODE> &K) {
+// Fills item `it` (clamped to the last) of the pairs from pair0 on; called by one lane per item.
+template <int KIND>
+__device__ inline void load_item(const Geom &g, const Pair *__restrict__ pairs, const Freq *__restrict__ freqs, long long it,
+                                 int pair0, int nl, TouchItem &I) {
+    const Pair P = pairs[pair0 + (int)(it / nl)];
+    const Freq f = freqs[(int)(it % nl)];
+    const double *A = g.V + 3 * P.j1[0], *B = g.V + 3 * P.j1[1], *C = g.V + 3 * P.j1[2];
+    const double *Y1 = KIND == 3 ? g.V + 3 * P.j2[1] : B, *Y2 = KIND == 1 ? C : g.V + 3 * P.j2[2];
+    double dx0[3], dx1[3], dy0[3], dy1[3];
+    for (int k = 0; k < 3; k++) dx0[k] = B[k] - A[k], dx1[k] = C[k] - B[k], dy0[k] = Y1[k] - A[k], dy1[k] = Y2[k] - Y1[k];
+    auto area2 = [](const double *u, const double *v) {
+        const double c[3] = {u[1] * v[2] - u[2] * v[1], u[2] * v[0] - u[0] * v[2], u[0] * v[1] - u[1] * v[0]};
+        return sqrt(c[0] * c[0] + c[1] * c[1] + c[2] * c[2]);
+    };
+    I.jac = area2(dx0, dx1) * area2(dy0, dy1);
+    const double il = 1.0 / sqrt(dy0[0] * dy0[0] + dy0[1] * dy0[1] + dy0[2] * dy0[2]);
+    double n[3], t1[3], t2[3];
+    for (int k = 0; k < 3; k++) n[k] = g.N[3 * P.f2 + k], t1[k] = dy0[k] * il;
+    for (int k = 0; k < 3; k++) t2[k] = n[(k + 1) % 3] * t1[(k + 2) % 3] - n[(k + 2) % 3] * t1[(k + 1) % 3];
+    auto dot = [](const double *u, const double *v) { return u[0] * v[0] + u[1] * v[1] + u[2] * v[2]; };
+    I.dx0[0] = dot(dx0, t1), I.dx0[1] = dot(dx0, t2), I.dx0[2] = KIND == 3 ? dot(dx0, n) : 0.0;
+    I.dx1[0] = dot(dx1, t1), I.dx1[1] = dot(dx1, t2), I.dx1[2] = KIND == 1 ? 0.0 : dot(dx1, n);
+    I.dy0[0] = dot(dy0, t1), I.dy0[1] = dot(dy0, t2), I.dy1[0] = dot(dy1, t1), I.dy1[1] = dot(dy1, t2);
+    I.sc1 = f.sc1, I.sc2 = f.sc2, I.is2 = f.is2, I.is = f.is, I.s = f.s;
+    for (int k = 0; k < 3; k++) I.px[k] = A[k], I.gx0[k] = dx0[k], I.gx1[k] = dx1[k], I.gy0[k] = dy0[k], I.gy1[k] = dy1[k];
+    for (int k = 0; k < 3; k++) I.Q[0][k] = t1[k], I.Q[1][k] = t2[k], I.Q[2][k] = n[k];
+}
+
+// What the directions of one lane keep in the LDS while the xi rule runs: 1/|d|, the direction (a, b, c), the direction's
+// weight, the A operands of the linear and the quadratic basis, |d| and (e1, e2, e3).
+struct TouchDir {
+    double2 id_a, bc, wA1, A2_len, e12, e3_;
+};
+
+// Direction dd (0 .. n^3 - 1) of region r for a lane of item I: z_k at xi = 1, and the rest into D.  A direction past
+// the end has weight 0.
+template <int KIND>
+__device__ __forceinline__ void touch_direction(int r, int dd, int nline, const double2 *line, const TouchItem &I, int row,
+                                                cd &zd1, cd &zd2, TouchDir &D) {
+    const int n2 = nline * nline, nd = n2 * nline, p = min(dd, nd - 1);
+    const int ia = p / n2, ib = (p - ia * n2) / nline, ic = p - ia * n2 - ib * nline;
+    const double2 la = line[ia], lb = line[ib], lc = line[ic];
+    double a0, a1, b0, b1, wt;
+    region_point<KIND>(r, la.x, lb.x, lc.x, 1.0, dd < nd ? la.y * lb.y * lc.y : 0.0, a0, a1, b0, b1, wt);
+    double d[3];
+#pragma unroll
+    for (int k = 0; k < 2; k++) d[k] = fma(I.dy0[k], b0, I.dy1[k] * b1) - fma(I.dx0[k], a0, I.dx1[k] * a1);
+    d[2] = -fma(I.dx0[2], a0, I.dx1[2] * a1);
+    const double d2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+    const double id = rsqrt_nr(d2), len = d2 * id;
+    zd1 = I.sc1 * len, zd2 = I.sc2 * len;
+    const double x1 = a0 - a1, x2 = a1, y1 = b0 - b1, y2 = b1;
+    const double A1 = row < 2 ? (row == 0 ? x1 : x2) : (row == 2 ? y1 : y2);
+    const double A2 = (row < 2 ? x1 : x2) * (row & 1 ? y2 : y1);
+    D.id_a = make_double2(id, d[0] * id), D.bc = make_double2(d[1] * id, d[2] * id), D.wA1 = make_double2(wt, wt * A1);
+    D.A2_len = make_double2(wt * A2, len), D.e12 = make_double2(la.x, lb.x), D.e3_ = make_double2(lc.x, 0.0);
+}
+
+// |y - x| at one point of the rule, from the points' coordinates in the global axes.  Coincident and edge-adjacent
+// pairs have rule points so close that the rounding of z = s r / c decides, through the exponentials, the last digits
+// of what is left of A1 - A2, different at every frequency; the late weights amplify those digits by R^-n.  Their r is
+// therefore formed with the roundings of the per-point kernels.
+template <int KIND>
+__device__ __forceinline__ double touch_distance(int region, const TouchDir &D, double xi, const TouchItem &I) {
+    double a0, a1, b0, b1, wt, x[3], y[3];
+    region_point<KIND>(region, D.e12.x, D.e12.y, D.e3_.x, xi, 1.0, a0, a1, b0, b1, wt);
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        x[k] = I.px[k] + I.gx0[k] * a0 + I.gx1[k] * a1, y[k] = I.px[k] + I.gy0[k] * b0 + I.gy1[k] * b1;
     const double r0 = y[0] - x[0], r1 = y[1] - x[1], r2 = y[2] - x[2];
     const double d2 = r0 * r0 + r1 * r1 + r2 * r2;
-    const double ir = rsqrt_nr(d2), r = d2 * ir, ir2 = ir * ir;
-    const double h[3] = {r0 * ir, r1 * ir, r2 * ir};
-    const Expo E = expo(r, f, M);
-    if (MODE == 0) {
-        cd al, be;
-        g_coef(E, ir, ir2, m, al, be);
-        al = al * ir, be = be * ir;
-        K.v[0] = al.x, K.v[1] = al.y, K.v[2] = be.x, K.v[3] = be.y;
-        K.v[4] = h[0] * h[0], K.v[5] = h[1] * h[1], K.v[6] = h[2] * h[2];
-        K.v[7] = h[0] * h[1], K.v[8] = h[0] * h[2], K.v[9] = h[1] * h[2];
-    } else {
-        cd c1, c2, c4;
-        h_coef(E, ir, ir2, f, m, c1, c2, c4);
-        const double rn = h[0] * n[0] + h[1] * n[1] + h[2] * n[2];
-#pragma unroll
-        for (int p = 0; p < 3; p++)
-#pragma unroll
-            for (int b = 0; b < 3; b++) {
-                cd v = c1 * (h[p] * n[b]);
-                fma_cr(v, c2, n[p] * h[b] + (p == b ? rn : 0.0));
-                fma_cr(v, c4, rn * h[p] * h[b]);
-                K.v[2 * (p * 3 + b)] = v.x, K.v[2 * (p * 3 + b) + 1] = v.y;
-            }
-    }
-    constexpr int o = QuadK<MODE>::NK;
-#pragma unroll
-    for (int k = 0; k < 3; k++) K.v[o + k] = Lx[k], K.v[o + 3 + k] = Ly[k];
-    K.v[o + 6] = wt;
+    return d2 * rsqrt_nr(d2);
 }
 
-__device__ __forceinline__ double pick3(const double *a, int i) { return i == 0 ? a[0] : (i == 1 ? a[1] : a[2]); }
-
-template <int MODE>
-__device__ __forceinline__ void quad_acc(const QuadK<MODE> &K, const int ci[3], const int cj[3], const double cv[3],
-                                         cd (*acc)[MODE == 0 ? 7 : 9]) {
-    constexpr int o = QuadK<MODE>::NK;
-#pragma unroll
-    for (int s = 0; s < 3; s++) {
-        const double w = K.v[o + 6] * pick3(K.v + o, ci[s]) * pick3(K.v + o + 3, cj[s]) * cv[s];
-        if (MODE == 0) {
-            const cd aw = cd{K.v[0], K.v[1]} * w;
-#pragma unroll
-            for (int e = 0; e < 6; e++) fma_cr(acc[s][e], aw, K.v[4 + e]);
-            fma_cr(acc[s][6], cd{K.v[2], K.v[3]}, w);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 9; e++) fma_cr(acc[s][e], cd{K.v[2 * e], K.v[2 * e + 1]}, w);
-        }
-    }
+__device__ inline void mfma_acc(cd &acc, double A, const cd &T) {
+    acc.x = __builtin_amdgcn_mfma_f64_4x4x4f64(A, T.x, acc.x, 0, 0, 0);
+    acc.y = __builtin_amdgcn_mfma_f64_4x4x4f64(A, T.y, acc.y, 0, 0, 0);
 }
 
-// HALF (coincident pairs only): regions 1, 3, 5 of the six, whose exchanged images are the other three; the
-// exchanged half is added afterwards by k_gal_coincident_sym.
-template <int MODE, int KIND, bool HALF = false>
-__global__ void __launch_bounds__(64) k_gal_sing_quad(Geom g, const Pair *__restrict__ pairs, int pair0,
-                                                      const double2 *__restrict__ line, int nline,
-                                                      const Freq *__restrict__ freqs, Mat m, cd *__restrict__ out) {
-    constexpr int NE = MODE == 0 ? 7 : 9;
-    const int pi = pair0 + blockIdx.x, l = blockIdx.y;
-    const Pair P = pairs[pi];
-    const Freq f = freqs[l];
-    __shared__ MathTables mtab;  // tables of the exponentials
-    load_math_tables(&mtab);
-    __syncthreads();
-    const double n[3] = {g.N[3 * P.f2], g.N[3 * P.f2 + 1], g.N[3 * P.f2 + 2]};
-    double px[3], dx0[3], dx1[3], dy0[3], dy1[3], jac;
-    {
-        const double *A = g.V + 3 * P.j1[0], *B = g.V + 3 * P.j1[1], *Cc = g.V + 3 * P.j1[2];
-        for (int k = 0; k < 3; k++) px[k] = A[k];
-        if (KIND == 1) {
-            for (int k = 0; k < 3; k++) dx0[k] = dy0[k] = B[k] - A[k], dx1[k] = dy1[k] = Cc[k] - B[k];
-        } else if (KIND == 2) {
-            const double *Y2 = g.V + 3 * P.j2[2];
-            for (int k = 0; k < 3; k++) dx0[k] = dy0[k] = B[k] - A[k], dx1[k] = Cc[k] - B[k], dy1[k] = Y2[k] - B[k];
-        } else {
-            const double *Y1 = g.V + 3 * P.j2[1], *Y2 = g.V + 3 * P.j2[2];
-            for (int k = 0; k < 3; k++) dx0[k] = B[k] - A[k], dx1[k] = Cc[k] - B[k], dy0[k] = Y1[k] - A[k], dy1[k] = Y2[k] - Y1[k];
-        }
-        const double cx[3] = {dx0[1] * dx1[2] - dx0[2] * dx1[1], dx0[2] * dx1[0] - dx0[0] * dx1[2], dx0[0] * dx1[1] - dx0[1] * dx1[0]};
-        const double cy[3] = {dy0[1] * dy1[2] - dy0[2] * dy1[1], dy0[2] * dy1[0] - dy0[0] * dy1[2], dy0[0] * dy1[1] - dy0[1] * dy1[0]};
-        jac = sqrt(cx[0] * cx[0] + cx[1] * cx[1] + cx[2] * cx[2]) * sqrt(cy[0] * cy[0] + cy[1] * cy[1] + cy[2] * cy[2]);
-    }
-    // this lane's basis pairs c = q + 4 s (c = 9..11 are empty slots)
-    const int q = threadIdx.x & 3;
-    int ci[3], cj[3];
-    double cv[3];
-    for (int s = 0; s < 3; s++) {
-        const int c = q + 4 * s;
-        cv[s] = c < 9 ? 1.0 : 0.0;
-        ci[s] = (c < 9 ? c : 0) / 3, cj[s] = (c < 9 ? c : 0) % 3;
-    }
-    cd acc[3][NE];
-    for (int s = 0; s < 3; s++)
-        for (int e = 0; e < NE; e++) acc[s][e] = cd{0, 0};
-    const int n4 = nline * nline * nline * nline;
-    const int iters = (n4 + 63) / 64;  // every lane runs the same count: the quad exchanges need all four
-    for (int itr = 0; itr < iters; ++itr) {
-        int p = threadIdx.x + 64 * itr;
-        const double pw = p < n4 ? 1.0 : 0.0;  // past the end: a repeated point with weight 0
-        if (p >= n4) p = n4 - 1;
-        const int ia = p / (nline * nline * nline), ib = (p / (nline * nline)) % nline, ic = (p / nline) % nline, id = p % nline;
-        const double e1 = line[ia].x, e2 = line[ib].x, e3 = line[ic].x, xi = line[id].x;
-        const double w = line[ia].y * line[ib].y * line[ic].y * line[id].y * pw;
-        constexpr int NR = KIND == 1 ? (HALF ? 3 : 6) : (KIND == 2 ? 5 : 2);
-#pragma unroll 1
-        for (int r = 0; r < NR; r++) {
-            double a0, a1, b0, b1, wt;
-            region_point<KIND>(HALF ? 2 * r : r, e1, e2, e3, xi, w, a0, a1, b0, b1, wt);
-            double x[3], y[3];
-            for (int k = 0; k < 3; k++) x[k] = px[k] + dx0[k] * a0 + dx1[k] * a1, y[k] = px[k] + dy0[k] * b0 + dy1[k] * b1;
-            const double Lx[3] = {1.0 - a0, a0 - a1, a1}, Ly[3] = {1.0 - b0, b0 - b1, b1};
-            QuadK<MODE> K;
-            quad_point<MODE>(x, y, Lx, Ly, wt, n, f, m, &mtab, K);
-            quad_acc<MODE>(K, ci, cj, cv, acc);
-#pragma unroll 1
-            for (int rot = 0; rot < 3; rot++) {  // the next lane's point, then the one after, then the last
+// Adds the wave's sums of NC entries into the block's Phi[item][basis product][entry] (wave 0 stores), all over the four
+// blocks of their rows: c1 and (QUAD) c2 as rows of basis products, c0 with QUAD as rows of entries (entry 4 g + i in row
+// i of c0[g]), without it as one sum per lane.  Basis products: 1, Lx1, Lx2, Ly1, Ly2, then Lx_i Ly_j.
+template <int NC, bool QUAD>
+__device__ inline void touch_reduce(const cd *c0, const cd *c1, const cd *c2, int wave, int nwaves, cd *Phi) {
+    constexpr int NB = QUAD ? 9 : 5;
+    const int lane = threadIdx.x & 63, j = lane & 3, row = lane >> 4;
+    auto sum = [&](cd v, int last) {
+        for (int o = 4; o < last; o <<= 1) v.x += __shfl_xor(v.x, o, 64), v.y += __shfl_xor(v.y, o, 64);
+        return v;
+    };
+    for (int w = 0; w < nwaves; w++) {
+        if (w == wave) {
+            auto put = [&](int basis, int e, const cd &v) {
+                cd *p = Phi + (j * NB + basis) * NC + e;
+                *p = w == 0 ? v : cd{p->x + v.x, p->y + v.y};
+            };
 #pragma unroll
-                for (int k = 0; k < QuadK<MODE>::NK + 7; k++) K.v[k] = quad_rot<1>(K.v[k]);
-                quad_acc<MODE>(K, ci, cj, cv, acc);
-            }
-        }
-    }
-    // add the 16 quads' partial sums (lanes with the same q)
-    for (int s = 0; s < 3; s++)
-        for (int e = 0; e < NE; e++) {
-            double vx = acc[s][e].x, vy = acc[s][e].y;
-            for (int o = 4; o < 64; o <<= 1) vx += __shfl_xor(vx, o, 64), vy += __shfl_xor(vy, o, 64);
-            acc[s][e] = cd{vx * jac, vy * jac};
-        }
-    if (threadIdx.x >= 4) return;
-    cd *ob = out + ((long long)pi * gridDim.y + l) * kPairStride;
-    for (int s = 0; s < 3; s++) {
-        const int c = q + 4 * s;
-        if (c >= 9) continue;
-        const int i = c / 3, j = c % 3;
-        for (int p = 0; p < 3; p++)
-            for (int b = 0; b < 3; b++) {
-                if (MODE == 0) {
-                    cd v = acc[s][sidx(p, b)];
-                    if (p == b) v += acc[s][6];
-                    ob[kPairG + (3 * i + p) * 9 + 3 * j + b] = v;
-                } else {
-                    ob[kPairH + (3 * i + p) * 9 + 3 * j + b] = acc[s][p * 3 + b] * kInv4Pi;
+            for (int e = 0; e < NC; e++) {
+                const cd s1 = sum(c1[e], 16), s2 = QUAD ? sum(c2[e], 16) : cd{0, 0};
+                if ((lane & 12) == 0) {
+                    put(1 + row, e, s1);
+                    if (QUAD) put(5 + row, e, s2);
+                }
+                if (!QUAD) {
+                    const cd s0 = sum(c0[e], 64);
+                    if (lane < 4) put(0, e, s0);
+                } else if (e % 4 == 0) {
+                    const cd s0 = sum(c0[e / 4], 16);
+                    if ((lane & 12) == 0 && e + row < NC) put(0, e + row, s0);
                 }
             }
+        }
+        __syncthreads();
     }
 }
 
-// Vertex-adjacent mirror pairs.  The rule of (f2, f1) is that of (f1, f2) with the two faces' points exchanged
-// (integrator_galerkin.hpp:190-197: region 2 is region 1 with x and y swapped; the pair list orders both
-// faces from the shared vertex), and the G kernel is even in y - x, so the G block of the mirror pair at
-// (test corner i, row p; source corner j, column b) is the primary pair's at (j, p; i, b).  One thread per
-// (mirror, frequency, entry); mirrors[k] = (mirror pair, primary pair).
-__global__ void k_gal_mirror_g(const int2 *__restrict__ mirrors, int nm, int nl, cd *__restrict__ out) {
-    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (t >= (long long)nm * nl * 81) return;
-    const int e = (int)(t % 81);
-    const long long kl = t / 81;
-    const int l = (int)(kl % nl), k = (int)(kl / nl);
-    const int2 mp = mirrors[k];
-    const int i = e / 27, p = (e / 9) % 3, j = (e % 9) / 3, b = e % 3;
-    out[((long long)mp.x * nl + l) * kPairStride + kPairG + e] =
-        out[((long long)mp.y * nl + l) * kPairStride + kPairG + (3 * j + p) * 9 + 3 * i + b];
+// HALF (coincident pairs only): regions 1, 3, 5 of the six, whose exchanged images are the other three; the exchanged
+// half is added afterwards by k_gal_coincident_sym.  NW waves share a block's four items, each taking every NW-th group
+// of 16 directions.
+template <bool DG, bool DH, int KIND, bool HALF, int NW>
+__global__ void __launch_bounds__(64 * NW, 2) k_gal_touch(Geom g, const Pair *__restrict__ pairs, int pair0, long long nitems,
+                                                          const double2 *__restrict__ line, int nline,
+                                                          const double *__restrict__ xtab, const Freq *__restrict__ freqs,
+                                                          int nl, Mat m, cd *__restrict__ out) {
+    constexpr int NG = DG ? 6 : 0, NC = NG + (DH ? 8 : 0);
+    constexpr int NR = KIND == 1 ? (HALF ? 3 : 6) : (KIND == 2 ? 5 : 2);
+    __shared__ MathTables mtab;
+    __shared__ TouchItem item[4];
+    __shared__ double2 lin[kTouchMaxLine];
+    __shared__ TouchDir dir[64 * NW];
+    __shared__ cd Phi[4 * 9 * NC];
+    constexpr bool CLOSE = KIND != 3;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const long long it0 = 4LL * blockIdx.x;
+    load_math_tables(&mtab);
+    for (int k = tid; k < nline; k += 64 * NW) lin[k] = line[k];
+    if (tid < 4) load_item<KIND>(g, pairs, freqs, it0 + tid < nitems ? it0 + tid : nitems - 1, pair0, nl, item[tid]);
+    __syncthreads();
+    const int j = lane & 3, slot = lane >> 2;
+    const int nd = nline * nline * nline;
+    const const_double *xt = (const const_double *)xtab;
+    cd c0[(NC + 3) / 4], c1[NC], c2[NC];
+#pragma unroll
+    for (int e = 0; e < NC; e++) c0[e / 4] = c1[e] = c2[e] = cd{0, 0};
+#pragma unroll 1
+    for (int r = 0; r < NR; r++) {
+        const int region = HALF ? 2 * r : r;
+#pragma unroll 1
+        for (int d0 = 16 * wave; d0 < nd; d0 += 16 * NW) {
+            cd zd1, zd2;
+            touch_direction<KIND>(region, d0 + slot, nline, lin, item[j], j, zd1, zd2, dir[tid]);
+            // moments with w xi^3: powers p of xi from kE on for e1, e2 and from -4 on for the others
+            constexpr int kE = CLOSE ? -3 : -2, nE = 2 - kE;
+            cd e1[nE], e2[nE], ds[4], da[3];
+#pragma unroll
+            for (int k = 0; k < nE; k++) e1[k] = e2[k] = cd{0, 0};
+#pragma unroll
+            for (int k = 0; k < 4; k++) ds[k] = cd{0, 0};
+#pragma unroll
+            for (int k = 0; k < 3; k++) da[k] = cd{0, 0};
+#pragma unroll 1
+            for (int q = 0; q < nline; q++) {
+                const const_double *X = xt + kTouchXi * q;
+                cd z1, z2;
+                if (CLOSE) {
+                    int jj = j;
+                    asm volatile("" : "+v"(jj));  // the item stays in the LDS
+                    const TouchItem &I = item[jj];
+                    const double len = touch_distance<KIND>(region, dir[tid], X[0], I);
+                    z1 = I.sc1 * len, z2 = I.sc2 * len;
+                } else {
+                    z1 = zd1 * X[0], z2 = zd2 * X[0];
+                }
+                const cd E1 = cexp_neg_tab(z1, &mtab), E2 = cexp_neg_tab(z2, &mtab);
+                const cd dS = CLOSE ? E1 - E2 : (z1 * E1 + E1) - (z2 * E2 + E2);
+#pragma unroll
+                for (int k = 0; k < nE; k++) fma_cr(e1[k], E1, X[5 + kE + k]), fma_cr(e2[k], E2, X[5 + kE + k]);
+#pragma unroll
+                for (int k = 0; k < 4; k++) fma_cr(ds[k], dS, X[1 + k]);
+                if (DG && KIND == 1) {  // A1 - A2
+                    const cd is2 = item[j].is2;
+                    const cd A1 = (z1 + cd{1.0, 0.0}) * E1 * is2, A2 = (z2 + cd{1.0, 0.0}) * E2 * is2, dA = A1 - A2;
+#pragma unroll
+                    for (int k = 0; k < 3; k++) fma_cr(da[k], dA, X[2 + k]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            int ln = tid;  // read back, not kept in registers across the rule
+            asm volatile("" : "+v"(ln));
+            const TouchDir D = dir[ln];
+            const double a = D.id_a.y, b = D.bc.x, c = D.bc.y;
+            PointExpo E;
+            E.ir = D.id_a.x, E.ir2 = E.ir * E.ir;
+            const TouchItem &I = item[j];
+            const cd q1 = I.is * E.ir, q2 = CLOSE ? q1 * q1 : I.is2 * E.ir2;
+            if (CLOSE) zd1 = I.sc1 * D.A2_len.y, zd2 = I.sc2 * D.A2_len.y;
+            // (A1 - A2) / r^2 times xi^p: the moment ds[p + 4] of (z1 + 1) e1 - (z2 + 1) e2 over (s |d|)^2, or, for close
+            // pairs, q (e1 / c1 - e2 / c2) + q^2 (e1 - e2) with q = 1 / (s r)
+            auto dd = [&](int p) {
+                if (!CLOSE) return ds[p + 2] * q2;
+                return (e1[p - 1 - kE] * m.ic1 - e2[p - 1 - kE] * m.ic2) * q1 + ds[p + 2] * q2;
+            };
+            const double row0[4] = {j == 0 ? D.wA1.x : 0.0, j == 1 ? D.wA1.x : 0.0, j == 2 ? D.wA1.x : 0.0, j == 3 ? D.wA1.x : 0.0};
+#pragma unroll
+            for (int mm = 0; mm < 3; mm++) {
+                cd T[NC > 0 ? NC : 1];
+                if (DG) {
+                    E.e1 = e1[mm - 1 - kE], E.e2 = e2[mm - 1 - kE];
+                    E.dd = KIND == 1 ? da[mm] * E.ir2 : dd(mm - 1);
+                    point_g(E, a, b, c, m, T);
+                }
+                if (DH) {
+                    E.e1 = e1[mm - 2 - kE], E.e2 = e2[mm - 2 - kE], E.dd = dd(mm - 2);
+                    E.w1 = zd1 * e1[mm - 1 - kE], E.w2 = zd2 * e2[mm - 1 - kE];
+                    point_h(E, a, b, c, m, T + NG);
+                }
+#pragma unroll
+                for (int e = 0; e < NC; e++) {
+                    if (mm == 0) mfma_acc(c0[e / 4], row0[e % 4], T[e]);
+                    else if (mm == 1) mfma_acc(c1[e], D.wA1.y, T[e]);
+                    else mfma_acc(c2[e], D.A2_len.x, T[e]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    touch_reduce<NC, true>(c0, c1, c2, wave, NW, Phi);
+    // one lane per (item, test corner, source corner): the corner basis from the products, then the global axes
+    if (tid >= 36 || it0 + tid / 9 >= nitems) return;
+    const int jt = tid / 9, ti = (tid % 9) / 3, tj = tid % 3;
+    const cd *ph = Phi + jt * 9 * NC;
+    const TouchItem &I = item[jt];
+    double A[3][3];
+    for (int k = 0; k < 3; k++)
+        for (int d = 0; d < 3; d++) A[k][d] = I.Q[k][d] * I.jac;
+    auto corner = [&](int e) {
+        auto p = [&](int k) { return ph[k * NC + e]; };
+        if (ti && tj) return p(2 + 2 * ti + tj);
+        if (ti) return p(ti) - p(3 + 2 * ti) - p(4 + 2 * ti);
+        if (tj) return p(2 + tj) - p(4 + tj) - p(6 + tj);
+        return (p(0) - p(1) - p(2)) - (p(3) + p(4)) + ((p(5) + p(6)) + (p(7) + p(8)));
+    };
+    const long long it = it0 + jt;
+    cd *o = out + ((long long)(pair0 + (int)(it / nl)) * nl + (int)(it % nl)) * kPairStride;
+    if (DG) {
+        double Sx[6], Sy[6], Rx[6], Ry[6];
+        for (int e = 0; e < 6; e++) {
+            const cd v = corner(e);
+            Sx[e] = v.x, Sy[e] = v.y;
+        }
+        rotate_sym(Sx, I.Q, A, Rx), rotate_sym(Sy, I.Q, A, Ry);
+        for (int p = 0; p < 3; p++)
+            for (int b = 0; b < 3; b++)
+                o[kPairG + (3 * ti + p) * 9 + 3 * tj + b] = cd{Rx[sidx(p, b)], Ry[sidx(p, b)]} * m.g_scale;
+    }
+    if (DH) {
+        double Sx[8], Sy[8], Rx[9], Ry[9];
+        for (int e = 0; e < 8; e++) {
+            const cd v = corner(NG + e);
+            Sx[e] = v.x, Sy[e] = v.y;
+        }
+        rotate_gen(Sx, I.Q, A, Rx), rotate_gen(Sy, I.Q, A, Ry);
+        for (int p = 0; p < 3; p++)
+            for (int b = 0; b < 3; b++) o[kPairH + (3 * ti + p) * 9 + 3 * tj + b] = cd{Rx[p * 3 + b], Ry[p * 3 + b]} * kInv4Pi;
+    }
+}
+
+// The same for B_trans and B_angular, which have the test basis only: T_0 for 1 and T_1 for Lx1, Lx2 (and Ly1, Ly2).
+// Entries, in units of 1/(8 pi s^2): the odd ones t1 h (3) and t2 c, the even ones u1 h h + u12 I (6) and u3.  HALF
+// (coincident pairs): regions 1, 3, 5, each point standing for its exchanged image too, whose test basis is Ly: the odd
+// entries take Lx - Ly and the even ones Lx + Ly.
+template <int KIND, bool HALF, int NW>
+__global__ void __launch_bounds__(64 * NW, 2) k_gal_touch_b(Geom g, const Pair *__restrict__ pairs, int pair0, long long nitems,
+                                                            const double2 *__restrict__ line, int nline,
+                                                            const double *__restrict__ xtab, const Freq *__restrict__ freqs,
+                                                            int nl, Mat m, cd *__restrict__ out) {
+    constexpr int NC = 11, NO = 4;  // entries, of which the first NO are odd in y - x
+    constexpr int NR = KIND == 1 ? (HALF ? 3 : 6) : (KIND == 2 ? 5 : 2);
+    __shared__ MathTables mtab;
+    __shared__ TouchItem item[4];
+    __shared__ double2 lin[kTouchMaxLine];
+    __shared__ TouchDir dir[64 * NW];
+    __shared__ cd Phi[4 * 5 * NC];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const long long it0 = 4LL * blockIdx.x;
+    load_math_tables(&mtab);
+    for (int k = tid; k < nline; k += 64 * NW) lin[k] = line[k];
+    if (tid < 4) load_item<KIND>(g, pairs, freqs, it0 + tid < nitems ? it0 + tid : nitems - 1, pair0, nl, item[tid]);
+    __syncthreads();
+    const int j = lane & 3, slot = lane >> 2;
+    const int nd = nline * nline * nline;
+    const const_double *xt = (const const_double *)xtab;
+    cd c0[NC], c1[NC];
+#pragma unroll
+    for (int e = 0; e < NC; e++) c0[e] = c1[e] = cd{0, 0};
+#pragma unroll 1
+    for (int r = 0; r < NR; r++) {
+#pragma unroll 1
+        for (int d0 = 16 * wave; d0 < nd; d0 += 16 * NW) {
+            cd zd1, zd2;
+            touch_direction<KIND>(HALF ? 2 * r : r, d0 + slot, nline, lin, item[j], j, zd1, zd2, dir[tid]);
+            cd e1[2], e2[4], ds[3];  // xi^0, xi^1; xi^-2 .. xi^1; xi^-2 .. xi^0, with w xi^3
+            e1[0] = e1[1] = cd{0, 0};
+#pragma unroll
+            for (int k = 0; k < 4; k++) e2[k] = cd{0, 0};
+#pragma unroll
+            for (int k = 0; k < 3; k++) ds[k] = cd{0, 0};
+#pragma unroll 1
+            for (int q = 0; q < nline; q++) {
+                const const_double *X = xt + kTouchXi * q;
+                const cd z1 = zd1 * X[0], z2 = zd2 * X[0];
+                const cd E1 = cexp_neg_tab(z1, &mtab), E2 = cexp_neg_tab(z2, &mtab);
+                const cd dS = (z1 * E1 + E1) - (z2 * E2 + E2);
+                fma_cr(e1[0], E1, X[5]), fma_cr(e1[1], E1, X[6]);
+#pragma unroll
+                for (int k = 0; k < 4; k++) fma_cr(e2[k], E2, X[3 + k]);
+#pragma unroll
+                for (int k = 0; k < 3; k++) fma_cr(ds[k], dS, X[3 + k]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            int ln = tid;
+            asm volatile("" : "+v"(ln));
+            const TouchDir D = dir[ln];
+            const double id = D.id_a.x, id2 = id * id, h[3] = {D.id_a.y, D.bc.x, D.bc.y};
+            const cd s = item[j].s;
+#pragma unroll
+            for (int mm = 0; mm < 2; mm++) {
+                cd T[NC];
+                const cd t1 = ds[mm] * id2, u1 = ds[mm + 1] * id;
+                const cd v = e2[mm + 2] * m.ic2, S = s * (v - e1[mm] * m.ic1);
+                cd t2 = zd2 * e2[mm + 1] + e2[mm];
+                t2.x -= xt[kTouchXi * nline + mm];
+#pragma unroll
+                for (int k = 0; k < 3; k++) T[k] = t1 * h[k];
+                T[3] = t2 * (2.0 * id2 * h[2]);
+                const cd u12 = u1 + S;
+#pragma unroll
+                for (int p = 0; p < 3; p++)
+#pragma unroll
+                    for (int q = p; q < 3; q++) {
+                        cd w = p == q ? u12 : cd{0, 0};
+                        fma_cr(w, u1, h[p] * h[q]);
+                        T[NO + sidx(p, q)] = w;
+                    }
+                T[10] = s * v * 2.0;
+#pragma unroll
+                for (int e = 0; e < NC; e++) {
+                    if (mm == 0) fma_cr(c0[e], T[e], D.wA1.x);
+                    else mfma_acc(c1[e], D.wA1.y, T[e]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    touch_reduce<NC, false>(c0, c1, nullptr, wave, NW, Phi);
+    // one lane per (item, test corner)
+    if (tid >= 12 || it0 + tid / 3 >= nitems) return;
+    const int jt = tid / 3, ti = tid % 3;
+    const TouchItem &I = item[jt];
+    const cd *ph = Phi + jt * 5 * NC;
+    cd v[NC];
+    for (int e = 0; e < NC; e++) {
+        auto p = [&](int k) { return ph[k * NC + e]; };
+        const double sg = e < NO ? -1.0 : 1.0;  // weight of the exchanged image's basis
+        if (ti) {
+            v[e] = p(ti);
+            if (HALF) fma_cr(v[e], p(2 + ti), sg);
+        } else {
+            v[e] = cd{0, 0} - (p(1) + p(2));
+            if (HALF) fma_cr(v[e], p(3) + p(4), -sg);
+            fma_cr(v[e], p(0), HALF ? 1.0 + sg : 1.0);
+        }
+        v[e] = v[e] * I.is2 * (I.jac * kInv8Pi);
+    }
+    cd mt[3], M[6];
+    for (int d = 0; d < 3; d++) {
+        mt[d] = cd{0, 0};
+        for (int k = 0; k < 3; k++) fma_cr(mt[d], v[k], I.Q[k][d]);
+    }
+    double Sx[6], Sy[6], Rx[6], Ry[6];
+    for (int e = 0; e < 6; e++) Sx[e] = v[NO + e].x, Sy[e] = v[NO + e].y;
+    rotate_sym(Sx, I.Q, I.Q, Rx), rotate_sym(Sy, I.Q, I.Q, Ry);
+    for (int e = 0; e < 6; e++) M[e] = cd{Rx[e], Ry[e]};
+    const double *n = I.Q[2];
+    const long long it = it0 + jt;
+    cd *o = out + ((long long)(pair0 + (int)(it / nl)) * nl + (int)(it % nl)) * kPairStride;
+    for (int p = 0; p < 3; p++)
+        for (int b = 0; b < 3; b++) {
+            cd t = p == b ? v[3] : cd{0, 0};
+            fma_cr(t, mt[p], n[b]);
+            fma_cr(t, mt[b], n[p]);
+            o[kPairBt + (3 * ti + p) * 3 + b] = t;
+            for (int k = 0; k < 3; k++) {
+                cd u = {0, 0};
+                fma_cr(u, M[sidx(p, k)], n[b]);
+                fma_cr(u, M[sidx(b, k)], n[p]);
+                if (p == b) fma_cr(u, v[10], n[k]);
+                o[kPairBa + (3 * ti + p) * 9 + b * 3 + k] = u;
+            }
+        }
 }
 
 // Coincident pairs integrated over regions 1, 3, 5 only (sums S).  Regions 2, 4, 6 are those with x and y
@@ -1073,38 +1322,8 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
     int kind_off[4] = {0, 0, 0, 0};
     for (const Pair &p : pairs) kind_off[p.kind]++;
     kind_off[3] += kind_off[2] += kind_off[1];  // exclusive ends per kind: [0,k1) coincident, [k1,k2) edge, [k2,k3) vertex
-    // Vertex-adjacent mirrors: a pair (f1, f2) with f1 > f2 whose pair (f2, f1) is listed with both faces ordered from
-    // the same shared vertex (as the classification orders them on a consistently oriented mesh).  Its G block is
-    // the transpose of that primary's and is not integrated (quad kernels); the mirrors go after the other
-    // vertex-adjacent pairs, and a pair without such a primary is integrated in full.
-    std::vector<int2> mirrors;  // (mirror pair, primary pair)
-    int vprim = kind_off[3];    // end of the vertex-adjacent pairs that are integrated for G
-    {
-        auto key = [](const Pair &p) { return std::make_pair(p.f1, p.f2); };
-        std::map<std::pair<int, int>, int> at;
-        for (int k = kind_off[2]; k < kind_off[3]; k++) at[key(pairs[k])] = k;
-        auto mirrored = [&](const Pair &p) {
-            if (p.f1 < p.f2) return false;
-            auto it = at.find({p.f2, p.f1});
-            if (it == at.end()) return false;
-            const Pair &q = pairs[it->second];
-            for (int c = 0; c < 3; c++)
-                if (q.j1[c] != p.j2[c] || q.j2[c] != p.j1[c]) return false;
-            return true;
-        };
-        std::vector<char> mir(pairs.size(), 0);
-        for (int k = kind_off[2]; k < kind_off[3]; k++) mir[k] = mirrored(pairs[k]) ? 1 : 0;
-        std::vector<Pair> prim, rest;
-        for (int k = kind_off[2]; k < kind_off[3]; k++) (mir[k] ? rest : prim).push_back(pairs[k]);
-        std::copy(prim.begin(), prim.end(), pairs.begin() + kind_off[2]);
-        std::copy(rest.begin(), rest.end(), pairs.begin() + kind_off[2] + (int)prim.size());
-        vprim = kind_off[2] + (int)prim.size();
-        at.clear();
-        for (int k = kind_off[2]; k < vprim; k++) at[key(pairs[k])] = k;
-        for (int k = vprim; k < kind_off[3]; k++) mirrors.push_back(make_int2(k, at.at({pairs[k].f2, pairs[k].f1})));
-    }
     const long long npairs = (long long)pairs.size();
-    DevVec dpairs, dscratch, dblocks, dptr, ditems, dvptr, dvitems, dmirrors;
+    DevVec dpairs, dscratch, dblocks, dptr, ditems, dvptr, dvitems, dxi;
     const Pair *dp = dpairs.up(pairs, st);
     dscratch.alloc((size_t)npairs * nl * kPairStride * sizeof(cd), "device allocation: touching-pair scratch");
     cd *scratch = (cd *)dscratch.p;
@@ -1118,38 +1337,45 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
         const char *sv = std::getenv("CQBEM_GALERKIN_SINGULAR");
         const bool lane = sv && !std::strcmp(sv, "lane");  // every region of every ordered pair integrated
         if (!lane) {
-#define CQBEM_SINGQ(MODE, KIND, HALF, E)                                                                              \
-    if ((E) > beg[KIND - 1])                                                                                          \
-        hipLaunchKernelGGL((k_gal_sing_quad<MODE, KIND, HALF>), dim3((unsigned)((E) - beg[KIND - 1]), nl), dim3(64), 0, \
-                           st, g, dp, beg[KIND - 1], job.line, job.nline, job.freqs, job.mat, scratch);
-            // coincident: half the regions, then the exchanged half; vertex-adjacent G: the primaries, then
-            // their mirrors' transposes
-            if (U) { CQBEM_SINGQ(0, 1, true, end[0]) CQBEM_SINGQ(0, 2, false, end[1]) CQBEM_SINGQ(0, 3, false, vprim) }
-            if (P) { CQBEM_SINGQ(1, 1, true, end[0]) CQBEM_SINGQ(1, 2, false, end[1]) CQBEM_SINGQ(1, 3, false, end[2]) }
-#undef CQBEM_SINGQ
-            if ((U || P) && end[0] > 0) {
+            dxi.alloc(sizeof(double) * (kTouchXi * job.nline + 2), "device allocation: xi table");
+            double *xtab = (double *)dxi.p;
+            hipLaunchKernelGGL(k_gal_xi, dim3(1), dim3(128), 0, st, job.line, job.nline, xtab);
+            // four waves per block while one wave per block would give fewer than 8 waves per SIMD
+#define CQBEM_TOUCH(KERNEL, KIND, ...)                                                                                \
+    if (end[KIND - 1] > beg[KIND - 1]) {                                                                              \
+        const long long items = (long long)(end[KIND - 1] - beg[KIND - 1]) * nl, blocks = (items + 3) / 4;            \
+        if (blocks < 8LL * 4 * job.num_cus)                                                                           \
+            hipLaunchKernelGGL((KERNEL<__VA_ARGS__, 4>), dim3((unsigned)blocks), dim3(256), 0, st, g, dp, beg[KIND - 1], items, \
+                               job.line, job.nline, xtab, job.freqs, nl, job.mat, scratch);                           \
+        else                                                                                                          \
+            hipLaunchKernelGGL((KERNEL<__VA_ARGS__, 1>), dim3((unsigned)blocks), dim3(64), 0, st, g, dp, beg[KIND - 1], items, \
+                               job.line, job.nline, xtab, job.freqs, nl, job.mat, scratch);                           \
+    }
+#define CQBEM_TOUCH_GH(DG, DH)                                                                                        \
+    {                                                                                                                 \
+        CQBEM_TOUCH(k_gal_touch, 1, DG, DH, 1, true)                                                                  \
+        CQBEM_TOUCH(k_gal_touch, 2, DG, DH, 2, false)                                                                 \
+        CQBEM_TOUCH(k_gal_touch, 3, DG, DH, 3, false)                                                                 \
+    }
+            if (U && P) CQBEM_TOUCH_GH(true, true)
+            else if (U) CQBEM_TOUCH_GH(true, false)
+            else if (P) CQBEM_TOUCH_GH(false, true)
+            if ((U || P) && end[0] > 0) {  // the coincident pairs' exchanged half
                 const long long n = (long long)end[0] * nl * 108;
                 hipLaunchKernelGGL(k_gal_coincident_sym, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, end[0], nl,
                                    U ? 1 : 0, P ? 1 : 0, scratch);
             }
-            if (U && !mirrors.empty()) {
-                const int2 *dm = dmirrors.up(mirrors, st);
-                const long long n = (long long)mirrors.size() * nl * 81;
-                hipLaunchKernelGGL(k_gal_mirror_g, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, dm, (int)mirrors.size(),
-                                   nl, scratch);
+            if (Bt && Ba) {
+                CQBEM_TOUCH(k_gal_touch_b, 1, 1, true)
+                CQBEM_TOUCH(k_gal_touch_b, 2, 2, false)
+                CQBEM_TOUCH(k_gal_touch_b, 3, 3, false)
             }
+#undef CQBEM_TOUCH_GH
+#undef CQBEM_TOUCH
         } else {
             if (U) { CQBEM_SING(0, 1) CQBEM_SING(0, 2) CQBEM_SING(0, 3) }
             if (P) { CQBEM_SING(1, 1) CQBEM_SING(1, 2) CQBEM_SING(1, 3) }
-        }
-        if (Bt && Ba) {
-            if (lane) {
-                CQBEM_SING(2, 1)
-            } else if (end[0] > beg[0]) {  // coincident B over half the regions, the exchanged half folded in
-                hipLaunchKernelGGL((k_gal_sing<2, 1, true>), dim3((unsigned)(end[0] - beg[0]), nl), dim3(64), 0, st, g, dp,
-                                   beg[0], job.line, job.nline, job.freqs, job.mat, scratch);
-            }
-            CQBEM_SING(2, 2) CQBEM_SING(2, 3)
+            if (Bt && Ba) { CQBEM_SING(2, 1) CQBEM_SING(2, 2) CQBEM_SING(2, 3) }
         }
 #undef CQBEM_SING
         check(hipGetLastError(), "k_gal_sing");

@@ -166,12 +166,6 @@ constexpr int kRmw = 8;             // slot words read at a time when a corner i
 constexpr int kNoStep = 0xff;       // sub-step code of a corner outside the patch
 constexpr int kFramePairs = 3;      // per lane, read at every point: the FaceFrame
 
-// Tables that no kernel writes, read through the constant address space: uniform indices become scalar loads also where
-// the pointer itself came from memory (scenes).
-typedef const __attribute__((address_space(4))) double const_double;
-typedef const __attribute__((address_space(4))) int const_int;
-__device__ inline const_double *as_const(const double4 *p) { return (const_double *)p; }
-__device__ inline const_int *as_const(const int4 *p) { return (const_int *)p; }
 // A pointer read from memory, known to be to global memory.
 template <class T> __device__ inline T *as_global(T *p) { return (T *)(__attribute__((address_space(1))) T *)p; }
 
