@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(64) k_colloc_gh(Geom g, const double4 *__restr
 // limit leaves): 292 VALU instructions per point, of which 84 are the corner
 // sums and 78 the two complex exponentials, and 1100 per face and row outside
 // the rule.  Icosphere level 4, L = 32, 28 points (6.2e9 unique evaluations):
-// 80.9 ms, 2.25 ms per point of the rule plus 18 ms.  The form it replaces, two
+// 80.2 ms, 2.25 ms per point of the rule plus 17 ms.  The form it replaces, two
 // lanes per face that swapped every point's 16 global entries through DPP, took
 // 128 ms at 516 instructions per point.  Tried and slower: the same with a
 // block barrier per sub-step (86.5 ms), the rotation inside the wave's turn
@@ -166,6 +166,12 @@ constexpr int kRmw = 8;             // slot words read at a time when a corner i
 constexpr int kNoStep = 0xff;       // sub-step code of a corner outside the patch
 constexpr int kFramePairs = 3;      // per lane, read at every point: the FaceFrame
 
+// A pointer that every lane holds alike, in scalar registers.
+template <class T> __device__ inline T *uniform_ptr(T *p) {
+    const unsigned long long v = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return (T *)((unsigned long long)hi << 32 | lo);
+}
 // A pointer read from memory, known to be to global memory.
 template <class T> __device__ inline T *as_global(T *p) { return (T *)(__attribute__((address_space(1))) T *)p; }
 
@@ -180,13 +186,19 @@ __device__ inline void wait_for(int *counter, int v) {
 // counters (2) and mtab are the block's LDS (mtab loaded); callers that run another tile on the same LDS synchronise
 // first.  The block has no barrier between its rows: a wave evaluates its first chunk of the next row before it writes
 // out (and clears) its 64 vertex slots of the last one, so neither the other waves' adds nor the stores are waited for.
-template <bool DG, bool DH, bool GAL>
+// `dest` returns where the rows go (PatchDest); it is called at each write-out, so that a caller that reads it from memory
+// need not hold it in registers.
+struct PatchDest {
+    const int *patch_verts;
+    cd *UG, *UH;
+    long long ld, lstride;
+};
+template <bool DG, bool DH, bool GAL, class Dest>
 __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, const double4 *__restrict__ ref_pts, int ref_npts,
                                  const Bands &bands, const Freq *__restrict__ freqs,
                                  int l0, const Mat &m, int row0, const double4 *__restrict__ tpts,
                                  const int *__restrict__ patch_chunk, const int4 *__restrict__ chunk_info,
-                                 const int4 *__restrict__ chunk_faces, const int *__restrict__ patch_verts,
-                                 cd *__restrict__ UG, cd *__restrict__ UH, long long ld, long long lstride, int pc, int l,
+                                 const int4 *__restrict__ chunk_faces, const Dest &dest, int pc, int l,
                                  int il0, int nr, double2 *acc, double2 *frame, int *counters, const MathTables &mtab) {
     constexpr int kWaves = kPatchThreads / 64;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -200,18 +212,20 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
     int *turns = counters, *cleared = counters + 1;  // chunks added so far; waves that cleared their slots, over all rows
     if (tid < 2) counters[tid] = 0;
     __syncthreads();
-    // Waves take the patch's chunks in turn.  With one or two chunks, 4 or 2 waves share a chunk, each taking every 4th
-    // or 2nd point of the rule, as long as 7 points are left to each.
-    const int c0 = patch_chunk[pc], nchunk = patch_chunk[pc + 1] - c0;
+    // With one or two chunks, 4 or 2 waves share a chunk, each taking every 4th or 2nd point of the rule, as long as 7
+    // points are left to each.
+    const_int *pch = (const_int *)(patch_chunk + pc);
+    const int c0 = pch[0], nchunk = pch[1] - c0;
     const int split = nchunk == 1 && ref_npts >= 28 ? 4 : nchunk <= 2 && ref_npts >= 14 ? 2 : 1;
     const int nturn = nchunk * split;
 
     // writes the G and H blocks of (row r of the tile, the wave's vertex slots) and clears the slots
     auto write_row = [&](int r) {
         wait_for(turns, (r + 1) * nturn);
-        const int j = patch_verts[pc * kPatchVerts + tid];
+        const PatchDest D = dest();
+        const int j = D.patch_verts[pc * kPatchVerts + tid];
         if (j >= 0) {
-            const long long obase = (long long)l * lstride + (long long)(3 * (il0 + r)) * ld + 3 * (long long)j;
+            const long long obase = (long long)l * D.lstride + (long long)(3 * (il0 + r)) * D.ld + 3 * (long long)j;
 #pragma unroll
             for (int p = 0; p < 3; p++) {
 #pragma unroll
@@ -219,11 +233,11 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
                     const int e = sidx(p, b);
                     if (DG) {
                         const double2 w = acc[e * kPatchVerts + tid];
-                        UG[obase + p * ld + b] = cd{w.x, w.y} * m.g_scale;
+                        D.UG[obase + p * D.ld + b] = cd{w.x, w.y} * m.g_scale;
                     }
                     if (DH) {
                         const double2 w = acc[(6 + p * 3 + b) * kPatchVerts + tid];
-                        UH[obase + p * ld + b] = cd{w.x, w.y} * kInv4Pi;
+                        D.UH[obase + p * D.ld + b] = cd{w.x, w.y} * kInv4Pi;
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -235,17 +249,20 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
         if (lane == 0) __hip_atomic_fetch_add(cleared, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
 
+    // turn t of the tile: chunk part t % nturn of row t / nturn; the waves take the turns round robin over all rows, so
+    // that a chunk count that is no multiple of the waves leaves none idle
+    int written = 0;  // rows the wave has written out
 #pragma unroll 1
-    for (int r = 0; r < nr; ++r) {
-        const int i = row0 + il0 + r;
-        // the row point: vertex i (collocation), or test point i with its face's corners t[] excluded (Galerkin)
+    for (int t = wave; t < nr * nturn; t += kWaves) {
+        const int r = t / nturn, turn = t - r * nturn, i = row0 + il0 + r;
+        // the row point: vertex i (collocation), or test point i with its face's corners tv[] excluded (Galerkin)
         double x0, x1, x2;
-        int t[3] = {i, i, i};
+        int tv[3] = {i, i, i};
         if (GAL) {
             const double4 T = tpts[i];
             x0 = T.x, x1 = T.y, x2 = T.z;
             const int f1 = (int)T.w;
-            t[0] = g.F[3 * f1], t[1] = g.F[3 * f1 + 1], t[2] = g.F[3 * f1 + 2];
+            tv[0] = g.F[3 * f1], tv[1] = g.F[3 * f1 + 1], tv[2] = g.F[3 * f1 + 2];
         } else {
             x0 = g.V[3 * i], x1 = g.V[3 * i + 1], x2 = g.V[3 * i + 2];
         }
@@ -255,145 +272,141 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
             if (__builtin_amdgcn_readfirstlane((int)beyond_sphere(x0, x1, x2, bands.sphere[pc])))
                 pts = bands.far_pts, npts = bands.far_npts;
         }
-        bool written = r == 0;  // whether the wave has written out the previous row
-#pragma unroll 1
-        for (int turn = wave; turn < nturn; turn += kWaves) {
-            const int part = turn % split;
-            const_int *ci = as_const(chunk_info + (c0 + turn / split));
-            const int4 info = make_int4(ci[0], ci[1], ci[2], 0);
-            // lanes past the chunk's faces repeat its last one; they and the faces touching the row point are not added
-            const int entry = info.x + min(lane, info.y - 1);
-            const int4 fe = chunk_faces[entry];
-            const int va[3] = {fe.x & 0xffffff, fe.y & 0xffffff, fe.z & 0xffffff};
-            bool active = lane < info.y;
-            for (int k = 0; k < (GAL ? 3 : 1); k++)
-                active = active && !(same_vertex(g, t[k], va[0]) || same_vertex(g, t[k], va[1]) || same_vertex(g, t[k], va[2]));
-            const unsigned long long act = __builtin_amdgcn_ballot_w64(active);
-            cd sg[3][6], sh[3][8];
-            if (act) {  // wave-uniform: no divergent merge of the sums
-                {
-                    double y[3][3];
+        pts = uniform_ptr(pts);
+        const int part = turn % split;
+        const_int *ci = as_const(chunk_info + (c0 + turn / split));
+        const int4 info = make_int4(ci[0], ci[1], ci[2], 0);
+        // lanes past the chunk's faces repeat its last one; they and the faces touching the row point are not added
+        const int entry = info.x + min(lane, info.y - 1);
+        const int4 fe = chunk_faces[entry];
+        const int va[3] = {fe.x & 0xffffff, fe.y & 0xffffff, fe.z & 0xffffff};
+        bool active = lane < info.y;
+        for (int k = 0; k < (GAL ? 3 : 1); k++)
+            active = active && !(same_vertex(g, tv[k], va[0]) || same_vertex(g, tv[k], va[1]) || same_vertex(g, tv[k], va[2]));
+        const unsigned long long act = __builtin_amdgcn_ballot_w64(active);
+        cd sg[3][6], sh[3][8];
+        if (act) {  // wave-uniform: no divergent merge of the sums
+            {
+                double y[3][3];
+#pragma unroll
+                for (int k = 0; k < 3; k++)
+#pragma unroll
+                    for (int d = 0; d < 3; d++) y[k][d] = g.V[3 * va[k] + d];
+                const FaceFrame F = face_frame(y, x0, x1, x2);
+                frame[tid] = make_double2(F.L1, F.u), frame[kPatchThreads + tid] = make_double2(F.v, F.xa);
+                frame[2 * kPatchThreads + tid] = make_double2(F.xb, F.cr);
+            }
+            // one point's entries into the sums; the first point starts them
+            auto point = [&](int q, auto first) __attribute__((always_inline)) {
+                // the lane is made opaque per point so that the frame stays in LDS (14 VGPRs otherwise)
+                int ln = tid;
+                asm volatile("" : "+v"(ln));
+                const double2 F0 = frame[ln], F1 = frame[kPatchThreads + ln], F2 = frame[2 * kPatchThreads + ln];
+                const_double *B = as_const(pts + 2 * q);  // b1, b2, -, -, w (phi_0, phi_1, phi_2, 1)
+                const double ar = fma(B[0], F0.x, fma(B[1], F0.y, F1.y)), br = fma(B[1], F1.x, F2.x), cr = F2.y;
+                const PointExpo E = point_expo(fma(ar, ar, fma(br, br, cr * cr)), f, &mtab);
+                const double w[3] = {B[4], B[5], B[6]};
+                const double a = ar * E.ir, b = br * E.ir, c = cr * E.ir;
+                auto add = [&](cd &s, const cd &v, double wk) {
+                    if (first()) s = v * wk;
+                    else fma_cr(s, v, wk);
+                };
+                // G and H one after the other, so that only one set of entries is live beside the sums
+                __builtin_amdgcn_sched_barrier(0);
+                if (DG) {
+                    cd G[6];
+                    point_g(E, a, b, c, m, G);
 #pragma unroll
                     for (int k = 0; k < 3; k++)
 #pragma unroll
-                        for (int d = 0; d < 3; d++) y[k][d] = g.V[3 * va[k] + d];
-                    const FaceFrame F = face_frame(y, x0, x1, x2);
-                    frame[tid] = make_double2(F.L1, F.u), frame[kPatchThreads + tid] = make_double2(F.v, F.xa);
-                    frame[2 * kPatchThreads + tid] = make_double2(F.xb, F.cr);
+                        for (int e = 0; e < 6; e++) add(sg[k][e], G[e], w[k]);
                 }
-                // one point's entries into the sums; the first point starts them
-                auto point = [&](int q, auto first) __attribute__((always_inline)) {
-                    // the lane is made opaque per point so that the frame stays in LDS (14 VGPRs otherwise)
-                    int ln = tid;
-                    asm volatile("" : "+v"(ln));
-                    const double2 F0 = frame[ln], F1 = frame[kPatchThreads + ln], F2 = frame[2 * kPatchThreads + ln];
-                    const_double *B = as_const(pts + 2 * q);  // b1, b2, -, -, w (phi_0, phi_1, phi_2, 1)
-                    const double ar = fma(B[0], F0.x, fma(B[1], F0.y, F1.y)), br = fma(B[1], F1.x, F2.x), cr = F2.y;
-                    const PointExpo E = point_expo(fma(ar, ar, fma(br, br, cr * cr)), f, &mtab);
-                    const double w[3] = {B[4], B[5], B[6]};
-                    const double a = ar * E.ir, b = br * E.ir, c = cr * E.ir;
-                    auto add = [&](cd &s, const cd &v, double wk) {
-                        if (first()) s = v * wk;
-                        else fma_cr(s, v, wk);
-                    };
-                    // G and H one after the other, so that only one set of entries is live beside the sums
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (DG) {
-                        cd G[6];
-                        point_g(E, a, b, c, m, G);
+                __builtin_amdgcn_sched_barrier(0);
+                if (DH) {
+                    cd H[8];
+                    point_h(E, a, b, c, m, H);
 #pragma unroll
-                        for (int k = 0; k < 3; k++)
+                    for (int k = 0; k < 3; k++)
 #pragma unroll
-                            for (int e = 0; e < 6; e++) add(sg[k][e], G[e], w[k]);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (DH) {
-                        cd H[8];
-                        point_h(E, a, b, c, m, H);
-#pragma unroll
-                        for (int k = 0; k < 3; k++)
-#pragma unroll
-                            for (int e = 0; e < 8; e++) add(sh[k][e], H[e], w[k]);
-                    }
-                };
-                point(part, std::true_type{});
+                        for (int e = 0; e < 8; e++) add(sh[k][e], H[e], w[k]);
+                }
+            };
+            point(part, std::true_type{});
 #pragma unroll 1
-                for (int q = part + split; q < npts; q += split) point(q, std::false_type{});
-            } else {
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-#pragma unroll
-                    for (int e = 0; e < 6; e++) sg[k][e] = cd{0, 0};
-#pragma unroll
-                    for (int e = 0; e < 8; e++) sh[k][e] = cd{0, 0};
-                }
-            }
-            if (!written) write_row(r - 1), written = true;
-            // rotate each corner's sums and add them in the scheduled sub-steps, after every earlier chunk of the row and
-            // once all slots are cleared
-            const int4 ge = chunk_faces[info.x + min(lane, info.y - 1)];
-            double Q[3][3], A[3][3];
-            {
-                double e1[3], e2[3], L1, area2;
-                const int v0 = ge.x & 0xffffff, v1 = ge.y & 0xffffff, v2 = ge.z & 0xffffff;
-                for (int d = 0; d < 3; d++) e1[d] = g.V[3 * v1 + d] - g.V[3 * v0 + d], e2[d] = g.V[3 * v2 + d] - g.V[3 * v0 + d];
-                face_axes(e1, e2, Q, &L1, &area2);
-                for (int j = 0; j < 3; j++)
-                    for (int k = 0; k < 3; k++) A[j][k] = Q[j][k] * (0.5 * area2);
-            }
-            double v[3][2 * kPatchPairs];
+            for (int q = part + split; q < npts; q += split) point(q, std::false_type{});
+        } else {
 #pragma unroll
             for (int k = 0; k < 3; k++) {
 #pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    if (DG) {
-                        double S[6], R[6];
+                for (int e = 0; e < 6; e++) sg[k][e] = cd{0, 0};
 #pragma unroll
-                        for (int e = 0; e < 6; e++) S[e] = p ? sg[k][e].y : sg[k][e].x;
-                        rotate_sym(S, Q, A, R);
-#pragma unroll
-                        for (int e = 0; e < 6; e++) v[k][2 * e + p] = R[e];
-                    }
-                    if (DH) {
-                        double S[8], R[9];
-#pragma unroll
-                        for (int e = 0; e < 8; e++) S[e] = p ? sh[k][e].y : sh[k][e].x;
-                        rotate_gen(S, Q, A, R);
-#pragma unroll
-                        for (int e = 0; e < 9; e++) v[k][12 + 2 * e + p] = R[e];
-                    }
-                }
-                // formed here, not sunk behind the waits below
-#pragma unroll
-                for (int e = DG ? 0 : 12; e < (DH ? 2 * kPatchPairs : 12); e++) asm volatile("" : "+v"(v[k][e]));
+                for (int e = 0; e < 8; e++) sh[k][e] = cd{0, 0};
             }
-            wait_for(cleared, kWaves * r);
-            wait_for(turns, r * nturn + turn);
-            const int corner[3] = {ge.x, ge.y, ge.z};
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const int slot = (unsigned)corner[k] >> 24;
-                const int step = (act >> lane) & 1 ? (ge.w >> (8 * k)) & 0xff : kNoStep;
-                const int nsub = (info.z >> (8 * k)) & 0xff;
-                for (int s = 0; s < nsub; ++s) {
-                    if (step != s) continue;
-                    // read-modify-write of the slot's words, kRmw reads in flight
-#pragma unroll
-                    for (int e0 = DG ? 0 : 6; e0 < (DH ? kPatchPairs : 6); e0 += kRmw) {
-                        double2 u[kRmw];
-#pragma unroll
-                        for (int e = e0; e < e0 + kRmw && e < (DH ? kPatchPairs : 6); e++) u[e - e0] = acc[e * kPatchVerts + slot];
-#pragma unroll
-                        for (int e = e0; e < e0 + kRmw && e < (DH ? kPatchPairs : 6); e++)
-                            acc[e * kPatchVerts + slot] = make_double2(u[e - e0].x + v[k][2 * e], u[e - e0].y + v[k][2 * e + 1]);
-                    }
-                }
-            }
-            __hip_atomic_store(turns, r * nturn + turn + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
-        if (!written) write_row(r - 1);  // a wave without a chunk in this patch
+        while (written < r) write_row(written++);
+        // rotate each corner's sums and add them in the scheduled sub-steps, after every earlier chunk of the row and
+        // once all slots are cleared
+        const int4 ge = chunk_faces[info.x + min(lane, info.y - 1)];
+        double Q[3][3], A[3][3];
+        {
+            double e1[3], e2[3], L1, area2;
+            const int v0 = ge.x & 0xffffff, v1 = ge.y & 0xffffff, v2 = ge.z & 0xffffff;
+            for (int d = 0; d < 3; d++) e1[d] = g.V[3 * v1 + d] - g.V[3 * v0 + d], e2[d] = g.V[3 * v2 + d] - g.V[3 * v0 + d];
+            face_axes(e1, e2, Q, &L1, &area2);
+            for (int j = 0; j < 3; j++)
+                for (int k = 0; k < 3; k++) A[j][k] = Q[j][k] * (0.5 * area2);
+        }
+        double v[3][2 * kPatchPairs];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                if (DG) {
+                    double S[6], R[6];
+#pragma unroll
+                    for (int e = 0; e < 6; e++) S[e] = p ? sg[k][e].y : sg[k][e].x;
+                    rotate_sym(S, Q, A, R);
+#pragma unroll
+                    for (int e = 0; e < 6; e++) v[k][2 * e + p] = R[e];
+                }
+                if (DH) {
+                    double S[8], R[9];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) S[e] = p ? sh[k][e].y : sh[k][e].x;
+                    rotate_gen(S, Q, A, R);
+#pragma unroll
+                    for (int e = 0; e < 9; e++) v[k][12 + 2 * e + p] = R[e];
+                }
+            }
+            // formed here, not sunk behind the waits below
+#pragma unroll
+            for (int e = DG ? 0 : 12; e < (DH ? 2 * kPatchPairs : 12); e++) asm volatile("" : "+v"(v[k][e]));
+        }
+        wait_for(cleared, kWaves * r);
+        wait_for(turns, t);
+        const int corner[3] = {ge.x, ge.y, ge.z};
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const int slot = (unsigned)corner[k] >> 24;
+            const int step = (act >> lane) & 1 ? (ge.w >> (8 * k)) & 0xff : kNoStep;
+            const int nsub = (info.z >> (8 * k)) & 0xff;
+            for (int s = 0; s < nsub; ++s) {
+                if (step != s) continue;
+                // read-modify-write of the slot's words, kRmw reads in flight
+#pragma unroll
+                for (int e0 = DG ? 0 : 6; e0 < (DH ? kPatchPairs : 6); e0 += kRmw) {
+                    double2 u[kRmw];
+#pragma unroll
+                    for (int e = e0; e < e0 + kRmw && e < (DH ? kPatchPairs : 6); e++) u[e - e0] = acc[e * kPatchVerts + slot];
+#pragma unroll
+                    for (int e = e0; e < e0 + kRmw && e < (DH ? kPatchPairs : 6); e++)
+                        acc[e * kPatchVerts + slot] = make_double2(u[e - e0].x + v[k][2 * e], u[e - e0].y + v[k][2 * e + 1]);
+                }
+            }
+        }
+        __hip_atomic_store(turns, t + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    write_row(nr - 1);
+    while (written < nr) write_row(written++);
 }
 
 // BANDED: the distance-banded rule (CQBEM_QUAD_BANDED) is compiled in; without it the tile rule check is not.
@@ -413,7 +426,7 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_colloc_gh_patch(Geom g, co
     __shared__ MathTables mtab;                       // tables of the exponentials
     load_math_tables(&mtab);
     patch_tile<DG, DH, GAL>(g, pts, npts, BANDED ? bands : Bands{}, freqs, l0, m, row0, tpts, patch_chunk, chunk_info,
-                           chunk_faces, patch_verts, UG, UH, ld, lstride, blockIdx.x, blockIdx.y, blockIdx.z * rpt,
+                           chunk_faces, [=] { return PatchDest{patch_verts, UG, UH, ld, lstride}; }, blockIdx.x, blockIdx.y, blockIdx.z * rpt,
                            min(rpt, nrows - (int)blockIdx.z * rpt), acc, frame, counters, mtab);
 }
 
@@ -433,6 +446,7 @@ __device__ __attribute__((always_inline)) inline void scene_tile(const ScenePiec
                                   const MathTables &mtab) {
     int pi = 0;
     while (pi + 1 < npieces && (unsigned)*(const_int *)&pieces[pi + 1].base <= t) ++pi;
+    pi = __builtin_amdgcn_readfirstlane(pi);
     ScenePiece P;  // held in scalar registers
     {
         static_assert(sizeof(ScenePiece) % 4 == 0, "copied in words");
@@ -444,12 +458,19 @@ __device__ __attribute__((always_inline)) inline void scene_tile(const ScenePiec
     }
     P.g.V = as_global(P.g.V), P.g.vmap = as_global(P.g.vmap);
     P.bands.sphere = as_global(P.bands.sphere);
+    auto dest = [pieces, pi] {
+        const ScenePiece *q = pieces + pi;
+        asm volatile("" : "+s"(q));
+        auto ptr = [](const void *field) { return *(const __attribute__((address_space(4))) unsigned long long *)field; };
+        return PatchDest{as_global((const int *)ptr(&q->patch_verts)), as_global((cd *)ptr(&q->UG)), as_global((cd *)ptr(&q->UH)),
+                         (long long)ptr(&q->ld), (long long)ptr(&q->lstride)};
+    };
     const unsigned local = t - P.base, np = (unsigned)P.npatches, nl = (unsigned)P.nl;
     const unsigned rest = local / np;
+    const int pc = __builtin_amdgcn_readfirstlane(local - rest * np), l = __builtin_amdgcn_readfirstlane(rest % nl),
+              r0 = __builtin_amdgcn_readfirstlane(rest / nl) * P.rpt;
     patch_tile<DG, DH, false>(P.g, P.pts, P.npts, P.bands, as_global(P.freqs), 0, P.m, P.row0, nullptr, as_global(P.patch_chunk),
-                              P.chunk_info, as_global(P.chunk_faces), as_global(P.patch_verts), as_global(P.UG), as_global(P.UH),
-                              P.ld, P.lstride, (int)(local - rest * np), (int)(rest % nl), (int)(rest / nl) * P.rpt,
-                              min(P.rpt, P.nrows - (int)(rest / nl) * P.rpt), acc, frame, counters, mtab);
+                              P.chunk_info, as_global(P.chunk_faces), dest, pc, l, r0, min(P.rpt, P.nrows - r0), acc, frame, counters, mtab);
 }
 
 template <bool DG, bool DH>
@@ -1278,8 +1299,9 @@ hipError_t launch_colloc_gh(const Geom &g, const double4 *quad, int npts, const 
 }
 
 
-// Rows per block of the patch kernel: enough to hide a row's start and write-out behind the next one's evaluation, and
-// still at least 8192 blocks (16 per resident block of 256 CUs) where there are as many tiles.
+// Rows per block of the patch kernel: enough to hide a row's start and write-out behind the next one's evaluation and to
+// even out chunk counts that are no multiple of 4, and still at least 4096 blocks (8 per resident block of 256 CUs) where
+// there are as many tiles.
 int patch_rows_per_tile(long long tiles) { return (int)std::min<long long>(16, std::max<long long>(1, tiles / 8192)); }
 
 hipError_t launch_colloc_gh_patch(const Geom &g, const double4 *pts, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
