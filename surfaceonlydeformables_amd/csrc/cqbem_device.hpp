@@ -43,6 +43,26 @@ __host__ __device__ inline void fma_cr(cd &a, cd b, double s) {
     a.y = fma(b.y, s, a.y);
 }
 
+// Two real values side by side, with component-wise products: one quantity at the two frequencies of the half spectrum
+// where s is real (l = 0, and l = L/2 for an even L).
+struct rp {
+    double x, y;
+};
+__host__ __device__ inline rp operator+(rp a, rp b) { return rp{a.x + b.x, a.y + b.y}; }
+__host__ __device__ inline rp operator-(rp a, rp b) { return rp{a.x - b.x, a.y - b.y}; }
+__host__ __device__ inline rp operator*(rp a, rp b) { return rp{a.x * b.x, a.y * b.y}; }
+__host__ __device__ inline rp operator*(rp a, double s) { return rp{a.x * s, a.y * s}; }
+__host__ __device__ inline rp operator*(double s, rp a) { return rp{a.x * s, a.y * s}; }
+__host__ __device__ inline rp &operator+=(rp &a, rp b) { return a = a + b; }
+__host__ __device__ inline rp &operator-=(rp &a, rp b) { return a = a - b; }
+__host__ __device__ inline void fma_cr(rp &a, rp b, double s) {
+    a.x = fma(b.x, s, a.x);
+    a.y = fma(b.y, s, a.y);
+}
+// v + 1 at one frequency, or at both
+__host__ __device__ inline cd add_one(cd v, double one) { return cd{v.x + one, v.y}; }
+__host__ __device__ inline rp add_one(rp v, double one) { return rp{v.x + one, v.y + one}; }
+
 // ---------------------------------------------------------------------------
 // FP64 elementary functions for the kernel arguments.  The CQ exponent
 // z = s r / c has Re z >= 0 (the BDF symbols are A-stable, so Re s_l > 0) and
@@ -242,6 +262,11 @@ __host__ __device__ inline cd cexp_neg_tab(cd z, const MathTables *M) {
     return cd{m * cs, -m * sn};
 }
 
+// The same at two real arguments.
+__host__ __device__ inline rp cexp_neg_tab(rp z, const MathTables *M) {
+    return rp{exp_tab_core(fmax(-z.x, -740.0), M->e), exp_tab_core(fmax(-z.y, -740.0), M->e)};
+}
+
 // exp(-z), Re z >= 0
 __device__ inline cd cexp_neg(cd z) {
     const double m = exp_neg(z.x);
@@ -265,6 +290,20 @@ struct Freq {
     cd is;   // 1 / s
     cd is2;  // 1 / s^2
 };
+
+// The constants that the regular-face kernels read, at one frequency (cd) or at the two real ones (rp), from the table
+// through the constant address space.
+template <class T> struct PointFreq {
+    T s, sc1, sc2, is2;
+};
+__device__ inline PointFreq<cd> point_freq(const Freq *f, int l, cd) {
+    const_double *p = (const_double *)(f + l);
+    return PointFreq<cd>{cd{p[0], p[1]}, cd{p[2], p[3]}, cd{p[4], p[5]}, cd{p[8], p[9]}};
+}
+__device__ inline PointFreq<rp> point_freq(const Freq *f, int hi, rp) {
+    const_double *p = (const_double *)f, *q = (const_double *)(f + hi);
+    return PointFreq<rp>{rp{p[0], q[0]}, rp{p[2], q[2]}, rp{p[4], q[4]}, rp{p[8], q[8]}};
+}
 
 // Material constants.
 struct Mat {
@@ -375,15 +414,15 @@ __device__ inline FaceFrame face_frame(const double y[3][3], double x0, double x
 // Frequency- and material-dependent factors of one point: with w_k = z_k e_k and dd = (A1 - A2) / r^2 every
 // coefficient is a short sum, the traction's in units of 1/r^2 (their static part 6 c2^2 dd is the first bracket of
 // H_collocation.cu:45-76, which the displacement kernel shares).
-struct PointExpo {
+template <class T> struct PointExpo {
     double ir, ir2, r;
-    cd e1, e2, w1, w2, s2, q2;  // s2 = (z2 + 1) e2, q2 = 1 / (s r)^2
-    cd dd;
+    T e1, e2, w1, w2, s2, q2;  // s2 = (z2 + 1) e2, q2 = 1 / (s r)^2
+    T dd;
 };
-__device__ inline PointExpo point_expo(double d2, const Freq &f, const MathTables *M) {
-    PointExpo E;
+template <class T> __device__ inline PointExpo<T> point_expo(double d2, const PointFreq<T> &f, const MathTables *M) {
+    PointExpo<T> E;
     E.ir = rsqrt_h3(d2), E.r = d2 * E.ir, E.ir2 = E.ir * E.ir;
-    const cd z1 = f.sc1 * E.r, z2 = f.sc2 * E.r;
+    const T z1 = f.sc1 * E.r, z2 = f.sc2 * E.r;
     E.e1 = cexp_neg_tab(z1, M), E.e2 = cexp_neg_tab(z2, M);
     E.w1 = z1 * E.e1, E.w2 = z2 * E.e2;
     E.s2 = E.w2 + E.e2, E.q2 = f.is2 * E.ir2;
@@ -393,25 +432,27 @@ __device__ inline PointExpo point_expo(double d2, const Freq &f, const MathTable
 
 // Local entries of one point in direction (a, b, c), not weighted: G (xx yy zz xy xz yz) = (alpha h h^T + beta I) / r
 // without 1/(4 pi rho), and H (xx yy zz xy xz yz zx zy) without 1/(4 pi).
-__device__ inline void point_g(const PointExpo &E, double a, double b, double c, const Mat &m, cd *G) {
-    const cd t = E.e2 * m.ic2s;
-    const cd al = (3.0 * E.dd + (E.e1 * m.ic1s - t)) * E.ir, be = (t - E.dd) * E.ir;
+template <class T>
+__device__ inline void point_g(const PointExpo<T> &E, double a, double b, double c, const Mat &m, T *G) {
+    const T t = E.e2 * m.ic2s;
+    const T al = (3.0 * E.dd + (E.e1 * m.ic1s - t)) * E.ir, be = (t - E.dd) * E.ir;
     G[0] = G[1] = G[2] = be;
     fma_cr(G[0], al, a * a), fma_cr(G[1], al, b * b), fma_cr(G[2], al, c * c);
     G[3] = al * (a * b), G[4] = al * (a * c), G[5] = al * (b * c);
 }
-__device__ inline void point_h(const PointExpo &E, double a, double b, double c, const Mat &m, cd *H) {
+template <class T>
+__device__ inline void point_h(const PointExpo<T> &E, double a, double b, double c, const Mat &m, T *H) {
     const double k = m.kap, a2 = a * E.ir2, b2 = b * E.ir2, c2 = c * E.ir2, cc = c * c;
-    const cd d6 = E.dd * m.six_c2s;
-    cd h1 = d6, h2 = d6, h4 = d6 * (-5.0);
+    const T d6 = E.dd * m.six_c2s;
+    T h1 = d6, h2 = d6, h4 = d6 * (-5.0);
     fma_cr(h1, E.e1, 4.0 * k - 1.0), fma_cr(h1, E.e2, -2.0), fma_cr(h1, E.w1, 2.0 * k - 1.0);
     fma_cr(h2, E.e1, 2.0 * k), fma_cr(h2, E.e2, -3.0), h2 -= E.w2;
     fma_cr(h4, E.e1, -12.0 * k), fma_cr(h4, E.e2, 12.0), fma_cr(h4, E.w1, -2.0 * k), fma_cr(h4, E.w2, 2.0);
-    const cd hc = h4 * c2;
+    const T hc = h4 * c2;
     H[0] = H[1] = h2 * c2;
     fma_cr(H[0], hc, a * a), fma_cr(H[1], hc, b * b);
     H[3] = hc * (a * b);
-    cd p1 = h1, p2 = h2;
+    T p1 = h1, p2 = h2;
     fma_cr(p1, h4, cc), fma_cr(p2, h4, cc);
     H[4] = p1 * a2, H[5] = p1 * b2, H[6] = p2 * a2, H[7] = p2 * b2;
     fma_cr(p1, h2, 2.0);

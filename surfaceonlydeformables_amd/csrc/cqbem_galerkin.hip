@@ -743,7 +743,7 @@ __global__ void __launch_bounds__(64 * NW, 2) k_gal_touch(Geom g, const Pair *__
             asm volatile("" : "+v"(ln));
             const TouchDir D = dir[ln];
             const double a = D.id_a.y, b = D.bc.x, c = D.bc.y;
-            PointExpo E;
+            PointExpo<cd> E;
             E.ir = D.id_a.x, E.ir2 = E.ir * E.ir;
             const TouchItem &I = item[j];
             const cd q1 = I.is * E.ir, q2 = CLOSE ? q1 * q1 : I.is2 * E.ir2;
@@ -1238,7 +1238,7 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
                         // the patch kernel at the test points: timed on its own, with its launches and its unique
                         // evaluations (test point, regular source face, source point, frequency)
                         EvTimer tp(st, &tm[2]);
-                        check(launch_colloc_gh_patch(g, job.patch_pts, npts, job.freqs, 0, nl, job.mat, row0, nrows,
+                        check(launch_colloc_gh_patch(g, job.patch_pts, npts, job.freqs, 0, nl, job.real_ends, job.mat, row0, nrows,
                                                     tpts, job.patch_chunk, job.chunk_info, job.chunk_faces, job.patch_verts,
                                                     job.npatches, sG, sH, n3, ls, st),
                               "k_colloc_gh_patch (test points)");
@@ -1255,7 +1255,7 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
                                                 cap_rows, st),
                               "k_colloc_b32 (test points)");
                     else
-                        check(launch_points_b(g, job.quad, npts, job.freqs, 0, nl, job.mat, tpts, row0, nrows, sBt, sBa,
+                        check(launch_points_b(g, job.quad, npts, job.freqs, 0, nl, job.real_ends, job.mat, tpts, row0, nrows, sBt, sBa,
                                               cap_rows, st),
                               "k_colloc_b (test points)");
                     project(sBt, 3, cap_rows * 3, faces + fi0, nfc, row0, Bt, n3 * 3);

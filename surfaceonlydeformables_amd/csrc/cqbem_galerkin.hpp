@@ -17,6 +17,7 @@ struct GalerkinJob {
     int nline;
     const Freq *freqs;    // first frequency of the job's range
     int nl;               // number of frequencies
+    bool real_ends;       // s is real at the first and the last of them (Prepared::real_ends)
     Mat mat;
     int num_cus;
     // patch-form tables of the collocation G/H kernel (column patches; see launch_colloc_gh_patch)

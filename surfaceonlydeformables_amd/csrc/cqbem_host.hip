@@ -207,6 +207,11 @@ struct Prepared {
     std::vector<Freq> freqs;
     std::vector<double2> tab;
     Mat mat;
+    // whether frequencies l0 .. l0 + nl - 1 are the half spectrum of an even L, or one real frequency of it: s is then
+    // real at the first and the last, and the kernels compute the two together, in the same arithmetic for both calls
+    bool real_ends(int l0, int nl) const {
+        return L % 2 == 0 && ((l0 == 0 && nl == Lf) || (nl == 1 && (l0 == 0 || l0 == Lf - 1)));
+    }
 };
 
 // CQBEM_QUAD_BANDED default: far when the row point is kBandKappa largest face diameters beyond the patch's bounding
@@ -590,7 +595,7 @@ hipError_t launch_gh(const DevMesh &d, const Prepared &P, const Freq *freqs, int
                      cd *UH, long long ld, long long lstride, hipStream_t st) {
     if (colloc_star() && P.far_patch_pts.empty())
         return launch_colloc_gh(d.g, d.quad.as<double4>(), P.npts, freqs, l0, nl, P.mat, row0, nrows, UG, UH, ld, lstride, st);
-    return launch_colloc_gh_patch(d.g, d.patch_pts.as<double4>(), P.npts, freqs, l0, nl, P.mat, row0, nrows,
+    return launch_colloc_gh_patch(d.g, d.patch_pts.as<double4>(), P.npts, freqs, l0, nl, P.real_ends(l0, nl), P.mat, row0, nrows,
                                  nullptr, d.patch_chunk.as<int>(), d.chunk_info.as<int4>(), d.chunk_faces.as<int4>(),
                                  d.patch_verts.as<int>(), P.npatches, UG, UH, ld, lstride, st, bands_of(d, P));
 }
@@ -814,7 +819,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
                     HIPCHK(launch_colloc_b32(g, quad, npts, freqs32, 0, Lf, mat32, 0, nv, specB.as<cd>(), specBa.as<cd>(), st,
                                              fbands_of(d, P)));
                 else
-                    HIPCHK(launch_colloc_b(g, quad, npts, freqs, 0, Lf, P.mat, 0, nv, specB.as<cd>(), specBa.as<cd>(), st,
+                    HIPCHK(launch_colloc_b(g, quad, npts, freqs, 0, Lf, P.real_ends(0, Lf), P.mat, 0, nv, specB.as<cd>(), specBa.as<cd>(), st,
                                            fbands_of(d, P)));
             }
             {
@@ -834,7 +839,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
                 HIPCHK(launch_add_c_colloc(H, dC.as<double>(), nv, st));
         }
     } else {
-        GalerkinJob gj{g, quad, npts, line, nline, freqs, Lf, P.mat, ctx->num_cus, d.patch_pts.as<double4>(),
+        GalerkinJob gj{g, quad, npts, line, nline, freqs, Lf, P.real_ends(0, Lf), P.mat, ctx->num_cus, d.patch_pts.as<double4>(),
                        d.patch_chunk.as<int>(), d.chunk_info.as<int4>(), d.chunk_faces.as<int4>(),
                        d.patch_verts.as<int>(), P.npatches, galerkin_budget(slab_budget)};
         if (mixed) gj.freqs32 = freqs32, gj.mat32 = mat32;  // far-field B at the test points in float
@@ -1112,19 +1117,20 @@ void run_scene(cqbem_context *ctx, hipStream_t st, int n, const cqbem_mesh *mesh
             // objects with the float G kernel: H through the shared launch, G through the float kernel
             const bool g_in_patch = o->wantG && !o->g32;
             if (!g_in_patch && !o->wantH) continue;
+            const bool ends = o->P.real_ends(0, o->P.Lf);
             ScenePiece sp{o->d.g, o->d.patch_pts.as<double4>(), o->P.npts, o->d.freqs.as<Freq>(), o->P.mat,
-                          pc.row0, pc.nrows, 1, o->P.Lf, o->P.npatches, o->d.patch_chunk.as<int>(),
+                          pc.row0, pc.nrows, 1, ends ? std::max(o->P.Lf - 1, 1) : o->P.Lf, ends ? o->P.Lf - 1 : -1, o->P.npatches, o->d.patch_chunk.as<int>(),
                           o->d.chunk_info.as<int4>(), o->d.chunk_faces.as<int4>(), o->d.patch_verts.as<int>(),
                           g_in_patch ? sG : nullptr, o->wantH ? sH : nullptr, n3, lstride, 0u, bands_of(o->d, o->P)};
             (g_in_patch ? (o->wantH ? gh : gonly) : honly).push_back(sp);
         }
         auto number = [](std::vector<ScenePiece> &v) {
             long long base = 0, tiles = 0;
-            for (auto &sp : v) tiles += (long long)sp.npatches * sp.nl * sp.nrows;
+            for (auto &sp : v) tiles += (long long)sp.npatches * sp.slots * sp.nrows;
             for (auto &sp : v) {
                 sp.rpt = patch_rows_per_tile(tiles);
                 sp.base = (unsigned)base;
-                base += (long long)sp.npatches * sp.nl * ((sp.nrows + sp.rpt - 1) / sp.rpt);
+                base += (long long)sp.npatches * sp.slots * ((sp.nrows + sp.rpt - 1) / sp.rpt);
             }
             if (base >= (1LL << 31)) throw Err{CQBEM_ERR_UNSUPPORTED, "assemble_scene: too many tiles in one wave"};
             return base;
@@ -1214,7 +1220,7 @@ void run_scene(cqbem_context *ctx, hipStream_t st, int n, const cqbem_mesh *mesh
                 HIPCHK(launch_colloc_b32(g, o->d.quad.as<double4>(), o->P.npts, o->dfreq32.as<FreqF>(), 0, Lf, o->mat32, 0, nv,
                                          o->specB.as<cd>(), o->specBa.as<cd>(), st, fbands_of(o->d, o->P)));
             else
-                HIPCHK(launch_colloc_b(g, o->d.quad.as<double4>(), o->P.npts, freqs, 0, Lf, o->P.mat, 0, nv, o->specB.as<cd>(),
+                HIPCHK(launch_colloc_b(g, o->d.quad.as<double4>(), o->P.npts, freqs, 0, Lf, o->P.real_ends(0, Lf), o->P.mat, 0, nv, o->specB.as<cd>(),
                                        o->specBa.as<cd>(), st, fbands_of(o->d, o->P)));
             HIPCHK(launch_colloc_singular(1, g, o->d.line.as<double2>(), (int)o->P.line.size(), freqs, 0, Lf, o->P.mat, 0, nv,
                                           nullptr, n3, 0, o->specB.as<cd>(), o->specBa.as<cd>(), st));
@@ -1596,13 +1602,13 @@ int cqbem_laplace(cqbem_context *ctx, const cqbem_mesh *mesh, const cqbem_params
                     HIPCHK(launch_colloc_b32(d.g, quad, npts, dfreq32.as<FreqF>(), l, 1, mat32, 0, nv, dBt.as<cd>(), dBa.as<cd>(), st,
                                              fbands_of(d, P)));
                 else
-                    HIPCHK(launch_colloc_b(d.g, quad, npts, freqs, l, 1, P.mat, 0, nv, dBt.as<cd>(), dBa.as<cd>(), st,
+                    HIPCHK(launch_colloc_b(d.g, quad, npts, freqs, l, 1, P.real_ends(l, 1), P.mat, 0, nv, dBt.as<cd>(), dBa.as<cd>(), st,
                                            fbands_of(d, P)));
                 HIPCHK(launch_colloc_singular(1, d.g, line, nline, freqs, l, 1, P.mat, 0, nv, nullptr, n3, 0, dBt.as<cd>(),
                                               dBa.as<cd>(), st));
             }
         } else {
-            GalerkinJob gj{d.g, quad, npts, line, nline, freqs + l, 1, P.mat, ctx->num_cus, d.patch_pts.as<double4>(),
+            GalerkinJob gj{d.g, quad, npts, line, nline, freqs + l, 1, P.real_ends(l, 1), P.mat, ctx->num_cus, d.patch_pts.as<double4>(),
                            d.patch_chunk.as<int>(), d.chunk_info.as<int4>(),
                            d.chunk_faces.as<int4>(), d.patch_verts.as<int>(), P.npatches, (size_t)1 << 30};
             if (mixed) gj.freqs32 = dfreq32.as<FreqF>() + l, gj.mat32 = mat32;

@@ -141,16 +141,19 @@ __global__ void __launch_bounds__(64) k_colloc_gh(Geom g, const double4 *__restr
 // different entries, and keeps the sums of all three corner basis functions in
 // registers (84 doubles with G and H); the rule's points and weights are
 // wave-uniform (scalar loads).  After the rule it rotates each corner's sums to
-// the global axes and adds them to per-vertex LDS accumulators.  The waves add in chunk order (an LDS turn counter) and, within a chunk, in
-// sub-steps that the host schedules so that no vertex is updated twice in one
-// sub-step: every sum has one order, whatever the hardware's.  The block then
-// writes each (row, column) block once.
+// the global axes and adds them to per-vertex LDS accumulators.  The waves add in
+// chunk order (an LDS turn counter) and, within a chunk, in sub-steps that the
+// host schedules so that no vertex is updated twice in one sub-step: every sum
+// has one order, whatever the hardware's.  The block then writes each (row,
+// column) block once.  The first and the last frequency of an even L, where s is
+// real, are one slot (T = rp: two real numbers in the place of a complex one).
 //
 // Bound by FP64 VALU issue (and, near full issue, by the clock that the power
 // limit leaves): 292 VALU instructions per point, of which 84 are the corner
 // sums and 78 the two complex exponentials, and 1100 per face and row outside
 // the rule.  Icosphere level 4, L = 32, 28 points (6.2e9 unique evaluations):
-// 80.2 ms, 2.25 ms per point of the rule plus 17 ms.  The form it replaces, two
+// 76.8 ms (80.8 with a slot for each real frequency), 2.25 ms per point of the
+// rule plus 17 ms at 17 slots.  The form it replaces, two
 // lanes per face that swapped every point's 16 global entries through DPP, took
 // 128 ms at 516 instructions per point.  Tried and slower: the same with a
 // block barrier per sub-step (86.5 ms), the rotation inside the wave's turn
@@ -182,6 +185,23 @@ __device__ inline void wait_for(int *counter, int v) {
         __builtin_amdgcn_s_sleep(1);
 }
 
+// Whether one of the first N vertices t and one of the face's corners c are the same mesh vertex (same_vertex of every
+// pair), without a branch per pair.
+template <int N>
+__device__ inline bool touches(const Geom &g, const int (&t)[3], const int (&c)[3]) {
+    int tt[3] = {t[0], t[1], t[2]}, cc[3] = {c[0], c[1], c[2]};
+    if (g.vmap) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) tt[k] = g.vmap[t[k]], cc[k] = g.vmap[c[k]];
+    }
+    bool any = false;
+#pragma unroll
+    for (int k = 0; k < N; k++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) any |= tt[k] == cc[j];
+    return any;
+}
+
 // The rows il0 .. il0 + nr - 1 of one (patch pc, frequency l) for a block of kPatchThreads threads.  acc, frame,
 // counters (2) and mtab are the block's LDS (mtab loaded); callers that run another tile on the same LDS synchronise
 // first.  The block has no barrier between its rows: a wave evaluates its first chunk of the next row before it writes
@@ -193,21 +213,14 @@ struct PatchDest {
     cd *UG, *UH;
     long long ld, lstride;
 };
-template <bool DG, bool DH, bool GAL, class Dest>
+template <class T, bool DG, bool DH, bool GAL, class Dest>
 __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, const double4 *__restrict__ ref_pts, int ref_npts,
-                                 const Bands &bands, const Freq *__restrict__ freqs,
-                                 int l0, const Mat &m, int row0, const double4 *__restrict__ tpts,
+                                 const Bands &bands, const PointFreq<T> &f, const Mat &m, int row0, const double4 *__restrict__ tpts,
                                  const int *__restrict__ patch_chunk, const int4 *__restrict__ chunk_info,
                                  const int4 *__restrict__ chunk_faces, const Dest &dest, int pc, int l,
                                  int il0, int nr, double2 *acc, double2 *frame, int *counters, const MathTables &mtab) {
     constexpr int kWaves = kPatchThreads / 64;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    Freq f;  // one frequency's constants, in scalar registers
-    {
-        const_double *src = (const_double *)(freqs + (l0 + l));
-        f.s = cd{src[0], src[1]}, f.sc1 = cd{src[2], src[3]}, f.sc2 = cd{src[4], src[5]}, f.is = cd{src[6], src[7]},
-        f.is2 = cd{src[8], src[9]};
-    }
     for (int k = tid; k < kPatchPairs * kPatchVerts; k += kPatchThreads) acc[k] = make_double2(0.0, 0.0);
     int *turns = counters, *cleared = counters + 1;  // chunks added so far; waves that cleared their slots, over all rows
     if (tid < 2) counters[tid] = 0;
@@ -225,20 +238,20 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
         const PatchDest D = dest();
         const int j = D.patch_verts[pc * kPatchVerts + tid];
         if (j >= 0) {
-            const long long obase = (long long)l * D.lstride + (long long)(3 * (il0 + r)) * D.ld + 3 * (long long)j;
+            // cd: one complex entry at frequency l; rp: the real entries at frequencies 0 and l
+            constexpr bool kReal = std::is_same<T, rp>::value;
+            const long long obase = (kReal ? 0 : (long long)l * D.lstride) + (long long)(3 * (il0 + r)) * D.ld + 3 * (long long)j;
+            auto put = [&](cd *o, const double2 &w, double scale) {
+                *o = kReal ? cd{w.x * scale, 0.0} : cd{w.x * scale, w.y * scale};
+                if (kReal) o[(long long)l * D.lstride] = cd{w.y * scale, 0.0};
+            };
 #pragma unroll
             for (int p = 0; p < 3; p++) {
 #pragma unroll
                 for (int b = 0; b < 3; b++) {
                     const int e = sidx(p, b);
-                    if (DG) {
-                        const double2 w = acc[e * kPatchVerts + tid];
-                        D.UG[obase + p * D.ld + b] = cd{w.x, w.y} * m.g_scale;
-                    }
-                    if (DH) {
-                        const double2 w = acc[(6 + p * 3 + b) * kPatchVerts + tid];
-                        D.UH[obase + p * D.ld + b] = cd{w.x, w.y} * kInv4Pi;
-                    }
+                    if (DG) put(D.UG + obase + p * D.ld + b, acc[e * kPatchVerts + tid], m.g_scale);
+                    if (DH) put(D.UH + obase + p * D.ld + b, acc[(6 + p * 3 + b) * kPatchVerts + tid], kInv4Pi);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -259,9 +272,9 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
         double x0, x1, x2;
         int tv[3] = {i, i, i};
         if (GAL) {
-            const double4 T = tpts[i];
-            x0 = T.x, x1 = T.y, x2 = T.z;
-            const int f1 = (int)T.w;
+            const double4 P = tpts[i];
+            x0 = P.x, x1 = P.y, x2 = P.z;
+            const int f1 = (int)P.w;
             tv[0] = g.F[3 * f1], tv[1] = g.F[3 * f1 + 1], tv[2] = g.F[3 * f1 + 2];
         } else {
             x0 = g.V[3 * i], x1 = g.V[3 * i + 1], x2 = g.V[3 * i + 2];
@@ -280,11 +293,10 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
         const int entry = info.x + min(lane, info.y - 1);
         const int4 fe = chunk_faces[entry];
         const int va[3] = {fe.x & 0xffffff, fe.y & 0xffffff, fe.z & 0xffffff};
-        bool active = lane < info.y;
-        for (int k = 0; k < (GAL ? 3 : 1); k++)
-            active = active && !(same_vertex(g, tv[k], va[0]) || same_vertex(g, tv[k], va[1]) || same_vertex(g, tv[k], va[2]));
+        const bool touch = touches<GAL ? 3 : 1>(g, tv, va);
+        const bool active = (lane < info.y) & !touch;
         const unsigned long long act = __builtin_amdgcn_ballot_w64(active);
-        cd sg[3][6], sh[3][8];
+        T sg[3][6], sh[3][8];
         if (act) {  // wave-uniform: no divergent merge of the sums
             {
                 double y[3][3];
@@ -304,17 +316,17 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
                 const double2 F0 = frame[ln], F1 = frame[kPatchThreads + ln], F2 = frame[2 * kPatchThreads + ln];
                 const_double *B = as_const(pts + 2 * q);  // b1, b2, -, -, w (phi_0, phi_1, phi_2, 1)
                 const double ar = fma(B[0], F0.x, fma(B[1], F0.y, F1.y)), br = fma(B[1], F1.x, F2.x), cr = F2.y;
-                const PointExpo E = point_expo(fma(ar, ar, fma(br, br, cr * cr)), f, &mtab);
+                const PointExpo<T> E = point_expo(fma(ar, ar, fma(br, br, cr * cr)), f, &mtab);
                 const double w[3] = {B[4], B[5], B[6]};
                 const double a = ar * E.ir, b = br * E.ir, c = cr * E.ir;
-                auto add = [&](cd &s, const cd &v, double wk) {
+                auto add = [&](T &s, const T &v, double wk) {
                     if (first()) s = v * wk;
                     else fma_cr(s, v, wk);
                 };
                 // G and H one after the other, so that only one set of entries is live beside the sums
                 __builtin_amdgcn_sched_barrier(0);
                 if (DG) {
-                    cd G[6];
+                    T G[6];
                     point_g(E, a, b, c, m, G);
 #pragma unroll
                     for (int k = 0; k < 3; k++)
@@ -323,7 +335,7 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 if (DH) {
-                    cd H[8];
+                    T H[8];
                     point_h(E, a, b, c, m, H);
 #pragma unroll
                     for (int k = 0; k < 3; k++)
@@ -338,9 +350,9 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
 #pragma unroll
             for (int k = 0; k < 3; k++) {
 #pragma unroll
-                for (int e = 0; e < 6; e++) sg[k][e] = cd{0, 0};
+                for (int e = 0; e < 6; e++) sg[k][e] = T{0, 0};
 #pragma unroll
-                for (int e = 0; e < 8; e++) sh[k][e] = cd{0, 0};
+                for (int e = 0; e < 8; e++) sh[k][e] = T{0, 0};
             }
         }
         while (written < r) write_row(written++);
@@ -419,15 +431,22 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_colloc_gh_patch(Geom g, co
                                                                   const int4 *__restrict__ chunk_faces,
                                                                   const int *__restrict__ patch_verts, cd *__restrict__ UG,
                                                                   cd *__restrict__ UH, long long ld, long long lstride,
-                                                                  int nrows, int rpt, Bands bands) {
+                                                                  int nrows, int rpt, int real_hi, Bands bands) {
     __shared__ double2 acc[kPatchPairs * kPatchVerts];      // [word][slot]
     __shared__ double2 frame[kFramePairs * kPatchThreads];
     __shared__ int counters[2];  // [word pair][lane]
     __shared__ MathTables mtab;                       // tables of the exponentials
     load_math_tables(&mtab);
-    patch_tile<DG, DH, GAL>(g, pts, npts, BANDED ? bands : Bands{}, freqs, l0, m, row0, tpts, patch_chunk, chunk_info,
-                           chunk_faces, [=] { return PatchDest{patch_verts, UG, UH, ld, lstride}; }, blockIdx.x, blockIdx.y, blockIdx.z * rpt,
-                           min(rpt, nrows - (int)blockIdx.z * rpt), acc, frame, counters, mtab);
+    auto dest = [=] { return PatchDest{patch_verts, UG, UH, ld, lstride}; };
+    const int r0 = blockIdx.z * rpt, nr = min(rpt, nrows - r0);
+    if (real_hi >= 0 && blockIdx.y == 0)
+        patch_tile<rp, DG, DH, GAL>(g, pts, npts, BANDED ? bands : Bands{}, point_freq(freqs + l0, real_hi, rp{}), m, row0, tpts,
+                                    patch_chunk, chunk_info, chunk_faces, dest, blockIdx.x, real_hi, r0, nr, acc, frame,
+                                    counters, mtab);
+    else
+        patch_tile<cd, DG, DH, GAL>(g, pts, npts, BANDED ? bands : Bands{}, point_freq(freqs, l0 + blockIdx.y, cd{}), m, row0, tpts,
+                                    patch_chunk, chunk_info, chunk_faces, dest, blockIdx.x, blockIdx.y, r0, nr, acc, frame,
+                                    counters, mtab);
 }
 
 // ------------------------------------------------------------------------
@@ -465,12 +484,18 @@ __device__ __attribute__((always_inline)) inline void scene_tile(const ScenePiec
         return PatchDest{as_global((const int *)ptr(&q->patch_verts)), as_global((cd *)ptr(&q->UG)), as_global((cd *)ptr(&q->UH)),
                          (long long)ptr(&q->ld), (long long)ptr(&q->lstride)};
     };
-    const unsigned local = t - P.base, np = (unsigned)P.npatches, nl = (unsigned)P.nl;
+    const unsigned local = t - P.base, np = (unsigned)P.npatches, nl = (unsigned)P.slots;
     const unsigned rest = local / np;
     const int pc = __builtin_amdgcn_readfirstlane(local - rest * np), l = __builtin_amdgcn_readfirstlane(rest % nl),
               r0 = __builtin_amdgcn_readfirstlane(rest / nl) * P.rpt;
-    patch_tile<DG, DH, false>(P.g, P.pts, P.npts, P.bands, as_global(P.freqs), 0, P.m, P.row0, nullptr, as_global(P.patch_chunk),
-                              P.chunk_info, as_global(P.chunk_faces), dest, pc, l, r0, min(P.rpt, P.nrows - r0), acc, frame, counters, mtab);
+    if (P.real_hi >= 0 && l == 0)
+        patch_tile<rp, DG, DH, false>(P.g, P.pts, P.npts, P.bands, point_freq(P.freqs, P.real_hi, rp{}), P.m, P.row0, nullptr,
+                                      as_global(P.patch_chunk), P.chunk_info, as_global(P.chunk_faces), dest, pc, P.real_hi, r0,
+                                      min(P.rpt, P.nrows - r0), acc, frame, counters, mtab);
+    else
+        patch_tile<cd, DG, DH, false>(P.g, P.pts, P.npts, P.bands, point_freq(P.freqs, l, cd{}), P.m, P.row0, nullptr,
+                                      as_global(P.patch_chunk), P.chunk_info, as_global(P.chunk_faces), dest, pc, l, r0,
+                                      min(P.rpt, P.nrows - r0), acc, frame, counters, mtab);
 }
 
 template <bool DG, bool DH>
@@ -509,68 +534,59 @@ __global__ void k_zero_counter(unsigned *counter) {
 }
 
 // ------------------------------------------------------------------------
-// B_trans and B_angular, regular faces.  Grid: (nl, rows), 256 threads; lanes
-// stride over the faces, then a wave shuffle reduction and one LDS pass.
+// B_trans and B_angular, regular faces.  NW waves per (row, frequency slot), 4 waves per block: the lanes stride over the
+// faces, then the 48 sums are reduced over the lanes and the NW waves.
 //
 // Bound by FP64 VALU issue.  A point adds to 12 complex moments of its face
 // (h, n.h, h h and two scalars, each times a function of r and s); every factor
 // that depends on the frequency alone (1/s^2, s, 1/s) waits until the face's
 // or the row's end, and the trace of the h h moment serves as the scalar moment
 // of the same function (|h| = 1).  156 instructions per point; with the factors
-// applied per point it was 203.  Icosphere level 4, L = 32: 34.0 ms (43.0).
+// applied per point it was 203.  The two real frequencies of an even L share a
+// slot in real arithmetic (133 per point for both).  Icosphere level 4, L = 32:
+// 31.9 ms (33.1 with a slot each, 43.0 at 203).
 // ------------------------------------------------------------------------
 constexpr int kBWords = 48;  // B_trans (6 sym complex) + B_angular (18 complex), as doubles
 
-// GAL: the rows are test points tpts[row0 + y] (x, y, z, face) whose face's corners are excluded, written to
-// rows 3y..3y+2 of an nv3-row buffer; otherwise collocation vertex i = row0 + y, written to rows 3i..3i+2.
+// One lane's sums over its faces: words 2 k, 2 k + 1 of out are entry k, in units of 1/(8 pi s^2).
+// GAL: the row is test point tpts[i] (x, y, z, face), whose face's corners are excluded; otherwise vertex i.
 // BANDED: each face takes the far rule or the reference rule (a lane then reads its own rule's points; without bands
 // they are wave-uniform).
-template <bool GAL, bool BANDED>
-__global__ void __launch_bounds__(256) k_colloc_b(Geom g, const double4 *__restrict__ quad, int npts,
-                                                   const Freq *__restrict__ freqs, int l0, Mat m, int row0,
-                                                   const double4 *__restrict__ tpts, cd *__restrict__ Bt,
-                                                   cd *__restrict__ Ba, long long nv3, FaceBands fb) {
-    __shared__ double red[4][kBWords];
-    __shared__ MathTables mtab;  // tables of the exponentials
-    load_math_tables(&mtab);
-    __syncthreads();
-    const int l = blockIdx.x;
-    const int i = row0 + blockIdx.y;
-    const Freq f = freqs[l0 + l];
+template <class T, bool GAL, bool BANDED>
+__device__ __attribute__((always_inline)) inline void b_sums(const Geom &g, const double4 *__restrict__ quad, int npts,
+                                                             const PointFreq<T> &f, const Mat &m, int i,
+                                                             const double4 *__restrict__ tpts, int first, int step,
+                                                             const FaceBands &fb, const MathTables &mtab, double (&out)[kBWords]) {
     double x[3];
     int t[3] = {i, i, i};
     if (GAL) {
-        const double4 T = tpts[i];
-        x[0] = T.x, x[1] = T.y, x[2] = T.z;
-        const int f1 = (int)T.w;
+        const double4 P = tpts[i];
+        x[0] = P.x, x[1] = P.y, x[2] = P.z;
+        const int f1 = (int)P.w;
         t[0] = g.F[3 * f1], t[1] = g.F[3 * f1 + 1], t[2] = g.F[3 * f1 + 2];
     } else {
         x[0] = g.V[3 * i], x[1] = g.V[3 * i + 1], x[2] = g.V[3 * i + 2];
     }
-    const int io = GAL ? (int)blockIdx.y : i;
-    cd bt[6], ba[18];  // the row's sums in units of 1/(8 pi s^2)
+    T bt[6], ba[18];  // the row's sums in units of 1/(8 pi s^2)
 #pragma unroll
-    for (int k = 0; k < 6; k++) bt[k] = cd{0, 0};
+    for (int k = 0; k < 6; k++) bt[k] = T{0, 0};
 #pragma unroll
-    for (int k = 0; k < 18; k++) ba[k] = cd{0, 0};
-    for (int fc = threadIdx.x; fc < g.nf; fc += 256) {
-        const int a0 = g.F[3 * fc], a1 = g.F[3 * fc + 1], a2 = g.F[3 * fc + 2];
-        bool touch = false;
-        for (int k = 0; k < (GAL ? 3 : 1); k++)
-            touch = touch || same_vertex(g, t[k], a0) || same_vertex(g, t[k], a1) || same_vertex(g, t[k], a2);
-        if (touch) continue;
+    for (int k = 0; k < 18; k++) ba[k] = T{0, 0};
+    for (int fc = first; fc < g.nf; fc += step) {
+        const int c[3] = {g.F[3 * fc], g.F[3 * fc + 1], g.F[3 * fc + 2]};
+        if (touches<GAL ? 3 : 1>(g, t, c)) continue;
         // y - x = o + b1 e1 + b2 e2, whose component along the normal is the same at every point
         double o[3], e1[3], e2[3];
         const double n[3] = {g.N[3 * fc], g.N[3 * fc + 1], g.N[3 * fc + 2]};
 #pragma unroll
         for (int k = 0; k < 3; k++)
-            o[k] = g.V[3 * a0 + k] - x[k], e1[k] = g.V[3 * a1 + k] - g.V[3 * a0 + k], e2[k] = g.V[3 * a2 + k] - g.V[3 * a0 + k];
+            o[k] = g.V[3 * c[0] + k] - x[k], e1[k] = g.V[3 * c[1] + k] - g.V[3 * c[0] + k], e2[k] = g.V[3 * c[2] + k] - g.V[3 * c[0] + k];
         const double4 *qf = quad;  // the face's rule
         int nq = npts;
         if (BANDED && beyond_sphere(x[0], x[1], x[2], fb.sphere[fc])) qf = fb.far_quad, nq = fb.far_npts;
-        cd mt[3] = {{0, 0}, {0, 0}, {0, 0}}, m2 = {0, 0}, M[6], S = {0, 0}, S3 = {0, 0};
+        T mt[3] = {{0, 0}, {0, 0}, {0, 0}}, m2 = {0, 0}, M[6], S = {0, 0}, S3 = {0, 0};
 #pragma unroll
-        for (int k = 0; k < 6; k++) M[k] = cd{0, 0};
+        for (int k = 0; k < 6; k++) M[k] = T{0, 0};
 #pragma unroll 1
         for (int q = 0; q < nq; ++q) {
             double b1, b2, w;
@@ -586,9 +602,9 @@ __global__ void __launch_bounds__(256) k_colloc_b(Geom g, const double4 *__restr
             for (int k = 0; k < 3; k++) d[k] = fma(b1, e1[k], fma(b2, e2[k], o[k]));
             const double d2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
             const double ir = rsqrt_h3(d2), r = d2 * ir;
-            const cd z1 = f.sc1 * r, z2 = f.sc2 * r;
-            const cd E1 = cexp_neg_tab(z1, &mtab), E2 = cexp_neg_tab(z2, &mtab);
-            const cd s2 = z2 * E2 + E2, dS = (z1 * E1 + E1) - s2;  // s^2 A2, s^2 (A1 - A2)
+            const T z1 = f.sc1 * r, z2 = f.sc2 * r;
+            const T E1 = cexp_neg_tab(z1, &mtab), E2 = cexp_neg_tab(z2, &mtab);
+            const T s2 = z2 * E2 + E2, dS = (z1 * E1 + E1) - s2;  // s^2 A2, s^2 (A1 - A2)
             const double w2 = (w * ir) * ir, w3 = w2 * ir;
             const double h[3] = {w3 * d[0], w3 * d[1], w3 * d[2]};  // w h / r^2
 #pragma unroll
@@ -597,9 +613,9 @@ __global__ void __launch_bounds__(256) k_colloc_b(Geom g, const double4 *__restr
 #pragma unroll
                 for (int b = a; b < 3; b++) fma_cr(M[sidx(a, b)], dS, h[a] * d[b]);  // w h h / r
             }
-            fma_cr(m2, cd{s2.x - 1.0, s2.y}, w3);
-            const cd v = E2 * m.ic2;
-            cd u = v;
+            fma_cr(m2, add_one(s2, -1.0), w3);
+            const T v = E2 * m.ic2;
+            T u = v;
             fma_cr(u, E1, -m.ic1);
             fma_cr(S, u, w);
             fma_cr(S3, v, w);
@@ -618,50 +634,103 @@ __global__ void __launch_bounds__(256) k_colloc_b(Geom g, const double4 *__restr
         for (int a = 0; a < 3; a++)
 #pragma unroll
             for (int b = a; b < 3; b++) {
-                cd &v = bt[sidx(a, b)];
+                T &v = bt[sidx(a, b)];
                 fma_cr(v, mt[a], n[b]);
                 fma_cr(v, mt[b], n[a]);
                 if (a == b) v += m2;
 #pragma unroll
                 for (int k = 0; k < 3; k++) {
-                    cd &u = ba[sidx(a, b) * 3 + k];
+                    T &u = ba[sidx(a, b) * 3 + k];
                     fma_cr(u, M[sidx(a, k)], n[b]);
                     fma_cr(u, M[sidx(b, k)], n[a]);
                     if (a == b) fma_cr(u, S3, n[k]);
                 }
             }
     }
-    // wave reduction of the 48 partial sums, then the 4 waves through LDS (fixed order)
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
-    for (int k = 0; k < kBWords; k++) {
-        double v = k < 12 ? (k & 1 ? bt[k >> 1].y : bt[k >> 1].x) : (k & 1 ? ba[(k - 12) >> 1].y : ba[(k - 12) >> 1].x);
+    for (int k = 0; k < 6; k++) out[2 * k] = bt[k].x, out[2 * k + 1] = bt[k].y;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        if (lane == 0) red[wave][k] = v;
+    for (int k = 0; k < 18; k++) out[12 + 2 * k] = ba[k].x, out[13 + 2 * k] = ba[k].y;
+}
+
+// Sums v over the 64 lanes: lanes 8 j .. 8 j + 7 get the sums of words 6 j .. 6 j + 5 in v[0..5].  Three steps halve the
+// words a lane holds (48, 24, 12, 6), the last three add the same 6: 60 exchanges, where 6 steps of 48 words are 288.
+__device__ __attribute__((always_inline)) inline void wave_sum48(double (&v)[kBWords], int lane) {
+#pragma unroll
+    for (int n = 24, o = 32; n >= 6; n /= 2, o /= 2) {
+        const bool hi = lane & o;
+#pragma unroll
+        for (int k = 0; k < n; k++) v[k] = (hi ? v[k + n] : v[k]) + __shfl_xor(hi ? v[k] : v[k + n], o, 64);
     }
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+        for (int k = 0; k < 6; k++) v[k] += __shfl_xor(v[k], o, 64);
+}
+
+// GAL: the rows are test points row0 + r, written to rows 3r..3r+2 of an nv3-row buffer; otherwise collocation vertices
+// i = row0 + r, written to rows 3i..3i+2.
+template <int NW, bool GAL, bool BANDED>
+__global__ void __launch_bounds__(256, 2) k_colloc_b(Geom g, const double4 *__restrict__ quad, int npts,
+                                                   const Freq *__restrict__ freqs, int l0, int slots, Mat m, int row0, int nrows,
+                                                   const double4 *__restrict__ tpts, cd *__restrict__ Bt,
+                                                   cd *__restrict__ Ba, long long nv3, int real_hi, FaceBands fb) {
+    __shared__ double red[4][kBWords];
+    __shared__ MathTables mtab;  // tables of the exponentials
+    load_math_tables(&mtab);
     __syncthreads();
-    if (threadIdx.x < kBWords) {
-        const int k = threadIdx.x;
-        const int c = k & 1, e0 = k & ~1;
-        auto total = [&](int j) { return (red[0][j] + red[1][j]) + (red[2][j] + red[3][j]); };
-        const cd sum = cd{total(e0), total(e0 + 1)} * f.is2;
-        const double v = (c ? sum.y : sum.x) * kInv8Pi;
-        // scatter the packed symmetric entries to their full positions
-        if (k < 12) {
-            const int e = k >> 1;
-            double *bt_out = reinterpret_cast<double *>(Bt + (long long)l * nv3 * 3 + (long long)(3 * io) * 3);
-            for (int a = 0; a < 3; a++)
-                for (int b = 0; b < 3; b++)
-                    if (sidx(a, b) == e) bt_out[2 * (a * 3 + b) + c] = v;
-        } else {
-            const int e = (k - 12) >> 1, sab = e / 3, kk = e % 3;
-            double *ba_out = reinterpret_cast<double *>(Ba + (long long)l * nv3 * 9 + (long long)(3 * io) * 9);
-            for (int a = 0; a < 3; a++)
-                for (int b = 0; b < 3; b++)
-                    if (sidx(a, b) == sab) ba_out[2 * (a * 9 + b * 3 + kk) + c] = v;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    // (row, slot) of this group of NW waves, numbered with the slots fastest; past the end: nothing to sum or write
+    const unsigned job = blockIdx.x * (4 / NW) + wave / NW;
+    const int r = job / (unsigned)slots, slot = job - (unsigned)r * slots, i = row0 + r;
+    const bool valid = r < nrows, real = real_hi >= 0 && slot == 0;
+    double v[kBWords];
+    if (valid) {
+        const int first = lane + 64 * (wave % NW);
+        if (real)
+            b_sums<rp, GAL, BANDED>(g, quad, npts, point_freq(freqs + l0, real_hi, rp{}), m, i, tpts, first, 64 * NW, fb, mtab, v);
+        else
+            b_sums<cd, GAL, BANDED>(g, quad, npts, point_freq(freqs, l0 + slot, cd{}), m, i, tpts, first, 64 * NW, fb, mtab, v);
+        wave_sum48(v, lane);
+    }
+    if (NW > 1) {  // the group's waves, in wave order
+        if (valid && (lane & 7) == 0) {
+#pragma unroll
+            for (int k = 0; k < 6; k++) red[wave][6 * (lane >> 3) + k] = v[k];
+        }
+        __syncthreads();
+        if (wave % NW) return;
+        if (valid) {
+#pragma unroll
+            for (int k = 0; k < 6; k++) {
+                v[k] = red[wave][6 * (lane >> 3) + k];
+#pragma unroll
+                for (int w = 1; w < NW; w++) v[k] += red[wave + w][6 * (lane >> 3) + k];
+            }
         }
     }
+    const int q = lane & 7;
+    if (!valid || q > 2) return;
+    // one entry per lane; scattered from the packed symmetric form to its full positions
+    const int k = 3 * (lane >> 3) + q;
+    const double sx = q == 0 ? v[0] : q == 1 ? v[2] : v[4], sy = q == 0 ? v[1] : q == 1 ? v[3] : v[5];
+    cd e0, e1{0, 0};  // the entry at frequency slot, or the two real entries at frequencies 0 and real_hi
+    if (real) {
+        const PointFreq<rp> f = point_freq(freqs + l0, real_hi, rp{});
+        e0 = cd{sx * f.is2.x * kInv8Pi, 0.0}, e1 = cd{sy * f.is2.y * kInv8Pi, 0.0};
+    } else {
+        e0 = cd{sx, sy} * point_freq(freqs, l0 + slot, cd{}).is2 * kInv8Pi;
+    }
+    const int io = GAL ? r : i, words = k < 6 ? 3 : 9;
+    const int ab = k < 6 ? k : (k - 6) / 3, c = k < 6 ? 0 : (k - 6) % 3;
+    cd *o = (k < 6 ? Bt : Ba) + (long long)(3 * io) * words;
+    for (int a = 0; a < 3; a++)
+        for (int b = 0; b < 3; b++)
+            if (sidx(a, b) == ab) {
+                cd *p = o + a * words + (k < 6 ? b : 3 * b + c);
+                p[slot * nv3 * words] = e0;
+                if (real) p[real_hi * nv3 * words] = e1;
+            }
 }
 
 // ------------------------------------------------------------------------
@@ -1304,17 +1373,18 @@ hipError_t launch_colloc_gh(const Geom &g, const double4 *quad, int npts, const 
 // there are as many tiles.
 int patch_rows_per_tile(long long tiles) { return (int)std::min<long long>(16, std::max<long long>(1, tiles / 8192)); }
 
-hipError_t launch_colloc_gh_patch(const Geom &g, const double4 *pts, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
+hipError_t launch_colloc_gh_patch(const Geom &g, const double4 *pts, int npts, const Freq *freqs, int l0, int nl, bool real_ends, const Mat &m,
                                  int row0, int nrows, const double4 *tpts, const int *patch_chunk, const int4 *chunk_info,
                                  const int4 *chunk_faces, const int *patch_verts, int npatches, cd *UG, cd *UH, long long ld,
                                  long long lstride, hipStream_t st, const Bands &bands) {
     if ((!UG && !UH) || npts <= 0 || nrows <= 0 || nrows > 65535) return hipErrorInvalidValue;
     if (bands.far_pts && (tpts || bands.far_npts <= 0 || !bands.sphere)) return hipErrorInvalidValue;
-    const int rpt = patch_rows_per_tile((long long)npatches * nl * nrows);
-    dim3 grid(npatches, nl, (nrows + rpt - 1) / rpt);
+    const int slots = real_ends ? std::max(nl - 1, 1) : nl, real_hi = real_ends ? nl - 1 : -1;
+    const int rpt = patch_rows_per_tile((long long)npatches * slots * nrows);
+    dim3 grid(npatches, slots, (nrows + rpt - 1) / rpt);
 #define CQBEM_PATCH(DG, DH, GAL, BANDED)                                                                                    \
     hipLaunchKernelGGL((k_colloc_gh_patch<DG, DH, GAL, BANDED>), grid, dim3(kPatchThreads), 0, st, g, pts, npts, freqs, \
-                       l0, m, row0, tpts, patch_chunk, chunk_info, chunk_faces, patch_verts, UG, UH, ld, lstride, nrows, rpt, bands)
+                       l0, m, row0, tpts, patch_chunk, chunk_info, chunk_faces, patch_verts, UG, UH, ld, lstride, nrows, rpt, real_hi, bands)
     if (tpts) {  // test points: never banded (refused above)
         if (UG && UH) CQBEM_PATCH(true, true, true, false);
         else if (UG) CQBEM_PATCH(true, false, true, false);
@@ -1367,24 +1437,31 @@ hipError_t launch_scene_gh(const ScenePiece *pieces, int npieces, long long ntil
 int patch_size() { return kPatchVerts; }
 int chunk_face_count() { return 64; }
 
-hipError_t launch_colloc_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
-                           int row0, int nrows, cd *Bt, cd *Ba, hipStream_t st, const FaceBands &fb) {
-    if (nrows <= 0 || nrows > 65535) return hipErrorInvalidValue;
-    if (fb.sphere)
-        hipLaunchKernelGGL((k_colloc_b<false, true>), dim3(nl, nrows), dim3(256), 0, st, g, quad, npts, freqs, l0, m, row0,
-                           (const double4 *)nullptr, Bt, Ba, 3LL * g.nv, fb);
-    else
-        hipLaunchKernelGGL((k_colloc_b<false, false>), dim3(nl, nrows), dim3(256), 0, st, g, quad, npts, freqs, l0, m, row0,
-                           (const double4 *)nullptr, Bt, Ba, 3LL * g.nv, fb);
+template <bool GAL, bool BANDED>
+static hipError_t launch_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, bool real_ends,
+                           const Mat &m, int row0, int nrows, const double4 *tpts, cd *Bt, cd *Ba, long long out_rows,
+                           hipStream_t st, const FaceBands &fb) {
+    const int slots = real_ends ? std::max(nl - 1, 1) : nl, real_hi = real_ends ? nl - 1 : -1;
+    const long long jobs = (long long)slots * nrows;
+    auto go = [&](auto kernel, int nw) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((jobs * nw + 3) / 4)), dim3(256), 0, st, g, quad, npts, freqs, l0, slots, m, row0,
+                           nrows, tpts, Bt, Ba, out_rows, real_hi, fb);
+    };
+    go(k_colloc_b<4, GAL, BANDED>, 4);
     return hipGetLastError();
 }
 
-hipError_t launch_points_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
+hipError_t launch_colloc_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, bool real_ends, const Mat &m,
+                           int row0, int nrows, cd *Bt, cd *Ba, hipStream_t st, const FaceBands &fb) {
+    if (nrows <= 0 || nrows > 65535) return hipErrorInvalidValue;
+    return fb.sphere ? launch_b<false, true>(g, quad, npts, freqs, l0, nl, real_ends, m, row0, nrows, nullptr, Bt, Ba, 3LL * g.nv, st, fb)
+                     : launch_b<false, false>(g, quad, npts, freqs, l0, nl, real_ends, m, row0, nrows, nullptr, Bt, Ba, 3LL * g.nv, st, fb);
+}
+
+hipError_t launch_points_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, bool real_ends, const Mat &m,
                            const double4 *tpts, int row0, int nrows, cd *Bt, cd *Ba, long long out_rows, hipStream_t st) {
     if (nrows <= 0 || nrows > 65535 || 3LL * nrows > out_rows) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_colloc_b<true, false>), dim3(nl, nrows), dim3(256), 0, st, g, quad, npts, freqs, l0, m, row0, tpts, Bt, Ba,
-                       out_rows, FaceBands{});
-    return hipGetLastError();
+    return launch_b<true, false>(g, quad, npts, freqs, l0, nl, real_ends, m, row0, nrows, tpts, Bt, Ba, out_rows, st, FaceBands{});
 }
 
 hipError_t launch_colloc_singular(int kind, const Geom &g, const double2 *line, int nline, const Freq *freqs, int l0, int nl,

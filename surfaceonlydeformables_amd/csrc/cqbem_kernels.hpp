@@ -51,10 +51,13 @@ struct FaceBands {
 // of corner 1 << 8 | of corner 2 << 16, 0); per face entry, for its corners k = 0..2 (the face's, from any of the
 // three), x, y, z = vertex | slot << 24 and w = the sub-steps, 8 bits each (255: outside the patch).
 // `pts` holds, for each point of the rule, (b1, b2, 0, 0) and w (b0, b1, b2, 1).
+// real_ends: s is real at the first and the last of the nl frequencies (the half spectrum of an even L, or one real
+// frequency), which then share one slot of the grid.
 // Rows are collocation vertices row0..row0+nrows-1 when tpts is null.  Otherwise they are the test points
 // tpts[row0..row0+nrows-1] = (x, y, z, test face), each excluding every face that shares a vertex with its
 // test face (the Galerkin non-singular set), and row r of the launch goes to rows 3r..3r+2 of UG/UH.
-hipError_t launch_colloc_gh_patch(const Geom &g, const double4 *pts, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
+hipError_t launch_colloc_gh_patch(const Geom &g, const double4 *pts, int npts, const Freq *freqs, int l0, int nl, bool real_ends,
+                                 const Mat &m,
                                  int row0, int nrows, const double4 *tpts, const int *patch_chunk, const int4 *chunk_info,
                                  const int4 *chunk_faces, const int *patch_verts, int npatches, cd *UG, cd *UH, long long ld,
                                  long long lstride, hipStream_t st, const Bands &bands = Bands{});
@@ -63,14 +66,15 @@ int chunk_face_count();  // faces per chunk
 int patch_rows_per_tile(long long tiles);  // rows per block for a job of `tiles` (patch, frequency, row) tiles
 
 // One object's row slab in a multi-object launch of the patch kernel (collocation rows row0..row0+nrows-1 at all
-// nl frequencies of `freqs`): its npatches x nl x ceil(nrows / rpt) tiles of rpt rows are numbered from base.
+// nl frequencies of `freqs`): its npatches x slots x ceil(nrows / rpt) tiles of rpt rows are numbered from base; slots: nl, or nl - 1 with
+// real_hi = nl - 1 when the first and the last frequency share one).
 struct ScenePiece {
     Geom g;
     const double4 *pts;
     int npts;
     const Freq *freqs;
     Mat m;
-    int row0, nrows, rpt, nl, npatches;
+    int row0, nrows, rpt, slots, real_hi, npatches;
     const int *patch_chunk;
     const int4 *chunk_info;
     const int4 *chunk_faces;
@@ -84,11 +88,13 @@ struct ScenePiece {
 // min(ntiles, 2 blocks per CU) blocks that take tiles from *counter (zeroed by the launcher with a kernel).
 hipError_t launch_scene_gh(const ScenePiece *pieces, int npieces, long long ntiles, unsigned *counter, bool G, bool H,
                                 int num_cus, hipStream_t st);
-hipError_t launch_colloc_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
+hipError_t launch_colloc_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, bool real_ends,
+                                 const Mat &m,
                            int row0, int nrows, cd *Bt, cd *Ba, hipStream_t st, const FaceBands &fb = FaceBands{});
 // B_trans / B_angular rows of the test points tpts[row0..row0+nrows-1] (Galerkin non-singular set, as above), into
 // rows 3r..3r+2 of Bt (out_rows x 3 per frequency) and Ba (out_rows x 9).
-hipError_t launch_points_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, const Mat &m,
+hipError_t launch_points_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, bool real_ends,
+                                 const Mat &m,
                            const double4 *tpts, int row0, int nrows, cd *Bt, cd *Ba, long long out_rows, hipStream_t st);
 hipError_t launch_colloc_singular(int kind, const Geom &g, const double2 *line, int nline, const Freq *freqs, int l0, int nl,
                                   const Mat &m, int row0, int nrows, cd *U, long long ld, long long lstride, cd *Bt,

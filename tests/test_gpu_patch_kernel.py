@@ -81,3 +81,35 @@ def test_rows_per_block_against_the_star_kernel(ctx, monkeypatch, nf, L):
     want = ctx.assemble(mesh, p, want=("G", "H"))
     for k in "GH":
         assert off(got[k], want[k]) <= 1e-8, k
+
+
+@pytest.mark.parametrize("galerkin", [False, True])
+@pytest.mark.parametrize("L", [2, 3, 4, 18])
+def test_real_frequencies_share_a_slot(ctx, galerkin, L):
+    """At an even L the first and the last frequency (real s) share one slot of the regular-face kernels; cqbem_laplace
+    computes each of them alone.  The weights must be the inverse transform of cqbem_laplace's matrices, plus
+    B_trans (x) x_v in B_angular: each within 1e-12 of the sum of its terms' magnitudes (the per-entry rounding above,
+    and a sum of at most 10 terms).  H from n = 1 (H_0 also holds the C matrix)."""
+    V, F = M.icosphere(1, 0.2)
+    V = M.center(M.jitter(V, F, 0.01, 3), F)
+    mesh, p = abi.make_mesh(V, F), params(L, 4, 1)
+    p.galerkin = int(galerkin)
+    p.which |= abi.B_TRANS | abi.B_ANGULAR
+    print(f"real frequencies L={L} galerkin={galerkin}", flush=True)
+    got = ctx.assemble(mesh, p, want=("G", "H", "B_trans", "B_angular"))
+    X = [ctx.laplace(mesh, p, l) for l in range(L // 2 + 1)]
+    mult = np.array([1.0 if l in (0, L / 2) else 2.0 for l in range(L // 2 + 1)])
+    ang = 2 * np.pi / L * np.outer(np.arange(L), np.arange(L // 2 + 1))
+    scale = p.R ** -np.arange(L, dtype=float)[:, None] / L
+    for k, name in (("U", "G"), ("P", "H"), ("Bt", "B_trans"), ("Ba", "B_angular")):
+        S = np.stack([x[k].reshape(-1) for x in X])
+        W = scale * ((mult * np.cos(ang)) @ S.real + (mult * np.sin(ang)) @ S.imag)
+        mag = scale * (mult @ np.abs(S))
+        if name == "B_trans":
+            Wt, mt = W, mag
+        elif name == "B_angular":
+            x = np.repeat(V, 3, axis=0)[None, :, None, :]
+            W = W + (Wt.reshape(L, -1, 3, 1) * x).reshape(L, -1)
+            mag = mag + (mt.reshape(L, -1, 3, 1) * np.abs(x)).reshape(L, -1)
+        first = name == "H"
+        assert (np.abs(got[name].reshape(L, -1) - W) <= 1e-12 * mag)[first:].all(), name
