@@ -1207,21 +1207,25 @@ __global__ void __launch_bounds__(256) k_history(const double *__restrict__ G, c
     }
 }
 
-// The same history sum for an even n3 with 16-byte aligned matrices and vectors (every row then starts on a 16-byte
-// boundary).  Each wavefront takes R consecutive rows, so a chunk of p and u loaded once serves R matrix rows
+// The same history sum in 16-byte loads.  A16: n3 is even and the matrices and vectors are 16-byte aligned (every row then
+// starts on a 16-byte boundary); otherwise the loads are declared 8-byte aligned, which the hardware takes at the price
+// of one more cache line per 1 KB, and an odd n3's last column is added on its own: n3 = 3489, 16 steps (3.1 GB) 516 us
+// (6.0 TB/s; 709 us in 8-byte loads, one row per wavefront).  Each wavefront takes R consecutive rows, so a chunk of p and u loaded once serves R matrix rows
 // (the vectors are re-read from L2 by every wavefront: with one row per wavefront that traffic equals the matrix
 // stream).  The matrix rows are streamed with 16-byte non-temporal loads: each weight is read once per step.  The
 // B terms are spread over the lanes before the wave reduction.  Matrix i starts at G + i * mat_stride (n3^2 for the
 // history; 0 with m = nh = 1 makes it y = A x).
 typedef double hist_d2 __attribute__((ext_vector_type(2)));
+typedef hist_d2 hist_d2u __attribute__((aligned(8)));
 typedef float hist_f2 __attribute__((ext_vector_type(2)));
-template <class S> struct HistPair;
-template <> struct HistPair<double> { typedef hist_d2 type; };
-template <> struct HistPair<float> { typedef hist_f2 type; };
+template <class S, bool A16> struct HistPair;
+template <> struct HistPair<double, true> { typedef hist_d2 type, vec; };
+template <> struct HistPair<double, false> { typedef hist_d2u type, vec; };
+template <> struct HistPair<float, true> { typedef hist_f2 type; typedef hist_d2 vec; };
 
 // S: the matrices' element type (double, or float for weights stored in single precision; the products and
 // sums are formed in double either way).
-template <class S, bool HG, bool HH, int R>
+template <class S, bool A16, bool HG, bool HH, int R>
 __global__ void __launch_bounds__(256) k_history_v2(const S *__restrict__ G, const S *__restrict__ H,
                                                      const double *__restrict__ B, const double *__restrict__ p,
                                                      const double *__restrict__ u, const double *__restrict__ acc,
@@ -1239,9 +1243,10 @@ __global__ void __launch_bounds__(256) k_history_v2(const S *__restrict__ G, con
     for (int k = 0; k < R; k++) s[k] = 0.0;
     for (int i = 1; i <= m; i++) {
         const long long mo = (long long)i * mat_stride;
-        const hist_d2 *xp = HG ? reinterpret_cast<const hist_d2 *>(p + (long long)(nh - i) * n3) : nullptr;
-        const hist_d2 *xu = HH ? reinterpret_cast<const hist_d2 *>(u + (long long)(nh - i) * n3) : nullptr;
-        typedef typename HistPair<S>::type s2;
+        typedef typename HistPair<S, A16>::type s2;
+        typedef typename HistPair<S, A16>::vec x2;
+        const x2 *xp = HG ? reinterpret_cast<const x2 *>(p + (long long)(nh - i) * n3) : nullptr;
+        const x2 *xu = HH ? reinterpret_cast<const x2 *>(u + (long long)(nh - i) * n3) : nullptr;
         const s2 *gr[R], *hr[R];
 #pragma unroll
         for (int k = 0; k < R; k++) {
@@ -1282,6 +1287,14 @@ __global__ void __launch_bounds__(256) k_history_v2(const S *__restrict__ G, con
                     const s2 h = __builtin_nontemporal_load(hr[k] + c);
                     s[k] = fma(-(double)h.y, y.y, fma(-(double)h.x, y.x, s[k]));
                 }
+            }
+        }
+        if (!A16 && (n3 & 1) && lane == 0) {  // the last column
+            const double x = HG ? p[(long long)(nh - i) * n3 + n3 - 1] : 0.0, y = HH ? u[(long long)(nh - i) * n3 + n3 - 1] : 0.0;
+#pragma unroll
+            for (int k = 0; k < R; k++) {
+                if (HG) s[k] = fma((double)G[mo + rr[k] * n3 + n3 - 1], x, s[k]);
+                if (HH) s[k] = fma(-(double)H[mo + rr[k] * n3 + n3 - 1], y, s[k]);
             }
         }
     }
@@ -1522,23 +1535,23 @@ hipError_t launch_transform(const cd *spec, long long E, long long spec_ls, int 
     return launch_transform_t(spec, E, spec_ls, Lf, tab, L, out, out_nstride, num_cus, st);
 }
 
-template <int R, class S>
+template <int R, bool A16, class S>
 static void launch_history_v2(const S *G, const S *H, const double *B, const double *p, const double *u,
                               const double *acc, long long n3, long long mat_stride, int m, int nh, double *b,
                               hipStream_t st) {
     const long long waves = (n3 + R - 1) / R;
     const dim3 grid((unsigned)((waves + 3) / 4));
     if (G && H)
-        hipLaunchKernelGGL((k_history_v2<S, true, true, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
+        hipLaunchKernelGGL((k_history_v2<S, A16, true, true, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
                            nh, b);
     else if (G)
-        hipLaunchKernelGGL((k_history_v2<S, true, false, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
+        hipLaunchKernelGGL((k_history_v2<S, A16, true, false, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
                            nh, b);
     else if (H)
-        hipLaunchKernelGGL((k_history_v2<S, false, true, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
+        hipLaunchKernelGGL((k_history_v2<S, A16, false, true, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
                            nh, b);
     else
-        hipLaunchKernelGGL((k_history_v2<S, false, false, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride,
+        hipLaunchKernelGGL((k_history_v2<S, A16, false, false, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride,
                            m, nh, b);
 }
 
@@ -1558,18 +1571,19 @@ hipError_t launch_history_f32(const float *G, const float *H, const double *B, c
     // single-precision matrices: 8-byte pairs of weights against 16-byte pairs of history entries
     if (n3 % 2 != 0 || (G && (!aligned8(G) || !aligned16(p))) || (H && (!aligned8(H) || !aligned16(u))))
         return hipErrorInvalidValue;
-    launch_history_v2<4>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
+    launch_history_v2<4, true>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
     return hipGetLastError();
 }
 
 hipError_t launch_history(const double *G, const double *H, const double *B, const double *p, const double *u,
                           const double *acc, long long n3, int m, int nh, double *b, hipStream_t st) {
     const int rows = history_rows();
-    if (rows > 1 && n3 % 2 == 0 && (!G || (aligned16(G) && aligned16(p))) && (!H || (aligned16(H) && aligned16(u)))) {
-        if (rows == 4)
-            launch_history_v2<4>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
-        else
-            launch_history_v2<2>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
+    if (rows > 1 && (!G || (aligned8(G) && aligned8(p))) && (!H || (aligned8(H) && aligned8(u)))) {
+        const bool a16 = n3 % 2 == 0 && (!G || (aligned16(G) && aligned16(p))) && (!H || (aligned16(H) && aligned16(u)));
+        if (a16 && rows == 4) launch_history_v2<4, true>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
+        else if (a16) launch_history_v2<2, true>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
+        else if (rows == 4) launch_history_v2<4, false>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
+        else launch_history_v2<2, false>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
         return hipGetLastError();
     }
     const dim3 grid((unsigned)((n3 + 3) / 4));
@@ -1586,11 +1600,12 @@ hipError_t launch_history(const double *G, const double *H, const double *B, con
 
 hipError_t launch_matvec(const double *A, const double *x, long long n, double *y, hipStream_t st) {
     const int rows = history_rows();
-    if (rows > 1 && n % 2 == 0 && aligned16(A) && aligned16(x)) {
-        if (rows == 4)
-            launch_history_v2<4, double>(A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
-        else
-            launch_history_v2<2, double>(A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
+    if (rows > 1 && aligned8(A) && aligned8(x)) {
+        const bool a16 = n % 2 == 0 && aligned16(A) && aligned16(x);
+        if (a16 && rows == 4) launch_history_v2<4, true, double>(A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
+        else if (a16) launch_history_v2<2, true, double>(A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
+        else if (rows == 4) launch_history_v2<4, false, double>(A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
+        else launch_history_v2<2, false, double>(A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(k_matvec, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, A, x, n, y);
