@@ -1011,27 +1011,22 @@ __global__ void k_gal_gather_gh(const int2 *__restrict__ blocks, const int *__re
         }
 }
 
+// The same for B, one lane per (vertex, frequency, entry): a pair's 36 entries per corner are read by neighbouring lanes
+// (icosphere level 2, L = 16: 40 us; one lane per (vertex, frequency) took 1070 us, 2754 lanes of strided 16-byte loads).
 __global__ void k_gal_gather_b(const int *__restrict__ vptr, const int *__restrict__ items, int nv, int nl,
                                const cd *__restrict__ scratch, cd *__restrict__ Bt, cd *__restrict__ Ba, long long nv3) {
     const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (t >= (long long)nv * nl) return;
-    const int u = (int)(t / nl), l = (int)(t % nl);
-    cd bt[9], ba[27];
-    for (int e = 0; e < 9; e++) bt[e] = cd{0, 0};
-    for (int e = 0; e < 27; e++) ba[e] = cd{0, 0};
+    if (t >= (long long)nv * nl * 36) return;
+    const int e = (int)(t % 36), l = (int)(t / 36 % nl), u = (int)(t / 36 / nl);
+    // entries 0..8 are B_trans's three rows, 9..35 B_angular's
+    const int off = e < 9 ? kPairBt + e : kPairBa + e - 9, corner = e < 9 ? 9 : 27;
+    cd s = {0, 0};
     for (int k = vptr[u]; k < vptr[u + 1]; k++) {
         const int it = items[k];
-        const int pi = it / 3, i = it % 3;
-        const cd *o = scratch + ((long long)pi * nl + l) * kPairStride;
-        for (int p = 0; p < 3; p++) {
-            for (int q = 0; q < 3; q++) bt[p * 3 + q] += o[kPairBt + (3 * i + p) * 3 + q];
-            for (int q = 0; q < 9; q++) ba[p * 9 + q] += o[kPairBa + (3 * i + p) * 9 + q];
-        }
+        s += scratch[((long long)(it / 3) * nl + l) * kPairStride + off + (it % 3) * corner];
     }
-    cd *bo = Bt + (long long)l * nv3 * 3 + (long long)(3 * u) * 3;
-    cd *ao = Ba + (long long)l * nv3 * 9 + (long long)(3 * u) * 9;
-    for (int e = 0; e < 9; e++) bo[e] += bt[e];
-    for (int e = 0; e < 27; e++) ao[e] += ba[e];
+    if (e < 9) Bt[(long long)l * nv3 * 3 + 9LL * u + e] += s;
+    else Ba[(long long)l * nv3 * 9 + 27LL * u + e - 9] += s;
 }
 
 // Test points of the faces faces[0..nfl) in that order: tpts[fi * npts + a] = (x_a, face) with x_a the a-th rule
@@ -1408,7 +1403,7 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
             check(hipGetLastError(), "k_gal_gather_gh");
         }
         if (Bt && Ba) {
-            const long long n = (long long)nv * nl;
+            const long long n = (long long)nv * nl * 36;
             hipLaunchKernelGGL(k_gal_gather_b, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, dvp, dvi, nv, nl, scratch, Bt, Ba, n3);
             check(hipGetLastError(), "k_gal_gather_b");
         }
