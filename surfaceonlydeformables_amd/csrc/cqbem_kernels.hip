@@ -1209,8 +1209,8 @@ __global__ void __launch_bounds__(256) k_history(const double *__restrict__ G, c
 
 // The same history sum in 16-byte loads.  A16: n3 is even and the matrices and vectors are 16-byte aligned (every row then
 // starts on a 16-byte boundary); otherwise the loads are declared 8-byte aligned, which the hardware takes at the price
-// of one more cache line per 1 KB, and an odd n3's last column is added on its own: n3 = 3489, 16 steps (3.1 GB) 516 us
-// (6.0 TB/s; 709 us in 8-byte loads, one row per wavefront).  Each wavefront takes R consecutive rows, so a chunk of p and u loaded once serves R matrix rows
+// of one more cache line per 1 KB, and an odd n3's last column is added on its own: n3 = 3489, 16 steps (3.1 GB) 530 us
+// (5.9 TB/s; 709 us in 8-byte loads, one row per wavefront).  SPLIT: history_split.  Each wavefront takes R consecutive rows, so a chunk of p and u loaded once serves R matrix rows
 // (the vectors are re-read from L2 by every wavefront: with one row per wavefront that traffic equals the matrix
 // stream).  The matrix rows are streamed with 16-byte non-temporal loads: each weight is read once per step.  The
 // B terms are spread over the lanes before the wave reduction.  Matrix i starts at G + i * mat_stride (n3^2 for the
@@ -1225,15 +1225,15 @@ template <> struct HistPair<float, true> { typedef hist_f2 type; typedef hist_d2
 
 // S: the matrices' element type (double, or float for weights stored in single precision; the products and
 // sums are formed in double either way).
-template <class S, bool A16, bool HG, bool HH, int R>
+template <class S, bool A16, bool SPLIT, bool HG, bool HH, int R>
 __global__ void __launch_bounds__(256) k_history_v2(const S *__restrict__ G, const S *__restrict__ H,
                                                      const double *__restrict__ B, const double *__restrict__ p,
                                                      const double *__restrict__ u, const double *__restrict__ acc,
                                                      long long n3, long long mat_stride, int m, int nh,
                                                      double *__restrict__ b) {
-    const long long r0 = ((long long)blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
-    const int lane = threadIdx.x & 63;
-    if (r0 >= n3) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const long long r0 = (SPLIT ? (long long)blockIdx.x : (long long)blockIdx.x * 4 + wave) * R;
+    if (r0 >= n3) return;  // SPLIT: of the whole block
     const long long nc = n3 >> 1;  // 16-byte columns
     long long rr[R];
 #pragma unroll
@@ -1241,7 +1241,7 @@ __global__ void __launch_bounds__(256) k_history_v2(const S *__restrict__ G, con
     double s[R];
 #pragma unroll
     for (int k = 0; k < R; k++) s[k] = 0.0;
-    for (int i = 1; i <= m; i++) {
+    for (int i = SPLIT ? 1 + wave : 1; i <= m; i += SPLIT ? 4 : 1) {
         const long long mo = (long long)i * mat_stride;
         typedef typename HistPair<S, A16>::type s2;
         typedef typename HistPair<S, A16>::vec x2;
@@ -1275,19 +1275,30 @@ __global__ void __launch_bounds__(256) k_history_v2(const S *__restrict__ G, con
                     if (HH) s[k] = fma(-(double)h[k][j].y, y[j].y, fma(-(double)h[k][j].x, y[j].x, s[k]));
                 }
         }
-        for (; c < nc; c += 64) {
-            const hist_d2 x = HG ? xp[c] : hist_d2{0.0, 0.0}, y = HH ? xu[c] : hist_d2{0.0, 0.0};
+        // the last, partial step: all its loads before the first product
+        {
+            x2 x[kHistUnroll], y[kHistUnroll];
+            s2 g[R][kHistUnroll], h[R][kHistUnroll];
 #pragma unroll
-            for (int k = 0; k < R; k++) {
-                if (HG) {
-                    const s2 g = __builtin_nontemporal_load(gr[k] + c);
-                    s[k] = fma((double)g.y, x.y, fma((double)g.x, x.x, s[k]));
+            for (int j = 0; j < kHistUnroll; j++)
+                if (c + 64 * j < nc) {
+                    if (HG) x[j] = xp[c + 64 * j];
+                    if (HH) y[j] = xu[c + 64 * j];
+#pragma unroll
+                    for (int k = 0; k < R; k++) {
+                        if (HG) g[k][j] = __builtin_nontemporal_load(gr[k] + c + 64 * j);
+                        if (HH) h[k][j] = __builtin_nontemporal_load(hr[k] + c + 64 * j);
+                    }
                 }
-                if (HH) {
-                    const s2 h = __builtin_nontemporal_load(hr[k] + c);
-                    s[k] = fma(-(double)h.y, y.y, fma(-(double)h.x, y.x, s[k]));
+#pragma unroll
+            for (int j = 0; j < kHistUnroll; j++)
+                if (c + 64 * j < nc) {
+#pragma unroll
+                    for (int k = 0; k < R; k++) {
+                        if (HG) s[k] = fma((double)g[k][j].y, x[j].y, fma((double)g[k][j].x, x[j].x, s[k]));
+                        if (HH) s[k] = fma(-(double)h[k][j].y, y[j].y, fma(-(double)h[k][j].x, y[j].x, s[k]));
+                    }
                 }
-            }
         }
         if (!A16 && (n3 & 1) && lane == 0) {  // the last column
             const double x = HG ? p[(long long)(nh - i) * n3 + n3 - 1] : 0.0, y = HH ? u[(long long)(nh - i) * n3 + n3 - 1] : 0.0;
@@ -1299,7 +1310,7 @@ __global__ void __launch_bounds__(256) k_history_v2(const S *__restrict__ G, con
         }
     }
     if (B)
-        for (int j = lane; j < 6 * m; j += 64) {
+        for (int j = SPLIT ? (int)threadIdx.x : lane; j < 6 * m; j += SPLIT ? 256 : 64) {
             const int i = j / 6 + 1, q = j - 6 * (i - 1);
             const double a = acc[(long long)(nh - i) * 6 + q];
 #pragma unroll
@@ -1309,6 +1320,16 @@ __global__ void __launch_bounds__(256) k_history_v2(const S *__restrict__ G, con
     for (int k = 0; k < R; k++)
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) s[k] += __shfl_xor(s[k], o, 64);
+    if (SPLIT) {  // the waves' sums, in wave order
+        __shared__ double part[4][R];
+        if (lane == 0)
+#pragma unroll
+            for (int k = 0; k < R; k++) part[wave][k] = s[k];
+        __syncthreads();
+        const int k = threadIdx.x;
+        if (k < R && r0 + k < n3) b[r0 + k] = (part[0][k] + part[1][k]) + (part[2][k] + part[3][k]);
+        return;
+    }
     if (lane == 0)
 #pragma unroll
         for (int k = 0; k < R; k++)
@@ -1535,32 +1556,75 @@ hipError_t launch_transform(const cd *spec, long long E, long long spec_ls, int 
     return launch_transform_t(spec, E, spec_ls, Lf, tab, L, out, out_nstride, num_cus, st);
 }
 
-template <int R, bool A16, class S>
-static void launch_history_v2(const S *G, const S *H, const double *B, const double *p, const double *u,
+// CQBEM_HISTORY_ROWS = 1 selects the 8-byte one-row history and matvec kernel, 2 or 4 that many rows per wavefront of the
+// 16-byte one, unsplit; anything else (0) the rule below.  Read at every call (a few hundred ns against a launch).
+static int history_rows() {
+    const char *e = std::getenv("CQBEM_HISTORY_ROWS");
+    const int v = e ? std::atoi(e) : 0;
+    return v == 1 || v == 2 || v == 4 ? v : 0;
+}
+
+// How the rows and the m steps (m = 1: a matvec) go over the wavefronts.  What counts below some 2000 wavefronts is how
+// many loads are in flight, beyond that how often the vectors are read again.  us per call, with 4 rows per wavefront and
+// no split first: n3 = 486, 31 steps 36 -> 10; 1158, 16 steps 34 -> 20 (22 at 4 rows); 1926, 16 steps 63 -> 42 (45 at
+// 2 rows); 7686, 31 steps 4660 and 4650.  One step: 1926 rows 19.7 -> 18.0 at one row, 3489 30.5 at 4 and 29.3 at 2,
+// 7686 89.7 at 4 and 95.4 at one.
+struct HistorySplit {
+    int rows;    // rows per wavefront; 0: the 8-byte kernel
+    bool split;  // a block's 4 waves share its rows and take every fourth step each
+};
+static HistorySplit history_split(long long n3, int m, bool a16) {
+    if (const int forced = history_rows()) return {forced == 1 ? 0 : forced, false};
+    // unaligned 16-byte loads pay from 4 steps or 2048 rows on (903 rows, 2 steps: 18.3 us in 8-byte loads, 19.4), for one
+    // step from 8192 (5001 rows: 40 and 47 us; 12289: 257 and 194)
+    if (m > 1 && (a16 || m >= 4 || n3 >= 2048)) {
+        // idle share of 256 CUs in the last round of blocks: 2 rows where that is clearly the smaller one (3489 rows, 16
+        // steps, unaligned: 528 us at 2 and 543 at 4 rows; 903: 57 and 53)
+        auto uneven = [&](long long r) {
+            const long long blocks = (n3 + r - 1) / r;
+            return (double)((blocks + 255) / 256) * 256 / (double)blocks;
+        };
+        return {uneven(4) > 1.06 * uneven(2) ? 2 : 4, true};
+    }
+    if (!a16 && n3 < 8192) return {0, false};
+    return {n3 < 3072 ? 1 : n3 < 6144 ? 2 : 4, false};
+}
+
+template <int R, bool A16, bool SPLIT, class S>
+static void launch_history_r(const S *G, const S *H, const double *B, const double *p, const double *u,
                               const double *acc, long long n3, long long mat_stride, int m, int nh, double *b,
                               hipStream_t st) {
     const long long waves = (n3 + R - 1) / R;
-    const dim3 grid((unsigned)((waves + 3) / 4));
+    const dim3 grid((unsigned)(SPLIT ? waves : (waves + 3) / 4));
     if (G && H)
-        hipLaunchKernelGGL((k_history_v2<S, A16, true, true, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
+        hipLaunchKernelGGL((k_history_v2<S, A16, SPLIT, true, true, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
                            nh, b);
     else if (G)
-        hipLaunchKernelGGL((k_history_v2<S, A16, true, false, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
+        hipLaunchKernelGGL((k_history_v2<S, A16, SPLIT, true, false, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
                            nh, b);
     else if (H)
-        hipLaunchKernelGGL((k_history_v2<S, A16, false, true, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
+        hipLaunchKernelGGL((k_history_v2<S, A16, SPLIT, false, true, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride, m,
                            nh, b);
     else
-        hipLaunchKernelGGL((k_history_v2<S, A16, false, false, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride,
+        hipLaunchKernelGGL((k_history_v2<S, A16, SPLIT, false, false, R>), grid, dim3(256), 0, st, G, H, B, p, u, acc, n3, mat_stride,
                            m, nh, b);
 }
 
-// Rows per wavefront of the 16-byte history and matvec kernel: CQBEM_HISTORY_ROWS = 1 selects the 8-byte one-row
-// kernel, 2 or 4 (default) the vectorized one.  Read at every call (a few hundred ns against a launch).
-static int history_rows() {
-    const char *e = std::getenv("CQBEM_HISTORY_ROWS");
-    const int v = e ? std::atoi(e) : 4;
-    return v == 1 || v == 2 ? v : 4;
+template <bool A16, class S>
+static void launch_history_v2(HistorySplit h, const S *G, const S *H, const double *B, const double *p, const double *u,
+                              const double *acc, long long n3, long long mat_stride, int m, int nh, double *b, hipStream_t st) {
+    auto go = [&](auto rows, auto split) {
+        launch_history_r<decltype(rows)::value, A16, decltype(split)::value>(G, H, B, p, u, acc, n3, mat_stride, m, nh, b, st);
+    };
+    using std::integral_constant;
+    if (h.split) {
+        if (h.rows == 4) go(integral_constant<int, 4>{}, std::true_type{});
+        else go(integral_constant<int, 2>{}, std::true_type{});
+    } else {
+        if (h.rows == 4) go(integral_constant<int, 4>{}, std::false_type{});
+        else if (h.rows == 2) go(integral_constant<int, 2>{}, std::false_type{});
+        else go(integral_constant<int, 1>{}, std::false_type{});
+    }
 }
 
 static bool aligned16(const double *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
@@ -1571,19 +1635,20 @@ hipError_t launch_history_f32(const float *G, const float *H, const double *B, c
     // single-precision matrices: 8-byte pairs of weights against 16-byte pairs of history entries
     if (n3 % 2 != 0 || (G && (!aligned8(G) || !aligned16(p))) || (H && (!aligned8(H) || !aligned16(u))))
         return hipErrorInvalidValue;
-    launch_history_v2<4, true>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
+    HistorySplit h = history_split(n3, m, true);
+    if (h.rows == 0) h.rows = 4;  // there is no kernel of single loads
+    launch_history_v2<true>(h, G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
     return hipGetLastError();
 }
 
 hipError_t launch_history(const double *G, const double *H, const double *B, const double *p, const double *u,
                           const double *acc, long long n3, int m, int nh, double *b, hipStream_t st) {
-    const int rows = history_rows();
-    if (rows > 1 && (!G || (aligned8(G) && aligned8(p))) && (!H || (aligned8(H) && aligned8(u)))) {
-        const bool a16 = n3 % 2 == 0 && (!G || (aligned16(G) && aligned16(p))) && (!H || (aligned16(H) && aligned16(u)));
-        if (a16 && rows == 4) launch_history_v2<4, true>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
-        else if (a16) launch_history_v2<2, true>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
-        else if (rows == 4) launch_history_v2<4, false>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
-        else launch_history_v2<2, false>(G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
+    const bool a16 = n3 % 2 == 0 && (!G || (aligned16(G) && aligned16(p))) && (!H || (aligned16(H) && aligned16(u)));
+    const bool a8 = (!G || (aligned8(G) && aligned8(p))) && (!H || (aligned8(H) && aligned8(u)));
+    const HistorySplit h = history_split(n3, m, a16);
+    if (h.rows && a8) {
+        if (a16) launch_history_v2<true>(h, G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
+        else launch_history_v2<false>(h, G, H, B, p, u, acc, n3, n3 * n3, m, nh, b, st);
         return hipGetLastError();
     }
     const dim3 grid((unsigned)((n3 + 3) / 4));
@@ -1599,13 +1664,11 @@ hipError_t launch_history(const double *G, const double *H, const double *B, con
 }
 
 hipError_t launch_matvec(const double *A, const double *x, long long n, double *y, hipStream_t st) {
-    const int rows = history_rows();
-    if (rows > 1 && aligned8(A) && aligned8(x)) {
-        const bool a16 = n % 2 == 0 && aligned16(A) && aligned16(x);
-        if (a16 && rows == 4) launch_history_v2<4, true, double>(A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
-        else if (a16) launch_history_v2<2, true, double>(A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
-        else if (rows == 4) launch_history_v2<4, false, double>(A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
-        else launch_history_v2<2, false, double>(A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
+    const bool a16 = n % 2 == 0 && aligned16(A) && aligned16(x);
+    const HistorySplit h = history_split(n, 1, a16);
+    if (h.rows && aligned8(A) && aligned8(x)) {
+        if (a16) launch_history_v2<true, double>(h, A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
+        else launch_history_v2<false, double>(h, A, nullptr, nullptr, x, nullptr, nullptr, n, 0, 1, 1, y, st);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(k_matvec, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, A, x, n, y);
