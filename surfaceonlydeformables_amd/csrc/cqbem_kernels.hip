@@ -149,11 +149,11 @@ __global__ void __launch_bounds__(64) k_colloc_gh(Geom g, const double4 *__restr
 // real, are one slot (T = rp: two real numbers in the place of a complex one).
 //
 // Bound by FP64 VALU issue (and, near full issue, by the clock that the power
-// limit leaves): 292 VALU instructions per point, of which 84 are the corner
-// sums and 78 the two complex exponentials, and 1100 per face and row outside
-// the rule.  Icosphere level 4, L = 32, 28 points (6.2e9 unique evaluations):
-// 76.8 ms (80.8 with a slot for each real frequency), 2.25 ms per point of the
-// rule plus 17 ms at 17 slots.  The form it replaces, two
+// limit leaves): 260 VALU instructions per point, of which 84 are the corner
+// sums and 47 the two complex exponentials (exp_pair), and 1100 per face and row
+// outside the rule.  Icosphere level 4, L = 32, 28 points (6.2e9 unique
+// evaluations): 70.8 ms; 76.8 at 292 instructions, with the exponentials through
+// reductions and e^x, sin, cos; 80.8 with a slot for each real frequency.  The form it replaces, two
 // lanes per face that swapped every point's 16 global entries through DPP, took
 // 128 ms at 516 instructions per point.  Tried and slower: the same with a
 // block barrier per sub-step (86.5 ms), the rotation inside the wave's turn
@@ -203,7 +203,7 @@ __device__ inline bool touches(const Geom &g, const int (&t)[3], const int (&c)[
 }
 
 // The rows il0 .. il0 + nr - 1 of one (patch pc, frequency l) for a block of kPatchThreads threads.  acc, frame,
-// counters (2) and mtab are the block's LDS (mtab loaded); callers that run another tile on the same LDS synchronise
+// exps (the table of the exponentials) are the block's LDS; callers that run another tile on the same LDS synchronise
 // first.  The block has no barrier between its rows: a wave evaluates its first chunk of the next row before it writes
 // out (and clears) its 64 vertex slots of the last one, so neither the other waves' adds nor the stores are waited for.
 // `dest` returns where the rows go (PatchDest); it is called at each write-out, so that a caller that reads it from memory
@@ -218,12 +218,16 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
                                  const Bands &bands, const PointFreq<T> &f, const Mat &m, int row0, const double4 *__restrict__ tpts,
                                  const int *__restrict__ patch_chunk, const int4 *__restrict__ chunk_info,
                                  const int4 *__restrict__ chunk_faces, const Dest &dest, int pc, int l,
-                                 int il0, int nr, double2 *acc, double2 *frame, int *counters, const MathTables &mtab) {
+                                 int il0, int nr, double2 *acc, double2 *frame, double2 *exps) {
     constexpr int kWaves = kPatchThreads / 64;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     for (int k = tid; k < kPatchPairs * kPatchVerts; k += kPatchThreads) acc[k] = make_double2(0.0, 0.0);
-    int *turns = counters, *cleared = counters + 1;  // chunks added so far; waves that cleared their slots, over all rows
-    if (tid < 2) counters[tid] = 0;
+    static_assert(kPatchThreads == kExpNodes, "one node per thread");
+    fill_exp_table(f, exps);
+    // chunks added so far; waves that cleared their slots, over all rows: in the table's unused place, so that
+    // two blocks fill a CU's LDS exactly
+    int *turns = reinterpret_cast<int *>(exps + 2 * (kExpNodes - kExpFine - 1)), *cleared = turns + 1;
+    if (tid < 2) turns[tid] = 0;
     __syncthreads();
     // With one or two chunks, 4 or 2 waves share a chunk, each taking every 4th or 2nd point of the rule, as long as 7
     // points are left to each.
@@ -316,7 +320,7 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
                 const double2 F0 = frame[ln], F1 = frame[kPatchThreads + ln], F2 = frame[2 * kPatchThreads + ln];
                 const_double *B = as_const(pts + 2 * q);  // b1, b2, -, -, w (phi_0, phi_1, phi_2, 1)
                 const double ar = fma(B[0], F0.x, fma(B[1], F0.y, F1.y)), br = fma(B[1], F1.x, F2.x), cr = F2.y;
-                const PointExpo<T> E = point_expo(fma(ar, ar, fma(br, br, cr * cr)), f, &mtab);
+                const PointExpo<T> E = point_expo(fma(ar, ar, fma(br, br, cr * cr)), f, exps);
                 const double w[3] = {B[4], B[5], B[6]};
                 const double a = ar * E.ir, b = br * E.ir, c = cr * E.ir;
                 auto add = [&](T &s, const T &v, double wk) {
@@ -434,19 +438,17 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_colloc_gh_patch(Geom g, co
                                                                   int nrows, int rpt, int real_hi, Bands bands) {
     __shared__ double2 acc[kPatchPairs * kPatchVerts];      // [word][slot]
     __shared__ double2 frame[kFramePairs * kPatchThreads];
-    __shared__ int counters[2];  // [word pair][lane]
-    __shared__ MathTables mtab;                       // tables of the exponentials
-    load_math_tables(&mtab);
+    __shared__ double2 exps[2 * kExpNodes];
     auto dest = [=] { return PatchDest{patch_verts, UG, UH, ld, lstride}; };
     const int r0 = blockIdx.z * rpt, nr = min(rpt, nrows - r0);
     if (real_hi >= 0 && blockIdx.y == 0)
         patch_tile<rp, DG, DH, GAL>(g, pts, npts, BANDED ? bands : Bands{}, point_freq(freqs + l0, real_hi, rp{}), m, row0, tpts,
                                     patch_chunk, chunk_info, chunk_faces, dest, blockIdx.x, real_hi, r0, nr, acc, frame,
-                                    counters, mtab);
+                                    exps);
     else
         patch_tile<cd, DG, DH, GAL>(g, pts, npts, BANDED ? bands : Bands{}, point_freq(freqs, l0 + blockIdx.y, cd{}), m, row0, tpts,
                                     patch_chunk, chunk_info, chunk_faces, dest, blockIdx.x, blockIdx.y, r0, nr, acc, frame,
-                                    counters, mtab);
+                                    exps);
 }
 
 // ------------------------------------------------------------------------
@@ -461,8 +463,7 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_colloc_gh_patch(Geom g, co
 //     persistent selects it, for comparison).
 // ------------------------------------------------------------------------
 template <bool DG, bool DH>
-__device__ __attribute__((always_inline)) inline void scene_tile(const ScenePiece *__restrict__ pieces, int npieces, unsigned t, double2 *acc, double2 *frame, int *counters,
-                                  const MathTables &mtab) {
+__device__ __attribute__((always_inline)) inline void scene_tile(const ScenePiece *__restrict__ pieces, int npieces, unsigned t, double2 *acc, double2 *frame, double2 *exps) {
     int pi = 0;
     while (pi + 1 < npieces && (unsigned)*(const_int *)&pieces[pi + 1].base <= t) ++pi;
     pi = __builtin_amdgcn_readfirstlane(pi);
@@ -491,11 +492,11 @@ __device__ __attribute__((always_inline)) inline void scene_tile(const ScenePiec
     if (P.real_hi >= 0 && l == 0)
         patch_tile<rp, DG, DH, false>(P.g, P.pts, P.npts, P.bands, point_freq(P.freqs, P.real_hi, rp{}), P.m, P.row0, nullptr,
                                       as_global(P.patch_chunk), P.chunk_info, as_global(P.chunk_faces), dest, pc, P.real_hi, r0,
-                                      min(P.rpt, P.nrows - r0), acc, frame, counters, mtab);
+                                      min(P.rpt, P.nrows - r0), acc, frame, exps);
     else
         patch_tile<cd, DG, DH, false>(P.g, P.pts, P.npts, P.bands, point_freq(P.freqs, l, cd{}), P.m, P.row0, nullptr,
                                       as_global(P.patch_chunk), P.chunk_info, as_global(P.chunk_faces), dest, pc, l, r0,
-                                      min(P.rpt, P.nrows - r0), acc, frame, counters, mtab);
+                                      min(P.rpt, P.nrows - r0), acc, frame, exps);
 }
 
 template <bool DG, bool DH>
@@ -503,10 +504,8 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_scene_gh_tiles(const Scene
                                                                   unsigned t0) {
     __shared__ double2 acc[kPatchPairs * kPatchVerts];
     __shared__ double2 frame[kFramePairs * kPatchThreads];
-    __shared__ int counters[2];
-    __shared__ MathTables mtab;
-    load_math_tables(&mtab);
-    scene_tile<DG, DH>(pieces, npieces, t0 + blockIdx.x, acc, frame, counters, mtab);
+    __shared__ double2 exps[2 * kExpNodes];
+    scene_tile<DG, DH>(pieces, npieces, t0 + blockIdx.x, acc, frame, exps);
 }
 
 template <bool DG, bool DH>
@@ -514,17 +513,15 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_scene_gh_persistent(const 
                                                                  unsigned ntiles, unsigned *__restrict__ counter) {
     __shared__ double2 acc[kPatchPairs * kPatchVerts];
     __shared__ double2 frame[kFramePairs * kPatchThreads];
-    __shared__ int counters[2];
-    __shared__ MathTables mtab;
+    __shared__ double2 exps[2 * kExpNodes];
     __shared__ unsigned next_tile;
-    load_math_tables(&mtab);
     for (;;) {
         __syncthreads();  // the previous tile's write-out has read acc; next_tile is free
         if (threadIdx.x == 0) next_tile = atomicAdd(counter, 1u);
         __syncthreads();
         const unsigned t = __builtin_amdgcn_readfirstlane(next_tile);
         if (t >= ntiles) break;  // uniform across the block: every wave leaves
-        scene_tile<DG, DH>(pieces, npieces, t, acc, frame, counters, mtab);
+        scene_tile<DG, DH>(pieces, npieces, t, acc, frame, exps);
     }
 }
 
@@ -534,17 +531,18 @@ __global__ void k_zero_counter(unsigned *counter) {
 }
 
 // ------------------------------------------------------------------------
-// B_trans and B_angular, regular faces.  NW waves per (row, frequency slot), 4 waves per block: the lanes stride over the
-// faces, then the 48 sums are reduced over the lanes and the NW waves.
+// B_trans and B_angular, regular faces.  Grid: (frequency slots, rows), 256 threads: the lanes stride over the faces, then
+// the 48 sums are reduced over the lanes and the waves.
 //
 // Bound by FP64 VALU issue.  A point adds to 12 complex moments of its face
 // (h, n.h, h h and two scalars, each times a function of r and s); every factor
 // that depends on the frequency alone (1/s^2, s, 1/s) waits until the face's
 // or the row's end, and the trace of the h h moment serves as the scalar moment
-// of the same function (|h| = 1).  156 instructions per point; with the factors
-// applied per point it was 203.  The two real frequencies of an even L share a
-// slot in real arithmetic (133 per point for both).  Icosphere level 4, L = 32:
-// 31.9 ms (33.1 with a slot each, 43.0 at 203).
+// of the same function (|h| = 1).  123 instructions per point, 156 before the
+// exponentials were tabulated (exp_pair), 203 with the factors applied per point.
+// The two real frequencies of an even L share a slot in real arithmetic.
+// Icosphere level 4, L = 32: 25.4 ms (31.9 at 156, 33.1 with a slot for each real
+// frequency, 43.0 at 203).
 // ------------------------------------------------------------------------
 constexpr int kBWords = 48;  // B_trans (6 sym complex) + B_angular (18 complex), as doubles
 
@@ -555,8 +553,8 @@ constexpr int kBWords = 48;  // B_trans (6 sym complex) + B_angular (18 complex)
 template <class T, bool GAL, bool BANDED>
 __device__ __attribute__((always_inline)) inline void b_sums(const Geom &g, const double4 *__restrict__ quad, int npts,
                                                              const PointFreq<T> &f, const Mat &m, int i,
-                                                             const double4 *__restrict__ tpts, int first, int step,
-                                                             const FaceBands &fb, const MathTables &mtab, double (&out)[kBWords]) {
+                                                             const double4 *__restrict__ tpts,
+                                                             const FaceBands &fb, const double2 *exps, double (&out)[kBWords]) {
     double x[3];
     int t[3] = {i, i, i};
     if (GAL) {
@@ -572,7 +570,7 @@ __device__ __attribute__((always_inline)) inline void b_sums(const Geom &g, cons
     for (int k = 0; k < 6; k++) bt[k] = T{0, 0};
 #pragma unroll
     for (int k = 0; k < 18; k++) ba[k] = T{0, 0};
-    for (int fc = first; fc < g.nf; fc += step) {
+    for (int fc = threadIdx.x; fc < g.nf; fc += 256) {
         const int c[3] = {g.F[3 * fc], g.F[3 * fc + 1], g.F[3 * fc + 2]};
         if (touches<GAL ? 3 : 1>(g, t, c)) continue;
         // y - x = o + b1 e1 + b2 e2, whose component along the normal is the same at every point
@@ -603,7 +601,8 @@ __device__ __attribute__((always_inline)) inline void b_sums(const Geom &g, cons
             const double d2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
             const double ir = rsqrt_h3(d2), r = d2 * ir;
             const T z1 = f.sc1 * r, z2 = f.sc2 * r;
-            const T E1 = cexp_neg_tab(z1, &mtab), E2 = cexp_neg_tab(z2, &mtab);
+            T E1, E2;
+            exp_pair(r, f, exps, E1, E2);
             const T s2 = z2 * E2 + E2, dS = (z1 * E1 + E1) - s2;  // s^2 A2, s^2 (A1 - A2)
             const double w2 = (w * ir) * ir, w3 = w2 * ir;
             const double h[3] = {w3 * d[0], w3 * d[1], w3 * d[2]};  // w h / r^2
@@ -670,47 +669,38 @@ __device__ __attribute__((always_inline)) inline void wave_sum48(double (&v)[kBW
 
 // GAL: the rows are test points row0 + r, written to rows 3r..3r+2 of an nv3-row buffer; otherwise collocation vertices
 // i = row0 + r, written to rows 3i..3i+2.
-template <int NW, bool GAL, bool BANDED>
+template <bool GAL, bool BANDED>
 __global__ void __launch_bounds__(256, 2) k_colloc_b(Geom g, const double4 *__restrict__ quad, int npts,
-                                                   const Freq *__restrict__ freqs, int l0, int slots, Mat m, int row0, int nrows,
+                                                   const Freq *__restrict__ freqs, int l0, Mat m, int row0,
                                                    const double4 *__restrict__ tpts, cd *__restrict__ Bt,
                                                    cd *__restrict__ Ba, long long nv3, int real_hi, FaceBands fb) {
     __shared__ double red[4][kBWords];
-    __shared__ MathTables mtab;  // tables of the exponentials
-    load_math_tables(&mtab);
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    // (row, slot) of this group of NW waves, numbered with the slots fastest; past the end: nothing to sum or write
-    const unsigned job = blockIdx.x * (4 / NW) + wave / NW;
-    const int r = job / (unsigned)slots, slot = job - (unsigned)r * slots, i = row0 + r;
-    const bool valid = r < nrows, real = real_hi >= 0 && slot == 0;
+    __shared__ double2 exps[2 * kExpNodes];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = blockIdx.y, slot = blockIdx.x, i = row0 + r;
+    const bool real = real_hi >= 0 && slot == 0;
     double v[kBWords];
-    if (valid) {
-        const int first = lane + 64 * (wave % NW);
-        if (real)
-            b_sums<rp, GAL, BANDED>(g, quad, npts, point_freq(freqs + l0, real_hi, rp{}), m, i, tpts, first, 64 * NW, fb, mtab, v);
-        else
-            b_sums<cd, GAL, BANDED>(g, quad, npts, point_freq(freqs, l0 + slot, cd{}), m, i, tpts, first, 64 * NW, fb, mtab, v);
-        wave_sum48(v, lane);
-    }
-    if (NW > 1) {  // the group's waves, in wave order
-        if (valid && (lane & 7) == 0) {
-#pragma unroll
-            for (int k = 0; k < 6; k++) red[wave][6 * (lane >> 3) + k] = v[k];
-        }
+    auto sums = [&](auto f) {
+        fill_exp_table(f, exps);
         __syncthreads();
-        if (wave % NW) return;
-        if (valid) {
+        b_sums<decltype(f.s), GAL, BANDED>(g, quad, npts, f, m, i, tpts, fb, exps, v);
+    };
+    if (real) sums(point_freq(freqs + l0, real_hi, rp{}));
+    else sums(point_freq(freqs, l0 + slot, cd{}));
+    wave_sum48(v, lane);
+    if ((lane & 7) == 0) {
 #pragma unroll
-            for (int k = 0; k < 6; k++) {
-                v[k] = red[wave][6 * (lane >> 3) + k];
+        for (int k = 0; k < 6; k++) red[wave][6 * (lane >> 3) + k] = v[k];
+    }
+    __syncthreads();
+    if (wave) return;
 #pragma unroll
-                for (int w = 1; w < NW; w++) v[k] += red[wave + w][6 * (lane >> 3) + k];
-            }
-        }
+    for (int k = 0; k < 6; k++) {  // the waves' sums, in wave order
+        const int w = 6 * (lane >> 3) + k;
+        v[k] = (red[0][w] + red[1][w]) + (red[2][w] + red[3][w]);
     }
     const int q = lane & 7;
-    if (!valid || q > 2) return;
+    if (q > 2) return;
     // one entry per lane; scattered from the packed symmetric form to its full positions
     const int k = 3 * (lane >> 3) + q;
     const double sx = q == 0 ? v[0] : q == 1 ? v[2] : v[4], sy = q == 0 ? v[1] : q == 1 ? v[3] : v[5];
@@ -1476,12 +1466,8 @@ static hipError_t launch_b(const Geom &g, const double4 *quad, int npts, const F
                            const Mat &m, int row0, int nrows, const double4 *tpts, cd *Bt, cd *Ba, long long out_rows,
                            hipStream_t st, const FaceBands &fb) {
     const int slots = real_ends ? std::max(nl - 1, 1) : nl, real_hi = real_ends ? nl - 1 : -1;
-    const long long jobs = (long long)slots * nrows;
-    auto go = [&](auto kernel, int nw) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)((jobs * nw + 3) / 4)), dim3(256), 0, st, g, quad, npts, freqs, l0, slots, m, row0,
-                           nrows, tpts, Bt, Ba, out_rows, real_hi, fb);
-    };
-    go(k_colloc_b<4, GAL, BANDED>, 4);
+    hipLaunchKernelGGL((k_colloc_b<GAL, BANDED>), dim3(slots, nrows), dim3(256), 0, st, g, quad, npts, freqs, l0, m, row0, tpts, Bt,
+                       Ba, out_rows, real_hi, fb);
     return hipGetLastError();
 }
 

@@ -113,3 +113,24 @@ def test_real_frequencies_share_a_slot(ctx, galerkin, L):
             mag = mag + (mt.reshape(L, -1, 3, 1) * np.abs(x)).reshape(L, -1)
         first = name == "H"
         assert (np.abs(got[name].reshape(L, -1) - W) <= 1e-12 * mag)[first:].all(), name
+
+
+@pytest.mark.parametrize("galerkin", [False, True])
+@pytest.mark.parametrize("dt,R,l", [(1e-2, 0.5, 1), (1e-3, 0.5, 3), (2e-5, 0.9999, 1), (2e-5, 0.9999, 8), (1e-6, 0.9999, 1),
+                                    (1e-6, 0.9999, 0)])
+def test_tabulated_exponentials_over_arguments(ctx, oracle, galerkin, dt, R, l):
+    """|s r / c| from below 1 to 1e4 over the mesh (up to 7 squarings of the tabulated values), complex and real s, against
+    the oracle's exponentials.  Its arguments are rounded to half an ulp, so a value at |z| is good to |z| 1.1e-16 there;
+    four times that (two exponentials, two roundings each) on top of the bounds of a moderate argument: 1e-13, and 1e-10
+    for the finite-part rule of P."""
+    L, rho = 16, 1000.0
+    V, F = M.icosphere(1, 0.2)
+    V = M.center(M.jitter(V, F, 0.01, 6), F)
+    _, c1, c2 = M.material_speeds(1e6, 0.35, rho)
+    s = oracle.frequencies(L, R, dt, 2)[l]
+    z = abs(s) * 0.42 / c2
+    print(f"exponentials dt={dt} l={l} |z|={z:.3g} galerkin={galerkin}", flush=True)
+    g = ctx.laplace(abi.make_mesh(V, F), abi.make_params(c1, c2, rho, 0.35, dt, R, L, order=2, subdivision=1, galerkin=galerkin), l)
+    o = oracle.laplace(V, F, oracle.params(c1, c2, rho, 0.35, dt, R, L, order=2, subdiv=1, galerkin=galerkin, nthreads=8), s)
+    for k, tol in (("U", 1e-13), ("P", 1e-10), ("Bt", 1e-13), ("Ba", 1e-13)):
+        assert off(g[k], o[k]) <= tol + 4 * z * 1.1e-16, k
