@@ -1105,23 +1105,6 @@ void zero(cd *p, long long n, int num_cus, hipStream_t st) {
     check(hipGetLastError(), "k_fill_zero");
 }
 
-struct EvTimer {
-    hipEvent_t a = nullptr, b = nullptr;
-    hipStream_t st;
-    double *acc;
-    bool on;
-    EvTimer(hipStream_t s, double *d) : st(s), acc(d), on(phase_timers_on()) {
-        if (on) (void)hipEventCreate(&a), (void)hipEventCreate(&b), (void)hipEventRecord(a, st);
-    }
-    ~EvTimer() {
-        if (!on) return;
-        float ms = 0;
-        if (hipEventRecord(b, st) == hipSuccess && hipEventSynchronize(b) == hipSuccess && hipEventElapsedTime(&ms, a, b) == hipSuccess)
-            *acc += ms;
-        (void)hipEventDestroy(a), (void)hipEventDestroy(b);
-    }
-};
-
 }  // namespace
 
 int galerkin_chunk_faces(int nv, int nf, int npts, int nl, bool G, bool H, bool B, size_t budget) {
@@ -1196,7 +1179,7 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
         // Test-point rows: the collocation kernels evaluate, for every rule point x_a of the test faces of a
         // chunk, the row sum over the source faces not touching x_a's face; k_gal_project then weights the
         // rows by the test basis.  Chunks are runs of one colour class, so their faces share no vertex.
-        EvTimer t(st, &tm[1]);
+        PhaseTimer t(st, &tm[1]);
         const int npts = job.npts;
         const long long ntp = (long long)nf * npts;
         DevVec dtp, dpsi, dsG, dsH, dsBt, dsBa;
@@ -1232,7 +1215,7 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
                     {
                         // the patch kernel at the test points: timed on its own, with its launches and its unique
                         // evaluations (test point, regular source face, source point, frequency)
-                        EvTimer tp(st, &tm[2]);
+                        PhaseTimer tp(st, &tm[2]);
                         check(launch_colloc_gh_patch(g, job.patch_pts, npts, job.freqs, 0, nl, job.real_ends, job.mat, row0, nrows,
                                                     tpts, job.patch_chunk, job.chunk_info, job.chunk_faces, job.patch_verts,
                                                     job.npatches, sG, sH, n3, ls, st),
@@ -1259,7 +1242,7 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
             }
         }
     } else if (U || P || Bt || Ba) {
-        EvTimer t(st, &tm[1]);
+        PhaseTimer t(st, &tm[1]);
         for (size_t c = 0; c < classes.size(); c++) {
             const int cnt = cls_off[c + 1] - cls_off[c];
             const int *fc = faces + cls_off[c];
@@ -1323,7 +1306,7 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
     dscratch.alloc((size_t)npairs * nl * kPairStride * sizeof(cd), "device allocation: touching-pair scratch");
     cd *scratch = (cd *)dscratch.p;
     {
-        EvTimer t(st, &tm[3]);
+        PhaseTimer t(st, &tm[3]);
         const int beg[3] = {0, kind_off[1], kind_off[2]}, end[3] = {kind_off[1], kind_off[2], kind_off[3]};
 #define CQBEM_SING(MODE, KIND)                                                                                        \
     if (end[KIND - 1] > beg[KIND - 1])                                                                                \
@@ -1395,7 +1378,7 @@ void run_galerkin(const GalerkinJob &job, const int *F, const int *vmap, cd *U, 
     const int2 *db = dblocks.up(blocks, st);
     const int *dpt = dptr.up(ptr, st), *dit = ditems.up(items, st), *dvp = dvptr.up(vptr, st), *dvi = dvitems.up(vitems, st);
     {
-        EvTimer t(st, &tm[3]);
+        PhaseTimer t(st, &tm[3]);
         if (U || P) {
             const long long n = (long long)blocks.size() * nl;
             hipLaunchKernelGGL(k_gal_gather_gh, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, db, dpt, dit, (int)blocks.size(), nl,

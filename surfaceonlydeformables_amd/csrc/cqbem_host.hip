@@ -74,7 +74,35 @@ struct DBuf {
         bytes = n;
         if (n) HIPCHK(dev_alloc(&p, n, &pooled));
     }
+    // a part of another buffer, which outlives it
+    void view(void *q, size_t n) { dev_free(p, pooled), p = q, bytes = n, pooled = true; }
     template <class T> T *as() const { return reinterpret_cast<T *>(p); }
+};
+
+// Several arrays in one device buffer and one copy: add() them, then send().  The host side stays until this is destroyed.
+class PackedUpload {
+  public:
+    template <class T> void add(DBuf &b, const T *v, size_t n) {
+        const size_t off = (host_.size() + 255) & ~(size_t)255;
+        host_.resize(off + n * sizeof(T));
+        if (n) std::memcpy(host_.data() + off, v, n * sizeof(T));
+        parts_.push_back(Part{&b, off, n * sizeof(T)});
+    }
+    template <class T> void add(DBuf &b, const std::vector<T> &v) { add(b, v.data(), v.size()); }
+    void send(hipStream_t st) {
+        all_.alloc(host_.size());
+        HIPCHK(hipMemcpyAsync(all_.p, host_.data(), host_.size(), hipMemcpyHostToDevice, st));
+        for (const Part &p : parts_) p.buf->view(p.bytes ? (char *)all_.p + p.off : nullptr, p.bytes);
+    }
+
+  private:
+    struct Part {
+        DBuf *buf;
+        size_t off, bytes;
+    };
+    std::vector<char> host_;
+    std::vector<Part> parts_;
+    DBuf all_;
 };
 
 template <class T> void upload(DBuf &b, const std::vector<T> &v, hipStream_t st) {
@@ -575,6 +603,7 @@ struct DevMesh {
     DBuf V, F, N, area, vs_ptr, vs_face, sg_ptr, sg_face, vmap, quad, line, freqs, tab;
     DBuf patch_chunk, chunk_info, chunk_faces, patch_verts, patch_pts;
     DBuf far_pts, patch_sphere, far_quad, face_sphere;  // CQBEM_QUAD_BANDED
+    PackedUpload all;  // holds the above
     Geom g;
 };
 
@@ -644,25 +673,21 @@ hipError_t launch_gh(const DevMesh &d, const Prepared &P, const Freq *freqs, int
                                  d.patch_verts.as<int>(), P.npatches, UG, UH, ld, lstride, st, bands_of(d, P));
 }
 
+// One copy of all arrays: each copy of its own cost 10 us of launch and gap, 17 of them 165 us of a small job's 400.
 void upload_mesh(DevMesh &d, const cqbem_mesh *mesh, const Prepared &P, hipStream_t st) {
-    d.V.alloc(sizeof(double) * 3 * P.nv);
-    HIPCHK(hipMemcpyAsync(d.V.p, mesh->V, sizeof(double) * 3 * P.nv, hipMemcpyHostToDevice, st));
-    d.F.alloc(sizeof(int) * 3 * P.nf);
-    HIPCHK(hipMemcpyAsync(d.F.p, mesh->F, sizeof(int) * 3 * P.nf, hipMemcpyHostToDevice, st));
-    if (mesh->vertex_map_inverse) {
-        d.vmap.alloc(sizeof(int) * P.nv);
-        HIPCHK(hipMemcpyAsync(d.vmap.p, mesh->vertex_map_inverse, sizeof(int) * P.nv, hipMemcpyHostToDevice, st));
-    }
-    upload(d.N, P.N, st), upload(d.area, P.area, st), upload(d.vs_ptr, P.vs_ptr, st), upload(d.vs_face, P.vs_face, st);
-    upload(d.sg_ptr, P.sg_ptr, st), upload(d.sg_face, P.sg_face, st), upload(d.quad, P.quad, st), upload(d.line, P.line, st);
-    upload(d.freqs, P.freqs, st), upload(d.tab, P.tab, st);
-    upload(d.patch_chunk, P.patch_chunk, st), upload(d.chunk_info, P.chunk_info, st);
-    upload(d.chunk_faces, P.chunk_faces, st), upload(d.patch_verts, P.patch_verts, st);
-    upload(d.patch_pts, P.patch_pts, st);
+    PackedUpload &u = d.all;
+    u.add(d.V, mesh->V, 3 * (size_t)P.nv), u.add(d.F, mesh->F, 3 * (size_t)P.nf);
+    if (mesh->vertex_map_inverse) u.add(d.vmap, mesh->vertex_map_inverse, P.nv);
+    u.add(d.N, P.N), u.add(d.area, P.area), u.add(d.vs_ptr, P.vs_ptr), u.add(d.vs_face, P.vs_face);
+    u.add(d.sg_ptr, P.sg_ptr), u.add(d.sg_face, P.sg_face), u.add(d.quad, P.quad), u.add(d.line, P.line);
+    u.add(d.freqs, P.freqs), u.add(d.tab, P.tab);
+    u.add(d.patch_chunk, P.patch_chunk), u.add(d.chunk_info, P.chunk_info);
+    u.add(d.chunk_faces, P.chunk_faces), u.add(d.patch_verts, P.patch_verts), u.add(d.patch_pts, P.patch_pts);
     if (!P.far_patch_pts.empty()) {
-        upload(d.far_pts, P.far_patch_pts, st), upload(d.patch_sphere, P.patch_sphere, st);
-        if (!P.face_sphere.empty()) upload(d.far_quad, P.far_quad, st), upload(d.face_sphere, P.face_sphere, st);
+        u.add(d.far_pts, P.far_patch_pts), u.add(d.patch_sphere, P.patch_sphere);
+        if (!P.face_sphere.empty()) u.add(d.far_quad, P.far_quad), u.add(d.face_sphere, P.face_sphere);
     }
+    u.send(st);
     Geom &g = d.g;
     g.V = d.V.as<double>(), g.F = d.F.as<int>(), g.N = d.N.as<double>(), g.area = d.area.as<double>();
     g.vs_ptr = d.vs_ptr.as<int>(), g.vs_face = d.vs_face.as<int>(), g.sg_ptr = d.sg_ptr.as<int>(), g.sg_face = d.sg_face.as<int>();
@@ -679,28 +704,6 @@ int slab_rows(int nv, int Lf, int nmat, size_t bytes) {
     rows = std::min<size_t>(std::max<size_t>(rows, 1), (size_t)nv);
     return (int)std::min<size_t>(rows, 65535);
 }
-
-struct Timer {
-    hipEvent_t a = nullptr, b = nullptr;
-    hipStream_t st;
-    double *acc;
-    bool on;
-    Timer(hipStream_t s, double *dst) : st(s), acc(dst), on(phase_timers_on()) {
-        if (!on) return;
-        HIPCHK(hipEventCreate(&a));
-        HIPCHK(hipEventCreate(&b));
-        HIPCHK(hipEventRecord(a, st));
-    }
-    ~Timer() {
-        if (!on) return;
-        if (hipEventRecord(b, st) == hipSuccess && hipEventSynchronize(b) == hipSuccess) {
-            float ms = 0;
-            if (hipEventElapsedTime(&ms, a, b) == hipSuccess) *acc += ms;
-        }
-        (void)hipEventDestroy(a);
-        (void)hipEventDestroy(b);
-    }
-};
 
 // Bound of the Galerkin per-test-point row scratch within a job's scratch budget: larger chunks only save
 // launches, the traffic per face is the same.
@@ -740,9 +743,11 @@ uint64_t footprint(const cqbem_mesh *mesh, const cqbem_params *p, int outputs_on
 void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const cqbem_params *p, const cqbem_outputs *out,
              size_t slab_budget, double *tm, bool sync_outputs, JobArena *fixed_arena = nullptr,
              const std::atomic<int> *cancel = nullptr) {
-    // a cancelled serving job ends at the next check (the arena then waits for the work already launched)
-    auto check_cancel = [cancel]() {
-        if (cancel && cancel->load()) throw Err{CQBEM_ERR_CANCELLED, "job cancelled"};
+    // a cancelled serving job ends at the next check, before which the work launched so far is waited for
+    auto check_cancel = [cancel, st]() {
+        if (!cancel) return;
+        HIPCHK(hipStreamSynchronize(st));
+        if (cancel->load()) throw Err{CQBEM_ERR_CANCELLED, "job cancelled"};
     };
     // every device buffer of the job comes from the context's pool and goes back to it when the stream is done
     // (CQBEM_POOL=0: plain hipMalloc / hipFree per buffer), or from the caller's fixed region
@@ -752,6 +757,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
     }();
     JobArena arena(&ctx->pool, st);
     ArenaScope arena_scope(fixed_arena ? fixed_arena : use_pool ? &arena : nullptr);
+    PhaseEvents phases;
     const auto t_host0 = std::chrono::steady_clock::now();
     Prepared P = prepare(mesh, p);
     const int nv = P.nv, L = P.L, Lf = P.Lf;
@@ -826,7 +832,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
                 check_cancel();
                 const int nr = std::min(rows, nv - r0);
                 {
-                    Timer t(st, &tm[1]);
+                    PhaseTimer t(st, &tm[1]);
                     if (!g32) {
                         HIPCHK(launch_gh(d, P, freqs, 0, Lf, r0, nr, specG.as<cd>(), specH.as<cd>(), n3, lstride, st));
                     } else {
@@ -839,7 +845,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
                 tm[6] += 1;
                 for (int i = r0; i < r0 + nr; i++) tm[7] += regular_evals(P, mesh->V, i);
                 {
-                    Timer t(st, &tm[3]);
+                    PhaseTimer t(st, &tm[3]);
                     if (wantG)
                         HIPCHK(launch_colloc_singular(0, g, line, nline, freqs, 0, Lf, P.mat, r0, nr, specG.as<cd>(), n3,
                                                       lstride, nullptr, nullptr, st));
@@ -848,7 +854,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
                                                       lstride, nullptr, nullptr, st));
                 }
                 {
-                    Timer t(st, &tm[4]);
+                    PhaseTimer t(st, &tm[4]);
                     const long long E = 3LL * nr * n3;
                     if (wantG) HIPCHK(transform_into(G, specG.as<cd>(), E, lstride, 3LL * r0 * n3));
                     if (wantH) HIPCHK(transform_into(H, specH.as<cd>(), E, lstride, 3LL * r0 * n3));
@@ -858,7 +864,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
         if (wantB) {
             check_cancel();
             {
-                Timer t(st, &tm[2]);
+                PhaseTimer t(st, &tm[2]);
                 if (mixed)
                     HIPCHK(launch_colloc_b32(g, quad, npts, freqs32, 0, Lf, mat32, 0, nv, specB.as<cd>(), specBa.as<cd>(), st,
                                              fbands_of(d, P)));
@@ -867,7 +873,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
                                            fbands_of(d, P)));
             }
             {
-                Timer t(st, &tm[3]);
+                PhaseTimer t(st, &tm[3]);
                 HIPCHK(launch_colloc_singular(1, g, line, nline, freqs, 0, Lf, P.mat, 0, nv, nullptr, n3, 0, specB.as<cd>(),
                                               specBa.as<cd>(), st));
             }
@@ -897,7 +903,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
             if (wantH) specH.alloc((size_t)Lf * lstride * sizeof(cd));
             run_galerkin(gj, mesh->F, mesh->vertex_map_inverse, specG.as<cd>(), specH.as<cd>(),
                          wantB ? specB.as<cd>() : nullptr, wantB ? specBa.as<cd>() : nullptr, tm, st);
-            Timer t(st, &tm[4]);
+            PhaseTimer t(st, &tm[4]);
             if (wantG) HIPCHK(transform_into(G, specG.as<cd>(), n3 * n3, n3 * n3, 0));
             if (wantH) HIPCHK(transform_into(H, specH.as<cd>(), n3 * n3, n3 * n3, 0));
         }
@@ -923,7 +929,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
         }
     }
     if (wantB) {
-        Timer t(st, &tm[4]);
+        PhaseTimer t(st, &tm[4]);
         HIPCHK(launch_transform(specB.as<cd>(), n3 * 3, n3 * 3, Lf, tab, L, Wbt, n3 * 3, ctx->num_cus, st));
         HIPCHK(launch_transform(specBa.as<cd>(), n3 * 9, n3 * 9, Lf, tab, L, Wba, n3 * 9, ctx->num_cus, st));
         HIPCHK(launch_b_post(Wbt, Wba, W6, g.V, nv, L, st));
@@ -939,6 +945,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
         tm[5] += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
     HIPCHK(hipStreamSynchronize(st));
+    phases.resolve();
 }
 
 // Stream capture of a launch sequence into a HIP graph that is launched once and waited for.  With capture off

@@ -126,6 +126,61 @@ inline bool &phase_timers_on() {
     return on;
 }
 
+// The phase timers of the job running on this thread: event pairs around the phases, read once the job's stream is done,
+// so that no phase waits for the one before it.
+class PhaseEvents {
+  public:
+    PhaseEvents() : prev_(current()) { current() = this; }
+    ~PhaseEvents() {
+        current() = prev_;
+        for (Pair &p : pairs_) (void)hipEventDestroy(p.a), (void)hipEventDestroy(p.b);
+    }
+    PhaseEvents(const PhaseEvents &) = delete;
+    PhaseEvents &operator=(const PhaseEvents &) = delete;
+    void add(hipEvent_t a, hipEvent_t b, double *ms) { pairs_.push_back(Pair{a, b, ms}); }
+    // Adds every phase's milliseconds to its sum; the stream has been synchronised.
+    void resolve() {
+        for (Pair &p : pairs_) {
+            float ms = 0;
+            if (hipEventElapsedTime(&ms, p.a, p.b) == hipSuccess) *p.ms += ms;
+        }
+    }
+    static PhaseEvents *&current() {
+        static thread_local PhaseEvents *c = nullptr;
+        return c;
+    }
+
+  private:
+    struct Pair {
+        hipEvent_t a, b;
+        double *ms;
+    };
+    std::vector<Pair> pairs_;
+    PhaseEvents *prev_;
+};
+
+// Times the launches of a scope on stream s into *ms (off without a PhaseEvents on this thread).
+class PhaseTimer {
+  public:
+    PhaseTimer(hipStream_t s, double *ms) : st_(s), ms_(ms) {
+        if (!phase_timers_on() || !PhaseEvents::current()) return;
+        if (hipEventCreate(&a_) != hipSuccess) a_ = nullptr;
+        else if (hipEventCreate(&b_) != hipSuccess) b_ = nullptr;
+        if (b_) (void)hipEventRecord(a_, st_);
+    }
+    ~PhaseTimer() {
+        if (b_) (void)hipEventRecord(b_, st_), PhaseEvents::current()->add(a_, b_, ms_);
+        else if (a_) (void)hipEventDestroy(a_);
+    }
+    PhaseTimer(const PhaseTimer &) = delete;
+    PhaseTimer &operator=(const PhaseTimer &) = delete;
+
+  private:
+    hipEvent_t a_ = nullptr, b_ = nullptr;
+    hipStream_t st_;
+    double *ms_;
+};
+
 // The arena of the job running on this thread (set for the duration of a job), or null.
 inline JobArena *&current_arena() {
     static thread_local JobArena *a = nullptr;
