@@ -732,11 +732,27 @@ __global__ void __launch_bounds__(256, 2) k_colloc_b(Geom g, const double4 *__re
 // ------------------------------------------------------------------------
 constexpr int kSingMaxFaces = 16;  // singular faces per batch of one (row, frequency) wavefront
 
-// Sum of v over lanes lane .. lane + gs - 1, in lane order (the group leader's value is the group's sum).
-__device__ inline cd group_sum(cd v, int lane, int gs) {
-    double sx = v.x, sy = v.y;
-    for (int q = 1; q < gs; q++) sx += __shfl(v.x, lane + q), sy += __shfl(v.y, lane + q);
-    return cd{sx, sy};
+// Sums v over the groups of gs lanes, in lane order: sum[group][k] for the first ngroups groups.  Through LDS, 9 words of
+// every lane at a time, each sum taken by one lane; a single wave per block.  (By shuffles, each lane read its gs - 1
+// successors' words: 36 cross-lane moves per entry at gs = 10.)
+template <int N, int NE>
+__device__ __attribute__((always_inline)) inline void group_sums(const cd (&v)[N], cd (*sum)[NE], cd (*part)[64], int lane, int gs, int ngroups) {
+#pragma unroll
+    for (int k0 = 0; k0 < N; k0 += 9) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 9; k++)
+            if (k0 + k < N) part[k][lane] = v[k0 + k];
+        __syncthreads();
+        const int n = N - k0 < 9 ? N - k0 : 9;
+        for (int o = lane; o < n * ngroups; o += 64) {
+            const int grp = o / n, k = o - grp * n;
+            cd t = part[k][grp * gs];
+            for (int q = 1; q < gs; q++) t += part[k][grp * gs + q];
+            sum[grp][k0 + k] = t;
+        }
+    }
+    __syncthreads();
 }
 
 __device__ inline void unit3(double v[3]) {
@@ -750,7 +766,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
                                                          int nrows, cd *__restrict__ U, long long ld, long long lstride,
                                                          cd *__restrict__ Bt, cd *__restrict__ Ba, long long nv3) {
     constexpr int NE = KIND == 1 ? 36 : 27;  // per face: B 9 + 27 entries; G/H 3 corners x 3 x 3
-    __shared__ cd fsum[kSingMaxFaces][NE];
+    __shared__ cd fsum[kSingMaxFaces][NE], part[9][64];
     __shared__ int fj[kSingMaxFaces][3], umap[kSingMaxFaces][3], ucol[3 * kSingMaxFaces + 1];
     const int il = blockIdx.x / nl, l = blockIdx.x % nl;
     const int i = row0 + il;
@@ -771,7 +787,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
             y1[k] = g.V[3 * j[0] + k], y2[k] = g.V[3 * j[1] + k], y3[k] = g.V[3 * j[2] + k], n[k] = g.N[3 * fc + k];
         double v1[3], v2[3];
         for (int k = 0; k < 3; k++) v1[k] = y2[k] - y1[k], v2[k] = y3[k] - y1[k];
-        const bool leader = active && t == 0;  // holds the face's sums after group_sum
+        const bool leader = active && t == 0;  // turns the face's sums (group_sums) into its entries
         if (KIND == 0 || KIND == 1) {
             // polar frame around y1
             double u1[3] = {v1[0], v1[1], v1[2]}, u2[3] = {v2[0], v2[1], v2[2]};
@@ -859,22 +875,36 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
                 }
             }
             if (KIND == 0) {
+                cd v[21];
+#pragma unroll
                 for (int k = 0; k < 3; k++) {
-                    gb[k] = group_sum(gb[k], lane, GS);
-                    for (int e2 = 0; e2 < 6; e2++) ga[k][e2] = group_sum(ga[k][e2], lane, GS);
+                    v[7 * k + 6] = gb[k];
+#pragma unroll
+                    for (int e2 = 0; e2 < 6; e2++) v[7 * k + e2] = ga[k][e2];
                 }
-                if (leader)
+                group_sums(v, fsum, part, lane, GS, nb);
+                if (leader) {
+#pragma unroll
+                    for (int k = 0; k < 21; k++) v[k] = fsum[slot][k];
+#pragma unroll
                     for (int k = 0; k < 3; k++)
+#pragma unroll
                         for (int a2 = 0; a2 < 3; a2++)
+#pragma unroll
                             for (int b = 0; b < 3; b++) {
-                                cd v = ga[k][sidx(a2, b)];
-                                if (a2 == b) v += gb[k];
-                                fsum[slot][k * 9 + a2 * 3 + b] = v;
+                                cd u = v[7 * k + sidx(a2, b)];
+                                if (a2 == b) u += v[7 * k + 6];
+                                fsum[slot][k * 9 + a2 * 3 + b] = u;
                             }
+                }
             } else {
-                for (int k = 0; k < 3; k++) mt[k] = group_sum(mt[k], lane, GS);
-                for (int k = 0; k < 6; k++) M[k] = group_sum(M[k], lane, GS);
-                m2 = group_sum(m2, lane, GS), S = group_sum(S, lane, GS), S3 = group_sum(S3, lane, GS);
+                cd v12s[12] = {mt[0], mt[1], mt[2], M[0], M[1], M[2], M[3], M[4], M[5], m2, S, S3};
+                group_sums(v12s, fsum, part, lane, GS, nb);
+                if (leader) {
+                    for (int k = 0; k < 3; k++) mt[k] = fsum[slot][k];
+                    for (int k = 0; k < 6; k++) M[k] = fsum[slot][3 + k];
+                    m2 = fsum[slot][9], S = fsum[slot][10], S3 = fsum[slot][11];
+                }
                 if (leader)
                 for (int a2 = 0; a2 < 3; a2++)
                     for (int b = 0; b < 3; b++) {
@@ -945,11 +975,12 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
                         }
                     }
             }
-            for (int e = 0; e < 27; e++) out[e] = group_sum(out[e], lane, GS);
-            if (leader)
-                for (int p = 0; p < 3; p++)
-                    for (int qq = 0; qq < 3; qq++)
-                        for (int k = 0; k < 3; k++) fsum[slot][k * 9 + p * 3 + qq] = out[(p * 3 + qq) * 3 + k];
+            cd v[27];  // in fsum's order
+#pragma unroll
+            for (int e = 0; e < 9; e++)
+#pragma unroll
+                for (int k = 0; k < 3; k++) v[k * 9 + e] = out[e * 3 + k];
+            group_sums(v, fsum, part, lane, GS, nb);
         }
         if (leader)
             for (int k = 0; k < 3; k++) fj[slot][k] = j[k];
