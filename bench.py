@@ -651,7 +651,7 @@ def main():
         ctx.assemble_device(mesh, params, ptrs)
         lat.append((time.perf_counter() - t0) * 1e3)
         tm = ctx.last_timings()
-        gh_ms += tm["regular_b" if params.galerkin else "regular_gh"]  # Galerkin: the pair kernel at the test points
+        gh_ms += tm["regular_b" if params.galerkin else "regular_gh"]  # Galerkin: the patch kernel at the test points
         gh_evals += tm["gh_evaluations"]
         gh_launches += int(tm["gh_launches"])
     torch.cuda.synchronize()
@@ -667,7 +667,7 @@ def main():
     history = history_step(ctx, ptrs, n3, L, torch, dev)
 
     phase_keys = ("regular_gh", "regular_b", "singular", "transform", "host")
-    if params.galerkin:  # non-singular G/H/B with the test projection in one phase, of which the G/H pair kernel
+    if params.galerkin:  # non-singular G/H/B with the test projection in one phase, of which the G/H patch kernel
         phases = {"nonsingular": last["regular_gh"], "nonsingular_gh_pair_kernel": last["regular_b"],
                   "singular_pairs": last["singular"], "transform": last["transform"], "host": last["host"]}
     else:
@@ -700,14 +700,14 @@ def main():
         line["banded_vs_reference_rule"] = cmp
         if roof:
             roof["note"] = "banded: evaluations counted per tile's rule"
-            roof["kernel"] = "k_colloc_gh_pair<true,true,false,true>"
+            roof["kernel"] = "k_colloc_gh_patch<true,true,false,true>"
     if args.precision == "mixed":
         line["mixed_vs_fp64"] = mixed_against_fp64(ctx, mesh, params, outs, ms_per_step, torch, dev)
         if roof and os.environ.get("CQBEM_MIXED_G") == "float":
-            roof["note"] = "mixed, float G: the timed G/H phase is the double H pair kernel plus the float G kernel"
-            roof["kernel"] = "k_colloc_gh_pair<false,true,false,false> + k_colloc_g32"
+            roof["note"] = "mixed, float G: the timed G/H phase is the double H patch kernel plus the float G kernel"
+            roof["kernel"] = "k_colloc_gh_patch<false,true,false,false> + k_colloc_g32"
         elif roof:
-            roof["note"] = "mixed: G and H in the double pair kernel, the far-field B in float"
+            roof["note"] = "mixed: G and H in the double patch kernel, the far-field B in float"
     if args.precision == "fp64" and args.quad == "reference" and not params.galerkin:
         # the metric's comparison, in the same run after the timed FP64 steps: the mixed-precision job, alone and
         # with the distance-banded rule, against the FP64 outputs just assembled
@@ -726,7 +726,7 @@ def main():
 
 def galerkin_line(ctx, torch, dev, steps=1):
     """The icosphere-L3 Galerkin workload (L = 64, 1926 x 1926 complex matrices per frequency) in the same run: one
-    warm-up and `steps` timed assemblies into device outputs, its phases and the pair kernel's roofline at the test
+    warm-up and `steps` timed assemblies into device outputs, its phases and the patch kernel's roofline at the test
     points."""
     from surfaceonlydeformables_amd import abi
     V, F, params, desc = workload("ico3-galerkin", "fp64")
@@ -788,7 +788,7 @@ def variant_against_fp64(ctx, mesh, params, outs, fp64_ms, torch, precision, ban
             "rel_err_stack": stack, "rel_err_max_per_weight": worst,
             "gh_within_1e-6": stack["G"] <= 1e-6 and stack["H"] <= 1e-6,
             "note": ("far-field B_trans and B_angular in float (Kahan-compensated face sums); G and H in the double "
-                     "pair kernel" + ("; G/H tiles beyond the band threshold on the far rule" if banded else "")
+                     "patch kernel" + ("; G/H tiles beyond the band threshold on the far rule" if banded else "")
                      + "; H, singular faces and the inverse transform in double")}
 
 
@@ -824,15 +824,15 @@ def mixed_against_fp64(ctx, mesh, params, outs, mixed_ms, torch, dev, steps=3):
 
 def roofline(gh_ms, gh_evals, gh_launches, with_traffic, galerkin=False):
     """VALU roofline of the dominant kernel from the library's HIP-event timers; the HBM traffic per launch is
-    the committed counter measurement of the icosphere-L4 shape.  Galerkin: the same pair kernel at the test
+    the committed counter measurement of the icosphere-L4 shape.  Galerkin: the same patch kernel at the test
     points, per (test point, regular source face, source point, frequency)."""
     achieved = FLOPS_PER_EVAL_GH * gh_evals / (gh_ms * 1e-3) / 1e12
-    kernel = "k_colloc_gh_pair<true,true,true,false>" if galerkin else "k_colloc_gh_pair<true,true,false,false>"
+    kernel = "k_colloc_gh_patch<true,true,true,false>" if galerkin else "k_colloc_gh_patch<true,true,false,false>"
     roof = {"bound": "valu", "kernel": kernel, "achieved": achieved, "peak": PEAK_FP64_TFLOPS,
             "unit": "TFLOP/s", "frac": achieved / PEAK_FP64_TFLOPS, "traffic": None,
             "launch_ms": gh_ms / max(gh_launches, 1),
             "flops_per_launch": FLOPS_PER_EVAL_GH * gh_evals / max(gh_launches, 1)}
-    prof = os.path.join(ROOT, "profiles", "k_colloc_gh_pair_icosphere_l4_traffic.json")
+    prof = os.path.join(ROOT, "profiles", "k_colloc_gh_patch_icosphere_l4_traffic.json")
     if with_traffic and os.path.exists(prof):
         with open(prof) as fh:
             roof["traffic"] = json.load(fh).get("hbm_bytes_per_launch")

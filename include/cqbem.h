@@ -46,7 +46,7 @@ enum { CQBEM_BDF1 = 1, CQBEM_BDF2 = 2 };
 /* CQBEM_MIXED (collocation): far-field B_trans and B_angular integrated in float, as the reference's typedefs do
  * (B_trans_collocation.cu:14, B_angular_collocation.cu:14), with Kahan-compensated face sums; H, the singular faces
  * and the inverse transform in double.  Far-field G stays in double by default: it shares H's exponentials in the
- * pair kernel, which costs less than a float kernel of its own; the environment variable CQBEM_MIXED_G=float
+ * patch kernel, which costs less than a float kernel of its own; the environment variable CQBEM_MIXED_G=float
  * selects the reference's float G (G_collocation.cu:14-15) instead.  Galerkin: the far-field B at the test points
  * in float, G and H in double (CQBEM_MIXED_G=float with Galerkin returns CQBEM_ERR_UNSUPPORTED). */
 enum { CQBEM_FP64 = 0, CQBEM_MIXED = 1 };
@@ -135,7 +135,7 @@ int cqbem_assemble_noalloc(cqbem_context *ctx, const cqbem_mesh *mesh, const cqb
 /* All objects of a scene in one call (device outputs only).  No counterpart in the reference, whose
  * Simulator::init assembles one object group after another (simulator.cpp:101-125).  The G/H regular-face tiles
  * of every collocation object -- (column patch, frequency, row) tiles of all objects, largest objects first --
- * run in shared launches of the pair kernel, in waves whose Laplace-domain spectra fit the HBM budget; each
+ * run in shared launches of the patch kernel, in waves whose Laplace-domain spectra fit the HBM budget; each
  * wave (the shared launch, the float G kernel of CQBEM_MIXED objects, the singular faces and the transforms of
  * every object slab) is captured in one HIP graph and launched once, and B, C and the B post-processing of all
  * objects follow in one more graph.  Galerkin objects run after them, one by one, as cqbem_assemble runs them.
@@ -209,7 +209,7 @@ int cqbem_frequencies(int32_t L, double R, double dt, int32_t bdf, double *s_out
 /* Statistics of the last cqbem_assemble on this context (device times from HIP events on the context's
  * stream, milliseconds): [0] total wall, [1] regular G/H quadrature (the dominant kernel; Galerkin: all
  * non-singular quadrature, G, H and B, with the test-basis projection), [2] regular B_trans/B_angular
- * quadrature (collocation; Galerkin: the G/H pair kernel at the test points, a part of [1]), [3] singular
+ * quadrature (collocation; Galerkin: the G/H patch kernel at the test points, a part of [1]), [3] singular
  * kernels (collocation: faces at the point; Galerkin: touching pairs and their gather), [4] inverse transform
  * and post-processing, [5] host preparation and staging, [6] launches of the dominant G/H kernel (the pair
  * kernel; Galerkin: at the test points), [7] far-field kernel evaluations (collocation point or test point,
