@@ -262,11 +262,6 @@ __host__ __device__ inline cd cexp_neg_tab(cd z, const MathTables *M) {
     return cd{m * cs, -m * sn};
 }
 
-// The same at two real arguments.
-__host__ __device__ inline rp cexp_neg_tab(rp z, const MathTables *M) {
-    return rp{exp_tab_core(fmax(-z.x, -740.0), M->e), exp_tab_core(fmax(-z.y, -740.0), M->e)};
-}
-
 // exp(-z), Re z >= 0
 __device__ inline cd cexp_neg(cd z) {
     const double m = exp_neg(z.x);
