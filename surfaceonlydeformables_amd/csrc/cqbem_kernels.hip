@@ -1029,55 +1029,15 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
 // entry, NC weights per pass; the table index is uniform (scalar loads).
 // ------------------------------------------------------------------------
 // Inverse CQ transform of one chunk of NC weights n0 .. n0+NC-1: out[n][e] = sum_l Re(X_l(e) T(n, l)), with
-// T(n, l) = (2 or 1) R^-n / L exp(-2 pi i n l / L) (the half-spectrum table).  One lane per entry e; the
-// chunk's table lives in LDS (read as broadcasts) and the spectrum is read LC frequencies at a time so
-// that LC loads per lane are in flight.
-constexpr int kTransformNC = 32, kTransformLC = 8, kTransformMaxLf = 64;
+// T(n, l) = (2 or 1) R^-n / L exp(-2 pi i n l / L) (the half-spectrum table).  The chunk's table lives in LDS (read as
+// broadcasts) and the spectrum is read LC frequencies at a time so that their loads are in flight together.
+constexpr int kTransformNC = 32, kTransformMaxLf = 64;
 
-// OutT: double, or float for resident weights stored in single precision (the sum is formed in double and
-// rounded once).
-template <int NC, int LC, class OutT>
-__global__ void __launch_bounds__(256) k_transform(const cd *__restrict__ spec, long long E, long long spec_ls, int Lf,
-                                                    const double2 *__restrict__ tab, int L, int n0,
-                                                    OutT *__restrict__ out, long long out_nstride) {
-    __shared__ double2 T[NC * kTransformMaxLf];  // [l][k]
-    for (int t = threadIdx.x; t < NC * Lf; t += 256) {
-        const int l = t / NC, k = t % NC;
-        T[t] = n0 + k < L ? tab[(long long)(n0 + k) * Lf + l] : make_double2(0.0, 0.0);
-    }
-    __syncthreads();
-    const long long stride = (long long)gridDim.x * 256;
-    for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < E; e += stride) {
-        double acc[NC];
-#pragma unroll
-        for (int k = 0; k < NC; k++) acc[k] = 0.0;
-        for (int l0 = 0; l0 < Lf; l0 += LC) {
-            cd X[LC];
-#pragma unroll
-            for (int c = 0; c < LC; c++) {
-                // each spectrum value is read once: streaming (non-temporal) loads
-                const double *src = reinterpret_cast<const double *>(spec + (long long)(l0 + c) * spec_ls + e);
-                X[c] = l0 + c < Lf ? cd{__builtin_nontemporal_load(src), __builtin_nontemporal_load(src + 1)} : cd{0.0, 0.0};
-            }
-#pragma unroll
-            for (int c = 0; c < LC; c++) {
-                if (l0 + c >= Lf) break;
-                const double2 *Tl = T + (l0 + c) * NC;
-#pragma unroll
-                for (int k = 0; k < NC; k++) acc[k] = fma(X[c].x, Tl[k].x, fma(-X[c].y, Tl[k].y, acc[k]));
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < NC; k++) {
-            const int n = n0 + k;
-            if (n < L) __builtin_nontemporal_store((OutT)acc[k], out + (long long)n * out_nstride + e);  // written once
-        }
-    }
-}
-
-// The same sums for two adjacent entries per lane (E, spec_ls and out_nstride even, out 16-byte aligned): each
+// OutT: double, or float for resident weights stored in single precision (the sum is formed in double and rounded once).
+// Two adjacent entries per lane (ALIGNED: E and out_nstride even, out aligned to a pair; otherwise the stores are
+// declared unaligned and an odd E's last entry is alone): each
 // frequency's two complex values in one 32-byte read, each weight's two values in one 16-byte store (the store
-// width HBM writes best), and a grid that covers every pair at once.  Each weight is k_transform's sum, term for
+// width HBM writes best), and a grid that covers every pair at once.  Each weight is the same sum, term for
 // term.  LC = 2 frequencies per batch of loads keeps the kernel within 168 VGPRs: 3 waves per SIMD (with 4 it takes
 // 181 VGPRs and 2 waves, 2.6% slower).
 typedef double d2v __attribute__((ext_vector_type(2)));
@@ -1089,7 +1049,7 @@ template <> struct Pair2<double> {
 template <> struct Pair2<float> {
     typedef f2v type;
 };
-template <int LC, class OutT>
+template <int LC, bool ALIGNED, class OutT>
 __global__ void __launch_bounds__(256, 3) k_transform_pair(const cd *__restrict__ spec, long long E, long long spec_ls, int Lf,
                                                         const double2 *__restrict__ tab, int L, int n0,
                                                         OutT *__restrict__ out, long long out_nstride) {
@@ -1113,7 +1073,7 @@ __global__ void __launch_bounds__(256, 3) k_transform_pair(const cd *__restrict_
             const d2v *src = reinterpret_cast<const d2v *>(spec + (long long)(l0 + c) * spec_ls + e);
             if (l0 + c < Lf) {
                 X0[c] = __builtin_nontemporal_load(src);
-                X1[c] = __builtin_nontemporal_load(src + 1);
+                X1[c] = ALIGNED || e + 1 < E ? __builtin_nontemporal_load(src + 1) : d2v{0.0, 0.0};
             } else {
                 X0[c] = d2v{0.0, 0.0}, X1[c] = d2v{0.0, 0.0};
             }
@@ -1134,8 +1094,12 @@ __global__ void __launch_bounds__(256, 3) k_transform_pair(const cd *__restrict_
     for (int k = 0; k < NC; k++) {
         const int n = n0 + k;
         if (n < L) {
+            typedef V2 V2u __attribute__((aligned(sizeof(OutT))));
             const V2 w = {(OutT)a0[k], (OutT)a1[k]};
-            __builtin_nontemporal_store(w, reinterpret_cast<V2 *>(out + (long long)n * out_nstride + e));  // written once
+            OutT *o = out + (long long)n * out_nstride + e;  // written once
+            if (ALIGNED) __builtin_nontemporal_store(w, reinterpret_cast<V2 *>(o));
+            else if (e + 1 < E) __builtin_nontemporal_store(w, reinterpret_cast<V2u *>(o));
+            else __builtin_nontemporal_store(w.x, o);
         }
     }
 }
@@ -1536,13 +1500,18 @@ hipError_t launch_colloc_singular(int kind, const Geom &g, const double2 *line, 
 template <class OutT>
 static hipError_t launch_transform_t(const cd *spec, long long E, long long spec_ls, int Lf, const double2 *tab, int L,
                                      OutT *out, long long out_nstride, int num_cus, hipStream_t st) {
-    // two entries per lane when the pairs stay aligned: even sizes and strides, a 2-value-aligned output
-    if (Lf <= kTransformMaxLf && E % 2 == 0 && spec_ls % 2 == 0 && out_nstride % 2 == 0 &&
-        reinterpret_cast<uintptr_t>(out) % (2 * sizeof(OutT)) == 0 && E / 2 <= 256LL * 0x7fffffffLL) {
-        const long long pblocks = (E / 2 + 255) / 256;
+    // two entries per lane.  Where the pairs' stores are not aligned (odd sizes or strides, an output at an odd value) they
+    // are declared so; one entry per lane with stores of one value took 2.0 ms where this takes 1.64 (3291 x 3291, L = 21, G and H)
+    if (Lf <= kTransformMaxLf) {
+        const bool aligned = E % 2 == 0 && out_nstride % 2 == 0 && reinterpret_cast<uintptr_t>(out) % (2 * sizeof(OutT)) == 0;
+        const long long pblocks = ((E + 1) / 2 + 255) / 256;
         for (int n0 = 0; n0 < L; n0 += kTransformNC) {
-            hipLaunchKernelGGL((k_transform_pair<2, OutT>), dim3((unsigned)pblocks), dim3(256), 0, st, spec, E, spec_ls, Lf,
-                               tab, L, n0, out, out_nstride);
+            if (aligned)
+                hipLaunchKernelGGL((k_transform_pair<2, true, OutT>), dim3((unsigned)pblocks), dim3(256), 0, st, spec, E, spec_ls,
+                                   Lf, tab, L, n0, out, out_nstride);
+            else
+                hipLaunchKernelGGL((k_transform_pair<2, false, OutT>), dim3((unsigned)pblocks), dim3(256), 0, st, spec, E, spec_ls,
+                                   Lf, tab, L, n0, out, out_nstride);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
         }
@@ -1553,12 +1522,8 @@ static hipError_t launch_transform_t(const cd *spec, long long E, long long spec
     if (blocks > cap) blocks = cap;
     if (blocks < 1) blocks = 1;
     for (int n0 = 0; n0 < L; n0 += kTransformNC) {
-        if (Lf <= kTransformMaxLf)
-            hipLaunchKernelGGL((k_transform<kTransformNC, kTransformLC, OutT>), dim3((unsigned)blocks), dim3(256), 0, st, spec,
-                               E, spec_ls, Lf, tab, L, n0, out, out_nstride);
-        else
-            hipLaunchKernelGGL((k_transform_wide<kTransformNC, OutT>), dim3((unsigned)blocks), dim3(256), 0, st, spec, E,
-                               spec_ls, Lf, tab, L, n0, out, out_nstride);
+        hipLaunchKernelGGL((k_transform_wide<kTransformNC, OutT>), dim3((unsigned)blocks), dim3(256), 0, st, spec, E, spec_ls, Lf,
+                           tab, L, n0, out, out_nstride);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -134,3 +134,29 @@ def test_tabulated_exponentials_over_arguments(ctx, oracle, galerkin, dt, R, l):
     o = oracle.laplace(V, F, oracle.params(c1, c2, rho, 0.35, dt, R, L, order=2, subdiv=1, galerkin=galerkin, nthreads=8), s)
     for k, tol in (("U", 1e-13), ("P", 1e-10), ("Bt", 1e-13), ("Ba", 1e-13)):
         assert off(g[k], o[k]) <= tol + 4 * z * 1.1e-16, k
+
+
+@pytest.mark.parametrize("nf,L", [(62, 5), (62, 16), (66, 33)])
+def test_transform_of_odd_sizes(ctx, nf, L):
+    """99 or 105 rows: the transform's pairs of entries are unaligned and the last entry has none.  Against the transform of
+    cqbem_laplace's matrices (1e-12 of the terms, as above), and in float storage the same weights rounded once."""
+    import torch
+    V, F = sphere_with(nf)
+    V = M.center(V, F)
+    n3 = 3 * len(V)
+    assert n3 % 2 == 1
+    mesh, p = abi.make_mesh(V, F), params(L, 2, 1, abi.G)
+    print(f"transform of odd sizes n3={n3} L={L}", flush=True)
+    got = ctx.assemble(mesh, p, want=("G",))["G"].reshape(L, -1)
+    S = np.stack([ctx.laplace(mesh, p, l)["U"].reshape(-1) for l in range(L // 2 + 1)])
+    mult = np.array([1.0 if l in (0, L / 2) else 2.0 for l in range(L // 2 + 1)])
+    ang = 2 * np.pi / L * np.outer(np.arange(L), np.arange(L // 2 + 1))
+    scale = p.R ** -np.arange(L, dtype=float)[:, None] / L
+    W = scale * ((mult * np.cos(ang)) @ S.real + (mult * np.sin(ang)) @ S.imag)
+    assert (np.abs(got - W) <= 1e-12 * scale * (mult @ np.abs(S))).all()
+    p.storage = abi.STORE_F32
+    out = torch.full((L * n3 * n3 + 1,), float("nan"), dtype=torch.float32, device="cuda:0")
+    torch.cuda.synchronize()
+    ctx.assemble_device(mesh, p, {"G": out.data_ptr()})
+    assert np.array_equal(out[:-1].cpu().numpy(), got.astype(np.float32).reshape(-1))
+    assert bool(torch.isnan(out[-1]))  # nothing behind the last weight
