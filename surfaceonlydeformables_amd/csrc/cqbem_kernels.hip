@@ -230,7 +230,7 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
     if (tid < 2) turns[tid] = 0;
     __syncthreads();
     // With one or two chunks, 4 or 2 waves share a chunk, each taking every 4th or 2nd point of the rule, as long as 7
-    // points are left to each.
+    // points of the reference rule are left to each (a far row may leave a wave none: part_has_points).
     const_int *pch = (const_int *)(patch_chunk + pc);
     const int c0 = pch[0], nchunk = pch[1] - c0;
     const int split = nchunk == 1 && ref_npts >= 28 ? 4 : nchunk <= 2 && ref_npts >= 14 ? 2 : 1;
@@ -301,7 +301,7 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
         const bool active = (lane < info.y) & !touch;
         const unsigned long long act = __builtin_amdgcn_ballot_w64(active);
         T sg[3][6], sh[3][8];
-        if (act) {  // wave-uniform: no divergent merge of the sums
+        if (act && part_has_points(npts, part)) {  // wave-uniform: no divergent merge of the sums
             {
                 double y[3][3];
 #pragma unroll
@@ -347,9 +347,7 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
                         for (int e = 0; e < 8; e++) add(sh[k][e], H[e], w[k]);
                 }
             };
-            point(part, std::true_type{});
-#pragma unroll 1
-            for (int q = part + split; q < npts; q += split) point(q, std::false_type{});
+            each_part_point(npts, split, part, point);
         } else {
 #pragma unroll
             for (int k = 0; k < 3; k++) {

@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "cqbem_device.hpp"
 
 namespace cqbem {
@@ -37,6 +39,15 @@ __host__ __device__ inline bool beyond_sphere(double x0, double x1, double x2, c
 #pragma clang fp contract(off)
     const double dx = x0 - S.x, dy = x1 - S.y, dz = x2 - S.z;
     return dx * dx + dy * dy + dz * dz >= S.w * S.w;
+}
+// Of the waves that share a chunk of the patch kernel, wave `part` takes the rule's points from `part` on.  A far rule may
+// have fewer points than the waves that the reference rule calls for: the last ones then have none.
+__host__ __device__ inline bool part_has_points(int npts, int part) { return part < npts; }
+// The points that it takes, every split-th one; the first is told apart (it starts the sums).  part_has_points.
+template <class Point> __host__ __device__ __attribute__((always_inline)) inline void each_part_point(int npts, int split, int part, const Point &point) {
+    point(part, std::true_type{});
+#pragma unroll 1
+    for (int q = part + split; q < npts; q += split) point(q, std::false_type{});
 }
 // Distance bands of the B kernels' regular-face rule (CQBEM_QUAD_BANDED).  Face f takes the far rule for row point x
 // at every frequency when |x - centre_f| >= radius_f + kappa h_f (h_f: its longest edge); otherwise the reference
