@@ -178,6 +178,14 @@ template <class T> __device__ inline T *uniform_ptr(T *p) {
 // A pointer read from memory, known to be to global memory.
 template <class T> __device__ inline T *as_global(T *p) { return (T *)(__attribute__((address_space(1))) T *)p; }
 
+// Orders the LDS accesses of the lanes of a wave: what any lane wrote before it, every lane reads after it.  No instruction
+// (a wave's LDS accesses complete in order); it holds the compiler, which otherwise orders one lane's accesses only.
+__device__ inline void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Waits until the LDS counter holds `v`.  Every wave of the block is resident and every wave's waits are for events that
 // earlier program points of the others raise, so each wait ends.
 __device__ inline void wait_for(int *counter, int v) {
@@ -262,7 +270,7 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
         }
 #pragma unroll
         for (int e = DG ? 0 : 6; e < (DH ? kPatchPairs : 6); e++) acc[e * kPatchVerts + tid] = make_double2(0.0, 0.0);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        wave_sync();  // every lane's words are cleared
         if (lane == 0) __hip_atomic_fetch_add(cleared, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
 
@@ -404,8 +412,7 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
             const int slot = (unsigned)corner[k] >> 24;
             const int step = (act >> lane) & 1 ? (ge.w >> (8 * k)) & 0xff : kNoStep;
             const int nsub = (info.z >> (8 * k)) & 0xff;
-            for (int s = 0; s < nsub; ++s) {
-                if (step != s) continue;
+            in_sub_steps(nsub, step, wave_sync, [&]() __attribute__((always_inline)) {
                 // read-modify-write of the slot's words, kRmw reads in flight
 #pragma unroll
                 for (int e0 = DG ? 0 : 6; e0 < (DH ? kPatchPairs : 6); e0 += kRmw) {
@@ -416,8 +423,9 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
                     for (int e = e0; e < e0 + kRmw && e < (DH ? kPatchPairs : 6); e++)
                         acc[e * kPatchVerts + slot] = make_double2(u[e - e0].x + v[k][2 * e], u[e - e0].y + v[k][2 * e + 1]);
                 }
-            }
+            });
         }
+        wave_sync();  // every lane's adds before the turn is given on
         __hip_atomic_store(turns, t + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     while (written < nr) write_row(written++);

@@ -49,6 +49,15 @@ template <class Point> __host__ __device__ __attribute__((always_inline)) inline
 #pragma unroll 1
     for (int q = part + split; q < npts; q += split) point(q, std::false_type{});
 }
+// The update of every lane whose sub-step is `step`, the sub-steps one after another: sync() orders the lanes of the wave,
+// so that an update sees those of the sub-steps before it, whichever lanes made them.
+template <class Sync, class Update>
+__host__ __device__ __attribute__((always_inline)) inline void in_sub_steps(int nsub, int step, const Sync &sync, const Update &update) {
+    for (int s = 0; s < nsub; ++s) {
+        sync();
+        if (step == s) update();
+    }
+}
 // Distance bands of the B kernels' regular-face rule (CQBEM_QUAD_BANDED).  Face f takes the far rule for row point x
 // at every frequency when |x - centre_f| >= radius_f + kappa h_f (h_f: its longest edge); otherwise the reference
 // rule.  sphere == nullptr: the reference rule for every face.
