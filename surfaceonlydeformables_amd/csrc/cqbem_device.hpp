@@ -349,16 +349,9 @@ template <class T> __device__ inline void fill_exp_table(const PointFreq<T> &f, 
     const T e1 = node_exp(f.sc1 * down, r), e2 = node_exp(f.sc2 * down, r);
     tab[2 * k] = make_double2(e1.x, e1.y), tab[2 * k + 1] = make_double2(e2.x, e2.y);
 }
-// d q[0] + .. + d^5 q[4], one component.  Written out with the coefficient as the FMA's scalar addend: the compiler's choice
-// was the two-address form, with two moves per coefficient.
+// d q[0] + .. + d^5 q[4], one component.
 __device__ inline double exp_poly(double d, double q1, double q2, double q3, double q4, double q5) {
-    double p;
-    asm("v_mul_f64 %0, %1, %2" : "=v"(p) : "v"(d), "s"(q5));
-    asm("v_add_f64 %0, %1, %2" : "=v"(p) : "v"(p), "s"(q4));
-    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(p) : "v"(p), "v"(d), "s"(q3));
-    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(p) : "v"(p), "v"(d), "s"(q2));
-    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(p) : "v"(p), "v"(d), "s"(q1));
-    return p * d;
+    return fma(fma(fma(fma(d, q5, q4), d, q3), d, q2), d, q1) * d;
 }
 template <class T> __device__ inline T exp_poly(double d, const T (&q)[kExpDeg]) {
     return T{exp_poly(d, q[0].x, q[1].x, q[2].x, q[3].x, q[4].x), exp_poly(d, q[0].y, q[1].y, q[2].y, q[3].y, q[4].y)};
