@@ -14,6 +14,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "cqbem_math_tables.hpp"
 
 namespace cqbem {
@@ -89,8 +92,9 @@ constexpr double kTrigArgMax = 1.0e6;
 // e^{-a}, a >= -700.  k = rint(-a / ln 2); f + c = -a - k ln 2 with |f| <= ln2/2 (the k kLn2Hi part
 // is exact by Sterbenz); e^(f+c) = (1 + f) + (f^2 p(f) + c (1 + f)) with p the Taylor series of
 // (e^f - 1 - f) / f^2 through f^11 (next term < 5e-18); 1 + f is split exactly.  Scaled by 2^k;
-// -a is clamped at -740, where the result has underflowed to 0.
-__device__ inline double exp_neg(double a) {
+// -a is clamped at -740, where the result has underflowed to 0.  With `lo`, what the rounding of the result left out goes
+// there (good to 2^-57 of the result).
+__host__ __device__ inline double exp_neg(double a, double *lo = nullptr) {
 #pragma clang fp contract(off)
     const double t = fmin(fmax(-a, -740.0), 700.0);
     const double k = rint(t * kLog2e);
@@ -111,15 +115,17 @@ __device__ inline double exp_neg(double a) {
     p = fma(p, f, 1.0 / 6.0);
     p = fma(p, f, 0.5);
     const double tail = fma(f * f, p, fma(c, f, c));
-    const double s1 = 1.0 + f, e1 = (1.0 - s1) + f;
-    return ldexp(s1 + (e1 + tail), (int)k);
+    const double s1 = 1.0 + f, e1 = ((1.0 - s1) + f) + tail, m = s1 + e1;
+    if (lo) *lo = ldexp((s1 - m) + e1, (int)k);
+    return ldexp(m, (int)k);
 }
 
 // sin y, cos y for |y| < kTrigArgMax.  k = rint(2y/pi); r + rr = y - k pi/2 to ~1e-30 (three-part
 // pi/2, the first two products exact, the subtraction split by TwoSum); sin r through r^17 and
 // cos r through r^18 (next terms < 1e-19), first-order in rr; 1 - r^2/2 split exactly.  The
-// quadrant k mod 4 then selects and signs them.
-__device__ inline void cq_sincos(double y, double *s, double *c) {
+// quadrant k mod 4 then selects and signs them.  With `lo`, lo[0] and lo[1] are what the roundings of s and c left out
+// (good to 2^-57).
+__host__ __device__ inline void cq_sincos(double y, double *s, double *c, double *lo = nullptr) {
 #pragma clang fp contract(off)
     const double k = rint(y * kTwoOverPi);
     const double r1 = fma(-k, kPio2A, y);
@@ -145,15 +151,19 @@ __device__ inline void cq_sincos(double y, double *s, double *c) {
     pc = fma(pc, x, 1.0 / 40320.0);
     pc = fma(pc, x, -1.0 / 720.0);
     pc = fma(pc, x, 1.0 / 24.0);
-    const double sr = r + fma(r * x, ps, rr * fma(-0.5, x, 1.0));
+    const double st = fma(r * x, ps, rr * fma(-0.5, x, 1.0)), sr = r + st;
     const double xl = fma(r, r, -x);
     const double hz = 0.5 * x;
-    const double w = 1.0 - hz, ew = (1.0 - w) - hz;
-    const double cr = w + (ew + fma(x * x, pc, -fma(0.5, xl, rr * r)));
+    const double w = 1.0 - hz, ct = ((1.0 - w) - hz) + fma(x * x, pc, -fma(0.5, xl, rr * r)), cr = w + ct;
     const int q = (int)k;
     const double so = (q & 1) ? cr : sr, co = (q & 1) ? sr : cr;
     *s = (q & 2) ? -so : so;
     *c = ((q + 1) & 2) ? -co : co;
+    if (lo) {
+        const double sl = (r - sr) + st, cl = (w - cr) + ct, sv = (q & 1) ? cl : sl, cv = (q & 1) ? sl : cl;
+        lo[0] = (q & 2) ? -sv : sv;
+        lo[1] = ((q + 1) & 2) ? -cv : cv;
+    }
 }
 
 // 1/sqrt(d), d > 0: hardware estimate refined by two Newton steps y += y (1 - d y^2) / 2.
@@ -278,9 +288,13 @@ __device__ inline const_double *as_const(const double4 *p) { return (const_doubl
 __device__ inline const_int *as_const(const int4 *p) { return (const_int *)p; }
 
 // Per-frequency constants, uniform across a wavefront (loaded with scalar loads).
-constexpr int kExpNodes = 256;  // entries of the exponentials' table: 127 coarse nodes, one place not used, 128 fine ones
-constexpr int kExpFine = 128;
-constexpr int kExpCells = (kExpNodes - kExpFine - 1) * kExpFine;
+// The table of the regular kernels' exponentials (exp_pair): four arrays of coarse nodes (a pair's values, then what their
+// rounding left out, relative to them), whose last place is left to the block's counters, and two of fine nodes.  Arrays, not
+// records: lanes at different nodes meet in an LDS bank only where the nodes are 16 apart.
+constexpr int kExpCoarse = 64, kExpFine = 128;
+constexpr int kExpWords = 4 * kExpCoarse + 2 * kExpFine;
+constexpr int kExpCells = (kExpCoarse - 1) * kExpFine - kExpFine / 2;
+constexpr int kExpCounters = 4 * kExpCoarse - 1;  // the word of the block's counters
 constexpr int kExpDeg = 5;  // of the polynomial in the rest
 struct Freq {
     cd s;    // s_l
@@ -288,92 +302,171 @@ struct Freq {
     cd sc2;  // s / c2
     cd is;   // 1 / s
     cd is2;  // 1 / s^2
-    // The regular kernels' exponentials (exp_pair): the cell h and 1 / h, the coefficients of d, .., d^5 in
-    // e^{-s d / (2^sq c)} for c1 and c2, |d| <= h / 2.
+    // The regular kernels' exponentials (exp_pair): the cell h and 1 / h, the coefficients of d, .., d^5 in e^{-s d / c} for
+    // c1 and c2, |d| <= h / 2; direct: s is beyond the table's reach.
     double h, ih;
     cd q[2][kExpDeg];
-    int sq, pad;
+    int direct, pad;
 };
+
+// The cell over distances up to `reach` (n h is exact for every n + 1/2 up to kExpCells), and the largest |s / c| H that the
+// table is used for, with H = h / 2 (+ 1/16: the cell index is rounded).  The polynomial of e^{-x d}, |d| <= H, is the
+// Taylor series through d^6 with the last term economized (d^6 -> (48 H^2 d^4 - 18 H^4 d^2 + H^6) / 32, T. J. Rivlin,
+// "Chebyshev Polynomials", 1990): its error 2 |x H|^6 / (32 6!), constant term left out included, is below 1e-17.  The line is
+// at |s| reach / c = 99, where a fine node's value is e^{+-0.8} at most: up to there the table's values are no less exact than
+// the direct functions' in any range of arguments (at 124 they have 1.1 times their error for |s r / c| in 0.3 .. 1).
+inline double exp_table_cell(double reach) {
+    if (!(reach > 0.0)) return 1.0;
+    const double h = reach / (kExpCells - 1.5);
+    const float f = (float)h;
+    return f > 0.0f && f < INFINITY ? (double)__builtin_nextafterf(f, INFINITY) : h;
+}
+constexpr double kExpTableReach = 0.0066;
+inline double exp_table_width(double h) { return 0.5 * h * (1.0 + 1.0 / 16); }
+// Fills the fields of exp_pair from s / c1 and s / c2 and the cell.
+inline void exp_table_plan(Freq &f, double h) {
+    const double H = exp_table_width(h);
+    f.h = h, f.ih = 1.0 / h, f.pad = 0;
+    f.direct = !(H * std::max(std::hypot(f.sc1.x, f.sc1.y), std::hypot(f.sc2.x, f.sc2.y)) <= kExpTableReach);
+    for (int c = 0; c < 2; c++) {
+        const cd x = c ? f.sc2 : f.sc1, x2 = x * x, x4 = x2 * x2, x6 = x4 * x2;
+        f.q[c][0] = x * -1.0;
+        f.q[c][1] = x2 * 0.5 + x6 * (H * H * H * H / -1280.0);
+        f.q[c][2] = x * x2 * (-1.0 / 6.0);
+        f.q[c][3] = x4 * (1.0 / 24.0) + x6 * (H * H / 480.0);
+        f.q[c][4] = x * x4 * (-1.0 / 120.0);
+    }
+}
 
 // The constants that the regular-face kernels read, at one frequency (cd) or at the two real ones (rp), from the table
 // through the constant address space.
 template <class T> struct PointFreq {
+    typedef T value;
     T s, sc1, sc2, is2;
+};
+// A frequency within the reach of the exponentials' table.
+struct TableFreq : PointFreq<cd> {
     double h, ih;
-    T q[2][kExpDeg];
-    int sq;
+    cd q[2][kExpDeg];
 };
 __device__ inline PointFreq<cd> point_freq(const Freq *f, int l, cd) {
     const_double *p = (const_double *)(f + l);
-    PointFreq<cd> r{cd{p[0], p[1]}, cd{p[2], p[3]}, cd{p[4], p[5]}, cd{p[8], p[9]}, p[10], p[11]};
-#pragma unroll
-    for (int k = 0; k < 2 * kExpDeg; k++) r.q[k / kExpDeg][k % kExpDeg] = cd{p[12 + 2 * k], p[13 + 2 * k]};
-    r.sq = *(const_int *)&f[l].sq;
-    return r;
+    return PointFreq<cd>{cd{p[0], p[1]}, cd{p[2], p[3]}, cd{p[4], p[5]}, cd{p[8], p[9]}};
 }
 __device__ inline PointFreq<rp> point_freq(const Freq *f, int hi, rp) {
     const_double *p = (const_double *)f, *q = (const_double *)(f + hi);
-    PointFreq<rp> r{rp{p[0], q[0]}, rp{p[2], q[2]}, rp{p[4], q[4]}, rp{p[8], q[8]}, p[10], p[11]};
+    return PointFreq<rp>{rp{p[0], q[0]}, rp{p[2], q[2]}, rp{p[4], q[4]}, rp{p[8], q[8]}};
+}
+__device__ inline TableFreq table_freq(const Freq *f, int l) {
+    const_double *p = (const_double *)(f + l);
+    TableFreq r{point_freq(f, l, cd{}), p[10], p[11]};
 #pragma unroll
-    for (int k = 0; k < 2 * kExpDeg; k++) r.q[k / kExpDeg][k % kExpDeg] = rp{p[12 + 2 * k], q[12 + 2 * k]};
-    r.sq = *(const_int *)&f->sq;
+    for (int k = 0; k < 2 * kExpDeg; k++) r.q[k / kExpDeg][k % kExpDeg] = cd{p[12 + 2 * k], p[13 + 2 * k]};
     return r;
 }
+__device__ inline bool beyond_table(const Freq *f, int l) { return *(const_int *)&f[l].direct; }
 
 // ---------------------------------------------------------------------------
 // The regular kernels' exponentials e^{-s r / c1} and e^{-s r / c2}.  Both depend on the distance r alone once the
-// frequency is fixed, so a block tabulates them: r = (128 k + j + 1/2) h + d with |d| <= h / 2 over the mesh's extent,
-// e^{-s r / c} = coarse_k fine_j (1 + u(d)), u a polynomial of degree 5 in the real d with uniform coefficients.  47
-// instructions per point and pair, against 78 for two reductions with e^x, sin and cos.  The nodes' arguments carry their
-// rounding errors, so the pair is good to 2 ulp of the result also where s r / c is large (a rounded argument alone costs
-// |s r / c| / 2 ulp).  Where s h is beyond the polynomial's reach everything is at s / 2^sq and squared back.
+// frequency is fixed, so a block tabulates them: r = 128 k h + (j - 63.5) h + d with |d| <= h / 2 over the mesh's
+// extent, e^{-s r / c} = C_k (1 + g_j) (1 + u(d)), g_j = e^{..} - 1 and u a polynomial of degree 5 in the real d with uniform
+// coefficients, whose constant term is the relative rounding error of C_k, the lane's own.  It is summed as C + C v,
+// v = g + (1 + g) u, so that a value carries the last sum's roundings and |v| (at most about 1, and small near r = 0, where C
+// is 1) times the ones before: 0.3 to 0.7 units of 2^-53 rms over all arguments up to the table's reach (kExpTableReach), where
+// the direct functions, whose argument s r / c is rounded, have 0.5 to 0.95 below |s r / c| = 3 and 22 at 100.  49
+// instructions per point and pair, against 78 for two reductions with e^x, sin and cos, which remain beyond the reach.
 // ---------------------------------------------------------------------------
-constexpr double kNodeMagic = 211106232532992.0;  // 1.5 2^47: the low word of r / h + this holds 32 floor(r / h) + 5 bits
-__device__ inline cd node_exp(cd sc, double r) {
-    const cd z = sc * r;
-    const cd e = cexp_neg(cd{fmin(z.x, 740.0), z.y});
-    return e - e * cd{fma(sc.x, r, -z.x), fma(sc.y, r, -z.y)};
+constexpr double kNodeMagic = 422212465065984.0 + kExpFine / 2;  // 1.5 2^48 + 64: the low word of r / h + this holds 16 cell + 4 bits
+// e^{-sc r} as the sum of two doubles, r exact.
+__host__ __device__ inline cd node_exp(cd sc, double r, cd &lo) {
+#pragma clang fp contract(off)
+    const cd z{sc.x * r, sc.y * r};
+    double m, ml, s, c, sl[2];
+    m = exp_neg(z.x, &ml), cq_sincos(z.y, &s, &c, sl);
+    const cd e{m * c, -m * s};
+    // what the products, their factors' low parts and the argument's roundings add
+    const cd t{fma(sc.x, r, -z.x), fma(sc.y, r, -z.y)};
+    const cd l{fma(m, c, -e.x) + (m * sl[1] + ml * c) - (e.x * t.x - e.y * t.y),
+               fma(-m, s, -e.y) - (m * sl[0] + ml * s) - (e.x * t.y + e.y * t.x)};
+    const cd v{e.x + l.x, e.y + l.y};
+    lo = cd{(e.x - v.x) + l.x, (e.y - v.y) + l.y};
+    return v;
 }
-__device__ inline rp node_exp(rp sc, double r) {
-    const rp z = sc * r;
-    const rp e{exp_neg(fmin(z.x, 740.0)), exp_neg(fmin(z.y, 740.0))};
-    return e - e * rp{fma(sc.x, r, -z.x), fma(sc.y, r, -z.y)};
+// a / b, to a few units of the last place
+__host__ __device__ inline cd over(cd a, cd b) {
+    const double i = 1.0 / (b.x * b.x + b.y * b.y);
+    return cd{(a.x * b.x + a.y * b.y) * i, (a.y * b.x - a.x * b.y) * i};
 }
-// Fills entry threadIdx.x of `tab` (2 words per entry), blockDim.x == kExpNodes: coarse nodes, then fine ones; the last
-// coarse entry's place is left alone.
-template <class T> __device__ inline void fill_exp_table(const PointFreq<T> &f, double2 *tab) {
-    const int k = threadIdx.x;
-    if (k == kExpNodes - kExpFine - 1) return;
-    const double r = (k < kExpNodes - kExpFine ? (double)(k * kExpFine) : k - (kExpNodes - kExpFine) + 0.5) * f.h;
-    const double down = ldexp(1.0, -f.sq);
-    const T e1 = node_exp(f.sc1 * down, r), e2 = node_exp(f.sc2 * down, r);
-    tab[2 * k] = make_double2(e1.x, e1.y), tab[2 * k + 1] = make_double2(e2.x, e2.y);
+// v - 1 from v's two parts
+__host__ __device__ inline cd minus_one(cd v, cd lo) { return cd{(v.x - 1.0) + lo.x, v.y + lo.y}; }
+// Node n of the table: coarse nodes, then fine ones, kExpCoarse - 1 + kExpFine in all.
+__host__ __device__ inline void fill_exp_node(const TableFreq &f, int n, double2 *tab) {
+    const bool fine = n >= kExpCoarse - 1;
+    const int j = n - (kExpCoarse - 1);
+    const double r = (fine ? j + (0.5 - kExpFine / 2) : (double)(n * kExpFine)) * f.h;
+    cd l1, l2;
+    const cd e1 = node_exp(f.sc1, r, l1), e2 = node_exp(f.sc2, r, l2);
+    if (fine) {
+        const cd g1 = minus_one(e1, l1), g2 = minus_one(e2, l2);
+        double2 *p = tab + 4 * kExpCoarse + j;
+        p[0] = make_double2(g1.x, g1.y), p[kExpFine] = make_double2(g2.x, g2.y);
+    } else {
+        const cd q1 = over(l1, e1), q2 = over(l2, e2);
+        double2 *p = tab + n;
+        p[0] = make_double2(e1.x, e1.y), p[kExpCoarse] = make_double2(e2.x, e2.y);
+        p[2 * kExpCoarse] = make_double2(q1.x, q1.y), p[3 * kExpCoarse] = make_double2(q2.x, q2.y);
+    }
 }
-// d q[0] + .. + d^5 q[4], one component.
-__device__ inline double exp_poly(double d, double q1, double q2, double q3, double q4, double q5) {
-    return fma(fma(fma(fma(d, q5, q4), d, q3), d, q2), d, q1) * d;
+static_assert(sizeof(MathTables) <= sizeof(double2) * kExpCounters, "the direct functions' tables fit in the same place");
+// Fills `tab` (kExpWords words but the last coarse entry's, which are left alone): with the nodes, or with the direct
+// functions' tables.
+__device__ inline void fill_exp_table(const TableFreq &f, double2 *tab) {
+    for (int n = threadIdx.x; n < kExpCoarse - 1 + kExpFine; n += blockDim.x) fill_exp_node(f, n, tab);
 }
-template <class T> __device__ inline T exp_poly(double d, const T (&q)[kExpDeg]) {
-    return T{exp_poly(d, q[0].x, q[1].x, q[2].x, q[3].x, q[4].x), exp_poly(d, q[0].y, q[1].y, q[2].y, q[3].y, q[4].y)};
+template <class T> __device__ inline void fill_exp_table(const PointFreq<T> &, double2 *tab) {
+    load_math_tables(reinterpret_cast<MathTables *>(tab));
 }
-__device__ inline cd times_one_plus(cd n, cd u) {
-    return cd{fma(n.x, u.x, fma(-n.y, u.y, n.x)), fma(n.x, u.y, fma(n.y, u.x, n.y))};
+// q0 + d q[0] + .. + d^5 q[4], one component.
+__host__ __device__ inline double exp_poly(double d, double q0, double q1, double q2, double q3, double q4, double q5) {
+    return fma(fma(fma(fma(fma(d, q5, q4), d, q3), d, q2), d, q1), d, q0);
 }
-__device__ inline rp times_one_plus(rp n, rp u) { return rp{fma(n.x, u.x, n.x), fma(n.y, u.y, n.y)}; }
-template <class T>
-__device__ __attribute__((always_inline)) inline void exp_pair(double r, const PointFreq<T> &f, const double2 *tab, T &e1, T &e2) {
+__host__ __device__ inline cd exp_poly(double d, double2 q0, const cd (&q)[kExpDeg]) {
+    return cd{exp_poly(d, q0.x, q[0].x, q[1].x, q[2].x, q[3].x, q[4].x), exp_poly(d, q0.y, q[0].y, q[1].y, q[2].y, q[3].y, q[4].y)};
+}
+// C (1 + g) (1 + u)
+__host__ __device__ inline cd node_value(cd C, cd g, cd u) {
+    const double fx = g.x + 1.0;
+    const cd v{fma(fx, u.x, fma(-g.y, u.y, g.x)), fma(fx, u.y, fma(g.y, u.x, g.y))};
+    return cd{fma(C.x, v.x, fma(-C.y, v.y, C.x)), fma(C.x, v.y, fma(C.y, v.x, C.y))};
+}
+// The pair at distance r; z1 = s r / c1 and z2 = s r / c2, rounded.
+__host__ __device__ __attribute__((always_inline)) inline void exp_pair(double r, const cd &, const cd &, const TableFreq &f,
+                                                                        const double2 *tab, cd &e1, cd &e2) {
     const unsigned long long t = __builtin_bit_cast(unsigned long long, fma(r, f.ih, kNodeMagic));
-    const unsigned lo = (unsigned)t & ~31u;
+    const unsigned lo = (unsigned)t & ~15u;
     const double n = __builtin_bit_cast(double, (t & 0xffffffff00000000ull) | lo) - (kNodeMagic - 0.5);
     const double d = fma(-f.h, n, r);
-    // byte offsets of the two entries, in bounds whatever r
-    const unsigned j = lo & (32u * (kExpFine - 1)), k = (lo / kExpFine) & (32u * (kExpNodes - kExpFine - 1));
-    const double2 *fine = reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(tab + 2 * (kExpNodes - kExpFine)) + j);
+    // byte offsets of the two nodes, in bounds whatever r
+    const unsigned j = lo & (16u * (kExpFine - 1)), k = (lo / kExpFine) & (16u * (kExpCoarse - 1));
+    const double2 *fine = reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(tab + 4 * kExpCoarse) + j);
     const double2 *coarse = reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(tab) + k);
-    const double2 a1 = coarse[0], a2 = coarse[1], b1 = fine[0], b2 = fine[1];
-    e1 = times_one_plus(T{a1.x, a1.y} * T{b1.x, b1.y}, exp_poly(d, f.q[0]));
-    e2 = times_one_plus(T{a2.x, a2.y} * T{b2.x, b2.y}, exp_poly(d, f.q[1]));
-    for (int k = 0; k < f.sq; k++) e1 = e1 * e1, e2 = e2 * e2;
+    const double2 a1 = coarse[0], a2 = coarse[kExpCoarse], l1 = coarse[2 * kExpCoarse], l2 = coarse[3 * kExpCoarse];
+    const double2 b1 = fine[0], b2 = fine[kExpFine];
+    e1 = node_value(cd{a1.x, a1.y}, cd{b1.x, b1.y}, exp_poly(d, l1, f.q[0]));
+    e2 = node_value(cd{a2.x, a2.y}, cd{b2.x, b2.y}, exp_poly(d, l2, f.q[1]));
+}
+// The same directly, for a frequency beyond the table's reach, and for the two real ones, where there are no trigonometric
+// functions to save and e^x is exact to half an ulp of the rounded argument's.
+__host__ __device__ __attribute__((always_inline)) inline void exp_pair(double, const cd &z1, const cd &z2, const PointFreq<cd> &,
+                                                                        const double2 *tab, cd &e1, cd &e2) {
+    const MathTables *M = reinterpret_cast<const MathTables *>(tab);
+    e1 = cexp_neg_tab(z1, M), e2 = cexp_neg_tab(z2, M);
+}
+__host__ __device__ __attribute__((always_inline)) inline void exp_pair(double, const rp &z1, const rp &z2, const PointFreq<rp> &,
+                                                                        const double2 *tab, rp &e1, rp &e2) {
+    const double2 *T = reinterpret_cast<const MathTables *>(tab)->e;
+    auto e = [T](double z) { return exp_tab_core(fmax(-z, -740.0), T); };
+    e1 = rp{e(z1.x), e(z1.y)}, e2 = rp{e(z2.x), e(z2.y)};
 }
 
 // Material constants.
@@ -490,11 +583,12 @@ template <class T> struct PointExpo {
     T e1, e2, w1, w2, s2, q2;  // s2 = (z2 + 1) e2, q2 = 1 / (s r)^2
     T dd;
 };
-template <class T> __device__ inline PointExpo<T> point_expo(double d2, const PointFreq<T> &f, const double2 *tab) {
+template <class F> __device__ inline PointExpo<typename F::value> point_expo(double d2, const F &f, const double2 *tab) {
+    typedef typename F::value T;
     PointExpo<T> E;
     E.ir = rsqrt_h3(d2), E.r = d2 * E.ir, E.ir2 = E.ir * E.ir;
     const T z1 = f.sc1 * E.r, z2 = f.sc2 * E.r;
-    exp_pair(E.r, f, tab, E.e1, E.e2);
+    exp_pair(E.r, z1, z2, f, tab, E.e1, E.e2);
     E.w1 = z1 * E.e1, E.w2 = z2 * E.e2;
     E.s2 = E.w2 + E.e2, E.q2 = f.is2 * E.ir2;
     E.dd = ((E.w1 + E.e1) - E.s2) * E.q2;

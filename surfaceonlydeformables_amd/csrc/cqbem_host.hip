@@ -268,32 +268,6 @@ double mesh_reach(const cqbem_mesh *mesh) {
     return 2.0 * std::sqrt(d2) * (1.0 + 1e-9);
 }
 
-// The tables of the regular kernels' exponentials over distances up to `reach`: the cell, and per frequency the polynomial
-// of e^{-x d}, x = s / (2^sq c), for |d| <= H = h / 2 (+ 1/32: the cell index is rounded): the Taylor series through d^6,
-// the last term economized (d^6 -> (48 H^2 d^4 - 18 H^4 d^2 + H^6) / 32, T. J. Rivlin, "Chebyshev Polynomials", 1990).
-// With |x H| <= 0.0085 the error 2 |x H|^6 / (32 6!), constant term left out included, is below 4e-17.  The
-// frequencies of a pair (real_pair: the first and the last) take the same scale.
-void exp_table_plan(std::vector<Freq> &freqs, bool real_pair, double reach) {
-    const double h = reach > 0.0 ? (double)std::nextafter((float)(reach / (kExpCells - 1.5)), INFINITY) : 1.0;  // n h is exact
-    const double H = 0.5 * h * (1.0 + 1.0 / 32);
-    auto largest = [&](const Freq &f) { return H * std::max(std::hypot(f.sc1.x, f.sc1.y), std::hypot(f.sc2.x, f.sc2.y)); };
-    for (size_t l = 0; l < freqs.size(); l++) {
-        Freq &f = freqs[l];
-        double w = largest(f);
-        if (real_pair && (l == 0 || l + 1 == freqs.size())) w = std::max(largest(freqs.front()), largest(freqs.back()));
-        f.h = h, f.ih = 1.0 / h, f.sq = f.pad = 0;
-        for (; w > 0.0085; w *= 0.5) f.sq++;
-        for (int c = 0; c < 2; c++) {
-            const cd x = (c ? f.sc2 : f.sc1) * std::ldexp(1.0, -f.sq), x2 = x * x, x4 = x2 * x2, x6 = x4 * x2;
-            f.q[c][0] = x * -1.0;
-            f.q[c][1] = x2 * 0.5 + x6 * (H * H * H * H / -1280.0);
-            f.q[c][2] = x * x2 * (-1.0 / 6.0);
-            f.q[c][3] = x4 * (1.0 / 24.0) + x6 * (H * H / 480.0);
-            f.q[c][4] = x * x4 * (-1.0 / 120.0);
-        }
-    }
-}
-
 Prepared prepare(const cqbem_mesh *mesh, const cqbem_params *p) {
     Prepared P;
     P.nv = (int)mesh->nv, P.nf = (int)mesh->nf, P.L = p->L, P.Lf = p->L / 2 + 1;
@@ -580,16 +554,16 @@ Prepared prepare(const cqbem_mesh *mesh, const cqbem_params *p) {
     }
     for (auto &xw : composite_line01(p->order, p->subdivision)) P.line.push_back(make_double2(xw.first, xw.second));
     const auto s = cq_frequencies(p->L, p->R, p->dt, p->bdf);
-    const double reach = mesh_reach(mesh);
+    const double cell = exp_table_cell(mesh_reach(mesh));
     for (auto sl : s) {
         Freq f;
         f.s = mkc(sl.real(), sl.imag());
         const std::complex<double> a = sl / p->c1, b = sl / p->c2, is = 1.0 / sl, is2 = is * is;
         f.sc1 = mkc(a.real(), a.imag()), f.sc2 = mkc(b.real(), b.imag());
         f.is = mkc(is.real(), is.imag()), f.is2 = mkc(is2.real(), is2.imag());
+        exp_table_plan(f, cell);
         P.freqs.push_back(f);
     }
-    exp_table_plan(P.freqs, P.L % 2 == 0, reach);
     for (auto t : transform_table(p->L, p->R)) P.tab.push_back(make_double2(t.real(), t.imag()));
     Mat &m = P.mat;
     m.c1 = p->c1, m.c2 = p->c2, m.rho = p->rho;

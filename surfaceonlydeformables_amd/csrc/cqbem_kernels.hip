@@ -149,11 +149,12 @@ __global__ void __launch_bounds__(64) k_colloc_gh(Geom g, const double4 *__restr
 // real, are one slot (T = rp: two real numbers in the place of a complex one).
 //
 // Bound by FP64 VALU issue (and, near full issue, by the clock that the power
-// limit leaves): 260 VALU instructions per point, of which 84 are the corner
-// sums and 47 the two complex exponentials (exp_pair), and 1100 per face and row
+// limit leaves): 268 VALU instructions per point, of which 84 are the corner
+// sums and 49 the two complex exponentials (exp_pair), and 1100 per face and row
 // outside the rule.  Icosphere level 4, L = 32, 28 points (6.2e9 unique
-// evaluations): 70.8 ms; 76.8 at 292 instructions, with the exponentials through
-// reductions and e^x, sin, cos; 80.8 with a slot for each real frequency.  The form it replaces, two
+// evaluations): 72 ms; 77 at 296 instructions, with the exponentials through
+// reductions and e^x, sin, cos, as frequencies beyond the table's reach still
+// have them; 81 with a slot for each real frequency.  The form it replaces, two
 // lanes per face that swapped every point's 16 global entries through DPP, took
 // 128 ms at 516 instructions per point.  Tried and slower: the same with a
 // block barrier per sub-step (86.5 ms), the rotation inside the wave's turn
@@ -221,20 +222,20 @@ struct PatchDest {
     cd *UG, *UH;
     long long ld, lstride;
 };
-template <class T, bool DG, bool DH, bool GAL, class Dest>
+template <bool DG, bool DH, bool GAL, class F, class Dest>
 __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, const double4 *__restrict__ ref_pts, int ref_npts,
-                                 const Bands &bands, const PointFreq<T> &f, const Mat &m, int row0, const double4 *__restrict__ tpts,
+                                 const Bands &bands, const F &f, const Mat &m, int row0, const double4 *__restrict__ tpts,
                                  const int *__restrict__ patch_chunk, const int4 *__restrict__ chunk_info,
                                  const int4 *__restrict__ chunk_faces, const Dest &dest, int pc, int l,
                                  int il0, int nr, double2 *acc, double2 *frame, double2 *exps) {
+    typedef typename F::value T;
     constexpr int kWaves = kPatchThreads / 64;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     for (int k = tid; k < kPatchPairs * kPatchVerts; k += kPatchThreads) acc[k] = make_double2(0.0, 0.0);
-    static_assert(kPatchThreads == kExpNodes, "one node per thread");
     fill_exp_table(f, exps);
     // chunks added so far; waves that cleared their slots, over all rows: in the table's unused place, so that
     // two blocks fill a CU's LDS exactly
-    int *turns = reinterpret_cast<int *>(exps + 2 * (kExpNodes - kExpFine - 1)), *cleared = turns + 1;
+    int *turns = reinterpret_cast<int *>(exps + kExpCounters), *cleared = turns + 1;
     if (tid < 2) turns[tid] = 0;
     __syncthreads();
     // With one or two chunks, 4 or 2 waves share a chunk, each taking every 4th or 2nd point of the rule, as long as 7
@@ -316,16 +317,18 @@ __device__ __attribute__((always_inline)) inline void patch_tile(const Geom &g, 
                 for (int k = 0; k < 3; k++)
 #pragma unroll
                     for (int d = 0; d < 3; d++) y[k][d] = g.V[3 * va[k] + d];
-                const FaceFrame F = face_frame(y, x0, x1, x2);
-                frame[tid] = make_double2(F.L1, F.u), frame[kPatchThreads + tid] = make_double2(F.v, F.xa);
-                frame[2 * kPatchThreads + tid] = make_double2(F.xb, F.cr);
+                const FaceFrame ff = face_frame(y, x0, x1, x2);
+                frame[tid] = make_double2(ff.L1, ff.u), frame[kPatchThreads + tid] = make_double2(ff.v, ff.xa);
+                frame[2 * kPatchThreads + tid] = make_double2(ff.xb, ff.cr);
             }
             // one point's entries into the sums; the first point starts them
             auto point = [&](int q, auto first) __attribute__((always_inline)) {
-                // the lane is made opaque per point so that the frame stays in LDS (14 VGPRs otherwise)
-                int ln = tid;
-                asm volatile("" : "+v"(ln));
-                const double2 F0 = frame[ln], F1 = frame[kPatchThreads + ln], F2 = frame[2 * kPatchThreads + ln];
+                // the lane is found anew at each point, so that neither the frame (12 VGPRs) nor the lane's number is held
+                // through the loop
+                unsigned all = ~0u;
+                asm volatile("" : "+s"(all));
+                const double2 *fr = frame + 64 * wave + __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
+                const double2 F0 = fr[0], F1 = fr[kPatchThreads], F2 = fr[2 * kPatchThreads];
                 const_double *B = as_const(pts + 2 * q);  // b1, b2, -, -, w (phi_0, phi_1, phi_2, 1)
                 const double ar = fma(B[0], F0.x, fma(B[1], F0.y, F1.y)), br = fma(B[1], F1.x, F2.x), cr = F2.y;
                 const PointExpo<T> E = point_expo(fma(ar, ar, fma(br, br, cr * cr)), f, exps);
@@ -444,17 +447,16 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_colloc_gh_patch(Geom g, co
                                                                   int nrows, int rpt, int real_hi, Bands bands) {
     __shared__ double2 acc[kPatchPairs * kPatchVerts];      // [word][slot]
     __shared__ double2 frame[kFramePairs * kPatchThreads];
-    __shared__ double2 exps[2 * kExpNodes];
+    __shared__ double2 exps[kExpWords];
     auto dest = [=] { return PatchDest{patch_verts, UG, UH, ld, lstride}; };
     const int r0 = blockIdx.z * rpt, nr = min(rpt, nrows - r0);
-    if (real_hi >= 0 && blockIdx.y == 0)
-        patch_tile<rp, DG, DH, GAL>(g, pts, npts, BANDED ? bands : Bands{}, point_freq(freqs + l0, real_hi, rp{}), m, row0, tpts,
-                                    patch_chunk, chunk_info, chunk_faces, dest, blockIdx.x, real_hi, r0, nr, acc, frame,
-                                    exps);
-    else
-        patch_tile<cd, DG, DH, GAL>(g, pts, npts, BANDED ? bands : Bands{}, point_freq(freqs, l0 + blockIdx.y, cd{}), m, row0, tpts,
-                                    patch_chunk, chunk_info, chunk_faces, dest, blockIdx.x, blockIdx.y, r0, nr, acc, frame,
-                                    exps);
+    auto tile = [&](const auto &f, int l) {
+        patch_tile<DG, DH, GAL>(g, pts, npts, BANDED ? bands : Bands{}, f, m, row0, tpts, patch_chunk, chunk_info, chunk_faces, dest,
+                                blockIdx.x, l, r0, nr, acc, frame, exps);
+    };
+    if (real_hi >= 0 && blockIdx.y == 0) tile(point_freq(freqs + l0, real_hi, rp{}), real_hi);
+    else if (beyond_table(freqs, l0 + blockIdx.y)) tile(point_freq(freqs, l0 + blockIdx.y, cd{}), blockIdx.y);
+    else tile(table_freq(freqs, l0 + blockIdx.y), blockIdx.y);
 }
 
 // ------------------------------------------------------------------------
@@ -495,14 +497,13 @@ __device__ __attribute__((always_inline)) inline void scene_tile(const ScenePiec
     const unsigned rest = local / np;
     const int pc = __builtin_amdgcn_readfirstlane(local - rest * np), l = __builtin_amdgcn_readfirstlane(rest % nl),
               r0 = __builtin_amdgcn_readfirstlane(rest / nl) * P.rpt;
-    if (P.real_hi >= 0 && l == 0)
-        patch_tile<rp, DG, DH, false>(P.g, P.pts, P.npts, P.bands, point_freq(P.freqs, P.real_hi, rp{}), P.m, P.row0, nullptr,
-                                      as_global(P.patch_chunk), P.chunk_info, as_global(P.chunk_faces), dest, pc, P.real_hi, r0,
-                                      min(P.rpt, P.nrows - r0), acc, frame, exps);
-    else
-        patch_tile<cd, DG, DH, false>(P.g, P.pts, P.npts, P.bands, point_freq(P.freqs, l, cd{}), P.m, P.row0, nullptr,
-                                      as_global(P.patch_chunk), P.chunk_info, as_global(P.chunk_faces), dest, pc, l, r0,
-                                      min(P.rpt, P.nrows - r0), acc, frame, exps);
+    auto tile = [&](const auto &f, int lf) {
+        patch_tile<DG, DH, false>(P.g, P.pts, P.npts, P.bands, f, P.m, P.row0, nullptr, as_global(P.patch_chunk), P.chunk_info,
+                                  as_global(P.chunk_faces), dest, pc, lf, r0, min(P.rpt, P.nrows - r0), acc, frame, exps);
+    };
+    if (P.real_hi >= 0 && l == 0) tile(point_freq(P.freqs, P.real_hi, rp{}), P.real_hi);
+    else if (beyond_table(P.freqs, l)) tile(point_freq(P.freqs, l, cd{}), l);
+    else tile(table_freq(P.freqs, l), l);
 }
 
 template <bool DG, bool DH>
@@ -510,7 +511,7 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_scene_gh_tiles(const Scene
                                                                   unsigned t0) {
     __shared__ double2 acc[kPatchPairs * kPatchVerts];
     __shared__ double2 frame[kFramePairs * kPatchThreads];
-    __shared__ double2 exps[2 * kExpNodes];
+    __shared__ double2 exps[kExpWords];
     scene_tile<DG, DH>(pieces, npieces, t0 + blockIdx.x, acc, frame, exps);
 }
 
@@ -519,7 +520,7 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_scene_gh_persistent(const 
                                                                  unsigned ntiles, unsigned *__restrict__ counter) {
     __shared__ double2 acc[kPatchPairs * kPatchVerts];
     __shared__ double2 frame[kFramePairs * kPatchThreads];
-    __shared__ double2 exps[2 * kExpNodes];
+    __shared__ double2 exps[kExpWords];
     __shared__ unsigned next_tile;
     for (;;) {
         __syncthreads();  // the previous tile's write-out has read acc; next_tile is free
@@ -544,10 +545,10 @@ __global__ void k_zero_counter(unsigned *counter) {
 // (h, n.h, h h and two scalars, each times a function of r and s); every factor
 // that depends on the frequency alone (1/s^2, s, 1/s) waits until the face's
 // or the row's end, and the trace of the h h moment serves as the scalar moment
-// of the same function (|h| = 1).  123 instructions per point, 156 before the
-// exponentials were tabulated (exp_pair), 203 with the factors applied per point.
+// of the same function (|h| = 1).  126 instructions per point, 156 beyond the
+// reach of the exponentials' table (exp_pair), 203 with the factors applied per point.
 // The two real frequencies of an even L share a slot in real arithmetic.
-// Icosphere level 4, L = 32: 25.4 ms (31.9 at 156, 33.1 with a slot for each real
+// Icosphere level 4, L = 32: 25.6 ms (31.9 at 156, 33.1 with a slot for each real
 // frequency, 43.0 at 203).
 // ------------------------------------------------------------------------
 constexpr int kBWords = 48;  // B_trans (6 sym complex) + B_angular (18 complex), as doubles
@@ -556,11 +557,12 @@ constexpr int kBWords = 48;  // B_trans (6 sym complex) + B_angular (18 complex)
 // GAL: the row is test point tpts[i] (x, y, z, face), whose face's corners are excluded; otherwise vertex i.
 // BANDED: each face takes the far rule or the reference rule (a lane then reads its own rule's points; without bands
 // they are wave-uniform).
-template <class T, bool GAL, bool BANDED>
+template <bool GAL, bool BANDED, class F>
 __device__ __attribute__((always_inline)) inline void b_sums(const Geom &g, const double4 *__restrict__ quad, int npts,
-                                                             const PointFreq<T> &f, const Mat &m, int i,
+                                                             const F &f, const Mat &m, int i,
                                                              const double4 *__restrict__ tpts,
                                                              const FaceBands &fb, const double2 *exps, double (&out)[kBWords]) {
+    typedef typename F::value T;
     double x[3];
     int t[3] = {i, i, i};
     if (GAL) {
@@ -608,7 +610,7 @@ __device__ __attribute__((always_inline)) inline void b_sums(const Geom &g, cons
             const double ir = rsqrt_h3(d2), r = d2 * ir;
             const T z1 = f.sc1 * r, z2 = f.sc2 * r;
             T E1, E2;
-            exp_pair(r, f, exps, E1, E2);
+            exp_pair(r, z1, z2, f, exps, E1, E2);
             const T s2 = z2 * E2 + E2, dS = (z1 * E1 + E1) - s2;  // s^2 A2, s^2 (A1 - A2)
             const double w2 = (w * ir) * ir, w3 = w2 * ir;
             const double h[3] = {w3 * d[0], w3 * d[1], w3 * d[2]};  // w h / r^2
@@ -681,18 +683,19 @@ __global__ void __launch_bounds__(256, 2) k_colloc_b(Geom g, const double4 *__re
                                                    const double4 *__restrict__ tpts, cd *__restrict__ Bt,
                                                    cd *__restrict__ Ba, long long nv3, int real_hi, FaceBands fb) {
     __shared__ double red[4][kBWords];
-    __shared__ double2 exps[2 * kExpNodes];
+    __shared__ double2 exps[kExpWords];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = blockIdx.y, slot = blockIdx.x, i = row0 + r;
     const bool real = real_hi >= 0 && slot == 0;
     double v[kBWords];
-    auto sums = [&](auto f) {
+    auto sums = [&](const auto &f) {
         fill_exp_table(f, exps);
         __syncthreads();
-        b_sums<decltype(f.s), GAL, BANDED>(g, quad, npts, f, m, i, tpts, fb, exps, v);
+        b_sums<GAL, BANDED>(g, quad, npts, f, m, i, tpts, fb, exps, v);
     };
     if (real) sums(point_freq(freqs + l0, real_hi, rp{}));
-    else sums(point_freq(freqs, l0 + slot, cd{}));
+    else if (beyond_table(freqs, l0 + slot)) sums(point_freq(freqs, l0 + slot, cd{}));
+    else sums(table_freq(freqs, l0 + slot));
     wave_sum48(v, lane);
     if ((lane & 7) == 0) {
 #pragma unroll
