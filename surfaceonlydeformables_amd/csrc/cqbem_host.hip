@@ -909,6 +909,7 @@ void run_job(cqbem_context *ctx, hipStream_t st, const cqbem_mesh *mesh, const c
         HIPCHK(launch_b_post(Wbt, Wba, W6, g.V, nv, L, st));
     }
     if (!out->on_device && sync_outputs) {
+        HIPCHK(hipStreamSynchronize(st));  // the copies wait for the kernels anyway; their time is not the staging's
         const auto t0 = std::chrono::steady_clock::now();
         if (wantG) HIPCHK(hipMemcpyAsync(out->G, G, matrix_bytes(nv, L), hipMemcpyDeviceToHost, st));
         if (wantH) HIPCHK(hipMemcpyAsync(out->H, H, matrix_bytes(nv, L), hipMemcpyDeviceToHost, st));
