@@ -133,16 +133,27 @@ class PhaseEvents {
     PhaseEvents() : prev_(current()) { current() = this; }
     ~PhaseEvents() {
         current() = prev_;
-        for (Pair &p : pairs_) (void)hipEventDestroy(p.a), (void)hipEventDestroy(p.b);
+        for (Pair &p : pairs_) {
+            if (p.a) (void)hipEventDestroy(p.a);
+            if (p.b) (void)hipEventDestroy(p.b);
+        }
     }
     PhaseEvents(const PhaseEvents &) = delete;
     PhaseEvents &operator=(const PhaseEvents &) = delete;
-    void add(hipEvent_t a, hipEvent_t b, double *ms) { pairs_.push_back(Pair{a, b, ms}); }
+    // Starts a phase on stream s; its end event is to be recorded when it ends (null: it is not timed).
+    hipEvent_t begin(hipStream_t s, double *ms) {
+        pairs_.push_back(Pair{nullptr, nullptr, ms});
+        Pair &p = pairs_.back();
+        if (hipEventCreate(&p.a) != hipSuccess) p.a = nullptr;
+        else if (hipEventCreate(&p.b) != hipSuccess) p.b = nullptr;
+        if (p.b) (void)hipEventRecord(p.a, s);
+        return p.b;
+    }
     // Adds every phase's milliseconds to its sum; the stream has been synchronised.
     void resolve() {
         for (Pair &p : pairs_) {
             float ms = 0;
-            if (hipEventElapsedTime(&ms, p.a, p.b) == hipSuccess) *p.ms += ms;
+            if (p.b && hipEventElapsedTime(&ms, p.a, p.b) == hipSuccess) *p.ms += ms;
         }
     }
     static PhaseEvents *&current() {
@@ -159,26 +170,22 @@ class PhaseEvents {
     PhaseEvents *prev_;
 };
 
-// Times the launches of a scope on stream s into *ms (off without a PhaseEvents on this thread).
+// Times the launches of a scope on stream s into *ms (off without a PhaseEvents on this thread).  What may throw is done
+// when the scope begins.
 class PhaseTimer {
   public:
-    PhaseTimer(hipStream_t s, double *ms) : st_(s), ms_(ms) {
-        if (!phase_timers_on() || !PhaseEvents::current()) return;
-        if (hipEventCreate(&a_) != hipSuccess) a_ = nullptr;
-        else if (hipEventCreate(&b_) != hipSuccess) b_ = nullptr;
-        if (b_) (void)hipEventRecord(a_, st_);
+    PhaseTimer(hipStream_t s, double *ms) : st_(s) {
+        if (phase_timers_on() && PhaseEvents::current()) end_ = PhaseEvents::current()->begin(s, ms);
     }
     ~PhaseTimer() {
-        if (b_) (void)hipEventRecord(b_, st_), PhaseEvents::current()->add(a_, b_, ms_);
-        else if (a_) (void)hipEventDestroy(a_);
+        if (end_) (void)hipEventRecord(end_, st_);
     }
     PhaseTimer(const PhaseTimer &) = delete;
     PhaseTimer &operator=(const PhaseTimer &) = delete;
 
   private:
-    hipEvent_t a_ = nullptr, b_ = nullptr;
+    hipEvent_t end_ = nullptr;
     hipStream_t st_;
-    double *ms_;
 };
 
 // The arena of the job running on this thread (set for the duration of a job), or null.
