@@ -709,7 +709,7 @@ uint64_t footprint(const cqbem_mesh *mesh, const cqbem_params *p, int outputs_on
                                         galerkin_budget(slab_budget));
     }
     bytes += (uint64_t)Lf * 3 * nv * 12 * sizeof(cd) + (uint64_t)L * 3 * nv * 18 * sizeof(double);
-    bytes += (uint64_t)mesh->nf * 64 + (uint64_t)nv * 64 + (1 << 20);
+    bytes += (uint64_t)mesh->nf * 64 + (uint64_t)nv * 64 + (uint64_t)Lf * sizeof(Freq) + (1 << 20);
     return bytes;
 }
 
