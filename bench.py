@@ -668,7 +668,7 @@ def main():
 
     phase_keys = ("regular_gh", "regular_b", "singular", "transform", "host")
     if params.galerkin:  # non-singular G/H/B with the test projection in one phase, of which the G/H patch kernel
-        phases = {"nonsingular": last["regular_gh"], "nonsingular_gh_pair_kernel": last["regular_b"],
+        phases = {"nonsingular": last["regular_gh"], "nonsingular_gh_patch_kernel": last["regular_b"],
                   "singular_pairs": last["singular"], "transform": last["transform"], "host": last["host"]}
     else:
         phases = {k: last[k] for k in phase_keys}
@@ -751,7 +751,7 @@ def galerkin_line(ctx, torch, dev, steps=1):
     del outs
     torch.cuda.empty_cache()
     return {"workload": desc, "steps": steps, "warmup": 1, "ms_per_step": ms, "entries_per_s": 2.0 * n3 * n3 * L * 1e3 / ms,
-            "phases_ms_last_step": {"nonsingular": tm["regular_gh"], "nonsingular_gh_pair_kernel": tm["regular_b"],
+            "phases_ms_last_step": {"nonsingular": tm["regular_gh"], "nonsingular_gh_patch_kernel": tm["regular_b"],
                                     "singular_pairs": tm["singular"], "transform": tm["transform"], "host": tm["host"]},
             "roofline": roofline(gh_ms, gh_evals, int(gh_launches), with_traffic=False, galerkin=True)}
 

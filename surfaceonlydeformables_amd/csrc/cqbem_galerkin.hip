@@ -1,22 +1,20 @@
 // Galerkin assembly on gfx950.
 //
-// Regular (non-touching) face pairs, G and H: one lane per (test face f1, source
-// vertex j, frequency l).  The lane walks f1's test points and, for each, j's
-// vertex star with j's basis function (integrate_galerkin_nonsingular,
-// integrator_galerkin.hpp:214-260, restricted to one source corner), then
-// projects onto f1's three test basis functions.  Test faces are launched by
-// vertex-disjoint colour classes, so the three row blocks a lane adds into are
-// owned by that lane alone within a launch: plain read-modify-write, no atomics,
-// a fixed summation order.
+// Regular (non-touching) face pairs (integrate_galerkin_nonsingular,
+// integrator_galerkin.hpp:214-260): the collocation kernels run with every test
+// quadrature point as a row that excludes the faces touching its test face, and
+// k_gal_project weights the rows by the test basis.  Test faces are taken by
+// vertex-disjoint colour classes, so that the row blocks a projection adds into
+// are its own within a launch: plain read-modify-write, no atomics, a fixed
+// summation order.  The star kernels (k_gal_gh: one lane per test face, source
+// vertex and frequency; k_gal_b: one block per test face and frequency) form
+// point rows and projection in one; CQBEM_GALERKIN_KERNEL=star selects them.
 //
-// Regular pairs, B_trans / B_angular: one 256-lane block per (test face, l); lanes
-// stride over source faces per test point, a block reduction per test point,
-// test-basis projection kept in LDS.
-//
-// Touching pairs (Sauter-Schwab, integrator_galerkin.hpp:42-212): one 64-lane
-// block per (pair, l); lanes split the 4D tensor rule, reduce, and write the
-// pair's corner blocks to a per-pair scratch.  A gather kernel then owns each
-// output block and adds its pairs' contributions in a fixed order.
+// Touching pairs (Sauter-Schwab, integrator_galerkin.hpp:42-212): one lane per
+// direction of the 4D rule (k_gal_touch, k_gal_touch_b), or one lane per point of
+// it (k_gal_sing, CQBEM_GALERKIN_SINGULAR=lane), reduced to the pair's corner
+// blocks in a per-pair scratch.  A gather kernel then owns each output block and
+// adds its pairs' contributions in a fixed order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

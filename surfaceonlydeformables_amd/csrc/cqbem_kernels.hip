@@ -1,13 +1,15 @@
 // gfx950 kernels of the CQBEM precompute (collocation path, inverse CQ
 // transform, jump/B post-processing).
 //
-// Work decomposition (collocation, regular pairs): one lane owns one output
-// block (row vertex i, column vertex j, frequency l) and integrates the faces
-// of j's vertex star with the basis function of j's corner.  Each block is
-// therefore written exactly once, with no atomics and no read-modify-write;
-// lanes of a wavefront share (i, l), so x_i and the frequency constants live
-// in scalar registers.  Faces touching i (the singular ones) are skipped and
-// integrated by the singular kernels, which own rows (i, l) and add into them.
+// Work decomposition (collocation, regular pairs): a block owns the columns of
+// a patch of vertices for some rows i at one frequency l and evaluates every
+// face that touches the patch once, one lane per face (k_colloc_gh_patch).  Each
+// output block is written exactly once, with no atomics; x_i and the frequency
+// constants live in scalar registers.  The star form (k_colloc_gh,
+// CQBEM_COLLOC_KERNEL=star) has a lane per output block instead, which integrates
+// the faces of its column vertex's star.  Faces touching i (the singular ones)
+// are skipped and integrated by the singular kernels, which own rows (i, l) and
+// add into them.
 //
 // Reference counterparts: compute_elastodynamic_{G,H,B_trans,B_angular}_kernel_collocation
 // (src/elastodynamics_cqbem_*_collocation.cu) and the inverse transform loops
@@ -466,9 +468,9 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_colloc_gh_patch(Geom g, co
 //   k_scene_gh_tiles: one block per tile; the hardware's workgroup dispatcher hands tiles to CUs in tile order as
 //     they free up (pieces are ordered largest first by the host).  Same registers as the single-object kernel
 //     plus the piece lookup: 2 waves per SIMD.
-//   k_scene_gh_persistent: persistent blocks (2 per CU) that take tile numbers from a device counter with one atomic add
-//     per tile.  The loop-carried state costs 8 registers beyond 256, i.e. 1 wave per SIMD (CQBEM_SCENE_KERNEL=
-//     persistent selects it, for comparison).
+//   k_scene_gh_persistent: persistent blocks that take tile numbers from a device counter with one atomic add per tile.
+//     The loop-carried state takes it past 256 registers and 80 KB of LDS: one block per CU is resident, of the two per
+//     CU that are launched (CQBEM_SCENE_KERNEL=persistent selects it, for comparison).
 // ------------------------------------------------------------------------
 template <bool DG, bool DH>
 __device__ __attribute__((always_inline)) inline void scene_tile(const ScenePiece *__restrict__ pieces, int npieces, unsigned t, double2 *acc, double2 *frame, double2 *exps) {
@@ -1397,8 +1399,8 @@ hipError_t launch_colloc_gh(const Geom &g, const double4 *quad, int npts, const 
 
 
 // Rows per block of the patch kernel: enough to hide a row's start and write-out behind the next one's evaluation and to
-// even out chunk counts that are no multiple of 4, and still at least 4096 blocks (8 per resident block of 256 CUs) where
-// there are as many tiles.
+// even out chunk counts that are no multiple of 4, and still at least 8192 blocks (16 for each that is resident on 256 CUs)
+// where there are as many tiles.
 int patch_rows_per_tile(long long tiles) { return (int)std::min<long long>(16, std::max<long long>(1, tiles / 8192)); }
 
 hipError_t launch_colloc_gh_patch(const Geom &g, const double4 *pts, int npts, const Freq *freqs, int l0, int nl, bool real_ends, const Mat &m,
@@ -1567,7 +1569,9 @@ struct HistorySplit {
 static HistorySplit history_split(long long n3, int m, bool a16) {
     if (const int forced = history_rows()) return {forced == 1 ? 0 : forced, false};
     // unaligned 16-byte loads pay from 4 steps or 2048 rows on (903 rows, 2 steps: 18.3 us in 8-byte loads, 19.4), for one
-    // step from 8192 (5001 rows: 40 and 47 us; 12289: 257 and 194)
+    // step from 8192 (5001 rows: 40 and 47 us; 12289: 257 and 194).  That is for weights that come from memory (1503 rows,
+    // 5 steps: 95 and 60 us; 2601, 2 steps: 101 and 62); the same few steps repeated on weights that the 256 MB cache
+    // still holds are up to 1.15 times faster in 8-byte loads (51 and 57; 50 and 58)
     if (m > 1 && (a16 || m >= 4 || n3 >= 2048)) {
         // idle share of 256 CUs in the last round of blocks: 2 rows where that is clearly the smaller one (3489 rows, 16
         // steps, unaligned: 528 us at 2 and 543 at 4 rows; 903: 57 and 53)

@@ -104,8 +104,9 @@ struct ScenePiece {
     unsigned base;
     Bands bands;
 };
-// The pieces (device array, ascending base, all with the same G / H selection) in one persistent launch of
-// min(ntiles, 2 blocks per CU) blocks that take tiles from *counter (zeroed by the launcher with a kernel).
+// The pieces (device array, ascending base, all with the same G / H selection): one block per tile, or with
+// CQBEM_SCENE_KERNEL=persistent min(ntiles, 2 per CU) blocks that take tiles from *counter (zeroed by the launcher with a
+// kernel).
 hipError_t launch_scene_gh(const ScenePiece *pieces, int npieces, long long ntiles, unsigned *counter, bool G, bool H,
                                 int num_cus, hipStream_t st);
 hipError_t launch_colloc_b(const Geom &g, const double4 *quad, int npts, const Freq *freqs, int l0, int nl, bool real_ends,
