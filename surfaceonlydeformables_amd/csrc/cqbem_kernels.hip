@@ -449,7 +449,7 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_colloc_gh_patch(Geom g, co
                                                                   int nrows, int rpt, int real_hi, Bands bands) {
     __shared__ double2 acc[kPatchPairs * kPatchVerts];      // [word][slot]
     __shared__ double2 frame[kFramePairs * kPatchThreads];
-    __shared__ double2 exps[kExpWords];
+    __shared__ __align__(32) double2 exps[kExpWords];
     auto dest = [=] { return PatchDest{patch_verts, UG, UH, ld, lstride}; };
     const int r0 = blockIdx.z * rpt, nr = min(rpt, nrows - r0);
     auto tile = [&](const auto &f, int l) {
@@ -513,7 +513,7 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_scene_gh_tiles(const Scene
                                                                   unsigned t0) {
     __shared__ double2 acc[kPatchPairs * kPatchVerts];
     __shared__ double2 frame[kFramePairs * kPatchThreads];
-    __shared__ double2 exps[kExpWords];
+    __shared__ __align__(32) double2 exps[kExpWords];
     scene_tile<DG, DH>(pieces, npieces, t0 + blockIdx.x, acc, frame, exps);
 }
 
@@ -522,7 +522,7 @@ __global__ void __launch_bounds__(kPatchThreads, 2) k_scene_gh_persistent(const 
                                                                  unsigned ntiles, unsigned *__restrict__ counter) {
     __shared__ double2 acc[kPatchPairs * kPatchVerts];
     __shared__ double2 frame[kFramePairs * kPatchThreads];
-    __shared__ double2 exps[kExpWords];
+    __shared__ __align__(32) double2 exps[kExpWords];
     __shared__ unsigned next_tile;
     for (;;) {
         __syncthreads();  // the previous tile's write-out has read acc; next_tile is free
@@ -685,7 +685,7 @@ __global__ void __launch_bounds__(256, 2) k_colloc_b(Geom g, const double4 *__re
                                                    const double4 *__restrict__ tpts, cd *__restrict__ Bt,
                                                    cd *__restrict__ Ba, long long nv3, int real_hi, FaceBands fb) {
     __shared__ double red[4][kBWords];
-    __shared__ double2 exps[kExpWords];
+    __shared__ __align__(32) double2 exps[kExpWords];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = blockIdx.y, slot = blockIdx.x, i = row0 + r;
     const bool real = real_hi >= 0 && slot == 0;
